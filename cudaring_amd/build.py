@@ -17,7 +17,13 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libdpmring.so")
 
-SOURCES = ["dpm_kernels.hip", "dpm_adjoint.hip", "dpm_observe.hip", "dpm_api.hip"]
+# (source, object, defines): the step and FIRE kernels are one translation unit per (interaction,
+# potential), so that their instances compile side by side
+_PAIRS = [(i, p) for i in (0, 1, 3) for p in range(4)]
+UNITS = ([("dpm_step.hip", f"dpm_step_{i}_{p}.o", [f"-DSTEP_INTER={i}", f"-DSTEP_POT={p}"]) for i, p in _PAIRS] +
+         [("dpm_fire.hip", f"dpm_fire_{i}_{p}.o", [f"-DFIRE_INTER={i}", f"-DFIRE_POT={p}"]) for i, p in _PAIRS] +
+         [(s, os.path.splitext(s)[0] + ".o", [])
+          for s in ("dpm_kernels.hip", "dpm_adjoint.hip", "dpm_observe.hip", "dpm_api.hip")])
 
 # C++ class layer (DPM2D / FIRE / Simulator / ioDPMFile) and the drivers built on it: plain host
 # C++ over the C ABI, linked against libdpmring.so (found next to bin/ through the rpath)
@@ -38,9 +44,10 @@ FLAGS = [
 ]
 
 
-def _compile(src):
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(unit):
+    src, obj, defines = unit
+    obj = os.path.join(BUILD, obj)
+    cmd = [HIPCC, *FLAGS, *defines, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
@@ -78,8 +85,8 @@ def build_host(verbose=False):
 
 def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+    with ThreadPoolExecutor(max_workers=min(len(UNITS), os.cpu_count() or 1)) as ex:
+        objs = list(ex.map(_compile, UNITS))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)

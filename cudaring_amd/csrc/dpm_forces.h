@@ -1,0 +1,421 @@
+// dpm_forces.h -- device functions of the step and FIRE kernels: ring geometry and shape forces,
+// the interparticle gather, the step loop's cell lists and the rigid-ring moves.
+#pragma once
+
+#include "dpm_internal.h"
+#include "dpm_rows.h"
+#include "dpm_tile.h"
+
+namespace dpm {
+
+// wave-per-tile kernels (4 tiles per 256-thread block)
+__device__ __forceinline__ bool wave_tile_ctx(const View& V, Lane& L) {
+  const int tile = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  if (tile >= V.ntiles) return false;
+  lane_ctx(V, tile, threadIdx.x & (WAVE - 1), L);
+  return true;
+}
+
+// Ring geometry + shape force for one lane (wave-uniform call).  Restates
+// kernelCalcParticleShape (cudaKernel.cuh:1571-1606), calcParticlePos (365-388)
+// and kernelCalcShapeForceEnergy (474-529) with the area/perimeter/bending
+// terms of 429-471.  Writes theta, length and the ring area/perimeter/centre.
+struct ShapeOut {
+  double fx, fy, e;
+  double cx, cy;  // ring centre (calcParticlePos, cudaKernel.cuh:365-388)
+};
+
+// turning angle at a vertex from its own, next and previous positions (calcAngle 423-427)
+__device__ __forceinline__ double vertex_theta(const Box& B, double x, double y, double xn, double yn, double xp,
+                                               double yp) {
+  const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
+  const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
+  return atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);
+}
+
+__device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, const Lane& L, const Box& B,
+                                               double x, double y, bool write) {
+  ShapeOut o;
+  double xn, yn, xp, yp, theta, seglen, area, perim, comx, comy;
+  int vn = 0, vp = 0;
+  if (!L.wide) {
+    xn = shfl_d(x, L.nl); yn = shfl_d(y, L.nl);
+    xp = shfl_d(x, L.pl); yp = shfl_d(y, L.pl);
+    const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
+    // segments of the reference's unwrapped walk
+    const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
+    const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
+    theta = atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);  // calcAngle 423-427
+    seglen = sqrt(dnx * dnx + dny * dny);
+    // Unwrapped position relative to the first vertex: the reference walks the ring one
+    // minimum-image segment at a time; here that walk is an exclusive segmented scan of the
+    // segment vectors, valid for rings wider than half the box.
+    const double Ix = seg_scan(L.act ? dnx : 0.0, L.lane, L.segS);
+    const double Iy = seg_scan(L.act ? dny : 0.0, L.lane, L.segS);
+    const double ux = L.act ? Ix - dnx : 0.0;
+    const double uy = L.act ? Iy - dny : 0.0;
+    const double shoe = L.act ? (ux * dny - dnx * uy) : 0.0;  // shoelace: cur x next = cur x delta
+    perim = seg_sum(L.act ? seglen : 0.0, L.lane, L.segS, L.segE);
+    const double shoeSum = seg_sum(shoe, L.lane, L.segS, L.segE);
+    const double sux = seg_sum(ux, L.lane, L.segS, L.segE);
+    const double suy = seg_sum(uy, L.lane, L.segS, L.segE);
+    const double ind = 1.0 / (double)L.n;
+    area = fabs(shoeSum) * 0.5;
+    comx = xf + sux * ind;
+    comy = yf + suy * ind;
+  } else {
+    // a slice of a wide ring: ring neighbours from memory (this launch reads the current positions
+    // only), the ring's area, perimeter and centre from k_wide_rings, launched just before
+    vn = ring_next(L.v, L.f, L.n);
+    vp = ring_prev(L.v, L.f, L.n);
+    xn = V.x[vn]; yn = V.y[vn];
+    xp = V.x[vp]; yp = V.y[vp];
+    theta = vertex_theta(B, x, y, xn, yn, xp, yp);
+    const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
+    seglen = sqrt(dnx * dnx + dny * dny);
+    area = V.area[L.r];
+    perim = V.perim[L.r];
+    comx = V.cx[L.r];
+    comy = V.cy[L.r];
+  }
+  o.cx = comx;
+  o.cy = comy;
+  if (write && L.act) {
+    V.th[L.v] = theta;
+    V.len[L.v] = seglen;
+    if (L.lane == L.segS && !L.wide) {
+      V.area[L.r] = area;
+      V.perim[L.r] = perim;
+      V.cx[L.r] = comx;
+      V.cy[L.r] = comy;
+    }
+  }
+  const double ind = 1.0 / (double)L.n;
+  // positions relative to the ring centre (getRelativeVertexPos 273-279)
+  const double rvx = pbx(x - comx, B), rvy = pby(y - comy, B);
+  const double rnx = pbx(xn - comx, B), rny = pby(yn - comy, B);
+  const double rpx = pbx(xp - comx, B), rpy = pby(yp - comy, B);
+  const double a0 = V.a0[L.r];
+  // shape costs: the global ea, el, eb, or per-ring values when the caller set them
+  const double ea = V.kr ? V.kr[L.r] : P.ea;
+  const double el = V.kr ? V.kr[V.np + L.r] : P.el;
+  const double eb = V.kr ? V.kr[2 * V.np + L.r] : P.eb;
+  // area term (calcAreaForceEnergy 429-435)
+  const double deltaA = (area / a0) - 1.;
+  const double gmA = ea * deltaA / a0;
+  double fx = 0.5 * gmA * (rpy - rny);
+  double fy = 0.5 * gmA * (rnx - rpx);
+  double e = (0.5 * ea * deltaA * deltaA) * ind;
+  // perimeter term (calcPerimeterForceEnergy 437-447 / FENE 449-455)
+  const double nsx = rnx - rvx, nsy = rny - rvy;
+  const double qsx = rvx - rpx, qsy = rvy - rpy;
+  const double pLen = sqrt(qsx * qsx + qsy * qsy);
+  const double nLen = sqrt(nsx * nsx + nsy * nsy);
+  const double l0v = V.l0[L.v];
+  const double l0s = shfl_d(l0v, L.pl);
+  const double l0p = L.wide ? V.l0[vp] : l0s;
+  if (P.monomer == MONO_HARMONIC) {
+    const double pDelta = (pLen / l0p) - 1.;
+    const double nDelta = (nLen / l0v) - 1.;
+    const double cn = nDelta / (l0v * nLen), cp = pDelta / (l0p * pLen);
+    fx += el * ((cn * (rnx - rvx)) - (cp * (rvx - rpx)));
+    fy += el * ((cn * (rny - rvy)) - (cp * (rvy - rpy)));
+    e += (0.5 * el * pDelta * pDelta);
+  } else {
+    const double c = 2 * el * P.stiff * P.extSq;
+    fx += c * ((nLen / (P.extSq * l0v * l0v - nLen * nLen)) * (rnx - rvx) / nLen -
+               (pLen / (P.extSq * l0p * l0p - pLen * pLen)) * (rvx - rpx) / pLen);
+    fy += c * ((nLen / (P.extSq * l0v * l0v - nLen * nLen)) * (rny - rvy) / nLen -
+               (pLen / (P.extSq * l0p * l0p - pLen * pLen)) * (rvy - rpy) / pLen);
+    e += el * P.stiff * P.extSq * log(1 - pLen * pLen / (P.extSq * l0p * l0p));
+  }
+  // bending term (calcBendingForceEnergy 457-471)
+  const double D = theta - V.th0[L.v];
+  double Dp = shfl_d(D, L.pl), Dn = shfl_d(D, L.nl);
+  if (L.wide) {  // the neighbours' angles from their own neighbours, as their lanes form them
+    const int vpp = ring_prev(vp, L.f, L.n), vnn = ring_next(vn, L.f, L.n);
+    Dp = vertex_theta(B, xp, yp, x, y, V.x[vpp], V.y[vpp]) - V.th0[vp];
+    Dn = vertex_theta(B, xn, yn, V.x[vnn], V.y[vnn], x, y) - V.th0[vn];
+  }
+  const double preVar = (D - Dp) / (qsx * qsx + qsy * qsy);
+  const double nextVar = (D - Dn) / (nsx * nsx + nsy * nsy);
+  fx += eb * (preVar * qsy + nextVar * nsy);
+  fy += eb * (preVar * (-qsx) + nextVar * (-nsx));
+  e += (0.5 * eb * D * D);
+  o.fx = fx; o.fy = fy; o.e = e;
+  return o;
+}
+
+// The ring centre alone (calcParticlePos, cudaKernel.cuh:365-388), as ring_shape computes it,
+// stored by the ring's first lane: the rigid rings' shape pass
+__device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, const Box& B, double x, double y) {
+  ShapeOut o{0, 0, 0, 0, 0};
+  const double xn = shfl_d(x, L.nl), yn = shfl_d(y, L.nl);
+  const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
+  const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
+  const double Ix = seg_scan(L.act ? dnx : 0.0, L.lane, L.segS);
+  const double Iy = seg_scan(L.act ? dny : 0.0, L.lane, L.segS);
+  const double ux = L.act ? Ix - dnx : 0.0;
+  const double uy = L.act ? Iy - dny : 0.0;
+  const double sux = seg_sum(ux, L.lane, L.segS, L.segE);
+  const double suy = seg_sum(uy, L.lane, L.segS, L.segE);
+  const double ind = 1.0 / (double)L.n;
+  o.cx = xf + sux * ind;
+  o.cy = yf + suy * ind;
+  if (L.act && L.lane == L.segS) {
+    V.cx[L.r] = o.cx;
+    V.cy[L.r] = o.cy;
+  }
+  return o;
+}
+
+// Interparticle gather of lane L's vertex over entries k0, k0 + kstep, ... of its row:
+// accumulates the force on v, the vertex-vertex energy e, the smooth energy es and the share
+// (qx, qy) that v's `other` evaluation owes prev(v) (handed to prev(v)'s lane by the caller).
+// On the last lane of a wide ring's slice, whose next vertex lies in another tile, (qnx, qny)
+// accumulates the share that next(v)'s evaluations owe v, from next(v)'s row (complete before
+// the launch: wide sets rebuild rows in their own launch).
+template <int INTER, int POT>
+__device__ __forceinline__ void gather_pairs(const View& V, const Params& P, const Lane& L, const Box& B, double x,
+                                             double y, int k0, int kstep, double& fx, double& fy, double& e,
+                                             double& es, double& qx, double& qy, double& qnx, double& qny) {
+  const double radv = V.rad[L.v];
+  // Row entries are fetched one iteration ahead, the first one before the row length is known:
+  // rows are W entries wide (unused entries hold -1), so k < W keeps every fetch in bounds, and
+  // an entry is only used once k < ncnt is known.
+  if constexpr (INTER == INT_VV) {
+    // kernelCalcVertexInteraction, cudaKernel.cuh:690-722
+    int j = k0 < V.W ? V.nbr[(long)k0 * V.nv + L.v] : 0;
+    const int c = L.act ? V.ncnt[L.v] : 0;
+    for (int k = k0; k < c; k += kstep) {
+      const int kn = k + kstep;
+      const int jn = kn < V.W ? V.nbr[(long)kn * V.nv + L.v] : 0;
+      e += pair_force<POT>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
+      j = jn;
+    }
+  } else if constexpr (INTER == INT_SMOOTH) {
+    // kernelCalcSmoothInteraction, cudaKernel.cuh:922-975, as a gather: for every u in list(v),
+    // (v, segment of u) gives v's `this` share, and (u, segment (prev(v), v)) gives v's
+    // `other` share and prev(v)'s `previous` share (handed to prev(v)'s lane by the caller).
+    // Ring neighbours of v; inactive lanes past the tile end use v itself (in bounds).
+    int vp = L.act ? L.v0 + L.pl : L.v;
+    int vpp = L.act ? L.v0 + ((L.pl > L.segS) ? L.pl - 1 : L.segE) : L.v;
+    if (L.wide && L.act) {
+      vp = ring_prev(L.v, L.f, L.n);
+      vpp = ring_prev(vp, L.f, L.n);
+    }
+    const double xp = V.x[vp], yp = V.y[vp];
+    const double xpp = V.x[vpp], ypp = V.y[vpp];
+    int u = 0;
+    int2 pp = make_int2(0, 0);
+    if (k0 < V.W) {
+      u = V.nbr[(long)k0 * V.nv + L.v];
+      pp = V.nbrp[(long)k0 * V.nv + L.v];
+    }
+    const int c = L.act ? V.ncnt[L.v] : 0;
+    for (int k = k0; k < c; k += kstep) {
+      const int kn = k + kstep;
+      int un = 0;
+      int2 ppn = make_int2(0, 0);
+      if (kn < V.W) {
+        un = V.nbr[(long)kn * V.nv + L.v];
+        ppn = V.nbrp[(long)kn * V.nv + L.v];
+      }
+      const double xu = V.x[u], yu = V.y[u];
+      const double radSum = radv + V.rad[u];
+      es += smooth_pair<POT, ROLE_THIS>(P, B, x, y, xu, yu, V.x[pp.x], V.y[pp.x], V.x[pp.y], V.y[pp.y], radSum,
+                                        fx, fy);
+      es += smooth_pair_op<POT>(P, B, xu, yu, x, y, xp, yp, xpp, ypp, radSum, fx, fy, qx, qy);
+      u = un;
+      pp = ppn;
+    }
+    if (L.wide && L.act && L.lane == L.segE) {
+      // (u, segment (v, next(v))) for u in list(next(v)): next(v)'s `other` share is its own
+      // lane's; the `previous` share is v's (the energy is counted by next(v)'s lane)
+      const int j = ring_next(L.v, L.f, L.n);
+      const double xj = V.x[j], yj = V.y[j], radj = V.rad[j];
+      const int cj = V.ncnt[j];
+      for (int k = k0; k < cj; k += kstep) {
+        const int w = V.nbr[(long)k * V.nv + j];
+        double ox = 0, oy = 0;
+        (void)smooth_pair_op<POT>(P, B, V.x[w], V.y[w], xj, yj, x, y, xp, yp, radj + V.rad[w], ox, oy, qnx, qny);
+      }
+    }
+  } else {
+    // kernelCalcAllToAllVertexInteraction, cudaKernel.cuh:725-757 (test mode)
+    if (L.act) {
+      const int b0 = V.svoff[L.s], b1 = V.svoff[L.s + 1];
+      for (int j = b0 + k0; j < b1; j += kstep) {
+        if (V.vring[j] == L.r) continue;
+        e += pair_force<POT>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
+      }
+    }
+  }
+}
+
+// -------------------------------------------------------------- step ---
+// Waves of a tile: with nw > 1, wave 0 does the ring geometry, shape force and random draws
+// while waves 1..nw-1 share the neighbour gather; with nw == 1 wave 0 does both in turn.
+// A drift that moved a vertex more than cutoff / 3 marks its system FLAG_FAR: the next rebuild
+// cannot rely on the cells of its list positions (md_cells)
+__device__ __forceinline__ void far_test(const Params& P, const Box& B, double dx, double dy, int* flag) {
+  dx = pbx(dx, B);
+  dy = pby(dy, B);
+  if (3 * sqrt(dx * dx + dy * dy) > P.cutoff) atomicOr(flag, FLAG_FAR);
+}
+
+// The step loop's cell lists of a system whose list positions (the positions of its last
+// rebuild) have generation g: its rows are rebuilt from list g % 3, the rebuild bins its own
+// positions (the next list positions) into list (g + 1) % 3, cleared by the rebuild before, and
+// clears list (g + 2) % 3, which that rebuild read.  The cells are wide enough for a vertex 2
+// cutoff / 3 from its list position: at most cutoff / 3 before the drift that triggers the
+// rebuild (the displacement test) plus cutoff / 3 in that drift (else FLAG_FAR, all pairs).
+struct MdCells {
+  const int *cnt, *slots;  // read
+  int *binCnt, *binSlots;  // binned into
+  int* clear;              // cleared
+};
+__device__ __forceinline__ MdCells md_cells(const StepArgs& A, const CellGrid& G, int g) {
+  const long C = G.ncells, CS = (long)G.ncells * G.cap;
+  const int k0 = g % 3, k1 = (g + 1) % 3, k2 = (g + 2) % 3;
+  return MdCells{A.cellCur + k0 * C, A.slotsCur + k0 * CS, A.cellCur + k1 * C, A.slotsCur + k1 * CS,
+                 A.cellCur + k2 * C};
+}
+
+// a rebuilding vertex at (x, y) farther than 2 cutoff / 3 from its list position: its cells may
+// miss a neighbour (cannot happen while the displacement and far tests hold)
+__device__ __forceinline__ void md_stale_test(const View& V, const Params& P, const Box& B, int v, double x, double y,
+                                              int* err) {
+  const double ddx = pbx(x - V.lx[v], B), ddy = pby(y - V.ly[v], B);
+  if (3 * sqrt(ddx * ddx + ddy * ddy) > 2 * P.cutoff) atomicOr(err, ERR_STALE_BINS);
+}
+
+// ---------------------------------------------------------- rigid rings ---
+// Half kick of a rigid ring: RigidNVE::updateVelocity (Simulator.cu:348-366), or
+// RigidLangevin::updateVelocity (263-286) with its unit Gaussian pair (z0, z1) of the step and
+// d_thermalVel zero; the angular velocity takes the torque / moment of inertia.
+__device__ __forceinline__ void rigid_kick(bool langevin, double h, double gamma, double Fx, double Fy, double T,
+                                           double z0, double z1, double& vx, double& vy, double& w) {
+  if (langevin) {
+    vx += h * (Fx - vx * gamma);
+    vx -= 0.5 * h * h * (Fx - vx * gamma) / gamma;
+    vx += z0;
+    vy += h * (Fy - vy * gamma);
+    vy -= 0.5 * h * h * (Fy - vy * gamma) / gamma;
+    vy += z1;
+  } else {
+    vx += h * Fx;
+    vy += h * Fy;
+  }
+  w += h * T;
+}
+
+// A ring's vertex after the ring moved from centre (cx, cy) to (ncx, ncy) and turned by dth:
+// translateVertices then rotateVertices (kernelTranslateVertices / kernelRotateVertices,
+// cudaKernel.cuh:1678-1713), each difference a box distance.
+__device__ __forceinline__ void rigid_move(const Box& B, double x, double y, double cx, double cy, double ncx,
+                                           double ncy, double c, double sn, double& xn, double& yn) {
+  const double x1 = x + pbx(ncx - cx, B), y1 = y + pby(ncy - cy, B);
+  const double dx = pbx(x1 - ncx, B), dy = pby(y1 - ncy, B);
+  xn = x1 + ((dx * c - dy * sn) - dx);
+  yn = y1 + ((dx * sn + dy * c) - dy);
+}
+
+// Per-tile partials of the rigid FIRE sums over the rings whose first vertex is in the tile:
+// [0] v.F, [1] |v|^2, [2] |F|^2 (ring velocities and forces)
+__device__ __forceinline__ void rigid_fire_partials(const Lane& L, bool head, double vx, double vy, double Fx,
+                                                    double Fy, double* part) {
+  const double p0 = wave_sum(head ? vx * Fx + vy * Fy : 0.0);
+  const double p1 = wave_sum(head ? vx * vx + vy * vy : 0.0);
+  const double p2 = wave_sum(head ? Fx * Fx + Fy * Fy : 0.0);
+  if (L.lane == 0) {
+    part[L.tile * 4 + 0] = p0;
+    part[L.tile * 4 + 1] = p1;
+    part[L.tile * 4 + 2] = p2;
+  }
+}
+
+// Step-kernel epilogue of rigid rings (wave 0, one ring per lane segment): the interaction
+// forces' transfer to the ring (calcRigidForceEnergy, DPM2D.cu:2128-2142: torque r x f about
+// the centre, moment of inertia sum |r|^2, ring force sum f, ring torque sum (r x f) / I, ring
+// energy sum e for vertexVertex), then the second half kick of this step and, with MODE_START,
+// the next step's first half: last centre and angle stored, half kick with the next step's
+// draw, centre and angle advanced, vertices moved (RigidNVE / RigidLangevin::integrate,
+// Simulator.cu:241-252, 316-326).  With MODE_FIRE the half kick takes the system's FIRE step.
+template <int MODE, bool VV>
+__device__ __forceinline__ void rigid_epilogue(const View& V, const Params& P, const StepArgs& A, const Lane& L,
+                                               const Box& B, double x, double y, double fx, double fy, double e,
+                                               double cx, double cy, double lx, double ly, double z0, double z1) {
+  const Rigid R = *V.rg;
+  const double rx = pbx(x - cx, B), ry = pby(y - cy, B);
+  const double tq = rx * fy - ry * fx;
+  const double I = seg_sum(L.act ? rx * rx + ry * ry : 0.0, L.lane, L.segS, L.segE);
+  const double Fx = seg_sum(L.act ? fx : 0.0, L.lane, L.segS, L.segE);
+  const double Fy = seg_sum(L.act ? fy : 0.0, L.lane, L.segS, L.segE);
+  const double T = seg_sum(L.act ? tq : 0.0, L.lane, L.segS, L.segE) / I;
+  double E = 0;
+  if constexpr (VV) E = seg_sum(L.act ? e : 0.0, L.lane, L.segS, L.segE);
+  const bool head = L.act && L.lane == L.segS;
+  double vx = 0, vy = 0, w = 0;
+  if constexpr (MODE != MODE_RIGID) {
+    if (L.act) {
+      vx = R.pvx[L.r];
+      vy = R.pvy[L.r];
+      w = R.pw[L.r];
+    }
+  }
+  if constexpr ((MODE & MODE_FIRE) != 0) {
+    // the second half kick with the system's FIRE step, then the tile partials of the next
+    // iteration's sums (every lane takes part in the wave sums)
+    if (L.act) rigid_kick(false, 0.5 * A.fire[L.s].dt, 0.0, Fx, Fy, T, 0.0, 0.0, vx, vy, w);
+    rigid_fire_partials(L, head, vx, vy, Fx, Fy, A.part);
+  }
+  if (!L.act) return;
+  V.fx[L.v] = fx;
+  V.fy[L.v] = fy;
+  V.ev[L.v] = e;
+  R.vtq[L.v] = tq;
+  if (head) {
+    R.pfx[L.r] = Fx;
+    R.pfy[L.r] = Fy;
+    R.ptq[L.r] = T;
+    R.moi[L.r] = I;
+    if constexpr (VV) V.pe[L.r] = E;
+  }
+  if constexpr (MODE == MODE_RIGID) return;
+  if constexpr ((MODE & MODE_FIRE) == 0) {
+    rigid_kick(A.rigidLangevin, A.h, P.gamma, Fx, Fy, T, z0, z1, vx, vy, w);
+    if constexpr ((MODE & MODE_START) != 0) {
+      double n0 = 0, n1 = 0;
+      if (A.rigidLangevin)
+        gauss_pair(P.seed, (uint32_t)L.s, TAG_THERMAL, A.ctr[0] + (unsigned long long)A.ctrOffT + 1ull,
+                   (uint32_t)(L.r - V.sroff[L.s]), n0, n1);
+      rigid_kick(A.rigidLangevin, A.h, P.gamma, Fx, Fy, T, n0, n1, vx, vy, w);
+      const double ang = V.ang[L.r];
+      const double ncx = cx + A.dt * vx, ncy = cy + A.dt * vy, nang = ang + A.dt * w;
+      const double dth = nang - ang;
+      double xn, yn;
+      rigid_move(B, x, y, cx, cy, ncx, ncy, cos(dth), sin(dth), xn, yn);
+      A.xout[L.v] = xn;
+      A.yout[L.v] = yn;
+      const double ddx = pbx(xn - lx, B), ddy = pby(yn - ly, B);
+      if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
+        atomicOr(&A.flagOut[L.s], 1);
+        atomicOr(A.anyOut, 1);
+      }
+      far_test(P, B, xn - x, yn - y, A.flagOut + L.s);
+      if (head) {
+        V.ang[L.r] = nang;
+        V.cx[L.r] = ncx;
+        V.cy[L.r] = ncy;
+      }
+    }
+  }
+  if (head) {
+    R.pvx[L.r] = vx;
+    R.pvy[L.r] = vy;
+    R.pw[L.r] = w;
+  }
+}
+
+}  // namespace dpm

@@ -20,172 +20,10 @@
 // md_cells), so a step is one launch with no binning and no host
 // synchronisation; the FIRE graph path bins the current positions in a k_bin
 // launch before each step kernel.
-#include "dpm_internal.h"
-#include "dpm_rows.h"
-#include "dpm_tile.h"
+#include "dpm_forces.h"
+#include "dpm_launch.h"
 
 namespace dpm {
-
-// wave-per-tile kernels (4 tiles per 256-thread block)
-__device__ __forceinline__ bool wave_tile_ctx(const View& V, Lane& L) {
-  const int tile = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-  if (tile >= V.ntiles) return false;
-  lane_ctx(V, tile, threadIdx.x & (WAVE - 1), L);
-  return true;
-}
-
-// Ring geometry + shape force for one lane (wave-uniform call).  Restates
-// kernelCalcParticleShape (cudaKernel.cuh:1571-1606), calcParticlePos (365-388)
-// and kernelCalcShapeForceEnergy (474-529) with the area/perimeter/bending
-// terms of 429-471.  Writes theta, length and the ring area/perimeter/centre.
-struct ShapeOut {
-  double fx, fy, e;
-  double cx, cy;  // ring centre (calcParticlePos, cudaKernel.cuh:365-388)
-};
-
-// turning angle at a vertex from its own, next and previous positions (calcAngle 423-427)
-__device__ __forceinline__ double vertex_theta(const Box& B, double x, double y, double xn, double yn, double xp,
-                                               double yp) {
-  const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-  const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
-  return atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);
-}
-
-__device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, const Lane& L, const Box& B,
-                                               double x, double y, bool write) {
-  ShapeOut o;
-  double xn, yn, xp, yp, theta, seglen, area, perim, comx, comy;
-  int vn = 0, vp = 0;
-  if (!L.wide) {
-    xn = shfl_d(x, L.nl); yn = shfl_d(y, L.nl);
-    xp = shfl_d(x, L.pl); yp = shfl_d(y, L.pl);
-    const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
-    // segments of the reference's unwrapped walk
-    const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-    const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
-    theta = atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);  // calcAngle 423-427
-    seglen = sqrt(dnx * dnx + dny * dny);
-    // Unwrapped position relative to the first vertex: the reference walks the ring one
-    // minimum-image segment at a time; here that walk is an exclusive segmented scan of the
-    // segment vectors, valid for rings wider than half the box.
-    const double Ix = seg_scan(L.act ? dnx : 0.0, L.lane, L.segS);
-    const double Iy = seg_scan(L.act ? dny : 0.0, L.lane, L.segS);
-    const double ux = L.act ? Ix - dnx : 0.0;
-    const double uy = L.act ? Iy - dny : 0.0;
-    const double shoe = L.act ? (ux * dny - dnx * uy) : 0.0;  // shoelace: cur x next = cur x delta
-    perim = seg_sum(L.act ? seglen : 0.0, L.lane, L.segS, L.segE);
-    const double shoeSum = seg_sum(shoe, L.lane, L.segS, L.segE);
-    const double sux = seg_sum(ux, L.lane, L.segS, L.segE);
-    const double suy = seg_sum(uy, L.lane, L.segS, L.segE);
-    const double ind = 1.0 / (double)L.n;
-    area = fabs(shoeSum) * 0.5;
-    comx = xf + sux * ind;
-    comy = yf + suy * ind;
-  } else {
-    // a slice of a wide ring: ring neighbours from memory (this launch reads the current positions
-    // only), the ring's area, perimeter and centre from k_wide_rings, launched just before
-    vn = ring_next(L.v, L.f, L.n);
-    vp = ring_prev(L.v, L.f, L.n);
-    xn = V.x[vn]; yn = V.y[vn];
-    xp = V.x[vp]; yp = V.y[vp];
-    theta = vertex_theta(B, x, y, xn, yn, xp, yp);
-    const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-    seglen = sqrt(dnx * dnx + dny * dny);
-    area = V.area[L.r];
-    perim = V.perim[L.r];
-    comx = V.cx[L.r];
-    comy = V.cy[L.r];
-  }
-  o.cx = comx;
-  o.cy = comy;
-  if (write && L.act) {
-    V.th[L.v] = theta;
-    V.len[L.v] = seglen;
-    if (L.lane == L.segS && !L.wide) {
-      V.area[L.r] = area;
-      V.perim[L.r] = perim;
-      V.cx[L.r] = comx;
-      V.cy[L.r] = comy;
-    }
-  }
-  const double ind = 1.0 / (double)L.n;
-  // positions relative to the ring centre (getRelativeVertexPos 273-279)
-  const double rvx = pbx(x - comx, B), rvy = pby(y - comy, B);
-  const double rnx = pbx(xn - comx, B), rny = pby(yn - comy, B);
-  const double rpx = pbx(xp - comx, B), rpy = pby(yp - comy, B);
-  const double a0 = V.a0[L.r];
-  // shape costs: the global ea, el, eb, or per-ring values when the caller set them
-  const double ea = V.kr ? V.kr[L.r] : P.ea;
-  const double el = V.kr ? V.kr[V.np + L.r] : P.el;
-  const double eb = V.kr ? V.kr[2 * V.np + L.r] : P.eb;
-  // area term (calcAreaForceEnergy 429-435)
-  const double deltaA = (area / a0) - 1.;
-  const double gmA = ea * deltaA / a0;
-  double fx = 0.5 * gmA * (rpy - rny);
-  double fy = 0.5 * gmA * (rnx - rpx);
-  double e = (0.5 * ea * deltaA * deltaA) * ind;
-  // perimeter term (calcPerimeterForceEnergy 437-447 / FENE 449-455)
-  const double nsx = rnx - rvx, nsy = rny - rvy;
-  const double qsx = rvx - rpx, qsy = rvy - rpy;
-  const double pLen = sqrt(qsx * qsx + qsy * qsy);
-  const double nLen = sqrt(nsx * nsx + nsy * nsy);
-  const double l0v = V.l0[L.v];
-  const double l0s = shfl_d(l0v, L.pl);
-  const double l0p = L.wide ? V.l0[vp] : l0s;
-  if (P.monomer == MONO_HARMONIC) {
-    const double pDelta = (pLen / l0p) - 1.;
-    const double nDelta = (nLen / l0v) - 1.;
-    const double cn = nDelta / (l0v * nLen), cp = pDelta / (l0p * pLen);
-    fx += el * ((cn * (rnx - rvx)) - (cp * (rvx - rpx)));
-    fy += el * ((cn * (rny - rvy)) - (cp * (rvy - rpy)));
-    e += (0.5 * el * pDelta * pDelta);
-  } else {
-    const double c = 2 * el * P.stiff * P.extSq;
-    fx += c * ((nLen / (P.extSq * l0v * l0v - nLen * nLen)) * (rnx - rvx) / nLen -
-               (pLen / (P.extSq * l0p * l0p - pLen * pLen)) * (rvx - rpx) / pLen);
-    fy += c * ((nLen / (P.extSq * l0v * l0v - nLen * nLen)) * (rny - rvy) / nLen -
-               (pLen / (P.extSq * l0p * l0p - pLen * pLen)) * (rvy - rpy) / pLen);
-    e += el * P.stiff * P.extSq * log(1 - pLen * pLen / (P.extSq * l0p * l0p));
-  }
-  // bending term (calcBendingForceEnergy 457-471)
-  const double D = theta - V.th0[L.v];
-  double Dp = shfl_d(D, L.pl), Dn = shfl_d(D, L.nl);
-  if (L.wide) {  // the neighbours' angles from their own neighbours, as their lanes form them
-    const int vpp = ring_prev(vp, L.f, L.n), vnn = ring_next(vn, L.f, L.n);
-    Dp = vertex_theta(B, xp, yp, x, y, V.x[vpp], V.y[vpp]) - V.th0[vp];
-    Dn = vertex_theta(B, xn, yn, V.x[vnn], V.y[vnn], x, y) - V.th0[vn];
-  }
-  const double preVar = (D - Dp) / (qsx * qsx + qsy * qsy);
-  const double nextVar = (D - Dn) / (nsx * nsx + nsy * nsy);
-  fx += eb * (preVar * qsy + nextVar * nsy);
-  fy += eb * (preVar * (-qsx) + nextVar * (-nsx));
-  e += (0.5 * eb * D * D);
-  o.fx = fx; o.fy = fy; o.e = e;
-  return o;
-}
-
-// The ring centre alone (calcParticlePos, cudaKernel.cuh:365-388), as ring_shape computes it,
-// stored by the ring's first lane: the rigid rings' shape pass
-__device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, const Box& B, double x, double y) {
-  ShapeOut o{0, 0, 0, 0, 0};
-  const double xn = shfl_d(x, L.nl), yn = shfl_d(y, L.nl);
-  const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
-  const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-  const double Ix = seg_scan(L.act ? dnx : 0.0, L.lane, L.segS);
-  const double Iy = seg_scan(L.act ? dny : 0.0, L.lane, L.segS);
-  const double ux = L.act ? Ix - dnx : 0.0;
-  const double uy = L.act ? Iy - dny : 0.0;
-  const double sux = seg_sum(ux, L.lane, L.segS, L.segE);
-  const double suy = seg_sum(uy, L.lane, L.segS, L.segE);
-  const double ind = 1.0 / (double)L.n;
-  o.cx = xf + sux * ind;
-  o.cy = yf + suy * ind;
-  if (L.act && L.lane == L.segS) {
-    V.cx[L.r] = o.cx;
-    V.cy[L.r] = o.cy;
-  }
-  return o;
-}
 
 // --------------------------------------------------------- neighbours ---
 // cell_of, prev_pair, row_insert and build_row live in dpm_rows.h (shared with the adjoint).
@@ -224,529 +62,6 @@ __global__ void k_build_rows(View V, Params P, CellGrid G, const int* count, con
   if (countUpdates && L.tile == V.stile[L.s] && L.lane == 0) updateCount[L.s] += 1;
   if (!L.act) return;
   build_row(V, P, G, count, G.slots, L.v, L.s, box_of(V, L.s), err, maxcnt);
-}
-
-// Interparticle gather of lane L's vertex over entries k0, k0 + kstep, ... of its row:
-// accumulates the force on v, the vertex-vertex energy e, the smooth energy es and the share
-// (qx, qy) that v's `other` evaluation owes prev(v) (handed to prev(v)'s lane by the caller).
-// On the last lane of a wide ring's slice, whose next vertex lies in another tile, (qnx, qny)
-// accumulates the share that next(v)'s evaluations owe v, from next(v)'s row (complete before
-// the launch: wide sets rebuild rows in their own launch).
-template <int INTER, int POT>
-__device__ __forceinline__ void gather_pairs(const View& V, const Params& P, const Lane& L, const Box& B, double x,
-                                             double y, int k0, int kstep, double& fx, double& fy, double& e,
-                                             double& es, double& qx, double& qy, double& qnx, double& qny) {
-  const double radv = V.rad[L.v];
-  // Row entries are fetched one iteration ahead, the first one before the row length is known:
-  // rows are W entries wide (unused entries hold -1), so k < W keeps every fetch in bounds, and
-  // an entry is only used once k < ncnt is known.
-  if constexpr (INTER == INT_VV) {
-    // kernelCalcVertexInteraction, cudaKernel.cuh:690-722
-    int j = k0 < V.W ? V.nbr[(long)k0 * V.nv + L.v] : 0;
-    const int c = L.act ? V.ncnt[L.v] : 0;
-    for (int k = k0; k < c; k += kstep) {
-      const int kn = k + kstep;
-      const int jn = kn < V.W ? V.nbr[(long)kn * V.nv + L.v] : 0;
-      e += pair_force<POT>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
-      j = jn;
-    }
-  } else if constexpr (INTER == INT_SMOOTH) {
-    // kernelCalcSmoothInteraction, cudaKernel.cuh:922-975, as a gather: for every u in list(v),
-    // (v, segment of u) gives v's `this` share, and (u, segment (prev(v), v)) gives v's
-    // `other` share and prev(v)'s `previous` share (handed to prev(v)'s lane by the caller).
-    // Ring neighbours of v; inactive lanes past the tile end use v itself (in bounds).
-    int vp = L.act ? L.v0 + L.pl : L.v;
-    int vpp = L.act ? L.v0 + ((L.pl > L.segS) ? L.pl - 1 : L.segE) : L.v;
-    if (L.wide && L.act) {
-      vp = ring_prev(L.v, L.f, L.n);
-      vpp = ring_prev(vp, L.f, L.n);
-    }
-    const double xp = V.x[vp], yp = V.y[vp];
-    const double xpp = V.x[vpp], ypp = V.y[vpp];
-    int u = 0;
-    int2 pp = make_int2(0, 0);
-    if (k0 < V.W) {
-      u = V.nbr[(long)k0 * V.nv + L.v];
-      pp = V.nbrp[(long)k0 * V.nv + L.v];
-    }
-    const int c = L.act ? V.ncnt[L.v] : 0;
-    for (int k = k0; k < c; k += kstep) {
-      const int kn = k + kstep;
-      int un = 0;
-      int2 ppn = make_int2(0, 0);
-      if (kn < V.W) {
-        un = V.nbr[(long)kn * V.nv + L.v];
-        ppn = V.nbrp[(long)kn * V.nv + L.v];
-      }
-      const double xu = V.x[u], yu = V.y[u];
-      const double radSum = radv + V.rad[u];
-      es += smooth_pair<POT, ROLE_THIS>(P, B, x, y, xu, yu, V.x[pp.x], V.y[pp.x], V.x[pp.y], V.y[pp.y], radSum,
-                                        fx, fy);
-      es += smooth_pair_op<POT>(P, B, xu, yu, x, y, xp, yp, xpp, ypp, radSum, fx, fy, qx, qy);
-      u = un;
-      pp = ppn;
-    }
-    if (L.wide && L.act && L.lane == L.segE) {
-      // (u, segment (v, next(v))) for u in list(next(v)): next(v)'s `other` share is its own
-      // lane's; the `previous` share is v's (the energy is counted by next(v)'s lane)
-      const int j = ring_next(L.v, L.f, L.n);
-      const double xj = V.x[j], yj = V.y[j], radj = V.rad[j];
-      const int cj = V.ncnt[j];
-      for (int k = k0; k < cj; k += kstep) {
-        const int w = V.nbr[(long)k * V.nv + j];
-        double ox = 0, oy = 0;
-        (void)smooth_pair_op<POT>(P, B, V.x[w], V.y[w], xj, yj, x, y, xp, yp, radj + V.rad[w], ox, oy, qnx, qny);
-      }
-    }
-  } else {
-    // kernelCalcAllToAllVertexInteraction, cudaKernel.cuh:725-757 (test mode)
-    if (L.act) {
-      const int b0 = V.svoff[L.s], b1 = V.svoff[L.s + 1];
-      for (int j = b0 + k0; j < b1; j += kstep) {
-        if (V.vring[j] == L.r) continue;
-        e += pair_force<POT>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
-      }
-    }
-  }
-}
-
-// -------------------------------------------------------------- step ---
-// Waves of a tile: with nw > 1, wave 0 does the ring geometry, shape force and random draws
-// while waves 1..nw-1 share the neighbour gather; with nw == 1 wave 0 does both in turn.
-// A drift that moved a vertex more than cutoff / 3 marks its system FLAG_FAR: the next rebuild
-// cannot rely on the cells of its list positions (md_cells)
-__device__ __forceinline__ void far_test(const Params& P, const Box& B, double dx, double dy, int* flag) {
-  dx = pbx(dx, B);
-  dy = pby(dy, B);
-  if (3 * sqrt(dx * dx + dy * dy) > P.cutoff) atomicOr(flag, FLAG_FAR);
-}
-
-// The step loop's cell lists of a system whose list positions (the positions of its last
-// rebuild) have generation g: its rows are rebuilt from list g % 3, the rebuild bins its own
-// positions (the next list positions) into list (g + 1) % 3, cleared by the rebuild before, and
-// clears list (g + 2) % 3, which that rebuild read.  The cells are wide enough for a vertex 2
-// cutoff / 3 from its list position: at most cutoff / 3 before the drift that triggers the
-// rebuild (the displacement test) plus cutoff / 3 in that drift (else FLAG_FAR, all pairs).
-struct MdCells {
-  const int *cnt, *slots;  // read
-  int *binCnt, *binSlots;  // binned into
-  int* clear;              // cleared
-};
-__device__ __forceinline__ MdCells md_cells(const StepArgs& A, const CellGrid& G, int g) {
-  const long C = G.ncells, CS = (long)G.ncells * G.cap;
-  const int k0 = g % 3, k1 = (g + 1) % 3, k2 = (g + 2) % 3;
-  return MdCells{A.cellCur + k0 * C, A.slotsCur + k0 * CS, A.cellCur + k1 * C, A.slotsCur + k1 * CS,
-                 A.cellCur + k2 * C};
-}
-
-// a rebuilding vertex at (x, y) farther than 2 cutoff / 3 from its list position: its cells may
-// miss a neighbour (cannot happen while the displacement and far tests hold)
-__device__ __forceinline__ void md_stale_test(const View& V, const Params& P, const Box& B, int v, double x, double y,
-                                              int* err) {
-  const double ddx = pbx(x - V.lx[v], B), ddy = pby(y - V.ly[v], B);
-  if (3 * sqrt(ddx * ddx + ddy * ddy) > 2 * P.cutoff) atomicOr(err, ERR_STALE_BINS);
-}
-
-// ---------------------------------------------------------- rigid rings ---
-// Half kick of a rigid ring: RigidNVE::updateVelocity (Simulator.cu:348-366), or
-// RigidLangevin::updateVelocity (263-286) with its unit Gaussian pair (z0, z1) of the step and
-// d_thermalVel zero; the angular velocity takes the torque / moment of inertia.
-__device__ __forceinline__ void rigid_kick(bool langevin, double h, double gamma, double Fx, double Fy, double T,
-                                           double z0, double z1, double& vx, double& vy, double& w) {
-  if (langevin) {
-    vx += h * (Fx - vx * gamma);
-    vx -= 0.5 * h * h * (Fx - vx * gamma) / gamma;
-    vx += z0;
-    vy += h * (Fy - vy * gamma);
-    vy -= 0.5 * h * h * (Fy - vy * gamma) / gamma;
-    vy += z1;
-  } else {
-    vx += h * Fx;
-    vy += h * Fy;
-  }
-  w += h * T;
-}
-
-// A ring's vertex after the ring moved from centre (cx, cy) to (ncx, ncy) and turned by dth:
-// translateVertices then rotateVertices (kernelTranslateVertices / kernelRotateVertices,
-// cudaKernel.cuh:1678-1713), each difference a box distance.
-__device__ __forceinline__ void rigid_move(const Box& B, double x, double y, double cx, double cy, double ncx,
-                                           double ncy, double c, double sn, double& xn, double& yn) {
-  const double x1 = x + pbx(ncx - cx, B), y1 = y + pby(ncy - cy, B);
-  const double dx = pbx(x1 - ncx, B), dy = pby(y1 - ncy, B);
-  xn = x1 + ((dx * c - dy * sn) - dx);
-  yn = y1 + ((dx * sn + dy * c) - dy);
-}
-
-// Per-tile partials of the rigid FIRE sums over the rings whose first vertex is in the tile:
-// [0] v.F, [1] |v|^2, [2] |F|^2 (ring velocities and forces)
-__device__ __forceinline__ void rigid_fire_partials(const Lane& L, bool head, double vx, double vy, double Fx,
-                                                    double Fy, double* part) {
-  const double p0 = wave_sum(head ? vx * Fx + vy * Fy : 0.0);
-  const double p1 = wave_sum(head ? vx * vx + vy * vy : 0.0);
-  const double p2 = wave_sum(head ? Fx * Fx + Fy * Fy : 0.0);
-  if (L.lane == 0) {
-    part[L.tile * 4 + 0] = p0;
-    part[L.tile * 4 + 1] = p1;
-    part[L.tile * 4 + 2] = p2;
-  }
-}
-
-// Step-kernel epilogue of rigid rings (wave 0, one ring per lane segment): the interaction
-// forces' transfer to the ring (calcRigidForceEnergy, DPM2D.cu:2128-2142: torque r x f about
-// the centre, moment of inertia sum |r|^2, ring force sum f, ring torque sum (r x f) / I, ring
-// energy sum e for vertexVertex), then the second half kick of this step and, with MODE_START,
-// the next step's first half: last centre and angle stored, half kick with the next step's
-// draw, centre and angle advanced, vertices moved (RigidNVE / RigidLangevin::integrate,
-// Simulator.cu:241-252, 316-326).  With MODE_FIRE the half kick takes the system's FIRE step.
-template <int MODE, bool VV>
-__device__ __forceinline__ void rigid_epilogue(const View& V, const Params& P, const StepArgs& A, const Lane& L,
-                                               const Box& B, double x, double y, double fx, double fy, double e,
-                                               double cx, double cy, double lx, double ly, double z0, double z1) {
-  const Rigid R = *V.rg;
-  const double rx = pbx(x - cx, B), ry = pby(y - cy, B);
-  const double tq = rx * fy - ry * fx;
-  const double I = seg_sum(L.act ? rx * rx + ry * ry : 0.0, L.lane, L.segS, L.segE);
-  const double Fx = seg_sum(L.act ? fx : 0.0, L.lane, L.segS, L.segE);
-  const double Fy = seg_sum(L.act ? fy : 0.0, L.lane, L.segS, L.segE);
-  const double T = seg_sum(L.act ? tq : 0.0, L.lane, L.segS, L.segE) / I;
-  double E = 0;
-  if constexpr (VV) E = seg_sum(L.act ? e : 0.0, L.lane, L.segS, L.segE);
-  const bool head = L.act && L.lane == L.segS;
-  double vx = 0, vy = 0, w = 0;
-  if constexpr (MODE != MODE_RIGID) {
-    if (L.act) {
-      vx = R.pvx[L.r];
-      vy = R.pvy[L.r];
-      w = R.pw[L.r];
-    }
-  }
-  if constexpr ((MODE & MODE_FIRE) != 0) {
-    // the second half kick with the system's FIRE step, then the tile partials of the next
-    // iteration's sums (every lane takes part in the wave sums)
-    if (L.act) rigid_kick(false, 0.5 * A.fire[L.s].dt, 0.0, Fx, Fy, T, 0.0, 0.0, vx, vy, w);
-    rigid_fire_partials(L, head, vx, vy, Fx, Fy, A.part);
-  }
-  if (!L.act) return;
-  V.fx[L.v] = fx;
-  V.fy[L.v] = fy;
-  V.ev[L.v] = e;
-  R.vtq[L.v] = tq;
-  if (head) {
-    R.pfx[L.r] = Fx;
-    R.pfy[L.r] = Fy;
-    R.ptq[L.r] = T;
-    R.moi[L.r] = I;
-    if constexpr (VV) V.pe[L.r] = E;
-  }
-  if constexpr (MODE == MODE_RIGID) return;
-  if constexpr ((MODE & MODE_FIRE) == 0) {
-    rigid_kick(A.rigidLangevin, A.h, P.gamma, Fx, Fy, T, z0, z1, vx, vy, w);
-    if constexpr ((MODE & MODE_START) != 0) {
-      double n0 = 0, n1 = 0;
-      if (A.rigidLangevin)
-        gauss_pair(P.seed, (uint32_t)L.s, TAG_THERMAL, A.ctr[0] + (unsigned long long)A.ctrOffT + 1ull,
-                   (uint32_t)(L.r - V.sroff[L.s]), n0, n1);
-      rigid_kick(A.rigidLangevin, A.h, P.gamma, Fx, Fy, T, n0, n1, vx, vy, w);
-      const double ang = V.ang[L.r];
-      const double ncx = cx + A.dt * vx, ncy = cy + A.dt * vy, nang = ang + A.dt * w;
-      const double dth = nang - ang;
-      double xn, yn;
-      rigid_move(B, x, y, cx, cy, ncx, ncy, cos(dth), sin(dth), xn, yn);
-      A.xout[L.v] = xn;
-      A.yout[L.v] = yn;
-      const double ddx = pbx(xn - lx, B), ddy = pby(yn - ly, B);
-      if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
-        atomicOr(&A.flagOut[L.s], 1);
-        atomicOr(A.anyOut, 1);
-      }
-      far_test(P, B, xn - x, yn - y, A.flagOut + L.s);
-      if (head) {
-        V.ang[L.r] = nang;
-        V.cx[L.r] = ncx;
-        V.cy[L.r] = ncy;
-      }
-    }
-  }
-  if (head) {
-    R.pvx[L.r] = vx;
-    R.pvy[L.r] = vy;
-    R.pw[L.r] = w;
-  }
-}
-
-template <int INTER, int POT, int MODE>
-__global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepArgs A, CellGrid G) {
-  // partials of gather waves 1..nw-1: red[((w - 1) * 6 + q) * WAVE + lane], sized by the launch
-  extern __shared__ double red[];
-  const int w = threadIdx.x / WAVE;
-  const int nw = blockDim.x / WAVE;
-  Lane L;
-  constexpr bool WIDE = (MODE & MODE_WIDE) != 0;
-  constexpr int MB = MODE & ~MODE_WIDE;  // the integrator mode
-  // A step of a velocity-Verlet, Langevin or BAOAB loop other than its last consumes the force it
-  // computes in this launch (the closing and next opening half kicks); its force, energies, ring
-  // geometry and wall forces are stored by the loop's last step only.
-  constexpr bool STORE = (MODE & MODE_START) == 0 || (MODE & (MODE_BROWN | MODE_RIGID)) != 0;
-  lane_ctx<WIDE>(V, A.xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x, threadIdx.x & (WAVE - 1), L);
-  const Box B = box_of(V, L.s);
-  // own position first: the row rebuild below does not change it, so its load overlaps the
-  // rebuild-flag load instead of waiting behind it
-  const double x = V.x[L.v], y = V.y[L.v];
-
-  // loop bookkeeping: clear flags (and cells) for later steps, count this step's rebuild, rebuild rows
-  if (A.manage) {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (A.cellOther)
-      for (int c = gid; c < G.ncells; c += gridDim.x * blockDim.x) A.cellOther[c] = 0;
-    if (A.flagClear)
-      for (int t = gid; t < V.nsys; t += gridDim.x * blockDim.x) A.flagClear[t] = 0;
-    const int flag = A.flagCur[L.s];
-    const bool rebuild = (flag & 1) != 0;
-    // a system flagged FLAG_FAR searches all its vertices instead of cells that may miss a
-    // neighbour (the reference's all-pairs search)
-    const bool allPairs = A.staleCheck && (flag & FLAG_FAR) != 0;
-    const int* cells = A.cellCur;
-    const int* slots = A.slotsCur;
-    if (A.genCur) {
-      // step loop: rows from the cells of the list positions (md_cells)
-      const int g = A.genCur[L.s];
-      if (L.tile == V.stile[L.s] && threadIdx.x == 0) A.genOut[L.s] = rebuild ? g + 1 : g;
-      if (rebuild) {
-        const MdCells M = md_cells(A, G, g);
-        cells = M.cnt;
-        slots = M.slots;
-        if (!A.rowsBuilt) {
-          if (w == 0 && L.act && !allPairs) md_stale_test(V, P, B, L.v, x, y, A.err);
-          // these positions are the system's next list positions (its rows are built from them)
-          if (w == nw - 1 && L.act) bin_vertex(G, B, M.binCnt, M.binSlots, L.v, L.s, x, y, A.err);
-          if (!G.brute[L.s]) {
-            const int t0 = V.stile[L.s], nt = V.stile[L.s + 1] - t0;
-            const int n = G.ncx[L.s] * G.ncy[L.s];
-            int* clr = M.clear + G.coff[L.s];
-            for (int c = (L.tile - t0) * (int)blockDim.x + (int)threadIdx.x; c < n; c += nt * (int)blockDim.x)
-              clr[c] = 0;
-          }
-        }
-      }
-    }
-    if (rebuild && L.tile == V.stile[L.s] && threadIdx.x == 0) A.updateCount[L.s] += 1;
-    // the cell search shared by the tile's waves (rows in LDS) where the launch sized LDS for it
-    const bool tileBuild = rebuild && !A.rowsBuilt && !allPairs && A.rowsLdsW == V.W && !G.brute[L.s];
-    if (tileBuild) {
-      build_rows_tile(V, P, G, cells, slots, L.lane, L.v, L.r, L.s, L.act, w, nw, B, x, y, (int*)red, A.err,
-                      A.maxcnt);
-    } else if (rebuild && w == 0 && L.act && !A.rowsBuilt) {
-      build_row(V, P, G, cells, slots, L.v, L.s, B, A.err, A.maxcnt, allPairs);
-    }
-    if (rebuild) __syncthreads();
-  }
-  // wave 0's epilogue operands, fetched before the force work (lastPos after the rebuild above)
-  double vx = 0, vy = 0, lx = 0, ly = 0;
-  if (w == 0) {
-    if constexpr (MB != MODE_FORCE && (MODE & MODE_RIGID) == 0) {
-      vx = V.vx[L.v];
-      vy = V.vy[L.v];
-    }
-    if constexpr ((MODE & MODE_START) != 0) {
-      lx = V.lx[L.v];
-      ly = V.ly[L.v];
-    }
-  }
-
-  // gather partials: force on v, vertex-vertex energy, smooth energy, share for prev(v)
-  double fx = 0, fy = 0, e = 0, es = 0, qx = 0, qy = 0, qnx = 0, qny = 0;
-  const int g0 = nw > 1 ? 1 : 0;
-  const int ng = nw - g0;
-  // partials per gather wave: six, eight when the tile is a slice of a wide ring
-  constexpr int nq = (INTER == INT_SMOOTH && WIDE) ? 8 : 6;
-  if (w >= g0) gather_pairs<INTER, POT>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
-  if (nw > 1 && w > 0) {
-    double* r = red + (w - 1) * nq * WAVE + L.lane;
-    r[0 * WAVE] = fx;
-    r[1 * WAVE] = fy;
-    if constexpr (STORE) {  // energies are outputs only: a step that stores none leaves them out
-      r[2 * WAVE] = e;
-      r[3 * WAVE] = es;
-    }
-    r[4 * WAVE] = qx;
-    r[5 * WAVE] = qy;
-    if (nq == 8) {
-      r[6 * WAVE] = qnx;
-      r[7 * WAVE] = qny;
-    }
-  }
-
-  // ---- wave 0: work that does not need the gather, overlapped with it
-  ShapeOut so{0, 0, 0};
-  double zt0 = 0, zt1 = 0, ang = 0;
-  if (w == 0) {
-    if constexpr ((MODE & MODE_RIGID) != 0) so = ring_centre(V, L, B, x, y);
-    else so = ring_shape(V, P, L, B, x, y, STORE);
-    // one thermal draw per integrate call and ring: Langevin::updateThermalVel (Simulator.cu:54-77)
-    // and Brownian::updateThermalVel (156-179) after this call's force, counter = call index;
-    // BAOAB::updateThermalVel (122-144) in the next call's first half, whose index is one more
-    const unsigned long long callT = A.ctr[0] + (unsigned long long)A.ctrOffT;
-    const unsigned long long callA = A.ctr[1] + (unsigned long long)A.ctrOffA;
-    if constexpr ((MODE & MODE_LANGEVIN) != 0 || ((MODE & MODE_BAOAB) != 0 && (MODE & MODE_START) != 0))
-      gauss_pair(P.seed, (uint32_t)L.s, TAG_THERMAL, callT, (uint32_t)(L.r - V.sroff[L.s]), zt0, zt1);
-    // rigid Langevin: this step's pair (RigidLangevin::integrate draws it before its first half)
-    if constexpr ((MODE & MODE_RIGID) != 0 && (MODE & MODE_KICK) != 0)
-      if (A.rigidLangevin)
-        gauss_pair(P.seed, (uint32_t)L.s, TAG_THERMAL, callT, (uint32_t)(L.r - V.sroff[L.s]), zt0, zt1);
-    if (P.geometry != GEOM_NORMAL) {  // walls, after the interactions (DPM2D.cu:2090-2103)
-      double wfx, wfy;
-      so.e += wall_forces(P, B, x, y, V.rad[L.v], so.fx, so.fy, wfx, wfy);
-      if (STORE && L.act) {
-        V.wfx[L.v] = wfx;
-        V.wfy[L.v] = wfy;
-      }
-    }
-    if (P.particle == PART_ACTIVE_SHAPE && L.act) {  // updateRestLength, DPM2D.cu:2037-2056
-      double z0, z1;
-      gauss_pair(P.seed, (uint32_t)L.s, TAG_SHAPE, callA, (uint32_t)(L.r - V.sroff[L.s]), z0, z1);
-      const double l0v = V.l0[L.v];
-      V.l0[L.v] = l0v + ((l0v - V.l0r[L.v]) / P.l0Tau + sqrt(2. * P.l0Diff / P.dt) * z0) * P.dt;
-    }
-    if (P.particle == PART_ACTIVE) {  // addSelfPropulsion, DPM2D.cu:1995-2035
-      const double amplitude = (P.taup != 0) ? sqrt(2.0 * P.dt / P.taup) : 0.0;
-      double z0, z1;
-      gauss_pair(P.seed, (uint32_t)L.s, TAG_ACTIVE, callA, (uint32_t)(L.r - V.sroff[L.s]), z0, z1);
-      ang = V.ang[L.r];
-      ang += amplitude * z0;
-      ang = ang + kPI;
-      ang = ang - 2.0 * kPI * floor(ang / (2.0 * kPI));
-      ang = ang - kPI;
-      // the store depends on every lane's load of the old angle, which has returned
-      if (L.act && L.lane == L.segS) V.ang[L.r] = ang;
-    }
-  }
-  if (nw > 1) {
-    __syncthreads();
-    if (w > 0) return;
-    for (int q = 1; q < nw; q++) {
-      const double* r = red + (q - 1) * nq * WAVE + L.lane;
-      fx += r[0 * WAVE];
-      fy += r[1 * WAVE];
-      if constexpr (STORE) {
-        e += r[2 * WAVE];
-        es += r[3 * WAVE];
-      }
-      qx += r[4 * WAVE];
-      qy += r[5 * WAVE];
-      if (nq == 8) {
-        qnx += r[6 * WAVE];
-        qny += r[7 * WAVE];
-      }
-    }
-  }
-
-  // ---- wave 0: assemble F = shape + interparticle (+ shares from the next lane)
-  if constexpr (INTER == INT_SMOOTH) {
-    const double sx = shfl_d(qx, L.nl), sy = shfl_d(qy, L.nl);
-    const bool fromMemory = L.wide && L.lane == L.segE;  // next(v) in another tile
-    fx += fromMemory ? qnx : sx;
-    fy += fromMemory ? qny : sy;
-    if constexpr (STORE) {
-      const double pe = seg_sum(L.act ? es : 0.0, L.lane, L.segS, L.segE);
-      if (L.act) {
-        V.es[L.v] = es;
-        if (L.lane == L.segS && !L.wide) V.pe[L.r] = pe;  // wide rings: k_wide_pe sums es
-      }
-    }
-  }
-  if constexpr ((MODE & MODE_RIGID) != 0) {
-    rigid_epilogue<MB, INTER == INT_VV>(V, P, A, L, B, x, y, fx, fy, e, so.cx, so.cy, lx, ly, zt0, zt1);
-    return;
-  }
-  fx = so.fx + fx;
-  fy = so.fy + fy;
-  e = so.e + e;
-  if (P.particle == PART_ACTIVE) {
-    fx += P.driving * ((1 - 0) * cos(ang) + 0 * sin(ang));
-    fy += P.driving * ((1 - 1) * cos(ang) + 1 * sin(ang));
-  }
-
-  if constexpr ((MODE & MODE_LANGEVIN) != 0 && (MODE & MODE_BROWN) == 0) {
-    fx += P.noise * zt0 - P.gamma * vx;
-    fy += P.noise * zt1 - P.gamma * vy;
-  }
-  if constexpr ((MODE & MODE_FIRE) != 0) {
-    const FireState fs = A.fire[L.s];
-    const double h = 0.5 * fs.dt;
-    if (L.act && !fs.converged) {
-      vx += h * fx;
-      vy += h * fy;
-    }
-    const double pvf = L.act ? (vx * fx + vy * fy) : 0.0;
-    const double f2 = L.act ? fmax(fx * fx, fy * fy) : -1.0;
-    const double tP = wave_sum(pvf);
-    const double tM = wave_max(f2);
-    if (L.lane == 0) {
-      A.part[L.tile * 4 + 0] = tP;
-      A.part[L.tile * 4 + 3] = tM;
-    }
-    if (!L.act) return;
-    V.fx[L.v] = fx; V.fy[L.v] = fy; V.ev[L.v] = e;
-    V.vx[L.v] = vx; V.vy[L.v] = vy;
-    return;
-  }
-  if (!L.act) return;
-  if constexpr (STORE) {
-    V.fx[L.v] = fx;
-    V.fy[L.v] = fy;
-    V.ev[L.v] = e;
-  }
-  if constexpr (MB == MODE_FORCE) return;
-  if constexpr ((MODE & MODE_BROWN) != 0) {
-    // overdamped velocity (Brownian: (F + noise xi) / gamma; driven: F / gamma), then the drift
-    if constexpr ((MODE & MODE_LANGEVIN) != 0) {
-      vx = (fx + P.noise * zt0) / P.gamma;
-      vy = (fy + P.noise * zt1) / P.gamma;
-    } else {
-      vx = fx / P.gamma;
-      vy = fy / P.gamma;
-    }
-  }
-  if constexpr ((MODE & MODE_KICK) != 0) {
-    vx += A.h * fx;
-    vy += A.h * fy;
-  }
-  if constexpr ((MODE & MODE_START) != 0) {
-    double xn, yn;
-    if constexpr ((MODE & MODE_BROWN) != 0) {
-      xn = x + vx * A.dt;
-      yn = y + vy * A.dt;
-    } else if constexpr ((MODE & MODE_BAOAB) != 0) {
-      // B, A (half), O, A (half)
-      vx += A.h * fx;
-      vy += A.h * fy;
-      const double xa = x + vx * A.h, ya = y + vy * A.h;
-      vx = P.gamma * vx + P.noise * zt0;
-      vy = P.gamma * vy + P.noise * zt1;
-      xn = xa + vx * A.h;
-      yn = ya + vy * A.h;
-    } else {
-      vx += A.h * fx;
-      vy += A.h * fy;
-      xn = x + A.dt * vx;
-      yn = y + A.dt * vy;
-    }
-    A.xout[L.v] = xn;
-    A.yout[L.v] = yn;
-    if (A.recx) {
-      A.recx[L.v] = xn;
-      A.recy[L.v] = yn;
-    }
-    const double ddx = pbx(xn - lx, B), ddy = pby(yn - ly, B);
-    if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
-      atomicOr(&A.flagOut[L.s], 1);
-      atomicOr(A.anyOut, 1);
-    }
-    far_test(P, B, xn - x, yn - y, A.flagOut + L.s);
-  }
-  V.vx[L.v] = vx;
-  V.vy[L.v] = vy;
 }
 
 // ------------------------------------------------------------ wide rings ---
@@ -1450,317 +765,27 @@ __global__ void k_fire_resume(FireState* fs, int nsys) {
   if (s < nsys) fs[s].converged = 0;
 }
 
-// ------------------------------------------------------- persistent FIRE ---
-// One workgroup per system runs whole FIRE iterations (FIRE::minimizerVertexLoop,
-// FIRE.cu:397-411) back to back, separated by workgroup barriers only: systems share nothing,
-// so no grid-wide synchronisation is needed and a converged system's workgroup simply exits.
-// Each wave walks the system's ring-aligned tiles; the force phase is the step kernel's
-// (ring_shape + gather_pairs).  At most `chunk` iterations per launch; every thread decides the
-// loop exit from the same FIRE state, so all waves leave together.
-// Two builds: up to 8 waves per system (about 190 VGPRs, no spills) and up to 16 (the 1024-lane
-// workgroup caps a wave at 128 VGPRs, so 40-75 of them spill to scratch; halving the tiles each
-// wave walks still makes an iteration about 12% shorter on systems of 76 tiles).
-#define FS_WAVES 8
-#define FS_WAVES_WIDE 16
-
-// Workgroup reductions of the persistent kernel, with one barrier each: a caller alternates two
-// exchange buffers `red`, so that between two exchanges through the same buffer every thread
-// passes another barrier (no exchange overwrites one that a wave is still reading).
-// workgroup sum of a and maximum of b (fixed order: lanes by butterfly, waves by index)
-__device__ __forceinline__ void block_sum_max(double a, double b, double (*red)[2], double& sa, double& mb) {
-  const int w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-  a = wave_sum(a);
-  b = wave_max(b);
-  if ((threadIdx.x & (WAVE - 1)) == 0) {
-    red[w][0] = a;
-    red[w][1] = b;
-  }
-  __syncthreads();
-  double s = 0, m = -1;
-  for (int q = 0; q < nw; q++) {
-    s += red[q][0];
-    m = fmax(m, red[q][1]);
-  }
-  sa = s;
-  mb = m;
-}
-
-// workgroup sums of a and of b in one exchange (the order of block_sum_max's sum for each)
-__device__ __forceinline__ void block_sum_sum(double a, double b, double (*red)[2], double& sa, double& sb) {
-  const int w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-  a = wave_sum(a);
-  b = wave_sum(b);
-  if ((threadIdx.x & (WAVE - 1)) == 0) {
-    red[w][0] = a;
-    red[w][1] = b;
-  }
-  __syncthreads();
-  double s = 0, t = 0;
-  for (int q = 0; q < nw; q++) {
-    s += red[q][0];
-    t += red[q][1];
-  }
-  sa = s;
-  sb = t;
-}
-
-// P = v.F and max F_c^2 over the system's vertices
-__device__ __forceinline__ void fire_power(const View& V, int t0, int t1, double (*red)[2], double& P, double& Fm) {
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-  double p = 0, m = -1;
-  for (int t = t0 + w; t < t1; t += nw) {
-    const int v = V.tile_v0[t] + lane;
-    if (v < V.tile_v1[t]) {
-      const double fx = V.fx[v], fy = V.fy[v];
-      p += V.vx[v] * fx + V.vy[v] * fy;
-      m = fmax(m, fmax(fx * fx, fy * fy));
-    }
-  }
-  block_sum_max(p, m, red, P, Fm);
-}
-
-template <int INTER, int POT, int MAXW>
-__global__ __launch_bounds__(WAVE* MAXW) void k_fire_sys(View V, Params P, FireParams fp, CellGrid G,
-                                                         FireState* fst, int chunk, int* updateCount, int* err,
-                                                         int* maxcnt, const int* order) {
-  // exchange buffers: [0] for |v|^2 and |F|^2 after the half kick, [1] for P and max F_c^2 after
-  // the force (between two exchanges through one buffer every thread passes the other's barrier
-  // and the displacement test's)
-  __shared__ double red[2][MAXW][2];
-  const int s = order[blockIdx.x];
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-  const int t0 = V.stile[s], t1 = V.stile[s + 1];
-  const Box B = box_of(V, s);
-  // every thread carries the system's FIRE state and updates it from the same reduced values in
-  // the same order, so all hold the same state and take the same exit without a barrier
-  FireState fs = fst[s];
-  double Pv, Fm;
-  fire_power(V, t0, t1, red[1], Pv, Fm);
-  for (int it = 0; it < chunk; it++) {
-    // ---- checkFIREParams (FIRE.cu:338-371) and the stopping rule
-    if (!fs.converged && (sqrt(Fm) <= fp.tol || fs.iters >= fp.maxIter)) fs.converged = 1;
-    if (fs.converged) break;
-    int reset = 0;
-    fs.P = Pv;
-    if (Pv > 0) {
-      fs.numStep++;
-      if (fs.numStep > fp.minStep) {
-        fs.dt = fmin(fs.dt * fp.f_inc, fp.dt_max);
-        fs.a *= fp.f_a;
-      }
-    } else {
-      fs.numStep = 0;
-      fs.dt = fmax(fs.dt * fp.f_dec, fp.dt_max / 10);
-      fs.a = fp.a_start;
-      reset = 1;
-    }
-    fs.iters++;
-    const double dt = fs.dt, h = 0.5 * dt, fa = fs.a;
-    // ---- back-step on reset (with the decreased dt), half kick, |v|^2 and |F|^2
-    double vv = 0, ff = 0;
-    for (int t = t0 + w; t < t1; t += nw) {
-      const int v = V.tile_v0[t] + lane;
-      if (v < V.tile_v1[t]) {
-        double vx = V.vx[v], vy = V.vy[v];
-        const double fx = V.fx[v], fy = V.fy[v];
-        if (reset) {
-          V.x[v] -= h * vx;
-          V.y[v] -= h * vy;
-          vx = 0;
-          vy = 0;
-        }
-        vx += h * fx;
-        vy += h * fy;
-        V.vx[v] = vx;
-        V.vy[v] = vy;
-        vv += vx * vx + vy * vy;
-        ff += fx * fx + fy * fy;
-      }
-    }
-    double VV, FF;
-    block_sum_sum(vv, ff, red[0], VV, FF);
-    // ---- bendVertexVelocityTowardsForce (FIRE.cu:374-394), drift, displacement test
-    int moved = 0;
-    for (int t = t0 + w; t < t1; t += nw) {
-      const int v = V.tile_v0[t] + lane;
-      if (v < V.tile_v1[t]) {
-        double vx = V.vx[v], vy = V.vy[v];
-        if (FF > 0) {
-          const double ratio = sqrt(VV / FF);
-          vx = (1 - fa) * vx + fa * V.fx[v] * ratio;
-          vy = (1 - fa) * vy + fa * V.fy[v] * ratio;
-        }
-        const double xn = V.x[v] + dt * vx, yn = V.y[v] + dt * vy;
-        V.vx[v] = vx;
-        V.vy[v] = vy;
-        V.x[v] = xn;
-        V.y[v] = yn;
-        const double ddx = pbx(xn - V.lx[v], B), ddy = pby(yn - V.ly[v], B);
-        if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) moved = 1;
-      }
-    }
-    // ---- checkNeighbors: rebuild the system's rows from cells binned here (DPM2D.cu:1408-1423)
-    if (__syncthreads_or(moved)) {
-      const int ncx = G.ncx[s], ncy = G.ncy[s];
-      int* count = G.count[0];
-      if (!G.brute[s]) {
-        for (int t = t0 + w; t < t1; t += nw) {
-          const int v = V.tile_v0[t] + lane;
-          if (v < V.tile_v1[t]) {
-            int cx, cy;
-            cell_of(V.x[v], V.y[v], B, ncx, ncy, cx, cy);
-            const int c = G.coff[s] + cy * ncx + cx;
-            const int slot = atomicAdd(&count[c], 1);
-            if (slot < G.cap) G.slots[(long)c * G.cap + slot] = v;
-            else atomicOr(err, ERR_CELL_OVERFLOW);
-          }
-        }
-      }
-      __syncthreads();
-      for (int t = t0 + w; t < t1; t += nw) {
-        const int v = V.tile_v0[t] + lane;
-        if (v < V.tile_v1[t]) build_row(V, P, G, count, G.slots, v, s, B, err, maxcnt);
-      }
-      __syncthreads();
-      if (!G.brute[s])
-        for (int c = threadIdx.x; c < ncx * ncy; c += blockDim.x) count[G.coff[s] + c] = 0;
-      if (threadIdx.x == 0) updateCount[s] += 1;
-    }
-    // ---- calcForceEnergy (shape + interaction) and the second half kick
-    double p = 0, m = -1;
-    for (int t = t0 + w; t < t1; t += nw) {
-      Lane L;
-      lane_ctx(V, t, lane, L);
-      const double x = V.x[L.v], y = V.y[L.v];
-      double fx = 0, fy = 0, e = 0, es = 0, qx = 0, qy = 0;
-      double qnx = 0, qny = 0;  // sets with wide rings do not run this kernel
-      gather_pairs<INTER, POT>(V, P, L, B, x, y, 0, 1, fx, fy, e, es, qx, qy, qnx, qny);
-      const ShapeOut so = ring_shape(V, P, L, B, x, y, true);
-      if constexpr (INTER == INT_SMOOTH) {
-        fx += shfl_d(qx, L.nl);
-        fy += shfl_d(qy, L.nl);
-        const double pe = seg_sum(L.act ? es : 0.0, L.lane, L.segS, L.segE);
-        if (L.act) {
-          V.es[L.v] = es;
-          if (L.lane == L.segS) V.pe[L.r] = pe;
-        }
-      }
-      fx = so.fx + fx;
-      fy = so.fy + fy;
-      if (L.act) {
-        const double vx = V.vx[L.v] + h * fx, vy = V.vy[L.v] + h * fy;
-        V.fx[L.v] = fx;
-        V.fy[L.v] = fy;
-        V.ev[L.v] = so.e + e;
-        V.vx[L.v] = vx;
-        V.vy[L.v] = vy;
-        p += vx * fx + vy * fy;
-        m = fmax(m, fmax(fx * fx, fy * fy));
-      }
-    }
-    block_sum_max(p, m, red[1], Pv, Fm);
-  }
-  if (threadIdx.x == 0) fst[s] = fs;
-}
-
 // --------------------------------------------------------- launchers ---
-static inline int grid_v(long n) { return (int)((n + 255) / 256); }
-static inline int grid_w(int ntiles) { return (ntiles + 3) / 4; }
 
-// LDS of the step kernel: six partials per lane of each gather wave (eight with wide rings)
-static inline size_t step_lds(const dpm_set_s* S) {
-  const size_t red = (size_t)(S->split - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
-  const size_t rows = (S->split >= 2 && S->V.W <= 64) ? (size_t)(64 + 64 * S->V.W) * sizeof(int) : 0;
-  return red > rows ? red : rows;
-}
-
-// rigid-ring modes (sets of rings of at most 64 vertices only)
-template <int INTER, int POT>
-static hipError_t step_rigid(dpm_set_s* S, int mode, const StepArgs& A) {
-  const int g = S->V.ntiles;
-  const int b = WAVE * S->split;
-  const size_t sh = step_lds(S);
-  hipStream_t st = S->stream;
-  switch (mode) {
-    case MODE_RIGID: k_step<INTER, POT, MODE_RIGID><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_RIGID | MODE_KICK:
-      k_step<INTER, POT, MODE_RIGID | MODE_KICK><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_RIGID | MODE_KICK | MODE_START:
-      k_step<INTER, POT, MODE_RIGID | MODE_KICK | MODE_START><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_RIGID | MODE_FIRE:
-      k_step<INTER, POT, MODE_RIGID | MODE_FIRE><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-template <int INTER, int POT, int WB>
-static hipError_t step_mode(dpm_set_s* S, int mode, const StepArgs& A) {
-  if constexpr (WB != 0) {
-    if (mode & MODE_RIGID) return hipErrorInvalidValue;  // refused for wide sets before this point
-  } else {
-    if (mode & MODE_RIGID) return step_rigid<INTER, POT>(S, mode, A);
-  }
-  const int g = S->V.ntiles;
-  const int b = WAVE * S->split;
-  const size_t sh = step_lds(S);
-  hipStream_t st = S->stream;
-  switch (mode) {
-    case MODE_FORCE: k_step<INTER, POT, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_KICK: k_step<INTER, POT, MODE_KICK | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_KICK | MODE_LANGEVIN:
-      k_step<INTER, POT, MODE_KICK | MODE_LANGEVIN | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_KICK | MODE_START:
-      k_step<INTER, POT, MODE_KICK | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_KICK | MODE_LANGEVIN | MODE_START:
-      k_step<INTER, POT, MODE_KICK | MODE_LANGEVIN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_FIRE: k_step<INTER, POT, MODE_FIRE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_KICK | MODE_BAOAB:
-      k_step<INTER, POT, MODE_KICK | MODE_BAOAB | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_KICK | MODE_BAOAB | MODE_START:
-      k_step<INTER, POT, MODE_KICK | MODE_BAOAB | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_BROWN | MODE_START:
-      k_step<INTER, POT, MODE_BROWN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_BROWN | MODE_LANGEVIN | MODE_START:
-      k_step<INTER, POT, MODE_BROWN | MODE_LANGEVIN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-template <int INTER, int WB>
+template <int INTER>
 static hipError_t step_pot(dpm_set_s* S, int mode, const StepArgs& A) {
   switch (S->P.potential) {
-    case POT_HARMONIC: return step_mode<INTER, POT_HARMONIC, WB>(S, mode, A);
-    case POT_LJ: return step_mode<INTER, POT_LJ, WB>(S, mode, A);
-    case POT_ADHESIVE: return step_mode<INTER, POT_ADHESIVE, WB>(S, mode, A);
-    case POT_WCA: return step_mode<INTER, POT_WCA, WB>(S, mode, A);
+    case POT_HARMONIC: return step_launch<INTER, POT_HARMONIC>(S, mode, A);
+    case POT_LJ: return step_launch<INTER, POT_LJ>(S, mode, A);
+    case POT_ADHESIVE: return step_launch<INTER, POT_ADHESIVE>(S, mode, A);
+    case POT_WCA: return step_launch<INTER, POT_WCA>(S, mode, A);
   }
   return hipErrorInvalidValue;
 }
 
-template <int WB>
-static hipError_t step_all(dpm_set_s* S, const StepArgs& A) {
-  const int g = S->V.ntiles, b = WAVE * S->split;
-  const size_t sh = step_lds(S);
-  hipStream_t st = S->stream;
+template <int INTER>
+static hipError_t fire_pot(dpm_set_s* S, int chunk, int threads) {
   switch (S->P.potential) {
-    case POT_HARMONIC: k_step<INT_ALL, POT_HARMONIC, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case POT_LJ: k_step<INT_ALL, POT_LJ, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case POT_ADHESIVE: k_step<INT_ALL, POT_ADHESIVE, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case POT_WCA: k_step<INT_ALL, POT_WCA, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
+    case POT_HARMONIC: return fire_launch<INTER, POT_HARMONIC>(S, chunk, threads);
+    case POT_LJ: return fire_launch<INTER, POT_LJ>(S, chunk, threads);
+    case POT_ADHESIVE: return fire_launch<INTER, POT_ADHESIVE>(S, chunk, threads);
+    default: return fire_launch<INTER, POT_WCA>(S, chunk, threads);
   }
-  return hipGetLastError();
 }
 
 static hipError_t launch_step_kernel(dpm_set_s* S, int mode, const StepArgs& A);
@@ -1800,14 +825,10 @@ static hipError_t launch_step_kernel(dpm_set_s* S, int mode, const StepArgs& A0)
   if (A.manage && (!A.flagCur || !A.cellCur || !A.slotsCur || (A.genCur && !A.genOut) || !A.err || !A.maxcnt ||
                    !A.updateCount))
     return hipErrorInvalidValue;
-  const bool wide = S->nwide > 0;
   switch (S->P.interaction) {
-    case INT_VV: return wide ? step_pot<INT_VV, MODE_WIDE>(S, mode, A) : step_pot<INT_VV, 0>(S, mode, A);
-    case INT_SMOOTH:
-      return wide ? step_pot<INT_SMOOTH, MODE_WIDE>(S, mode, A) : step_pot<INT_SMOOTH, 0>(S, mode, A);
-    case INT_ALL:
-      if (mode != MODE_FORCE) return hipErrorInvalidValue;
-      return wide ? step_all<MODE_WIDE>(S, A) : step_all<0>(S, A);
+    case INT_VV: return step_pot<INT_VV>(S, mode, A);
+    case INT_SMOOTH: return step_pot<INT_SMOOTH>(S, mode, A);
+    case INT_ALL: return step_pot<INT_ALL>(S, mode, A);
   }
   return hipErrorInvalidValue;
 }
@@ -1995,35 +1016,12 @@ hipError_t launch_fire_partials(dpm_set_s* S) {
   return hipGetLastError();
 }
 
-template <int INTER, int POT>
-static hipError_t fire_sys_t(dpm_set_s* S, int chunk, int threads) {
-  if (threads > WAVE * FS_WAVES)
-    k_fire_sys<INTER, POT, FS_WAVES_WIDE><<<(unsigned)S->nsys, threads, 0, S->stream>>>(
-        S->V, S->P, S->fp, S->G, S->d_fire[S->fireCur], chunk, S->d_updateCount, S->d_err, S->d_maxcnt,
-        S->d_sysOrder);
-  else
-    k_fire_sys<INTER, POT, FS_WAVES><<<(unsigned)S->nsys, threads, 0, S->stream>>>(
-        S->V, S->P, S->fp, S->G, S->d_fire[S->fireCur], chunk, S->d_updateCount, S->d_err, S->d_maxcnt,
-        S->d_sysOrder);
-  return hipGetLastError();
-}
-
-template <int INTER>
-static hipError_t fire_sys_pot(dpm_set_s* S, int chunk, int threads) {
-  switch (S->P.potential) {
-    case POT_HARMONIC: return fire_sys_t<INTER, POT_HARMONIC>(S, chunk, threads);
-    case POT_LJ: return fire_sys_t<INTER, POT_LJ>(S, chunk, threads);
-    case POT_ADHESIVE: return fire_sys_t<INTER, POT_ADHESIVE>(S, chunk, threads);
-    default: return fire_sys_t<INTER, POT_WCA>(S, chunk, threads);
-  }
-}
-
 hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves) {
   const int threads = WAVE * (waves < 1 ? 1 : (waves > FS_WAVES_WIDE ? FS_WAVES_WIDE : waves));
   switch (S->P.interaction) {
-    case INT_VV: return fire_sys_pot<INT_VV>(S, chunk, threads);
-    case INT_SMOOTH: return fire_sys_pot<INT_SMOOTH>(S, chunk, threads);
-    default: return fire_sys_pot<INT_ALL>(S, chunk, threads);
+    case INT_VV: return fire_pot<INT_VV>(S, chunk, threads);
+    case INT_SMOOTH: return fire_pot<INT_SMOOTH>(S, chunk, threads);
+    default: return fire_pot<INT_ALL>(S, chunk, threads);
   }
 }
 

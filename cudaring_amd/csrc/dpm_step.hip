@@ -1,0 +1,374 @@
+// dpm_step.hip -- the step kernel, compiled once per (interaction, potential): STEP_INTER and
+// STEP_POT select the instance, whose launcher is a specialisation of step_launch.
+#include "dpm_forces.h"
+#include "dpm_launch.h"
+
+namespace dpm {
+
+template <int INTER, int POT, int MODE>
+__global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepArgs A, CellGrid G) {
+  // partials of gather waves 1..nw-1: red[((w - 1) * 6 + q) * WAVE + lane], sized by the launch
+  extern __shared__ double red[];
+  const int w = threadIdx.x / WAVE;
+  const int nw = blockDim.x / WAVE;
+  Lane L;
+  constexpr bool WIDE = (MODE & MODE_WIDE) != 0;
+  constexpr int MB = MODE & ~MODE_WIDE;  // the integrator mode
+  // A step of a velocity-Verlet, Langevin or BAOAB loop other than its last consumes the force it
+  // computes in this launch (the closing and next opening half kicks); its force, energies, ring
+  // geometry and wall forces are stored by the loop's last step only.
+  constexpr bool STORE = (MODE & MODE_START) == 0 || (MODE & (MODE_BROWN | MODE_RIGID)) != 0;
+  lane_ctx<WIDE>(V, A.xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x, threadIdx.x & (WAVE - 1), L);
+  const Box B = box_of(V, L.s);
+  // own position first: the row rebuild below does not change it, so its load overlaps the
+  // rebuild-flag load instead of waiting behind it
+  const double x = V.x[L.v], y = V.y[L.v];
+
+  // loop bookkeeping: clear flags (and cells) for later steps, count this step's rebuild, rebuild rows
+  if (A.manage) {
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+    if (A.cellOther)
+      for (int c = gid; c < G.ncells; c += gridDim.x * blockDim.x) A.cellOther[c] = 0;
+    if (A.flagClear)
+      for (int t = gid; t < V.nsys; t += gridDim.x * blockDim.x) A.flagClear[t] = 0;
+    const int flag = A.flagCur[L.s];
+    const bool rebuild = (flag & 1) != 0;
+    // a system flagged FLAG_FAR searches all its vertices instead of cells that may miss a
+    // neighbour (the reference's all-pairs search)
+    const bool allPairs = A.staleCheck && (flag & FLAG_FAR) != 0;
+    const int* cells = A.cellCur;
+    const int* slots = A.slotsCur;
+    if (A.genCur) {
+      // step loop: rows from the cells of the list positions (md_cells)
+      const int g = A.genCur[L.s];
+      if (L.tile == V.stile[L.s] && threadIdx.x == 0) A.genOut[L.s] = rebuild ? g + 1 : g;
+      if (rebuild) {
+        const MdCells M = md_cells(A, G, g);
+        cells = M.cnt;
+        slots = M.slots;
+        if (!A.rowsBuilt) {
+          if (w == 0 && L.act && !allPairs) md_stale_test(V, P, B, L.v, x, y, A.err);
+          // these positions are the system's next list positions (its rows are built from them)
+          if (w == nw - 1 && L.act) bin_vertex(G, B, M.binCnt, M.binSlots, L.v, L.s, x, y, A.err);
+          if (!G.brute[L.s]) {
+            const int t0 = V.stile[L.s], nt = V.stile[L.s + 1] - t0;
+            const int n = G.ncx[L.s] * G.ncy[L.s];
+            int* clr = M.clear + G.coff[L.s];
+            for (int c = (L.tile - t0) * (int)blockDim.x + (int)threadIdx.x; c < n; c += nt * (int)blockDim.x)
+              clr[c] = 0;
+          }
+        }
+      }
+    }
+    if (rebuild && L.tile == V.stile[L.s] && threadIdx.x == 0) A.updateCount[L.s] += 1;
+    // the cell search shared by the tile's waves (rows in LDS) where the launch sized LDS for it
+    const bool tileBuild = rebuild && !A.rowsBuilt && !allPairs && A.rowsLdsW == V.W && !G.brute[L.s];
+    if (tileBuild) {
+      build_rows_tile(V, P, G, cells, slots, L.lane, L.v, L.r, L.s, L.act, w, nw, B, x, y, (int*)red, A.err,
+                      A.maxcnt);
+    } else if (rebuild && w == 0 && L.act && !A.rowsBuilt) {
+      build_row(V, P, G, cells, slots, L.v, L.s, B, A.err, A.maxcnt, allPairs);
+    }
+    if (rebuild) __syncthreads();
+  }
+  // wave 0's epilogue operands, fetched before the force work (lastPos after the rebuild above)
+  double vx = 0, vy = 0, lx = 0, ly = 0;
+  if (w == 0) {
+    if constexpr (MB != MODE_FORCE && (MODE & MODE_RIGID) == 0) {
+      vx = V.vx[L.v];
+      vy = V.vy[L.v];
+    }
+    if constexpr ((MODE & MODE_START) != 0) {
+      lx = V.lx[L.v];
+      ly = V.ly[L.v];
+    }
+  }
+
+  // gather partials: force on v, vertex-vertex energy, smooth energy, share for prev(v)
+  double fx = 0, fy = 0, e = 0, es = 0, qx = 0, qy = 0, qnx = 0, qny = 0;
+  const int g0 = nw > 1 ? 1 : 0;
+  const int ng = nw - g0;
+  // partials per gather wave: six, eight when the tile is a slice of a wide ring
+  constexpr int nq = (INTER == INT_SMOOTH && WIDE) ? 8 : 6;
+  if (w >= g0) gather_pairs<INTER, POT>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
+  if (nw > 1 && w > 0) {
+    double* r = red + (w - 1) * nq * WAVE + L.lane;
+    r[0 * WAVE] = fx;
+    r[1 * WAVE] = fy;
+    if constexpr (STORE) {  // energies are outputs only: a step that stores none leaves them out
+      r[2 * WAVE] = e;
+      r[3 * WAVE] = es;
+    }
+    r[4 * WAVE] = qx;
+    r[5 * WAVE] = qy;
+    if (nq == 8) {
+      r[6 * WAVE] = qnx;
+      r[7 * WAVE] = qny;
+    }
+  }
+
+  // ---- wave 0: work that does not need the gather, overlapped with it
+  ShapeOut so{0, 0, 0};
+  double zt0 = 0, zt1 = 0, ang = 0;
+  if (w == 0) {
+    if constexpr ((MODE & MODE_RIGID) != 0) so = ring_centre(V, L, B, x, y);
+    else so = ring_shape(V, P, L, B, x, y, STORE);
+    // one thermal draw per integrate call and ring: Langevin::updateThermalVel (Simulator.cu:54-77)
+    // and Brownian::updateThermalVel (156-179) after this call's force, counter = call index;
+    // BAOAB::updateThermalVel (122-144) in the next call's first half, whose index is one more
+    const unsigned long long callT = A.ctr[0] + (unsigned long long)A.ctrOffT;
+    const unsigned long long callA = A.ctr[1] + (unsigned long long)A.ctrOffA;
+    if constexpr ((MODE & MODE_LANGEVIN) != 0 || ((MODE & MODE_BAOAB) != 0 && (MODE & MODE_START) != 0))
+      gauss_pair(P.seed, (uint32_t)L.s, TAG_THERMAL, callT, (uint32_t)(L.r - V.sroff[L.s]), zt0, zt1);
+    // rigid Langevin: this step's pair (RigidLangevin::integrate draws it before its first half)
+    if constexpr ((MODE & MODE_RIGID) != 0 && (MODE & MODE_KICK) != 0)
+      if (A.rigidLangevin)
+        gauss_pair(P.seed, (uint32_t)L.s, TAG_THERMAL, callT, (uint32_t)(L.r - V.sroff[L.s]), zt0, zt1);
+    if (P.geometry != GEOM_NORMAL) {  // walls, after the interactions (DPM2D.cu:2090-2103)
+      double wfx, wfy;
+      so.e += wall_forces(P, B, x, y, V.rad[L.v], so.fx, so.fy, wfx, wfy);
+      if (STORE && L.act) {
+        V.wfx[L.v] = wfx;
+        V.wfy[L.v] = wfy;
+      }
+    }
+    if (P.particle == PART_ACTIVE_SHAPE && L.act) {  // updateRestLength, DPM2D.cu:2037-2056
+      double z0, z1;
+      gauss_pair(P.seed, (uint32_t)L.s, TAG_SHAPE, callA, (uint32_t)(L.r - V.sroff[L.s]), z0, z1);
+      const double l0v = V.l0[L.v];
+      V.l0[L.v] = l0v + ((l0v - V.l0r[L.v]) / P.l0Tau + sqrt(2. * P.l0Diff / P.dt) * z0) * P.dt;
+    }
+    if (P.particle == PART_ACTIVE) {  // addSelfPropulsion, DPM2D.cu:1995-2035
+      const double amplitude = (P.taup != 0) ? sqrt(2.0 * P.dt / P.taup) : 0.0;
+      double z0, z1;
+      gauss_pair(P.seed, (uint32_t)L.s, TAG_ACTIVE, callA, (uint32_t)(L.r - V.sroff[L.s]), z0, z1);
+      ang = V.ang[L.r];
+      ang += amplitude * z0;
+      ang = ang + kPI;
+      ang = ang - 2.0 * kPI * floor(ang / (2.0 * kPI));
+      ang = ang - kPI;
+      // the store depends on every lane's load of the old angle, which has returned
+      if (L.act && L.lane == L.segS) V.ang[L.r] = ang;
+    }
+  }
+  if (nw > 1) {
+    __syncthreads();
+    if (w > 0) return;
+    for (int q = 1; q < nw; q++) {
+      const double* r = red + (q - 1) * nq * WAVE + L.lane;
+      fx += r[0 * WAVE];
+      fy += r[1 * WAVE];
+      if constexpr (STORE) {
+        e += r[2 * WAVE];
+        es += r[3 * WAVE];
+      }
+      qx += r[4 * WAVE];
+      qy += r[5 * WAVE];
+      if (nq == 8) {
+        qnx += r[6 * WAVE];
+        qny += r[7 * WAVE];
+      }
+    }
+  }
+
+  // ---- wave 0: assemble F = shape + interparticle (+ shares from the next lane)
+  if constexpr (INTER == INT_SMOOTH) {
+    const double sx = shfl_d(qx, L.nl), sy = shfl_d(qy, L.nl);
+    const bool fromMemory = L.wide && L.lane == L.segE;  // next(v) in another tile
+    fx += fromMemory ? qnx : sx;
+    fy += fromMemory ? qny : sy;
+    if constexpr (STORE) {
+      const double pe = seg_sum(L.act ? es : 0.0, L.lane, L.segS, L.segE);
+      if (L.act) {
+        V.es[L.v] = es;
+        if (L.lane == L.segS && !L.wide) V.pe[L.r] = pe;  // wide rings: k_wide_pe sums es
+      }
+    }
+  }
+  if constexpr ((MODE & MODE_RIGID) != 0) {
+    rigid_epilogue<MB, INTER == INT_VV>(V, P, A, L, B, x, y, fx, fy, e, so.cx, so.cy, lx, ly, zt0, zt1);
+    return;
+  }
+  fx = so.fx + fx;
+  fy = so.fy + fy;
+  e = so.e + e;
+  if (P.particle == PART_ACTIVE) {
+    fx += P.driving * ((1 - 0) * cos(ang) + 0 * sin(ang));
+    fy += P.driving * ((1 - 1) * cos(ang) + 1 * sin(ang));
+  }
+
+  if constexpr ((MODE & MODE_LANGEVIN) != 0 && (MODE & MODE_BROWN) == 0) {
+    fx += P.noise * zt0 - P.gamma * vx;
+    fy += P.noise * zt1 - P.gamma * vy;
+  }
+  if constexpr ((MODE & MODE_FIRE) != 0) {
+    const FireState fs = A.fire[L.s];
+    const double h = 0.5 * fs.dt;
+    if (L.act && !fs.converged) {
+      vx += h * fx;
+      vy += h * fy;
+    }
+    const double pvf = L.act ? (vx * fx + vy * fy) : 0.0;
+    const double f2 = L.act ? fmax(fx * fx, fy * fy) : -1.0;
+    const double tP = wave_sum(pvf);
+    const double tM = wave_max(f2);
+    if (L.lane == 0) {
+      A.part[L.tile * 4 + 0] = tP;
+      A.part[L.tile * 4 + 3] = tM;
+    }
+    if (!L.act) return;
+    V.fx[L.v] = fx; V.fy[L.v] = fy; V.ev[L.v] = e;
+    V.vx[L.v] = vx; V.vy[L.v] = vy;
+    return;
+  }
+  if (!L.act) return;
+  if constexpr (STORE) {
+    V.fx[L.v] = fx;
+    V.fy[L.v] = fy;
+    V.ev[L.v] = e;
+  }
+  if constexpr (MB == MODE_FORCE) return;
+  if constexpr ((MODE & MODE_BROWN) != 0) {
+    // overdamped velocity (Brownian: (F + noise xi) / gamma; driven: F / gamma), then the drift
+    if constexpr ((MODE & MODE_LANGEVIN) != 0) {
+      vx = (fx + P.noise * zt0) / P.gamma;
+      vy = (fy + P.noise * zt1) / P.gamma;
+    } else {
+      vx = fx / P.gamma;
+      vy = fy / P.gamma;
+    }
+  }
+  if constexpr ((MODE & MODE_KICK) != 0) {
+    vx += A.h * fx;
+    vy += A.h * fy;
+  }
+  if constexpr ((MODE & MODE_START) != 0) {
+    double xn, yn;
+    if constexpr ((MODE & MODE_BROWN) != 0) {
+      xn = x + vx * A.dt;
+      yn = y + vy * A.dt;
+    } else if constexpr ((MODE & MODE_BAOAB) != 0) {
+      // B, A (half), O, A (half)
+      vx += A.h * fx;
+      vy += A.h * fy;
+      const double xa = x + vx * A.h, ya = y + vy * A.h;
+      vx = P.gamma * vx + P.noise * zt0;
+      vy = P.gamma * vy + P.noise * zt1;
+      xn = xa + vx * A.h;
+      yn = ya + vy * A.h;
+    } else {
+      vx += A.h * fx;
+      vy += A.h * fy;
+      xn = x + A.dt * vx;
+      yn = y + A.dt * vy;
+    }
+    A.xout[L.v] = xn;
+    A.yout[L.v] = yn;
+    if (A.recx) {
+      A.recx[L.v] = xn;
+      A.recy[L.v] = yn;
+    }
+    const double ddx = pbx(xn - lx, B), ddy = pby(yn - ly, B);
+    if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
+      atomicOr(&A.flagOut[L.s], 1);
+      atomicOr(A.anyOut, 1);
+    }
+    far_test(P, B, xn - x, yn - y, A.flagOut + L.s);
+  }
+  V.vx[L.v] = vx;
+  V.vy[L.v] = vy;
+}
+
+// LDS of the step kernel: six partials per lane of each gather wave (eight with wide rings)
+static inline size_t step_lds(const dpm_set_s* S) {
+  const size_t red = (size_t)(S->split - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
+  const size_t rows = (S->split >= 2 && S->V.W <= 64) ? (size_t)(64 + 64 * S->V.W) * sizeof(int) : 0;
+  return red > rows ? red : rows;
+}
+
+// rigid-ring modes (sets of rings of at most 64 vertices only)
+template <int INTER, int POT>
+static hipError_t step_rigid(dpm_set_s* S, int mode, const StepArgs& A) {
+  const int g = S->V.ntiles;
+  const int b = WAVE * S->split;
+  const size_t sh = step_lds(S);
+  hipStream_t st = S->stream;
+  switch (mode) {
+    case MODE_RIGID: k_step<INTER, POT, MODE_RIGID><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
+    case MODE_RIGID | MODE_KICK:
+      k_step<INTER, POT, MODE_RIGID | MODE_KICK><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_RIGID | MODE_KICK | MODE_START:
+      k_step<INTER, POT, MODE_RIGID | MODE_KICK | MODE_START><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_RIGID | MODE_FIRE:
+      k_step<INTER, POT, MODE_RIGID | MODE_FIRE><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+template <int INTER, int POT, int WB>
+static hipError_t step_mode(dpm_set_s* S, int mode, const StepArgs& A) {
+  if constexpr (WB != 0) {
+    if (mode & MODE_RIGID) return hipErrorInvalidValue;  // refused for wide sets before this point
+  } else {
+    if (mode & MODE_RIGID) return step_rigid<INTER, POT>(S, mode, A);
+  }
+  const int g = S->V.ntiles;
+  const int b = WAVE * S->split;
+  const size_t sh = step_lds(S);
+  hipStream_t st = S->stream;
+  switch (mode) {
+    case MODE_FORCE: k_step<INTER, POT, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
+    case MODE_KICK: k_step<INTER, POT, MODE_KICK | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
+    case MODE_KICK | MODE_LANGEVIN:
+      k_step<INTER, POT, MODE_KICK | MODE_LANGEVIN | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_KICK | MODE_START:
+      k_step<INTER, POT, MODE_KICK | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_KICK | MODE_LANGEVIN | MODE_START:
+      k_step<INTER, POT, MODE_KICK | MODE_LANGEVIN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_FIRE: k_step<INTER, POT, MODE_FIRE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
+    case MODE_KICK | MODE_BAOAB:
+      k_step<INTER, POT, MODE_KICK | MODE_BAOAB | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_KICK | MODE_BAOAB | MODE_START:
+      k_step<INTER, POT, MODE_KICK | MODE_BAOAB | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_BROWN | MODE_START:
+      k_step<INTER, POT, MODE_BROWN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    case MODE_BROWN | MODE_LANGEVIN | MODE_START:
+      k_step<INTER, POT, MODE_BROWN | MODE_LANGEVIN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
+      break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+// all-pairs interaction (test mode): forces only
+template <int POT, int WB>
+static hipError_t step_all(dpm_set_s* S, int mode, const StepArgs& A) {
+  if (mode != MODE_FORCE) return hipErrorInvalidValue;
+  k_step<INT_ALL, POT, MODE_FORCE | WB><<<S->V.ntiles, WAVE * S->split, step_lds(S), S->stream>>>(S->V, S->P, A, S->G);
+  return hipGetLastError();
+}
+
+#if !defined(STEP_INTER) || !defined(STEP_POT)
+#error "compile with -DSTEP_INTER and -DSTEP_POT"
+#endif
+template <>
+hipError_t step_launch<STEP_INTER, STEP_POT>(dpm_set_s* S, int mode, const StepArgs& A) {
+#if STEP_INTER == 3
+  return S->nwide > 0 ? step_all<STEP_POT, MODE_WIDE>(S, mode, A) : step_all<STEP_POT, 0>(S, mode, A);
+#else
+  return S->nwide > 0 ? step_mode<STEP_INTER, STEP_POT, MODE_WIDE>(S, mode, A)
+                      : step_mode<STEP_INTER, STEP_POT, 0>(S, mode, A);
+#endif
+}
+
+}  // namespace dpm

@@ -8,6 +8,9 @@ namespace dpm {
 
 #define WAVE 64
 #define MAXSPLIT 8
+// waves per workgroup of the two persistent FIRE builds
+#define FS_WAVES 8
+#define FS_WAVES_WIDE 16
 
 __device__ __forceinline__ double shfl_d(double v, int src) { return __shfl(v, src, WAVE); }
 __device__ __forceinline__ int shfl_i(int v, int src) { return __shfl(v, src, WAVE); }
