@@ -53,15 +53,25 @@ __global__ void k_bin(View V, CellGrid G, int* count, const int* flagCur, const 
   else atomicOr(err, ERR_CELL_OVERFLOW);
 }
 
-// Host-driven rebuild of the flagged systems' rows (calcNeighborList / checkNeighbors).
-__global__ void k_build_rows(View V, Params P, CellGrid G, const int* count, const int* flagCur, int* updateCount,
-                             int countUpdates, int* err, int* maxcnt) {
+// Host-driven rebuild of the flagged systems' rows (calcNeighborList / checkNeighbors), one
+// workgroup per tile whose waves share the cell search (build_rows_tile), or, without LDS for rows
+// of width W (rowsLds = 0) or without cells, one lane per vertex (build_row).  Latency-bound: with
+// one lane per vertex throughout, a lane inserts its row entry by entry in memory.
+__global__ __launch_bounds__(WAVE* ROWS_WAVES) void k_build_rows(View V, Params P, CellGrid G, const int* count,
+                                                                 const int* flagCur, int* updateCount,
+                                                                 int countUpdates, int rowsLds, int* err, int* maxcnt) {
+  extern __shared__ int rows[];
+  const int w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
   Lane L;
-  if (!wave_tile_ctx(V, L)) return;
+  lane_ctx(V, blockIdx.x, threadIdx.x & (WAVE - 1), L);
   if (!flagCur[L.s]) return;
-  if (countUpdates && L.tile == V.stile[L.s] && L.lane == 0) updateCount[L.s] += 1;
-  if (!L.act) return;
-  build_row(V, P, G, count, G.slots, L.v, L.s, box_of(V, L.s), err, maxcnt);
+  if (countUpdates && L.tile == V.stile[L.s] && threadIdx.x == 0) updateCount[L.s] += 1;
+  const Box B = box_of(V, L.s);
+  if (rowsLds && !G.brute[L.s])
+    build_rows_tile(V, P, G, count, G.slots, L.lane, L.v, L.r, L.s, L.act, w, nw, B, V.x[L.v], V.y[L.v], rows, err,
+                    maxcnt);
+  else if (w == 0 && L.act)
+    build_row(V, P, G, count, G.slots, L.v, L.s, B, err, maxcnt);
 }
 
 // ------------------------------------------------------------ wide rings ---
@@ -892,19 +902,17 @@ hipError_t launch_bin_view(dpm_set_s* S, const View& Vn, int parity) {
 }
 
 hipError_t launch_build_rows(dpm_set_s* S, int countUpdates) {
-  const int b = S->cur;
-  k_build_rows<<<grid_w(S->V.ntiles), 256, 0, S->stream>>>(S->V, S->P, S->G, S->G.count[b], S->d_flag[b],
-                                                             S->d_updateCount, countUpdates, S->d_err,
-                                                             S->d_maxcnt);
-  return hipGetLastError();
+  return launch_build_rows_view(S, S->V, S->cur, countUpdates);
 }
 
 // k_build_rows on positions other than the set's current buffer (the list positions), with the
 // flags and cells of `parity`
 hipError_t launch_build_rows_view(dpm_set_s* S, const View& Vn, int parity, int countUpdates) {
-  k_build_rows<<<grid_w(S->V.ntiles), 256, 0, S->stream>>>(Vn, S->P, S->G, S->G.count[parity], S->d_flag[parity],
-                                                             S->d_updateCount, countUpdates, S->d_err,
-                                                             S->d_maxcnt);
+  const int rowsLds = Vn.W <= 64;
+  const size_t sh = rowsLds ? (size_t)(64 + 64 * Vn.W) * sizeof(int) : 0;
+  k_build_rows<<<Vn.ntiles, rowsLds ? WAVE * ROWS_WAVES : WAVE, sh, S->stream>>>(
+      Vn, S->P, S->G, S->G.count[parity], S->d_flag[parity], S->d_updateCount, countUpdates, rowsLds, S->d_err,
+      S->d_maxcnt);
   return hipGetLastError();
 }
 

@@ -20,8 +20,8 @@ __device__ __forceinline__ void cell_of(double x, double y, const Box& B, int nc
 
 // previous and second previous vertex of u in its ring (getPreviousId 233-243)
 __device__ __forceinline__ int2 prev_pair(const View& V, int u) {
-  const int ring = V.vring[u];
-  const int f = V.rfirst[ring], n = V.rnv[ring];
+  const int4 vi = V.vinfo[u];
+  const int f = vi.y, n = vi.z;
   const int p1 = (u == f) ? f + n - 1 : u - 1;
   const int p2 = (p1 == f) ? f + n - 1 : p1 - 1;
   return make_int2(p1, p2);
@@ -99,12 +99,15 @@ __device__ void build_row(const View& V, const Params& P, const CellGrid& G, con
 
 // The rows of a tile's vertices (lane = vertex, L.act lanes), built by all nw waves of its
 // workgroup: thread (w, lane) scans the cells w, w + nw, ... of the 3 x 3 block around its lane's
-// vertex and appends the hits to the lane's list in LDS (an LDS counter per lane, so the order
-// of arrival varies); after a barrier each lane of wave 0 sorts its list ascending, and all waves
-// write the sorted entries with their prev pairs into the ELL rows.  The same rows as build_row
-// from the same cells (its predicate, ascending order), with the dependent steps of an insertion
-// in LDS instead of memory.  Every thread of the workgroup calls it (it holds barriers); lds holds
+// vertex, four candidates at a time, and appends the hits to the lane's list in LDS (an LDS counter
+// per lane, so the order of arrival varies); after a barrier the waves share the entries of each
+// list, place every one by its rank (the number of smaller entries of the list) and write it with
+// its prev pair into the ELL row.  The same rows as build_row from the same cells (its predicate,
+// ascending order).  Every thread of the workgroup calls it (it holds barriers); lds holds
 // 64 + 64 W ints; the caller synchronises before reading the rows or reusing lds.
+//
+// Bound by latency: one candidate at a time costs two dependent loads each (its slot, then its
+// position), and sorting on one wave a chain of dependent LDS swaps.
 __device__ void build_rows_tile(const View& V, const Params& P, const CellGrid& G, const int* count,
                                 const int* slots, int lane, int v, int r, int s, bool act, int w, int nw,
                                 const Box& B, double x, double y, int* lds, int* err, int* maxcnt) {
@@ -119,18 +122,33 @@ __device__ void build_rows_tile(const View& V, const Params& P, const CellGrid& 
     int cx, cy;
     cell_of(x, y, B, ncx, ncy, cx, cy);
     for (int k = w; k < 9; k += nw) {
-      const int yy = (cy + k / 3 - 1 + ncy) % ncy;
-      const int xx = (cx + k % 3 - 1 + ncx) % ncx;
+      int yy = cy + k / 3 - 1, xx = cx + k % 3 - 1;
+      yy += yy < 0 ? ncy : (yy >= ncy ? -ncy : 0);
+      xx += xx < 0 ? ncx : (xx >= ncx ? -ncx : 0);
       const int cell = G.coff[s] + yy * ncx + xx;
       const int m = min(count[cell], G.cap);
-      for (int q = 0; q < m; q++) {
-        const int j = slots[(long)cell * G.cap + q];
-        if (V.vring[j] == r) continue;
-        const double dx = pbx(x - V.x[j], B), dy = pby(y - V.y[j], B);
-        const double d = sqrt(dx * dx + dy * dy);
-        if (-(1 - d / (rv + V.rad[j])) < P.cutDistance) {
-          const int idx = atomicAdd(&lcnt[lane], 1);
-          if (idx < W) lrow[idx * 64 + lane] = j;
+      const int* sl = slots + (long)cell * G.cap;
+      for (int q = 0; q < m; q += 4) {
+        int j[4], rj[4];
+        double xj[4], yj[4], radj[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) j[i] = sl[min(q + i, m - 1)];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          rj[i] = V.vring[j[i]];
+          xj[i] = V.x[j[i]];
+          yj[i] = V.y[j[i]];
+          radj[i] = V.rad[j[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          if (q + i >= m || rj[i] == r) continue;
+          const double dx = pbx(x - xj[i], B), dy = pby(y - yj[i], B);
+          const double d = sqrt(dx * dx + dy * dy);
+          if (-(1 - d / (rv + radj[i])) < P.cutDistance) {
+            const int idx = atomicAdd(&lcnt[lane], 1);
+            if (idx < W) lrow[idx * 64 + lane] = j[i];
+          }
         }
       }
     }
@@ -139,28 +157,19 @@ __device__ void build_rows_tile(const View& V, const Params& P, const CellGrid& 
   const int c = act ? lcnt[lane] : 0;
   const int n = c < W ? c : W;
   if (w == 0 && act) {
-    for (int a = 1; a < n; a++) {
-      const int key = lrow[a * 64 + lane];
-      int b = a - 1;
-      while (b >= 0 && lrow[b * 64 + lane] > key) {
-        lrow[(b + 1) * 64 + lane] = lrow[b * 64 + lane];
-        b--;
-      }
-      lrow[(b + 1) * 64 + lane] = key;
-    }
     if (c > W) atomicOr(err, ERR_LIST_OVERFLOW);
     atomicMax(maxcnt, c);
     V.ncnt[v] = n;
     V.lx[v] = x;
     V.ly[v] = y;
   }
-  __syncthreads();
-  if (act)
-    for (int k = w; k < n; k += nw) {
-      const int j = lrow[k * 64 + lane];
-      V.nbr[(long)k * V.nv + v] = j;
-      V.nbrp[(long)k * V.nv + v] = prev_pair(V, j);
-    }
+  for (int k = w; k < n; k += nw) {
+    const int j = lrow[k * 64 + lane];
+    int rank = 0;
+    for (int q = 0; q < n; q++) rank += lrow[q * 64 + lane] < j ? 1 : 0;
+    V.nbr[(long)rank * V.nv + v] = j;
+    V.nbrp[(long)rank * V.nv + v] = prev_pair(V, j);
+  }
 }
 
 // Bin vertex v at (x, y) of system s into a cell list (counts + slots of capacity G.cap);

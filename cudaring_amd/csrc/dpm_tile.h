@@ -8,6 +8,8 @@ namespace dpm {
 
 #define WAVE 64
 #define MAXSPLIT 8
+// waves per tile of the host-driven row build
+#define ROWS_WAVES 8
 // waves per workgroup of the two persistent FIRE builds
 #define FS_WAVES 8
 #define FS_WAVES_WIDE 16
