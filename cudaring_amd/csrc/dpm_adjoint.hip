@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "dpm_internal.h"
+#include "dpm_near.h"
 #include "dpm_rows.h"
 #include "dpm_tile.h"
 
@@ -212,8 +213,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_adj_hvp(View V, Params P, Ce
   if (A.flag) {
     const bool rebuild = A.flag[L.s] != 0;
     if (rebuild && A.rowsLdsW == V.W && !G.brute[L.s])  // the tile's waves share the cell search
-      build_rows_tile(V, P, G, A.count, G.slots, L.lane, L.v, L.r, L.s, L.act, w, nw, B, x, y, (int*)red, A.err,
-                      A.maxcnt);
+      build_rows_tile<-1>(V, P, G, A.count, G.slots, L, w, nw, B, x, y, (int*)red, A.err, A.maxcnt, NearRows{});
     else if (rebuild && w == 0 && L.act)
       build_row(V, P, G, A.count, G.slots, L.v, L.s, B, A.err, A.maxcnt);
     if (rebuild) __syncthreads();
@@ -542,11 +542,11 @@ hipError_t launch_adj_hvp(dpm_set_s* S, const View& Vn, AdjArgs A) {
   A.xcd = S->xcdMap;
   const unsigned g = (unsigned)S->V.ntiles, b = WAVE * S->split;
   hipStream_t st = S->stream;
-  // rows rebuilt by the whole workgroup need 64 + 64 W ints of LDS (launches of more than one
+  // rows rebuilt by the whole workgroup need rows_lds_ints of LDS (W <= 64), in the region the gather
   // wave, W <= 64), in the region the gather partials use afterwards
-  const bool tileRows = A.flag && S->split >= 2 && S->V.W <= 64;
+  const bool tileRows = A.flag && S->V.W <= 64;
   A.rowsLdsW = tileRows ? S->V.W : 0;
-  const size_t rows = tileRows ? (size_t)(64 + 64 * S->V.W) * sizeof(int) : 0;
+  const size_t rows = tileRows ? (size_t)rows_lds_ints(S->V.W, false) * sizeof(int) : 0;
   if (S->P.interaction == INT_SMOOTH) {
     const size_t sh = std::max((size_t)(S->split - 1) * 4 * WAVE * sizeof(double), rows);
     switch (S->P.potential) {

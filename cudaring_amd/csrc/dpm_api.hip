@@ -235,6 +235,24 @@ int configure_cells(dpm_set_s* S) {
   return DPM_OK;
 }
 
+// The near lists of the step loops (dpm_near.h): rings of at most 64 vertices, rows of at most 64
+// entries.  Without the memory for them the loops gather over whole rows.
+int alloc_near(dpm_set_s* S) {
+  hipFree(S->N.task);
+  S->N.task = nullptr;
+  if (S->nwide > 0 || S->V.W > 64) return DPM_OK;
+  const int cap = 64 * S->V.W;
+  if ((!S->N.tcnt && dalloc(&S->N.tcnt, S->V.ntiles) != hipSuccess) ||
+      (!S->N.span && dalloc(&S->N.span, 2 * S->nv) != hipSuccess) ||
+      dalloc(&S->N.task, 2L * cap * S->V.ntiles) != hipSuccess) {
+    S->N.task = nullptr;
+    (void)hipGetLastError();
+    return DPM_OK;
+  }
+  S->N.cap = cap;
+  return DPM_OK;
+}
+
 int alloc_list(dpm_set_s* S, int W) {
   HIPCHK(hipStreamSynchronize(S->stream));
   hipFree(S->V.nbr);
@@ -247,6 +265,8 @@ int alloc_list(dpm_set_s* S, int W) {
   HIPCHK(launch_fill_int((int*)S->V.nbrp, 0, 2L * W * S->nv, S->stream));
   HIPCHK(launch_fill_int(S->V.ncnt, 0, S->nv, S->stream));
   S->V.W = W;
+  int rc = alloc_near(S);
+  if (rc) return rc;
   S->listBuilt = false;
   bump(S);
   return DPM_OK;
@@ -473,8 +493,9 @@ int loop_step(dpm_set_s* S, int mode, int bumpT, double* recx = nullptr, double*
 // into the next cell list and clears the one after; no other step touches the cells, so the
 // loop needs no binning, in a launch of its own or in the step kernel.  Its draws use the call
 // indices ctr[k] + offset.
-StepArgs md_args(dpm_set_s* S, long r, long long offT, long long offA) {
+StepArgs md_args(dpm_set_s* S, long r, long long offT, long long offA, bool near) {
   StepArgs A = loop_args(S);
+  if (near) A.near = S->N;
   const int a = (int)(r % 3), b = (int)((r + 1) % 3), c = (int)((r + 2) % 3);
   A.flagCur = S->mdFlag[a];
   A.cellCur = S->mdCount[0];
@@ -489,6 +510,13 @@ StepArgs md_args(dpm_set_s* S, long r, long long offT, long long offA) {
   A.ctrOffT = offT;
   A.ctrOffA = offA;
   return A;
+}
+
+// Whether a loop of `steps` steps runs on near lists: building them costs its start kernel about what
+// they save in NEAR_STEPS steps.
+constexpr long NEAR_STEPS = 4;
+bool near_loop(const dpm_set_s* S, long steps) {
+  return S->N.task && steps >= NEAR_STEPS && (S->P.interaction == INT_VV || S->P.interaction == INT_SMOOTH);
 }
 
 // A step loop's cell protocol at its start: cell lists 0 and 1 cleared (the start kernel bins
@@ -512,7 +540,7 @@ long long active_draws(const dpm_set_s* S, long steps) { return S->P.particle !=
 // With `rec` (slots of 2 nv doubles, x then y), the position after step i is also written to
 // slot i + 1 (the adjoint's recomputed segment).
 int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullptr) {
-  const double h = 0.5 * S->P.dt;
+  const bool near = near_loop(S, steps);
   const long nv = S->nv;
   int rc = md_start(S);
   if (rc) return rc;
@@ -523,16 +551,16 @@ int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullp
     HIPCHK(launch_copy_d(S->V.lx, S->V.x, nv, S->stream));
     HIPCHK(launch_copy_d(S->V.ly, S->V.y, nv, S->stream));
   }
-  StepArgs A0 = md_args(S, 0, 0, 0);
+  StepArgs A0 = md_args(S, 0, 0, 0, near);
   A0.recx = rec ? rec + 2 * nv : nullptr;
   A0.recy = rec ? rec + 3 * nv : nullptr;
-  HIPCHK(launch_start_md(S, h, S->P.dt, A0));
+  HIPCHK(launch_start_md(S, A0));
   if (rec) HIPCHK(launch_fill_int(S->mdFlag[1], 1, S->nsys, S->stream));
   swap_pos(S);
   for (long i = 1; i <= steps; i++) {
     const bool more = i < steps;
-    const int mode = MODE_KICK | (langevin ? MODE_LANGEVIN : 0) | (more ? MODE_START : 0);
-    StepArgs A = md_args(S, i, i - 1, i - 1);
+    const int mode = MODE_KICK | (langevin ? MODE_LANGEVIN : 0) | (more ? MODE_START : 0) | (near ? MODE_NEAR : 0);
+    StepArgs A = md_args(S, i, i - 1, i - 1, near);
     if (rec && more) {
       A.recx = rec + (i + 1) * 2 * nv;
       A.recy = A.recx + nv;
@@ -548,14 +576,15 @@ int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullp
 // force, then per step [F(x'); v += dt/2 F; unless last: B A O A].  The O step of call k of the
 // loop draws at counter ctr[0] + k.
 int baoab_sequence(dpm_set_s* S, long steps) {
-  const double h = 0.5 * S->P.dt;
+  const bool near = near_loop(S, steps);
   int rc = md_start(S);
   if (rc) return rc;
-  HIPCHK(launch_start_baoab(S, h, md_args(S, 0, 0, 0)));
+  HIPCHK(launch_start_baoab(S, md_args(S, 0, 0, 0, near)));
   swap_pos(S);
   for (long i = 1; i <= steps; i++) {
     const bool more = i < steps;
-    HIPCHK(launch_step(S, MODE_KICK | MODE_BAOAB | (more ? MODE_START : 0), md_args(S, i, i, i - 1)));
+    HIPCHK(launch_step(S, MODE_KICK | MODE_BAOAB | (more ? MODE_START : 0) | (near ? MODE_NEAR : 0),
+                       md_args(S, i, i, i - 1, near)));
     if (more) swap_pos(S);
   }
   HIPCHK(launch_ctr_add(S, steps, active_draws(S, steps)));
@@ -571,10 +600,11 @@ int brown_sequence(dpm_set_s* S, long steps, bool noisy) {
   int rc = md_start(S);
   if (rc) return rc;
   HIPCHK(launch_fill_int(S->mdFlag[0], 0, S->nsys, S->stream));
-  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0]));
+  const bool near = near_loop(S, steps);
+  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   for (long i = 1; i <= steps; i++) {
-    const int mode = MODE_BROWN | MODE_START | (noisy ? MODE_LANGEVIN : 0);
-    StepArgs A = md_args(S, i - 1, i - 1, i - 1);
+    const int mode = MODE_BROWN | MODE_START | (noisy ? MODE_LANGEVIN : 0) | (near ? MODE_NEAR : 0);
+    StepArgs A = md_args(S, i - 1, i - 1, i - 1, near);
     HIPCHK(launch_step(S, mode, A));
     swap_pos(S);
   }
@@ -951,13 +981,14 @@ int rigid_clear(dpm_set_s* S) {
 int rigid_sequence(dpm_set_s* S, long steps, bool langevin) {
   int rc = md_start(S);
   if (rc) return rc;
-  HIPCHK(launch_rigid_start(S, langevin, md_args(S, 0, 0, 0)));
+  const bool near = near_loop(S, steps);
+  HIPCHK(launch_rigid_start(S, langevin, md_args(S, 0, 0, 0, near)));
   swap_pos(S);
   for (long i = 1; i <= steps; i++) {
     const bool more = i < steps;
-    StepArgs A = md_args(S, i, i - 1, 0);
+    StepArgs A = md_args(S, i, i - 1, 0, near);
     A.rigidLangevin = langevin ? 1 : 0;
-    HIPCHK(launch_step(S, MODE_RIGID | MODE_KICK | (more ? MODE_START : 0), A));
+    HIPCHK(launch_step(S, MODE_RIGID | MODE_KICK | (more ? MODE_START : 0) | (near ? MODE_NEAR : 0), A));
     if (more) swap_pos(S);
   }
   if (langevin) HIPCHK(launch_ctr_add(S, steps, 0));
@@ -990,16 +1021,17 @@ int rigid_fire_sequence(dpm_set_s* S, long iterations) {
   int rc = md_start(S);
   if (rc) return rc;
   HIPCHK(launch_fill_int(S->mdFlag[0], 0, S->nsys, S->stream));
-  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0]));
+  const bool near = near_loop(S, iterations);
+  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   HIPCHK(launch_rigid_fire_partials(S));
   for (long it = 0; it < iterations; it++) {
     HIPCHK(launch_rigid_fire_move(S, S->mdFlag[it % 3], S->d_any + 2));
     S->rfireCur = 1 - S->rfireCur;
     swap_pos(S);
-    StepArgs A = md_args(S, it, 0, 0);
+    StepArgs A = md_args(S, it, 0, 0, near);
     A.fire = S->d_rfire[S->rfireCur];
     A.part = S->d_part;
-    HIPCHK(launch_step(S, MODE_RIGID | MODE_FIRE, A));
+    HIPCHK(launch_step(S, MODE_RIGID | MODE_FIRE | (near ? MODE_NEAR : 0), A));
   }
   return DPM_OK;
 }
@@ -1198,7 +1230,7 @@ int dpm_destroy(dpm_set_t h) {
                   S->d_contacts, S->d_ccount, S->d_x0, S->d_obs, S->mdCount[0], S->mdSlots[0], S->mdFlag[0],
                   S->mdFlag[1], S->mdFlag[2], S->mdFlag[3], S->mdGen[0], S->mdGen[1], S->mdGen[2], S->R.pvx, S->R.pvy, S->R.pw, S->R.pfx, S->R.pfy, S->R.ptq, S->R.moi,
                   S->R.prad, S->R.plx, S->R.ply, S->R.pla, S->R.vtq, S->d_rfire[0], S->d_rfire[1], S->d_rg,
-                  S->d_snap, S->d_ftape, S->d_ftapeState, S->d_fadj, S->d_wide};
+                  S->d_snap, S->d_ftape, S->d_ftapeState, S->d_fadj, S->d_wide, S->N.task, S->N.tcnt, S->N.span};
   for (void* p : ptrs)
     if (p) hipFree(p);
   if (S->ownStream) hipStreamDestroy(S->ownStream);
@@ -2223,14 +2255,16 @@ int dpm_time_step_kernel(dpm_set_t h, long reps, double* avgUs, double* meanNeig
   // rebuild, and the drift writes into the other position buffer only
   HIPCHK(launch_fill_int(S->mdFlag[3], 0, S->nsys, S->stream));
   for (int r = 0; r < 3; r++) HIPCHK(launch_fill_int(S->mdGen[r], 0, S->nsys, S->stream));
+  const bool near = near_loop(S, NEAR_STEPS);
+  if (near) HIPCHK(launch_near(S));
   auto args = [&](long i) {
-    StepArgs A = md_args(S, i, 0, 0);
+    StepArgs A = md_args(S, i, 0, 0, near);
     A.flagCur = S->mdFlag[3];
     A.flagOut = S->d_flag[1 - S->cur];
     A.flagClear = nullptr;
     return A;
   };
-  const int mode = MODE_KICK | MODE_LANGEVIN | MODE_START;
+  const int mode = MODE_KICK | MODE_LANGEVIN | MODE_START | (near ? MODE_NEAR : 0);
   HIPCHK(launch_step(S, mode, args(0)));  // warm caches and code
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));

@@ -20,7 +20,8 @@ namespace dpm {
 // the per-system FIRE step when MODE_FIRE is)
 enum : int { MODE_FORCE = 0, MODE_KICK = 1, MODE_LANGEVIN = 2, MODE_START = 4, MODE_FIRE = 8, MODE_BAOAB = 16,
              MODE_BROWN = 32, MODE_RIGID = 64,
-             MODE_WIDE = 128 };  // the launch serves a set holding rings of more than 64 vertices
+             MODE_WIDE = 128,   // the launch serves a set holding rings of more than 64 vertices
+     MODE_NEAR = 256 };  // the gather evaluates the tiles' near lists (dpm_near.h) instead of whole rows
 
 // noise types, simControlStruct::noiseEnum order (include/DPM2D.h:27)
 enum : int { NOISE_LANGEVIN = 0, NOISE_BAOAB = 1, NOISE_BROWNIAN = 2, NOISE_DRIVEN_BROWNIAN = 3 };
@@ -60,6 +61,15 @@ struct CellGrid {
   int ncells, cap;
 };
 
+// Near lists of the tiles (dpm_near.h): per tile and role `cap` entries, their numbers per tile
+// (role 0, role 1), and per role and vertex the first entry | number << 16.
+struct NearRows {
+  int2* task;
+  int2* tcnt;
+  int* span;
+  int cap;
+};
+
 struct StepArgs {
   double h;                       // kick time step (0.5 dt)
   double dt;                      // drift time step
@@ -89,6 +99,7 @@ struct StepArgs {
   int xcd;                        // XCD-aware workgroup -> tile mapping
   int rowsBuilt;                  // inside loops: flagged rows already rebuilt (k_rows_loop)
   int rowsLdsW;                   // set by the launcher: list width the launch's LDS holds rows of
+  NearRows near;                  // step loops with near lists (MODE_NEAR); start kernels build them when task is set
 };
 
 // Up to kMaxCopySegs device-to-device copies in one launch (k_copy_segs): 4-byte words.
@@ -175,6 +186,7 @@ struct dpm_set_s {
   int* d_err = nullptr;
   int* d_maxcnt = nullptr;
   unsigned long long* d_ctr = nullptr;  // thermal, active
+  dpm::NearRows N{};                    // near lists of the step loops (null for wide sets and rows of over 64)
   bool listBuilt = false;
   bool cutSet = false;
 
@@ -249,9 +261,10 @@ namespace dpm {
 // launchers (dpm_kernels.hip); all return hipError_t of the last launch
 hipError_t launch_shape_only(dpm_set_s* S);
 hipError_t launch_step(dpm_set_s* S, int mode, const StepArgs& A);
-hipError_t launch_start_baoab(dpm_set_s* S, double h, const StepArgs& A);
-hipError_t launch_start_md(dpm_set_s* S, double h, double dt, const StepArgs& A);
-hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int* genOut);
+hipError_t launch_start_baoab(dpm_set_s* S, const StepArgs& A);
+hipError_t launch_start_md(dpm_set_s* S, const StepArgs& A);
+hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int* genOut, const NearRows& near);
+hipError_t launch_near(dpm_set_s* S);
 hipError_t launch_ctr_add(dpm_set_s* S, long long addT, long long addA);
 hipError_t launch_bin(dpm_set_s* S, int bumpThermal, int bumpActive);
 hipError_t launch_build_rows(dpm_set_s* S, int countUpdates);

@@ -22,6 +22,7 @@
 // launch before each step kernel.
 #include "dpm_forces.h"
 #include "dpm_launch.h"
+#include "dpm_near.h"
 
 namespace dpm {
 
@@ -68,8 +69,7 @@ __global__ __launch_bounds__(WAVE* ROWS_WAVES) void k_build_rows(View V, Params 
   if (countUpdates && L.tile == V.stile[L.s] && threadIdx.x == 0) updateCount[L.s] += 1;
   const Box B = box_of(V, L.s);
   if (rowsLds && !G.brute[L.s])
-    build_rows_tile(V, P, G, count, G.slots, L.lane, L.v, L.r, L.s, L.act, w, nw, B, V.x[L.v], V.y[L.v], rows, err,
-                    maxcnt);
+    build_rows_tile<-1>(V, P, G, count, G.slots, L, w, nw, B, V.x[L.v], V.y[L.v], rows, err, maxcnt, NearRows{});
   else if (w == 0 && L.act)
     build_row(V, P, G, count, G.slots, L.v, L.s, B, err, maxcnt);
 }
@@ -224,103 +224,96 @@ __device__ __forceinline__ void md_prologue(const View& V, const Params& P, cons
   }
 }
 
-// The step loop's first half step (velocity Verlet, or BAOAB's B A O A with the draw of call
-// ctr[0] + ctrOffT) from the stored force, with the loop's cell protocol (md_prologue on the
-// destination, whose flags go to A.flagOut; generation 0 into A.genOut; A.flagClear cleared)
-// (BAOAB::integrate, Simulator.cu:112-120, up to its force evaluation).
-template <bool BAOAB>
-__global__ void k_start_loop(View V, Params P, CellGrid G, double h, double dt, StepArgs A) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int t = v; t < V.nsys; t += gridDim.x * blockDim.x) {
-    A.flagClear[t] = 0;
-    A.genOut[t] = 0;
-  }
-  if (v >= V.nv) return;
-  const int s = V.vsys[v];
-  const Box B = box_of(V, s);
-  double vx = V.vx[v] + h * V.fx[v];
-  double vy = V.vy[v] + h * V.fy[v];
-  double xn, yn;
-  if constexpr (BAOAB) {
-    double z0, z1;
-    gauss_pair(P.seed, (uint32_t)s, TAG_THERMAL, A.ctr[0] + (unsigned long long)A.ctrOffT,
-               (uint32_t)(V.vring[v] - V.sroff[s]), z0, z1);
-    const double xa = V.x[v] + vx * h, ya = V.y[v] + vy * h;
-    vx = P.gamma * vx + P.noise * z0;
-    vy = P.gamma * vy + P.noise * z1;
-    xn = xa + vx * h;
-    yn = ya + vy * h;
-  } else {
-    xn = V.x[v] + dt * vx;
-    yn = V.y[v] + dt * vy;
-  }
-  V.vx[v] = vx;
-  V.vy[v] = vy;
-  A.xout[v] = xn;
-  A.yout[v] = yn;
-  if (A.recx) {
-    A.recx[v] = xn;
-    A.recy[v] = yn;
-  }
-  md_prologue(V, P, G, A, B, v, s, xn, yn, A.flagOut + s, A.anyOut);
-  far_test(P, B, xn - V.x[v], yn - V.y[v], A.flagOut + s);
-}
+// Start of a step loop, one workgroup per tile: wave 0 takes the loop's opening move, all waves
+// build the tile's near list from its rows at the list positions (when the loop uses them).
+//   START_VERLET, START_BAOAB: the first half step from the stored force (velocity Verlet, or
+//     BAOAB's B A O A with the draw of call ctr[0] + ctrOffT; BAOAB::integrate, Simulator.cu:112-120,
+//     up to its force evaluation) into A.xout;
+//   START_RIGID: the rigid loop's first half step from the stored ring force and torque (RigidNVE /
+//     RigidLangevin::integrate, Simulator.cu:241-252, 316-326, up to the vertex move), every lane
+//     moving its ring redundantly, the ring's first lane storing it;
+//   START_STAY: the overdamped loops and rigid FIRE, whose first step starts from the current positions;
+//   START_NEAR: the near lists only.
+// All but START_NEAR run the loop's cell protocol (md_prologue on the positions the first step
+// reads, whose flags go to A.flagOut; generation 0 into A.genOut; A.flagClear cleared).
+// Latency-bound.  The rigid start took one thread per ring, which moved its vertices one after another:
+// 48 us for 1,024 rings.
+enum : int { START_VERLET, START_BAOAB, START_RIGID, START_STAY, START_NEAR };
 
-// The rigid loop's first half step from the stored ring force and torque, one thread per ring
-// (RigidNVE / RigidLangevin::integrate, Simulator.cu:241-252, 316-326, up to the vertex move):
-// last centre and angle stored, half kick with the draw of call ctr[0] + ctrOffT, centre and
-// angle advanced, and each vertex moved into A.xout and tested into A.flagOut; in the step loop
-// (A.genCur) with its cell protocol (md_prologue, generation 0 into A.genOut), else A.cellOther
-// cleared; A.flagClear cleared when given.
-__global__ void k_rigid_start(View V, Params P, CellGrid G, StepArgs A) {
-  const Rigid R = *V.rg;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (A.cellOther)
-    for (int c = t; c < G.ncells; c += gridDim.x * blockDim.x) A.cellOther[c] = 0;
-  if (A.flagClear)
-    for (int q = t; q < V.nsys; q += gridDim.x * blockDim.x) A.flagClear[q] = 0;
-  if (A.genCur)
-    for (int q = t; q < V.nsys; q += gridDim.x * blockDim.x) A.genOut[q] = 0;
-  if (t >= V.np) return;
-  const int r = t, s = V.rsys[r];
+template <int KIND, int INTER>
+__global__ __launch_bounds__(WAVE* START_WAVES) void k_loop_start(View V, Params P, CellGrid G, StepArgs A) {
+  __shared__ unsigned long long mask[2 * WAVE];
+  const int w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
+  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+  Lane L;
+  lane_ctx(V, blockIdx.x, threadIdx.x & (WAVE - 1), L);
+  const int v = L.v, s = L.s;
   const Box B = box_of(V, s);
-  double vx = R.pvx[r], vy = R.pvy[r], w = R.pw[r];
-  double z0 = 0, z1 = 0;
-  if (A.rigidLangevin)
-    gauss_pair(P.seed, (uint32_t)s, TAG_THERMAL, A.ctr[0] + (unsigned long long)A.ctrOffT, (uint32_t)(r - V.sroff[s]),
-               z0, z1);
-  rigid_kick(A.rigidLangevin, A.h, P.gamma, R.pfx[r], R.pfy[r], R.ptq[r], z0, z1, vx, vy, w);
-  const double cx = V.cx[r], cy = V.cy[r], ang = V.ang[r];
-  const double ncx = cx + A.dt * vx, ncy = cy + A.dt * vy, nang = ang + A.dt * w;
-  const double dth = nang - ang, c = cos(dth), sn = sin(dth);
-  bool flag = false;
-  for (int v = V.rfirst[r]; v < V.rfirst[r] + V.rnv[r]; v++) {
-    const double x = V.x[v], y = V.y[v];
-    double xn, yn;
-    rigid_move(B, x, y, cx, cy, ncx, ncy, c, sn, xn, yn);
-    A.xout[v] = xn;
-    A.yout[v] = yn;
-    if (A.genCur) {
-      md_prologue(V, P, G, A, B, v, s, xn, yn, A.flagOut + s, nullptr);
-    } else {
-      const double ddx = pbx(xn - V.lx[v], B), ddy = pby(yn - V.ly[v], B);
-      flag = flag || 3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff;
+  if constexpr (KIND != START_NEAR) {
+    for (int t = gid; t < V.nsys; t += gridDim.x * blockDim.x) {
+      if (A.flagClear) A.flagClear[t] = 0;
+      A.genOut[t] = 0;
     }
-    far_test(P, B, xn - x, yn - y, A.flagOut + s);
   }
-  if (flag) {
-    atomicOr(&A.flagOut[s], 1);
-    atomicOr(A.anyOut, 1);
+  if (KIND != START_NEAR && w == 0 && L.act) {
+    const double x = V.x[v], y = V.y[v];
+    double xn = x, yn = y;
+    if constexpr (KIND == START_VERLET || KIND == START_BAOAB) {
+      double vx = V.vx[v] + A.h * V.fx[v];
+      double vy = V.vy[v] + A.h * V.fy[v];
+      if constexpr (KIND == START_BAOAB) {
+        double z0, z1;
+        gauss_pair(P.seed, (uint32_t)s, TAG_THERMAL, A.ctr[0] + (unsigned long long)A.ctrOffT,
+                   (uint32_t)(L.r - V.sroff[s]), z0, z1);
+        const double xa = x + vx * A.h, ya = y + vy * A.h;
+        vx = P.gamma * vx + P.noise * z0;
+        vy = P.gamma * vy + P.noise * z1;
+        xn = xa + vx * A.h;
+        yn = ya + vy * A.h;
+      } else {
+        xn = x + A.dt * vx;
+        yn = y + A.dt * vy;
+      }
+      V.vx[v] = vx;
+      V.vy[v] = vy;
+    }
+    if constexpr (KIND == START_RIGID) {
+      const Rigid R = *V.rg;
+      const int r = L.r;
+      double vx = R.pvx[r], vy = R.pvy[r], om = R.pw[r];
+      double z0 = 0, z1 = 0;
+      if (A.rigidLangevin)
+        gauss_pair(P.seed, (uint32_t)s, TAG_THERMAL, A.ctr[0] + (unsigned long long)A.ctrOffT,
+                   (uint32_t)(r - V.sroff[s]), z0, z1);
+      rigid_kick(A.rigidLangevin, A.h, P.gamma, R.pfx[r], R.pfy[r], R.ptq[r], z0, z1, vx, vy, om);
+      const double cx = V.cx[r], cy = V.cy[r], ang = V.ang[r];
+      const double ncx = cx + A.dt * vx, ncy = cy + A.dt * vy, nang = ang + A.dt * om;
+      const double dth = nang - ang;
+      rigid_move(B, x, y, cx, cy, ncx, ncy, cos(dth), sin(dth), xn, yn);
+      if (L.lane == L.segS) {  // every lane of the ring has read the old state
+        R.plx[r] = cx;
+        R.ply[r] = cy;
+        R.pla[r] = ang;
+        R.pvx[r] = vx;
+        R.pvy[r] = vy;
+        R.pw[r] = om;
+        V.ang[r] = nang;
+        V.cx[r] = ncx;
+        V.cy[r] = ncy;
+      }
+    }
+    if constexpr (KIND != START_STAY) {
+      A.xout[v] = xn;
+      A.yout[v] = yn;
+      if (A.recx) {
+        A.recx[v] = xn;
+        A.recy[v] = yn;
+      }
+      far_test(P, B, xn - x, yn - y, A.flagOut + s);
+    }
+    md_prologue(V, P, G, A, B, v, s, xn, yn, A.flagOut + s, A.anyOut);
   }
-  R.plx[r] = cx;
-  R.ply[r] = cy;
-  R.pla[r] = ang;
-  R.pvx[r] = vx;
-  R.pvy[r] = vy;
-  R.pw[r] = w;
-  V.ang[r] = nang;
-  V.cx[r] = ncx;
-  V.cy[r] = ncy;
+  if (A.near.task) build_near_tile<INTER>(V, P, A.near, L, w, nw, B, V.lx, V.ly, G.brute[s] != 0, mask);
 }
 
 // RigidLangevin::injectKineticEnergy (Simulator.cu:254-261), one workgroup per system: a
@@ -359,16 +352,6 @@ __global__ __launch_bounds__(256) void k_rigid_inject(View V, Params P, double a
     R.pvx[r] -= mx;
     R.pvy[r] -= my;
   }
-}
-
-// The overdamped loops' prologue: md_prologue on the current positions (their first step
-// rebuilds when flagged), flags into `flag`, generation 0 into `genOut`.
-__global__ void k_bin_flag(View V, Params P, CellGrid G, StepArgs A, int* flag) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < V.nsys) A.genOut[v] = 0;
-  if (v >= V.nv) return;
-  const int s = V.vsys[v];
-  md_prologue(V, P, G, A, box_of(V, s), v, s, V.x[v], V.y[v], flag + s, nullptr);
 }
 
 // RNG call counters advanced by the draws of a finished loop
@@ -824,10 +807,10 @@ hipError_t launch_step(dpm_set_s* S, int mode, const StepArgs& A0) {
 static hipError_t launch_step_kernel(dpm_set_s* S, int mode, const StepArgs& A0) {
   // refuse argument sets the chosen epilogue would dereference as null
   if (!A0.ctr) return hipErrorInvalidValue;
-  // in-loop rebuilds by the whole workgroup need LDS for the tile's rows: 64 + 64 W ints, in the
-  // region the gather partials use afterwards (launches of more than one wave, W <= 64)
+  // in-loop rebuilds by the whole workgroup need LDS for the tile's rows (rows_lds_ints), in the
+  // region the gather's results use afterwards (W <= 64)
   StepArgs A = A0;
-  A.rowsLdsW = (A.manage && S->split >= 2 && S->V.W <= 64) ? S->V.W : 0;
+  A.rowsLdsW = (A.manage && S->V.W <= 64) ? S->V.W : 0;
   if (S->P.particle == PART_ACTIVE_SHAPE && !S->V.l0r) return hipErrorInvalidValue;
   if ((mode & MODE_FIRE) && (!A.fire || !A.part)) return hipErrorInvalidValue;
   if ((mode & MODE_RIGID) && S->P.interaction == INT_ALL) return hipErrorInvalidValue;
@@ -853,29 +836,43 @@ hipError_t launch_shape_only(dpm_set_s* S) {
   return hipGetLastError();
 }
 
-hipError_t launch_start_baoab(dpm_set_s* S, double h, const StepArgs& A) {
-  if (!A.genOut || !A.flagClear || !A.flagOut || !A.anyOut || !A.cellCur || !A.slotsCur || !A.ctr)
+template <int KIND>
+static hipError_t loop_start(dpm_set_s* S, const StepArgs& A) {
+  if (KIND != START_NEAR && (!A.genOut || !A.flagOut || !A.anyOut || !A.cellCur || !A.slotsCur || !A.ctr))
     return hipErrorInvalidValue;
-  k_start_loop<true><<<grid_v(S->nv > S->G.ncells ? S->nv : S->G.ncells), 256, 0, S->stream>>>(S->V, S->P, S->G, h,
-                                                                                           S->P.dt, A);
+  if (KIND != START_NEAR && KIND != START_STAY && (!A.xout || !A.yout || !A.flagClear)) return hipErrorInvalidValue;
+  const int threads = WAVE * (A.near.task ? START_WAVES : 1);
+  if (S->P.interaction == INT_SMOOTH)
+    k_loop_start<KIND, INT_SMOOTH><<<S->V.ntiles, threads, 0, S->stream>>>(S->V, S->P, S->G, A);
+  else
+    k_loop_start<KIND, INT_VV><<<S->V.ntiles, threads, 0, S->stream>>>(S->V, S->P, S->G, A);
   return hipGetLastError();
 }
 
-hipError_t launch_start_md(dpm_set_s* S, double h, double dt, const StepArgs& A) {
-  if (!A.genOut || !A.flagClear || !A.flagOut || !A.anyOut || !A.cellCur || !A.slotsCur) return hipErrorInvalidValue;
-  k_start_loop<false><<<grid_v(S->nv > S->G.ncells ? S->nv : S->G.ncells), 256, 0, S->stream>>>(S->V, S->P, S->G, h,
-                                                                                            dt, A);
-  return hipGetLastError();
-}
+hipError_t launch_start_baoab(dpm_set_s* S, const StepArgs& A) { return loop_start<START_BAOAB>(S, A); }
 
-hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int* genOut) {
+hipError_t launch_start_md(dpm_set_s* S, const StepArgs& A) { return loop_start<START_VERLET>(S, A); }
+
+// the overdamped and rigid FIRE loops' start: flags of the current positions into `flag`, generation
+// 0 into `genOut`
+hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int* genOut, const NearRows& near) {
   StepArgs A{};
+  A.ctr = S->d_ctr;
   A.cellCur = count;
   A.slotsCur = slots;
+  A.flagOut = flag;
+  A.anyOut = S->d_any + 2;  // not read by the loop
   A.genOut = genOut;
   A.err = S->d_err;
-  k_bin_flag<<<grid_v(S->nv > S->nsys ? S->nv : S->nsys), 256, 0, S->stream>>>(S->V, S->P, S->G, A, flag);
-  return hipGetLastError();
+  A.near = near;
+  return loop_start<START_STAY>(S, A);
+}
+
+// the near lists at the list positions
+hipError_t launch_near(dpm_set_s* S) {
+  StepArgs A{};
+  A.near = S->N;
+  return loop_start<START_NEAR>(S, A);
 }
 
 hipError_t launch_ctr_add(dpm_set_s* S, long long addT, long long addA) {
@@ -909,7 +906,7 @@ hipError_t launch_build_rows(dpm_set_s* S, int countUpdates) {
 // flags and cells of `parity`
 hipError_t launch_build_rows_view(dpm_set_s* S, const View& Vn, int parity, int countUpdates) {
   const int rowsLds = Vn.W <= 64;
-  const size_t sh = rowsLds ? (size_t)(64 + 64 * Vn.W) * sizeof(int) : 0;
+  const size_t sh = rowsLds ? (size_t)rows_lds_ints(Vn.W, false) * sizeof(int) : 0;
   k_build_rows<<<Vn.ntiles, rowsLds ? WAVE * ROWS_WAVES : WAVE, sh, S->stream>>>(
       Vn, S->P, S->G, S->G.count[parity], S->d_flag[parity], S->d_updateCount, countUpdates, rowsLds, S->d_err,
       S->d_maxcnt);
@@ -970,15 +967,9 @@ hipError_t launch_scale_box(dpm_set_s* S) {
 }
 
 hipError_t launch_rigid_start(dpm_set_s* S, bool langevin, const StepArgs& A) {
-  if (!A.ctr || (A.genCur && (!A.genOut || !A.cellCur || !A.slotsCur)) || (!A.genCur && !A.cellOther) ||
-      !A.flagOut || !A.anyOut || !A.xout || !A.yout)
-    return hipErrorInvalidValue;
   StepArgs B = A;
   B.rigidLangevin = langevin ? 1 : 0;
-  long n = S->np > S->G.ncells ? S->np : S->G.ncells;
-  if (n < S->nsys) n = S->nsys;
-  k_rigid_start<<<grid_v(n), 256, 0, S->stream>>>(S->V, S->P, S->G, B);
-  return hipGetLastError();
+  return loop_start<START_RIGID>(S, B);
 }
 
 hipError_t launch_rigid_inject(dpm_set_s* S, double amplitude, unsigned long long call) {

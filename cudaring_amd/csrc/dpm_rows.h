@@ -97,81 +97,6 @@ __device__ void build_row(const View& V, const Params& P, const CellGrid& G, con
   V.ly[v] = y;
 }
 
-// The rows of a tile's vertices (lane = vertex, L.act lanes), built by all nw waves of its
-// workgroup: thread (w, lane) scans the cells w, w + nw, ... of the 3 x 3 block around its lane's
-// vertex, four candidates at a time, and appends the hits to the lane's list in LDS (an LDS counter
-// per lane, so the order of arrival varies); after a barrier the waves share the entries of each
-// list, place every one by its rank (the number of smaller entries of the list) and write it with
-// its prev pair into the ELL row.  The same rows as build_row from the same cells (its predicate,
-// ascending order).  Every thread of the workgroup calls it (it holds barriers); lds holds
-// 64 + 64 W ints; the caller synchronises before reading the rows or reusing lds.
-//
-// Bound by latency: one candidate at a time costs two dependent loads each (its slot, then its
-// position), and sorting on one wave a chain of dependent LDS swaps.
-__device__ void build_rows_tile(const View& V, const Params& P, const CellGrid& G, const int* count,
-                                const int* slots, int lane, int v, int r, int s, bool act, int w, int nw,
-                                const Box& B, double x, double y, int* lds, int* err, int* maxcnt) {
-  int* lcnt = lds;
-  int* lrow = lds + 64;
-  const int W = V.W;
-  if (w == 0) lcnt[lane] = 0;
-  __syncthreads();
-  if (act) {
-    const double rv = V.rad[v];
-    const int ncx = G.ncx[s], ncy = G.ncy[s];
-    int cx, cy;
-    cell_of(x, y, B, ncx, ncy, cx, cy);
-    for (int k = w; k < 9; k += nw) {
-      int yy = cy + k / 3 - 1, xx = cx + k % 3 - 1;
-      yy += yy < 0 ? ncy : (yy >= ncy ? -ncy : 0);
-      xx += xx < 0 ? ncx : (xx >= ncx ? -ncx : 0);
-      const int cell = G.coff[s] + yy * ncx + xx;
-      const int m = min(count[cell], G.cap);
-      const int* sl = slots + (long)cell * G.cap;
-      for (int q = 0; q < m; q += 4) {
-        int j[4], rj[4];
-        double xj[4], yj[4], radj[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) j[i] = sl[min(q + i, m - 1)];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          rj[i] = V.vring[j[i]];
-          xj[i] = V.x[j[i]];
-          yj[i] = V.y[j[i]];
-          radj[i] = V.rad[j[i]];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          if (q + i >= m || rj[i] == r) continue;
-          const double dx = pbx(x - xj[i], B), dy = pby(y - yj[i], B);
-          const double d = sqrt(dx * dx + dy * dy);
-          if (-(1 - d / (rv + radj[i])) < P.cutDistance) {
-            const int idx = atomicAdd(&lcnt[lane], 1);
-            if (idx < W) lrow[idx * 64 + lane] = j[i];
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();
-  const int c = act ? lcnt[lane] : 0;
-  const int n = c < W ? c : W;
-  if (w == 0 && act) {
-    if (c > W) atomicOr(err, ERR_LIST_OVERFLOW);
-    atomicMax(maxcnt, c);
-    V.ncnt[v] = n;
-    V.lx[v] = x;
-    V.ly[v] = y;
-  }
-  for (int k = w; k < n; k += nw) {
-    const int j = lrow[k * 64 + lane];
-    int rank = 0;
-    for (int q = 0; q < n; q++) rank += lrow[q * 64 + lane] < j ? 1 : 0;
-    V.nbr[(long)rank * V.nv + v] = j;
-    V.nbrp[(long)rank * V.nv + v] = prev_pair(V, j);
-  }
-}
-
 // Bin vertex v at (x, y) of system s into a cell list (counts + slots of capacity G.cap);
 // systems searched by brute force have no cells.
 __device__ __forceinline__ void bin_vertex(const CellGrid& G, const Box& B, int* count, int* slots, int v, int s,

@@ -2,6 +2,7 @@
 // STEP_POT select the instance, whose launcher is a specialisation of step_launch.
 #include "dpm_forces.h"
 #include "dpm_launch.h"
+#include "dpm_near.h"
 
 namespace dpm {
 
@@ -13,7 +14,8 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   const int nw = blockDim.x / WAVE;
   Lane L;
   constexpr bool WIDE = (MODE & MODE_WIDE) != 0;
-  constexpr int MB = MODE & ~MODE_WIDE;  // the integrator mode
+  constexpr bool NEAR = (MODE & MODE_NEAR) != 0;
+  constexpr int MB = MODE & ~(MODE_WIDE | MODE_NEAR);  // the integrator mode
   // A step of a velocity-Verlet, Langevin or BAOAB loop other than its last consumes the force it
   // computes in this launch (the closing and next opening half kicks); its force, energies, ring
   // geometry and wall forces are stored by the loop's last step only.
@@ -64,12 +66,17 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
     // the cell search shared by the tile's waves (rows in LDS) where the launch sized LDS for it
     const bool tileBuild = rebuild && !A.rowsBuilt && !allPairs && A.rowsLdsW == V.W && !G.brute[L.s];
     if (tileBuild) {
-      build_rows_tile(V, P, G, cells, slots, L.lane, L.v, L.r, L.s, L.act, w, nw, B, x, y, (int*)red, A.err,
-                      A.maxcnt);
+      build_rows_tile<NEAR ? INTER : -1>(V, P, G, cells, slots, L, w, nw, B, x, y, (int*)red, A.err, A.maxcnt, A.near);
     } else if (rebuild && w == 0 && L.act && !A.rowsBuilt) {
       build_row(V, P, G, cells, slots, L.v, L.s, B, A.err, A.maxcnt, allPairs);
     }
     if (rebuild) __syncthreads();
+    if constexpr (NEAR) {
+      if (rebuild && !tileBuild) {
+        build_near_tile<INTER>(V, P, A.near, L, w, nw, B, V.x, V.y, G.brute[L.s] != 0, red);
+        __syncthreads();
+      }
+    }
   }
   // wave 0's epilogue operands, fetched before the force work (lastPos after the rebuild above)
   double vx = 0, vy = 0, lx = 0, ly = 0;
@@ -90,20 +97,31 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   const int ng = nw - g0;
   // partials per gather wave: six, eight when the tile is a slice of a wide ring
   constexpr int nq = (INTER == INT_SMOOTH && WIDE) ? 8 : 6;
-  if (w >= g0) gather_pairs<INTER, POT>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
-  if (nw > 1 && w > 0) {
-    double* r = red + (w - 1) * nq * WAVE + L.lane;
-    r[0 * WAVE] = fx;
-    r[1 * WAVE] = fy;
-    if constexpr (STORE) {  // energies are outputs only: a step that stores none leaves them out
-      r[2 * WAVE] = e;
-      r[3 * WAVE] = es;
+  int2 cnt = make_int2(0, 0);
+  int spanT = 0, spanO = 0;
+  if constexpr (NEAR) {
+    cnt = A.near.tcnt[L.tile];
+    if (w == 0 && L.act) {
+      spanT = A.near.span[L.v];
+      if constexpr (INTER == INT_SMOOTH) spanO = A.near.span[V.nv + L.v];
     }
-    r[4 * WAVE] = qx;
-    r[5 * WAVE] = qy;
-    if (nq == 8) {
-      r[6 * WAVE] = qnx;
-      r[7 * WAVE] = qny;
+    if (w >= g0) eval_near<INTER, POT, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, 0, L.lane, w - g0, ng, red);
+  } else {
+    if (w >= g0) gather_pairs<INTER, POT>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
+    if (nw > 1 && w > 0) {
+      double* r = red + (w - 1) * nq * WAVE + L.lane;
+      r[0 * WAVE] = fx;
+      r[1 * WAVE] = fy;
+      if constexpr (STORE) {  // energies are outputs only: a step that stores none leaves them out
+        r[2 * WAVE] = e;
+        r[3 * WAVE] = es;
+      }
+      r[4 * WAVE] = qx;
+      r[5 * WAVE] = qy;
+      if (nq == 8) {
+        r[6 * WAVE] = qnx;
+        r[7 * WAVE] = qny;
+      }
     }
   }
 
@@ -151,7 +169,19 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       if (L.act && L.lane == L.segS) V.ang[L.r] = ang;
     }
   }
-  if (nw > 1) {
+  if constexpr (NEAR) {
+    // windows of NEAR_WIN evaluations per role (one, unless the tile is unusually crowded)
+    const int most = max(cnt.x, cnt.y);
+    for (int base = 0;;) {
+      __syncthreads();
+      if (w == 0) sum_near<INTER, STORE>(spanT, spanO, base, red, fx, fy, INTER == INT_SMOOTH ? es : e, qx, qy);
+      base += NEAR_WIN;
+      if (base >= most) break;
+      __syncthreads();
+      if (w >= g0) eval_near<INTER, POT, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, base, L.lane, w - g0, ng, red);
+    }
+    if (w > 0) return;
+  } else if (nw > 1) {
     __syncthreads();
     if (w > 0) return;
     for (int q = 1; q < nw; q++) {
@@ -280,82 +310,82 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
 }
 
 // LDS of the step kernel: six partials per lane of each gather wave (eight with wide rings)
+// (or the results of the near list's evaluations), and in the same region the rows under construction
+template <int INTER, int MODE>
 static inline size_t step_lds(const dpm_set_s* S) {
-  const size_t red = (size_t)(S->split - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
-  const size_t rows = (S->split >= 2 && S->V.W <= 64) ? (size_t)(64 + 64 * S->V.W) * sizeof(int) : 0;
+  constexpr bool STORE = (MODE & MODE_START) == 0 || (MODE & (MODE_BROWN | MODE_RIGID)) != 0;
+  const size_t red = (MODE & MODE_NEAR) ? (size_t)near_slots_bytes<INTER, STORE>()
+                                        : (size_t)(S->split - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
+  const size_t rows = S->V.W <= 64 ? (size_t)rows_lds_ints(S->V.W, (MODE & MODE_NEAR) != 0) * sizeof(int) : 0;
   return red > rows ? red : rows;
+}
+
+template <int INTER, int POT, int MODE>
+static hipError_t step_one(dpm_set_s* S, const StepArgs& A) {
+  k_step<INTER, POT, MODE>
+      <<<S->V.ntiles, WAVE * S->split, step_lds<INTER, MODE>(S), S->stream>>>(S->V, S->P, A, S->G);
+  return hipGetLastError();
 }
 
 // rigid-ring modes (sets of rings of at most 64 vertices only)
 template <int INTER, int POT>
 static hipError_t step_rigid(dpm_set_s* S, int mode, const StepArgs& A) {
-  const int g = S->V.ntiles;
-  const int b = WAVE * S->split;
-  const size_t sh = step_lds(S);
-  hipStream_t st = S->stream;
   switch (mode) {
-    case MODE_RIGID: k_step<INTER, POT, MODE_RIGID><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_RIGID | MODE_KICK:
-      k_step<INTER, POT, MODE_RIGID | MODE_KICK><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_RIGID | MODE_KICK | MODE_START:
-      k_step<INTER, POT, MODE_RIGID | MODE_KICK | MODE_START><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_RIGID | MODE_FIRE:
-      k_step<INTER, POT, MODE_RIGID | MODE_FIRE><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    default: return hipErrorInvalidValue;
+    case MODE_RIGID: return step_one<INTER, POT, MODE_RIGID>(S, A);
+    case MODE_RIGID | MODE_KICK: return step_one<INTER, POT, MODE_RIGID | MODE_KICK>(S, A);
+    case MODE_RIGID | MODE_KICK | MODE_START: return step_one<INTER, POT, MODE_RIGID | MODE_KICK | MODE_START>(S, A);
+    case MODE_RIGID | MODE_FIRE: return step_one<INTER, POT, MODE_RIGID | MODE_FIRE>(S, A);
+    case MODE_RIGID | MODE_KICK | MODE_NEAR: return step_one<INTER, POT, MODE_RIGID | MODE_KICK | MODE_NEAR>(S, A);
+    case MODE_RIGID | MODE_KICK | MODE_START | MODE_NEAR:
+      return step_one<INTER, POT, MODE_RIGID | MODE_KICK | MODE_START | MODE_NEAR>(S, A);
+    case MODE_RIGID | MODE_FIRE | MODE_NEAR: return step_one<INTER, POT, MODE_RIGID | MODE_FIRE | MODE_NEAR>(S, A);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
-template <int INTER, int POT, int WB>
-static hipError_t step_mode(dpm_set_s* S, int mode, const StepArgs& A) {
-  if constexpr (WB != 0) {
-    if (mode & MODE_RIGID) return hipErrorInvalidValue;  // refused for wide sets before this point
-  } else {
-    if (mode & MODE_RIGID) return step_rigid<INTER, POT>(S, mode, A);
-  }
-  const int g = S->V.ntiles;
-  const int b = WAVE * S->split;
-  const size_t sh = step_lds(S);
-  hipStream_t st = S->stream;
+// the loop modes, on whole rows (XB: 0 or MODE_WIDE) or on the near lists (XB: MODE_NEAR)
+template <int INTER, int POT, int XB>
+static hipError_t step_loop_mode(dpm_set_s* S, int mode, const StepArgs& A) {
   switch (mode) {
-    case MODE_FORCE: k_step<INTER, POT, MODE_FORCE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_KICK: k_step<INTER, POT, MODE_KICK | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_KICK | MODE_LANGEVIN:
-      k_step<INTER, POT, MODE_KICK | MODE_LANGEVIN | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_KICK | MODE_START:
-      k_step<INTER, POT, MODE_KICK | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
+    case MODE_KICK: return step_one<INTER, POT, MODE_KICK | XB>(S, A);
+    case MODE_KICK | MODE_LANGEVIN: return step_one<INTER, POT, MODE_KICK | MODE_LANGEVIN | XB>(S, A);
+    case MODE_KICK | MODE_START: return step_one<INTER, POT, MODE_KICK | MODE_START | XB>(S, A);
     case MODE_KICK | MODE_LANGEVIN | MODE_START:
-      k_step<INTER, POT, MODE_KICK | MODE_LANGEVIN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_FIRE: k_step<INTER, POT, MODE_FIRE | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G); break;
-    case MODE_KICK | MODE_BAOAB:
-      k_step<INTER, POT, MODE_KICK | MODE_BAOAB | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
+      return step_one<INTER, POT, MODE_KICK | MODE_LANGEVIN | MODE_START | XB>(S, A);
+    case MODE_KICK | MODE_BAOAB: return step_one<INTER, POT, MODE_KICK | MODE_BAOAB | XB>(S, A);
     case MODE_KICK | MODE_BAOAB | MODE_START:
-      k_step<INTER, POT, MODE_KICK | MODE_BAOAB | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    case MODE_BROWN | MODE_START:
-      k_step<INTER, POT, MODE_BROWN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
+      return step_one<INTER, POT, MODE_KICK | MODE_BAOAB | MODE_START | XB>(S, A);
+    case MODE_BROWN | MODE_START: return step_one<INTER, POT, MODE_BROWN | MODE_START | XB>(S, A);
     case MODE_BROWN | MODE_LANGEVIN | MODE_START:
-      k_step<INTER, POT, MODE_BROWN | MODE_LANGEVIN | MODE_START | WB><<<g, b, sh, st>>>(S->V, S->P, A, S->G);
-      break;
-    default: return hipErrorInvalidValue;
+      return step_one<INTER, POT, MODE_BROWN | MODE_LANGEVIN | MODE_START | XB>(S, A);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
+}
+
+template <int INTER, int POT>
+static hipError_t step_mode(dpm_set_s* S, int mode, const StepArgs& A) {
+  if (S->nwide > 0) {
+    if (mode & (MODE_RIGID | MODE_NEAR)) return hipErrorInvalidValue;  // refused for wide sets before this point
+    switch (mode) {
+      case MODE_FORCE: return step_one<INTER, POT, MODE_FORCE | MODE_WIDE>(S, A);
+      case MODE_FIRE: return step_one<INTER, POT, MODE_FIRE | MODE_WIDE>(S, A);
+    }
+    return step_loop_mode<INTER, POT, MODE_WIDE>(S, mode, A);
+  }
+  if (mode & MODE_RIGID) return step_rigid<INTER, POT>(S, mode, A);
+  if (mode & MODE_NEAR) return step_loop_mode<INTER, POT, MODE_NEAR>(S, mode & ~MODE_NEAR, A);
+  switch (mode) {
+    case MODE_FORCE: return step_one<INTER, POT, MODE_FORCE>(S, A);
+    case MODE_FIRE: return step_one<INTER, POT, MODE_FIRE>(S, A);
+  }
+  return step_loop_mode<INTER, POT, 0>(S, mode, A);
 }
 
 // all-pairs interaction (test mode): forces only
 template <int POT, int WB>
 static hipError_t step_all(dpm_set_s* S, int mode, const StepArgs& A) {
   if (mode != MODE_FORCE) return hipErrorInvalidValue;
-  k_step<INT_ALL, POT, MODE_FORCE | WB><<<S->V.ntiles, WAVE * S->split, step_lds(S), S->stream>>>(S->V, S->P, A, S->G);
-  return hipGetLastError();
+  return step_one<INT_ALL, POT, MODE_FORCE | WB>(S, A);
 }
 
 #if !defined(STEP_INTER) || !defined(STEP_POT)
@@ -366,8 +396,7 @@ hipError_t step_launch<STEP_INTER, STEP_POT>(dpm_set_s* S, int mode, const StepA
 #if STEP_INTER == 3
   return S->nwide > 0 ? step_all<STEP_POT, MODE_WIDE>(S, mode, A) : step_all<STEP_POT, 0>(S, mode, A);
 #else
-  return S->nwide > 0 ? step_mode<STEP_INTER, STEP_POT, MODE_WIDE>(S, mode, A)
-                      : step_mode<STEP_INTER, STEP_POT, 0>(S, mode, A);
+  return step_mode<STEP_INTER, STEP_POT>(S, mode, A);
 #endif
 }
 

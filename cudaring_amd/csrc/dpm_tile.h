@@ -10,6 +10,8 @@ namespace dpm {
 #define MAXSPLIT 8
 // waves per tile of the host-driven row build
 #define ROWS_WAVES 8
+// waves per tile of the loops' start kernel when it builds near lists
+#define START_WAVES 4
 // waves per workgroup of the two persistent FIRE builds
 #define FS_WAVES 8
 #define FS_WAVES_WIDE 16
