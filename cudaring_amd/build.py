@@ -4,6 +4,7 @@ Every HIP translation unit is compiled with:
   --offload-arch=gfx950            the MI355X ISA only
   -ffp-contract=off                no FMA contraction, so the kernels evaluate the
                                    same expression order as the host restatement
+                                   (functions that contract say so themselves)
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                    no packed FP32 instructions
 """

@@ -80,6 +80,33 @@ struct Box {
   double mx, my;  // image multipliers: 1/L along a periodic direction, 0 along a walled one
 };
 
+// ---------------------------------------------------------- reciprocals ---
+// 1 / x and 1 / sqrt(x) from the hardware's estimate (about 2^-24) and one third-order Newton step:
+// three and five operations, within an ulp or two, where the IEEE division takes eleven and the
+// square root and its reciprocal together over twenty-five.  The kernels' time is the length of
+// their instruction streams (fetched anew by every launch) as much as the arithmetic.
+__device__ __forceinline__ double recip(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, y, 1.0);
+  return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+__device__ __forceinline__ double rsqrt_n(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+
+// sqrt(x) from y = 1 / sqrt(x), and a / b from r near 1 / b: one remainder step, exact by FMA, rounds
+// both as the IEEE operations do (but for cases closer to a tie than r and y are to exact)
+__device__ __forceinline__ double sqrt_from(double x, double y) {
+  const double s = x * y;
+  return __builtin_fma(0.5 * y, __builtin_fma(-s, s, x), s);
+}
+__device__ __forceinline__ double div_from(double a, double b, double r) {
+  const double q = a * r;
+  return __builtin_fma(r, __builtin_fma(-q, b, a), q);
+}
+
 // ------------------------------------------------------------ geometry ---
 // pbcDistance, cudaKernel.cuh:70-74 (round = half away from zero)
 __device__ __forceinline__ double pbc(double delta, double size) {
@@ -115,10 +142,10 @@ __device__ __forceinline__ void gauss_pair(uint64_t seed, uint32_t sys, uint32_t
   philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
   double uA = u01(c[0], c[1]);
   double uB = u01(c[2], c[3]);
-  double r = sqrt(-2.0 * log(uA));
-  double a = 2.0 * kPI * uB;
-  z0 = r * cos(a);
-  z1 = r * sin(a);
+  double r = sqrt(-2.0 * log(uA)), s, c2;
+  sincospi(2.0 * uB, &s, &c2);
+  z0 = r * c2;
+  z1 = r * s;
 }
 
 // ---------------------------------------------------------- pair terms ---
@@ -427,6 +454,162 @@ __device__ __forceinline__ double smooth_pair_op(const Params& P, const Box& B, 
     }
   }
   return energy;
+}
+
+// ------------------------------------------------------- the loops' forms ---
+// The same terms for the step loops, with fewer instructions: ranges and projections compared without
+// roots and divisions, each reciprocal formed once (recip, rsqrt_n).  The forms above, in the
+// reference's order of operations with IEEE division and root, serve the single force calls and the
+// vertex FIRE step: a minimiser amplifies its last bits, and a packing relaxed from the same start
+// stays the same packing.
+// Scalar gradient multiple gm and directed-visit energy at squared distance d2 (id = 1 / distance)
+// for radius sum `sum`, false out of range: calcContactInteraction 531-544, calcLJInteraction
+// 562-583, calcAdhesiveInteraction 604-626, calcWCAInteraction 653-668 (SEG = false) and
+// calcGradMultipleAndEnergy, cudaKernel.cuh:806-858 (SEG = true).  The ranges are compared as
+// squares, so pairs out of range cost no root.  Distance and quotient are rounded as the
+// reference's, nothing contracted: near its cutoff a stiff potential is a difference of large terms.
+template <int POT, bool SEG>
+__device__ __forceinline__ bool pair_gm(const Params& P, double d2, double sum, double& gm, double& id, double& e) {
+#pragma clang fp contract(off)
+  if constexpr (POT == POT_HARMONIC) {
+    if (!(d2 < sum * sum)) return false;
+    id = rsqrt_n(d2);
+    const double is = recip(sum), d = d2 > 0 ? sqrt_from(d2, id) : 0.0, overlap = 1 - div_from(d, sum, is);
+    gm = P.ec * overlap * is;
+    e = 0.25 * P.ec * overlap * overlap;
+    return true;
+  } else if constexpr (POT == POT_ADHESIVE) {
+    const double s1 = fmax(1 + P.l1, 0.0) * sum, s2 = fmax(1 + P.l2, 0.0) * sum;
+    const bool in1 = d2 < s1 * s1, in2 = d2 < s2 * s2;
+    if (!(SEG ? (in1 || in2) : in2)) return false;
+    id = rsqrt_n(d2);
+    const double is = recip(sum), d = d2 > 0 ? sqrt_from(d2, id) : 0.0, overlap = 1 - div_from(d, sum, is);
+    if (in1) {
+      gm = P.ec * overlap * is;
+      e = 0.25 * P.ec * (overlap * overlap - P.l1 * P.l2);
+    } else {
+      const double k = P.ec * P.l1 / (P.l2 - P.l1);
+      gm = -k * (overlap + P.l2) * is;
+      e = -0.25 * k * (overlap + P.l2) * (overlap + P.l2);
+    }
+    return true;
+  } else {
+    const double rc = (POT == POT_LJ ? fmax(P.LJcutoff, 0.0) : kWCAcut) * sum;
+    if (!(d2 <= rc * rc)) return false;
+    id = rsqrt_n(d2);
+    const double d = sqrt_from(d2, id), ratio = div_from(sum, d, id);
+    const double r2 = ratio * ratio;
+    const double ratio6 = r2 * r2 * r2;
+    const double ratio12 = ratio6 * ratio6;
+    gm = (POT == POT_WCA && SEG ? 4 * P.ec * (12 * ratio12 - 6 * ratio6) : 24 * P.ec * (2 * ratio12 - ratio6)) * id;
+    if constexpr (POT == POT_LJ) {
+      const double forceShift = P.LJfshift * recip(sum);
+      gm -= forceShift;
+      e = 0.5 * (4 * P.ec * (ratio12 - ratio6) - P.LJecut - fabs(forceShift) * (d - rc));
+    } else {
+      e = 0.5 * P.ec * (4 * (ratio12 - ratio6) + 1);
+    }
+    return true;
+  }
+}
+
+// Directed pair on `this` from `other` at separation (dx, dy) = this - other: adds to (fx, fy) and
+// returns the directed-visit energy.
+template <int POT>
+__device__ __forceinline__ double pair_force_n(const Params& P, double dx, double dy, double radSum,
+                                             double& fx, double& fy) {
+#pragma clang fp contract(off)
+  double gm, id, e;
+  if (!pair_gm<POT, false>(P, dx * dx + dy * dy, radSum, gm, id, e)) return 0.0;
+  gm *= id;
+  fx += gm * dx;
+  fy += gm * dy;
+  return e;
+}
+
+// Side of a projection dot / l2: -1 below 0, 0 in [0, 1), 1 from 1 on, 2 for a segment of no length
+// (or NaN).  The quotient is formed, as the reference forms it, only where the comparison of dot
+// with l2 cannot tell.
+__device__ __forceinline__ int proj_side(double dot, double l2) {
+  if (fabs(dot - l2) > 1e-12 * l2) return dot < 0 ? -1 : (dot < l2 ? 0 : 1);
+  const double length = sqrt(l2), proj = dot / (length * length);
+  return proj < 0 ? -1 : (proj < 1 ? 0 : (proj >= 1 ? 1 : 2));
+}
+
+// Both with sg = r_j - r_p, ip = r_i - r_p and ps = r_q - r_p (each one minimum image): every difference
+// the reference forms is one of these, their difference or its negative, and the sign
+// cross / |cross| is a comparison.  THIS: the force on i into (fx, fy); otherwise the forces on j into (fx, fy) and on
+// prev(j) into (px, py).  Returns the energy e added to both rings.
+template <int POT, bool THIS>
+__device__ __forceinline__ double smooth_eval(const Params& P, const Box& B, double tix, double tiy, double tjx,
+                                              double tjy, double tpx, double tpy, double tqx, double tqy,
+                                              double radSum, double& fx, double& fy, double& px, double& py) {
+#pragma clang fp contract(off)
+  const double sgx = pbx(tjx - tpx, B), sgy = pby(tjy - tpy, B);
+  const double ipx = pbx(tix - tpx, B), ipy = pby(tiy - tpy, B);
+  const double psx = pbx(tqx - tpx, B), psy = pby(tqy - tpy, B);
+  const double iqx = pbx(tix - tqx, B), iqy = pby(tiy - tqy, B);
+  const double l2 = sgx * sgx + sgy * sgy, dot = ipx * sgx + ipy * sgy;
+  const int side = proj_side(dot, l2);
+  const int prevSide = proj_side(-(iqx * psx + iqy * psy), psx * psx + psy * psy);
+  double energy = 0.0, gm, id, e;
+  if (side == 0) {
+    // the projection and its point rounded as the reference rounds them (dot / length^2 with a
+    // rounded length; nothing contracted): a stiff contact turns the point's last bit into 1e-12 of
+    // the force, and both codes share that error
+    const double il = rsqrt_n(l2), length = sqrt_from(l2, il), proj = div_from(dot, length * length, il * il);
+    const double qx = tpx + proj * sgx, qy = tpy + proj * sgy;
+    const double dqx = pbx(tix - qx, B), dqy = pby(tiy - qy, B);
+    if (pair_gm<POT, true>(P, dqx * dqx + dqy * dqy, radSum, gm, id, e)) {
+      const double cross = sgx * ipy - ipx * sgy;
+      const double sign = cross > 0 ? 1.0 : (cross < 0 ? -1.0 : 0.0);
+      gm *= il;
+      if constexpr (THIS) {
+        gm *= sign;
+        fx -= gm * sgy;
+        fy += gm * sgx;
+      } else {
+        const double jtx = pbx(sgx - ipx, B), jty = pby(sgy - ipy, B);
+        const double c = fabs(cross) * (il * il);
+        fx += gm * (sign * ipy - c * sgx);
+        fy += gm * (sign * -ipx - c * sgy);
+        px += gm * (sign * jty + c * sgx);
+        py += gm * (sign * -jtx + c * sgy);
+      }
+      energy += e;
+    }
+  }
+  // the pair (i, prev(j)): subtracted in a concave notch, added at a convex corner
+  const double s = side == 0 && prevSide == 0 ? -1.0 : (side == -1 && prevSide == 1 ? 1.0 : 0.0);
+  if (s != 0 && pair_gm<POT, true>(P, ipx * ipx + ipy * ipy, radSum, gm, id, e)) {
+    gm *= s * id;
+    if constexpr (THIS) {
+      fx += gm * ipx;
+      fy += gm * ipy;
+    } else {
+      px -= gm * ipx;
+      py -= gm * ipy;
+    }
+    energy += s * e;
+  }
+  return energy;
+}
+
+// force on i
+template <int POT>
+__device__ __forceinline__ double smooth_this_n(const Params& P, const Box& B, double tix, double tiy, double tjx,
+                                              double tjy, double tpx, double tpy, double tqx, double tqy,
+                                              double radSum, double& fx, double& fy) {
+  double nx = 0, ny = 0;
+  return smooth_eval<POT, true>(P, B, tix, tiy, tjx, tjy, tpx, tpy, tqx, tqy, radSum, fx, fy, nx, ny);
+}
+
+// forces on j and on prev(j) in one pass; the caller owns j, so both receivers lie in its own ring
+template <int POT>
+__device__ __forceinline__ double smooth_op_n(const Params& P, const Box& B, double tix, double tiy, double tjx,
+                                                 double tjy, double tpx, double tpy, double tqx, double tqy,
+                                                 double radSum, double& ox, double& oy, double& px, double& py) {
+  return smooth_eval<POT, false>(P, B, tix, tiy, tjx, tjy, tpx, tpy, tqx, tqy, radSum, ox, oy, px, py);
 }
 
 }  // namespace dpm

@@ -148,8 +148,7 @@ __global__ __launch_bounds__(WAVE* MAXW) void k_fire_sys(View V, Params P, FireP
         V.vy[v] = vy;
         V.x[v] = xn;
         V.y[v] = yn;
-        const double ddx = pbx(xn - V.lx[v], B), ddy = pby(yn - V.ly[v], B);
-        if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) moved = 1;
+        if (moved_past(P, B, xn - V.lx[v], yn - V.ly[v])) moved = 1;
       }
     }
     // ---- checkNeighbors: rebuild the system's rows from cells binned here (DPM2D.cu:1408-1423)
@@ -187,7 +186,7 @@ __global__ __launch_bounds__(WAVE* MAXW) void k_fire_sys(View V, Params P, FireP
       const double x = V.x[L.v], y = V.y[L.v];
       double fx = 0, fy = 0, e = 0, es = 0, qx = 0, qy = 0;
       double qnx = 0, qny = 0;  // sets with wide rings do not run this kernel
-      gather_pairs<INTER, POT>(V, P, L, B, x, y, 0, 1, fx, fy, e, es, qx, qy, qnx, qny);
+      gather_pairs<INTER, POT, true>(V, P, L, B, x, y, 0, 1, fx, fy, e, es, qx, qy, qnx, qny);
       const ShapeOut so = ring_shape(V, P, L, B, x, y, true);
       if constexpr (INTER == INT_SMOOTH) {
         fx += shfl_d(qx, L.nl);

@@ -146,6 +146,124 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
   return o;
 }
 
+// Position (ux, uy) of the lane's vertex relative to its ring's first vertex along the reference's
+// walk, one minimum-image segment (dnx, dny) at a time.  The walk of a ring narrower than half the box
+// is the minimum image of the difference itself: taken when every segment of the wave's rings joins up
+// with it, else the walk is an exclusive segmented scan of the segments (six dependent levels more).
+__device__ __forceinline__ void ring_walk(const Lane& L, const Box& B, double x, double y, double xf, double yf,
+                                          double dnx, double dny, double& ux, double& uy) {
+  ux = L.act ? pbx(x - xf, B) : 0.0;
+  uy = L.act ? pby(y - yf, B) : 0.0;
+  const double gx = shfl_d(ux, L.nl) - ux - dnx, gy = shfl_d(uy, L.nl) - uy - dny;
+  if (__all(!L.act || (fabs(gx) < 0.25 * B.Lx && fabs(gy) < 0.25 * B.Ly))) return;
+  ux = L.act ? seg_scan(L.act ? dnx : 0.0, L.lane, L.segS) - dnx : 0.0;
+  uy = L.act ? seg_scan(L.act ? dny : 0.0, L.lane, L.segS) - dny : 0.0;
+}
+
+// ring_shape for the step loops.  With dn = (v, next) and ps = (prev, v): the centre-relative differences of the reference's terms
+// (getRelativeVertexPos 273-279) are sums of the two, so the force needs no centre; the previous
+// segment's factors are the previous lane's own.  `write`: theta, length, energy, and the ring's area,
+// perimeter and centre, which nothing inside a step needs.
+__device__ __forceinline__ ShapeOut ring_shape_n(const View& V, const Params& P, const Lane& L, const Box& B,
+                                                 double x, double y, bool write) {
+#pragma clang fp contract(fast)
+  ShapeOut o{0, 0, 0, 0, 0};
+  double xn, yn, xp, yp, area, perim = 0;
+  int vn = 0, vp = 0;
+  if (!L.wide) {
+    xn = shfl_d(x, L.nl); yn = shfl_d(y, L.nl);
+    xp = shfl_d(x, L.pl); yp = shfl_d(y, L.pl);
+  } else {
+    // a slice of a wide ring: ring neighbours from memory (this launch reads the current positions
+    // only), the ring's area, perimeter and centre from k_wide_rings, launched just before
+    vn = ring_next(L.v, L.f, L.n);
+    vp = ring_prev(L.v, L.f, L.n);
+    xn = V.x[vn]; yn = V.y[vn];
+    xp = V.x[vp]; yp = V.y[vp];
+  }
+  const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
+  const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
+  const double theta = atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);  // calcAngle 423-427
+  const double n2 = dnx * dnx + dny * dny, in = rsqrt_n(n2), seglen = n2 > 0 ? sqrt_from(n2, in) : n2;
+  if (!L.wide) {
+    const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
+    double ux, uy;
+    ring_walk(L, B, x, y, xf, yf, dnx, dny, ux, uy);
+    const double shoe = L.act ? (ux * dny - dnx * uy) : 0.0;  // shoelace: cur x next = cur x delta
+    area = fabs(seg_sum(shoe, L.lane, L.segS, L.segE)) * 0.5;
+    if (write) {
+      perim = seg_sum(L.act ? seglen : 0.0, L.lane, L.segS, L.segE);
+      const double ind = 1.0 / (double)L.n;
+      o.cx = xf + seg_sum(ux, L.lane, L.segS, L.segE) * ind;
+      o.cy = yf + seg_sum(uy, L.lane, L.segS, L.segE) * ind;
+    }
+  } else {
+    area = V.area[L.r];
+  }
+  if (write && L.act) {
+    V.th[L.v] = theta;
+    V.len[L.v] = seglen;
+    if (L.lane == L.segS && !L.wide) {
+      V.area[L.r] = area;
+      V.perim[L.r] = perim;
+      V.cx[L.r] = o.cx;
+      V.cy[L.r] = o.cy;
+    }
+  }
+  const double a0 = V.a0[L.r], ia0 = recip(a0);
+  // shape costs: the global ea, el, eb, or per-ring values when the caller set them
+  const double ea = V.kr ? V.kr[L.r] : P.ea;
+  const double el = V.kr ? V.kr[V.np + L.r] : P.el;
+  const double eb = V.kr ? V.kr[2 * V.np + L.r] : P.eb;
+  // area term (calcAreaForceEnergy 429-435)
+  const double deltaA = div_from(area, a0, ia0) - 1.;
+  const double gmA = ea * deltaA * ia0;
+  double fx = -0.5 * gmA * (psy + dny);
+  double fy = 0.5 * gmA * (dnx + psx);
+  // perimeter term (calcPerimeterForceEnergy 437-447 / FENE 449-455): each segment's factor cn
+  const double l0v = V.l0[L.v];
+  const bool harmonic = P.monomer == MONO_HARMONIC;
+  auto factor = [&](double l0, double d2, double len, double id) {
+    if (harmonic) {
+      const double il0 = recip(l0);
+      return (div_from(len, l0, il0) - 1.) * il0 * id;
+    }
+    return 2 * P.stiff * P.extSq * recip(P.extSq * l0 * l0 - d2);
+  };
+  const double cn = factor(l0v, n2, seglen, in), in2 = in * in;
+  const double D = theta - V.th0[L.v];
+  double cp = shfl_d(cn, L.pl), ip2 = shfl_d(in2, L.pl), Dp = shfl_d(D, L.pl), Dn = shfl_d(D, L.nl);
+  if (L.wide) {  // from memory; the neighbours' angles from their own neighbours, as their lanes form them
+    const double p2 = psx * psx + psy * psy, ip = rsqrt_n(p2);
+    cp = factor(V.l0[vp], p2, sqrt_from(p2, ip), ip);
+    ip2 = ip * ip;
+    const int vpp = ring_prev(vp, L.f, L.n), vnn = ring_next(vn, L.f, L.n);
+    Dp = vertex_theta(B, xp, yp, x, y, V.x[vpp], V.y[vpp]) - V.th0[vp];
+    Dn = vertex_theta(B, xn, yn, V.x[vnn], V.y[vnn], x, y) - V.th0[vn];
+  }
+  fx += el * (cn * dnx - cp * psx);
+  fy += el * (cn * dny - cp * psy);
+  // bending term (calcBendingForceEnergy 457-471)
+  const double preVar = (D - Dp) * ip2, nextVar = (D - Dn) * in2;
+  fx += eb * (preVar * psy + nextVar * dny);
+  fy -= eb * (preVar * psx + nextVar * dnx);
+  if (write) {  // the previous segment's perimeter energy
+    double l0p = shfl_d(l0v, L.pl);
+    if (L.wide) l0p = V.l0[vp];
+    const double p2 = psx * psx + psy * psy;
+    double e = 0.5 * ea * deltaA * deltaA / (double)L.n + 0.5 * eb * D * D;
+    if (harmonic) {
+      const double pDelta = sqrt(p2) / l0p - 1.;
+      e += 0.5 * el * pDelta * pDelta;
+    } else {
+      e += el * P.stiff * P.extSq * log(1 - p2 / (P.extSq * l0p * l0p));
+    }
+    o.e = e;
+  }
+  o.fx = fx; o.fy = fy;
+  return o;
+}
+
 // The ring centre alone (calcParticlePos, cudaKernel.cuh:365-388), as ring_shape computes it,
 // stored by the ring's first lane: the rigid rings' shape pass
 __device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, const Box& B, double x, double y) {
@@ -153,10 +271,8 @@ __device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, co
   const double xn = shfl_d(x, L.nl), yn = shfl_d(y, L.nl);
   const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
   const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-  const double Ix = seg_scan(L.act ? dnx : 0.0, L.lane, L.segS);
-  const double Iy = seg_scan(L.act ? dny : 0.0, L.lane, L.segS);
-  const double ux = L.act ? Ix - dnx : 0.0;
-  const double uy = L.act ? Iy - dny : 0.0;
+  double ux, uy;
+  ring_walk(L, B, x, y, xf, yf, dnx, dny, ux, uy);
   const double sux = seg_sum(ux, L.lane, L.segS, L.segE);
   const double suy = seg_sum(uy, L.lane, L.segS, L.segE);
   const double ind = 1.0 / (double)L.n;
@@ -169,13 +285,34 @@ __device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, co
   return o;
 }
 
+// the pair terms in the reference's order (REF) or in the loops' form
+template <int POT, bool REF>
+__device__ __forceinline__ double pair_of(const Params& P, double dx, double dy, double sum, double& fx, double& fy) {
+  if constexpr (REF) return pair_force<POT>(P, dx, dy, sum, fx, fy);
+  return pair_force_n<POT>(P, dx, dy, sum, fx, fy);
+}
+template <int POT, bool REF>
+__device__ __forceinline__ double smooth_this_of(const Params& P, const Box& B, double tix, double tiy, double tjx,
+                                                 double tjy, double tpx, double tpy, double tqx, double tqy,
+                                                 double sum, double& fx, double& fy) {
+  if constexpr (REF) return smooth_pair<POT, ROLE_THIS>(P, B, tix, tiy, tjx, tjy, tpx, tpy, tqx, tqy, sum, fx, fy);
+  return smooth_this_n<POT>(P, B, tix, tiy, tjx, tjy, tpx, tpy, tqx, tqy, sum, fx, fy);
+}
+template <int POT, bool REF>
+__device__ __forceinline__ double smooth_op_of(const Params& P, const Box& B, double tix, double tiy, double tjx,
+                                               double tjy, double tpx, double tpy, double tqx, double tqy, double sum,
+                                               double& fx, double& fy, double& px, double& py) {
+  if constexpr (REF) return smooth_pair_op<POT>(P, B, tix, tiy, tjx, tjy, tpx, tpy, tqx, tqy, sum, fx, fy, px, py);
+  return smooth_op_n<POT>(P, B, tix, tiy, tjx, tjy, tpx, tpy, tqx, tqy, sum, fx, fy, px, py);
+}
+
 // Interparticle gather of lane L's vertex over entries k0, k0 + kstep, ... of its row:
 // accumulates the force on v, the vertex-vertex energy e, the smooth energy es and the share
 // (qx, qy) that v's `other` evaluation owes prev(v) (handed to prev(v)'s lane by the caller).
 // On the last lane of a wide ring's slice, whose next vertex lies in another tile, (qnx, qny)
 // accumulates the share that next(v)'s evaluations owe v, from next(v)'s row (complete before
 // the launch: wide sets rebuild rows in their own launch).
-template <int INTER, int POT>
+template <int INTER, int POT, bool REF>
 __device__ __forceinline__ void gather_pairs(const View& V, const Params& P, const Lane& L, const Box& B, double x,
                                              double y, int k0, int kstep, double& fx, double& fy, double& e,
                                              double& es, double& qx, double& qy, double& qnx, double& qny) {
@@ -190,7 +327,7 @@ __device__ __forceinline__ void gather_pairs(const View& V, const Params& P, con
     for (int k = k0; k < c; k += kstep) {
       const int kn = k + kstep;
       const int jn = kn < V.W ? V.nbr[(long)kn * V.nv + L.v] : 0;
-      e += pair_force<POT>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
+      e += pair_of<POT, REF>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
       j = jn;
     }
   } else if constexpr (INTER == INT_SMOOTH) {
@@ -223,9 +360,8 @@ __device__ __forceinline__ void gather_pairs(const View& V, const Params& P, con
       }
       const double xu = V.x[u], yu = V.y[u];
       const double radSum = radv + V.rad[u];
-      es += smooth_pair<POT, ROLE_THIS>(P, B, x, y, xu, yu, V.x[pp.x], V.y[pp.x], V.x[pp.y], V.y[pp.y], radSum,
-                                        fx, fy);
-      es += smooth_pair_op<POT>(P, B, xu, yu, x, y, xp, yp, xpp, ypp, radSum, fx, fy, qx, qy);
+      es += smooth_this_of<POT, REF>(P, B, x, y, xu, yu, V.x[pp.x], V.y[pp.x], V.x[pp.y], V.y[pp.y], radSum, fx, fy);
+      es += smooth_op_of<POT, REF>(P, B, xu, yu, x, y, xp, yp, xpp, ypp, radSum, fx, fy, qx, qy);
       u = un;
       pp = ppn;
     }
@@ -238,7 +374,7 @@ __device__ __forceinline__ void gather_pairs(const View& V, const Params& P, con
       for (int k = k0; k < cj; k += kstep) {
         const int w = V.nbr[(long)k * V.nv + j];
         double ox = 0, oy = 0;
-        (void)smooth_pair_op<POT>(P, B, V.x[w], V.y[w], xj, yj, x, y, xp, yp, radj + V.rad[w], ox, oy, qnx, qny);
+        (void)smooth_op_of<POT, REF>(P, B, V.x[w], V.y[w], xj, yj, x, y, xp, yp, radj + V.rad[w], ox, oy, qnx, qny);
       }
     }
   } else {
@@ -247,7 +383,7 @@ __device__ __forceinline__ void gather_pairs(const View& V, const Params& P, con
       const int b0 = V.svoff[L.s], b1 = V.svoff[L.s + 1];
       for (int j = b0 + k0; j < b1; j += kstep) {
         if (V.vring[j] == L.r) continue;
-        e += pair_force<POT>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
+        e += pair_of<POT, REF>(P, pbx(x - V.x[j], B), pby(y - V.y[j], B), radv + V.rad[j], fx, fy);
       }
     }
   }
@@ -256,12 +392,19 @@ __device__ __forceinline__ void gather_pairs(const View& V, const Params& P, con
 // -------------------------------------------------------------- step ---
 // Waves of a tile: with nw > 1, wave 0 does the ring geometry, shape force and random draws
 // while waves 1..nw-1 share the neighbour gather; with nw == 1 wave 0 does both in turn.
+// Whether a displacement exceeds k cutoff / 3 (checkDisplacement, DPM2D.cu:1390-1406), by squares; a
+// negative cutoff is exceeded by any
+__device__ __forceinline__ bool moved_past(const Params& P, const Box& B, double dx, double dy, double k = 1.0) {
+  dx = pbx(dx, B);
+  dy = pby(dy, B);
+  const double c = k * P.cutoff;
+  return 9 * (dx * dx + dy * dy) > c * fabs(c);
+}
+
 // A drift that moved a vertex more than cutoff / 3 marks its system FLAG_FAR: the next rebuild
 // cannot rely on the cells of its list positions (md_cells)
 __device__ __forceinline__ void far_test(const Params& P, const Box& B, double dx, double dy, int* flag) {
-  dx = pbx(dx, B);
-  dy = pby(dy, B);
-  if (3 * sqrt(dx * dx + dy * dy) > P.cutoff) atomicOr(flag, FLAG_FAR);
+  if (moved_past(P, B, dx, dy)) atomicOr(flag, FLAG_FAR);
 }
 
 // The step loop's cell lists of a system whose list positions (the positions of its last
@@ -286,8 +429,7 @@ __device__ __forceinline__ MdCells md_cells(const StepArgs& A, const CellGrid& G
 // miss a neighbour (cannot happen while the displacement and far tests hold)
 __device__ __forceinline__ void md_stale_test(const View& V, const Params& P, const Box& B, int v, double x, double y,
                                               int* err) {
-  const double ddx = pbx(x - V.lx[v], B), ddy = pby(y - V.ly[v], B);
-  if (3 * sqrt(ddx * ddx + ddy * ddy) > 2 * P.cutoff) atomicOr(err, ERR_STALE_BINS);
+  if (moved_past(P, B, x - V.lx[v], y - V.ly[v], 2.0)) atomicOr(err, ERR_STALE_BINS);
 }
 
 // ---------------------------------------------------------- rigid rings ---
@@ -398,8 +540,7 @@ __device__ __forceinline__ void rigid_epilogue(const View& V, const Params& P, c
       rigid_move(B, x, y, cx, cy, ncx, ncy, cos(dth), sin(dth), xn, yn);
       A.xout[L.v] = xn;
       A.yout[L.v] = yn;
-      const double ddx = pbx(xn - lx, B), ddy = pby(yn - ly, B);
-      if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
+      if (moved_past(P, B, xn - lx, yn - ly)) {
         atomicOr(&A.flagOut[L.s], 1);
         atomicOr(A.anyOut, 1);
       }

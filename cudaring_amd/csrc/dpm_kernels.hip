@@ -216,10 +216,8 @@ __device__ __forceinline__ void md_prologue(const View& V, const Params& P, cons
                                             const Box& B, int v, int s, double x, double y, int* flag, int* any) {
   const double lx = V.lx[v], ly = V.ly[v];
   bin_vertex(G, B, A.cellCur, A.slotsCur, v, s, lx, ly, A.err);
-  const double ddx = pbx(x - lx, B), ddy = pby(y - ly, B);
-  const double d3 = 3 * sqrt(ddx * ddx + ddy * ddy);
-  if (d3 > P.cutoff) {
-    atomicOr(flag, d3 > 2 * P.cutoff ? 1 | FLAG_FAR : 1);
+  if (moved_past(P, B, x - lx, y - ly)) {
+    atomicOr(flag, moved_past(P, B, x - lx, y - ly, 2.0) ? 1 | FLAG_FAR : 1);
     if (any) atomicOr(any, 1);
   }
 }
@@ -616,8 +614,7 @@ __global__ void k_rigid_fire_move(View V, Params P, FireParams fp, const FireSta
   rigid_move(B, V.x[L.v], V.y[L.v], lcx, lcy, cx, cy, cos(dth), sin(dth), xn, yn);
   xo[L.v] = xn;
   yo[L.v] = yn;
-  const double ddx = pbx(xn - V.lx[L.v], B), ddy = pby(yn - V.ly[L.v], B);
-  if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
+  if (moved_past(P, B, xn - V.lx[L.v], yn - V.ly[L.v])) {
     atomicOr(&flagOut[L.s], 1);
     atomicOr(anyOut, 1);
   }
@@ -720,8 +717,7 @@ __global__ void k_fire_mid(View V, Params P, const FireState* fcur, const double
   xo[L.v] = xn;
   yo[L.v] = yn;
   const Box B = box_of(V, L.s);
-  const double ddx = pbx(xn - V.lx[L.v], B), ddy = pby(yn - V.ly[L.v], B);
-  if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
+  if (moved_past(P, B, xn - V.lx[L.v], yn - V.ly[L.v])) {
     atomicOr(&flagOut[L.s], 1);
     atomicOr(anyOut, 1);
   }

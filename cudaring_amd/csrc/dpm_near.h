@@ -288,10 +288,10 @@ __device__ __forceinline__ void eval_near(const View& V, const Params& P, const 
         const double sum = V.rad[v] + V.rad[u];
         double fx = 0, fy = 0, e;
         if constexpr (NR == 1) {
-          e = pair_force<POT>(P, pbx(x - xu, B), pby(y - yu, B), sum, fx, fy);
+          e = pair_force_n<POT>(P, pbx(x - xu, B), pby(y - yu, B), sum, fx, fy);
         } else {
           const int p1 = u - (((t.y >> 8) & 255) - 64), p2 = u - (((t.y >> 16) & 255) - 64);
-          e = smooth_pair<POT, ROLE_THIS>(P, B, x, y, xu, yu, V.x[p1], V.y[p1], V.x[p2], V.y[p2], sum, fx, fy);
+          e = smooth_this_n<POT>(P, B, x, y, xu, yu, V.x[p1], V.y[p1], V.x[p2], V.y[p2], sum, fx, fy);
         }
         fT[i] = make_double2(fx, fy);
         if constexpr (ENERGY) eT[i] = e;
@@ -302,7 +302,7 @@ __device__ __forceinline__ void eval_near(const View& V, const Params& P, const 
         const int v = v0 + (t.y & 63), u = t.x;
         const int p1 = v - (((t.y >> 8) & 255) - 64), p2 = v - (((t.y >> 16) & 255) - 64);
         double fx = 0, fy = 0, qx = 0, qy = 0;
-        const double e = smooth_pair_op<POT>(P, B, V.x[u], V.y[u], V.x[v], V.y[v], V.x[p1], V.y[p1], V.x[p2], V.y[p2],
+        const double e = smooth_op_n<POT>(P, B, V.x[u], V.y[u], V.x[v], V.y[v], V.x[p1], V.y[p1], V.x[p2], V.y[p2],
                                              V.rad[v] + V.rad[u], fx, fy, qx, qy);
         fO[i] = make_double2(fx, fy);
         qO[i] = make_double2(qx, qy);

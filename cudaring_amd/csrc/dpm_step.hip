@@ -15,6 +15,8 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   Lane L;
   constexpr bool WIDE = (MODE & MODE_WIDE) != 0;
   constexpr bool NEAR = (MODE & MODE_NEAR) != 0;
+  // single force calls and the vertex FIRE step keep the reference's order of operations
+  constexpr bool REF = (MODE & (MODE_KICK | MODE_BROWN)) == 0;
   constexpr int MB = MODE & ~(MODE_WIDE | MODE_NEAR);  // the integrator mode
   // A step of a velocity-Verlet, Langevin or BAOAB loop other than its last consumes the force it
   // computes in this launch (the closing and next opening half kicks); its force, energies, ring
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
     }
     if (w >= g0) eval_near<INTER, POT, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, 0, L.lane, w - g0, ng, red);
   } else {
-    if (w >= g0) gather_pairs<INTER, POT>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
+    if (w >= g0) gather_pairs<INTER, POT, REF>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
     if (nw > 1 && w > 0) {
       double* r = red + (w - 1) * nq * WAVE + L.lane;
       r[0 * WAVE] = fx;
@@ -130,7 +132,8 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   double zt0 = 0, zt1 = 0, ang = 0;
   if (w == 0) {
     if constexpr ((MODE & MODE_RIGID) != 0) so = ring_centre(V, L, B, x, y);
-    else so = ring_shape(V, P, L, B, x, y, STORE);
+    else if constexpr (REF) so = ring_shape(V, P, L, B, x, y, STORE);
+    else so = ring_shape_n(V, P, L, B, x, y, STORE);
     // one thermal draw per integrate call and ring: Langevin::updateThermalVel (Simulator.cu:54-77)
     // and Brownian::updateThermalVel (156-179) after this call's force, counter = call index;
     // BAOAB::updateThermalVel (122-144) in the next call's first half, whose index is one more
@@ -223,8 +226,10 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   fy = so.fy + fy;
   e = so.e + e;
   if (P.particle == PART_ACTIVE) {
-    fx += P.driving * ((1 - 0) * cos(ang) + 0 * sin(ang));
-    fy += P.driving * ((1 - 1) * cos(ang) + 1 * sin(ang));
+    double sn, cs;
+    sincos(ang, &sn, &cs);
+    fx += P.driving * cs;
+    fy += P.driving * sn;
   }
 
   if constexpr ((MODE & MODE_LANGEVIN) != 0 && (MODE & MODE_BROWN) == 0) {
@@ -298,8 +303,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       A.recx[L.v] = xn;
       A.recy[L.v] = yn;
     }
-    const double ddx = pbx(xn - lx, B), ddy = pby(yn - ly, B);
-    if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
+    if (moved_past(P, B, xn - lx, yn - ly)) {
       atomicOr(&A.flagOut[L.s], 1);
       atomicOr(A.anyOut, 1);
     }
