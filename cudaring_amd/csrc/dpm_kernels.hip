@@ -1012,7 +1012,7 @@ hipError_t launch_fire_partials(dpm_set_s* S) {
 }
 
 hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves) {
-  const int threads = WAVE * (waves < 1 ? 1 : (waves > FS_WAVES_WIDE ? FS_WAVES_WIDE : waves));
+  const int threads = WAVE * (waves < 1 ? 1 : (waves > FS_WAVES ? FS_WAVES : waves));
   switch (S->P.interaction) {
     case INT_VV: return fire_pot<INT_VV>(S, chunk, threads);
     case INT_SMOOTH: return fire_pot<INT_SMOOTH>(S, chunk, threads);

@@ -11,8 +11,7 @@
 // its task at an address that depends on nothing but the tile.
 #pragma once
 
-#include "dpm_rows.h"
-#include "dpm_tile.h"
+#include "dpm_forces.h"
 
 namespace dpm {
 
@@ -65,16 +64,16 @@ __host__ __device__ constexpr int rows_lds_ints(int W, bool near) {
   return near ? kNearMaskBytes / 4 + WAVE + 2 * WAVE * W : WAVE + WAVE * W;
 }
 
-// The task list of a tile from the masks of its lanes' row entries (complete in LDS), `entry(k)` the
-// lane's k-th neighbour in ascending order, of n.
-template <int INTER, class F>
+// The task list of a tile: `bits(q)` the lane's mask of near row entries of role q (complete),
+// `entry(k)` its k-th neighbour in ascending order, of n.
+template <int INTER, class M, class F>
 __device__ __forceinline__ void write_near_tile(const View& V, const NearRows& N, const Lane& L, int w, int nw, int n,
-                                                const unsigned long long* mask, F entry) {
+                                                M bits, F entry) {
   constexpr int NR = INTER == INT_SMOOTH ? 2 : 1;
   int total[2] = {0, 0};
 #pragma unroll
   for (int q = 0; q < NR; q++) {
-    const unsigned long long m = mask[q * WAVE + L.lane];
+    const unsigned long long m = bits(q);
     const int c = __popcll(m);
     int end = c;  // inclusive scan over the lanes: vertices in order
 #pragma unroll
@@ -149,7 +148,27 @@ __device__ __forceinline__ void build_near_tile(const View& V, const Params& P, 
     if (bits & 2) atomicOr(&mask[WAVE + L.lane], 1ull << k);
   }
   __syncthreads();
-  write_near_tile<INTER>(V, N, L, w, nw, n, mask, [&](int k) { return V.nbr[(long)k * V.nv + L.v]; });
+  write_near_tile<INTER>(V, N, L, w, nw, n, [&](int q) { return mask[q * WAVE + L.lane]; }, [&](int k) { return V.nbr[(long)k * V.nv + L.v]; });
+}
+
+// build_near_tile by one wave for its tile, each lane over its own row, the masks in registers.
+template <int INTER>
+__device__ __forceinline__ void build_near_wave(const View& V, const Params& P, const NearRows& N, const Lane& L,
+                                                const Box& B, const double* px, const double* py, bool keepAll) {
+  const int n = L.act ? V.ncnt[L.v] : 0;
+  const double x = px[L.v], y = py[L.v], radv = V.rad[L.v];
+  const NearReach R(P);
+  const int vp = L.act ? L.v0 + L.pl : L.v;
+  const double xp = px[vp], yp = py[vp];
+  unsigned long long mask[2] = {0, 0};
+  for (int k = 0; k < n; k++) {
+    const int bits =
+        keepAll ? 3 : near_bits<INTER>(V, R, B, x, y, radv, xp, yp, V.nbr[(long)k * V.nv + L.v], px, py);
+    mask[0] |= (unsigned long long)(bits & 1) << k;
+    mask[1] |= (unsigned long long)(bits >> 1) << k;
+  }
+  write_near_tile<INTER>(V, N, L, 0, 1, n, [&](int q) { return mask[q]; },
+                         [&](int k) { return V.nbr[(long)k * V.nv + L.v]; });
 }
 
 // The rows of a tile's vertices (lane = vertex, L.act lanes), built by all nw waves of its
@@ -252,7 +271,7 @@ __device__ __forceinline__ void build_rows_tile(const View& V, const Params& P, 
   }
   if constexpr (NEAR >= 0) {
     __syncthreads();
-    write_near_tile<NEAR>(V, N, L, w, nw, n, mask, [&](int k) { return srow[k * WAVE + lane]; });
+    write_near_tile<NEAR>(V, N, L, w, nw, n, [&](int q) { return mask[q * WAVE + lane]; }, [&](int k) { return srow[k * WAVE + lane]; });
   }
 }
 
@@ -341,6 +360,66 @@ __device__ __forceinline__ void sum_near(int spanT, int spanO, int base, const v
       qx += q.x;
       qy += q.y;
       if constexpr (ENERGY) e += eO[k];
+    }
+  }
+}
+
+// One wave's evaluation of its tile's near list, 64 at a time, positions through pos(v) (a double2), the
+// chunk's results handed to their lanes through `res` (near_wave_doubles of LDS, the wave's own).
+template <int INTER>
+__host__ __device__ constexpr int near_wave_doubles() {
+  return WAVE * (INTER == INT_SMOOTH ? 5 : 3);
+}
+template <int INTER, int POT, bool REF, bool ENERGY, class X>
+__device__ __forceinline__ void near_wave(const View& V, const Params& P, const NearRows& N, const Box& B,
+                                          const Lane& L, X pos, double* res, double& fx, double& fy, double& e,
+                                          double& qx, double& qy) {
+  constexpr int NR = INTER == INT_SMOOTH ? 2 : 1;
+  double2* f = (double2*)res;
+  double2* g = f + WAVE;
+  double* en = (double*)(f + NR * WAVE);
+  const int2 cnt = N.tcnt[L.tile];
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const int total = q ? cnt.y : cnt.x, span = L.act ? N.span[(long)q * V.nv + L.v] : 0;
+    const int2* list = N.task + ((long)L.tile * 2 + q) * N.cap;
+    for (int base = 0; base < total; base += WAVE) {
+      if (base + L.lane < total) {
+        const int2 t = list[base + L.lane];
+        const int v = L.v0 + (t.y & 63), u = t.x;
+        const double2 a = pos(v), b = pos(u);
+        const double sum = V.rad[v] + V.rad[u];
+        double ax = 0, ay = 0, bx = 0, by = 0, ee;
+        if constexpr (NR == 1) {
+          ee = pair_of<POT, REF>(P, pbx(a.x - b.x, B), pby(a.y - b.y, B), sum, ax, ay);
+        } else {
+          const int j = q ? v : u;
+          const double2 p1 = pos(j - (((t.y >> 8) & 255) - 64)), p2 = pos(j - (((t.y >> 16) & 255) - 64));
+          if (q == 0)
+            ee = smooth_this_of<POT, REF>(P, B, a.x, a.y, b.x, b.y, p1.x, p1.y, p2.x, p2.y, sum, ax, ay);
+          else
+            ee = smooth_op_of<POT, REF>(P, B, b.x, b.y, a.x, a.y, p1.x, p1.y, p2.x, p2.y, sum, ax, ay, bx, by);
+        }
+        f[L.lane] = make_double2(ax, ay);
+        if (q == 1) g[L.lane] = make_double2(bx, by);
+        if constexpr (ENERGY) en[L.lane] = ee;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int s = (span & 0xffff) - base, k0 = max(s, 0), k1 = min(s + (span >> 16), WAVE);
+      for (int k = k0; k < k1; k++) {
+        const double2 a = f[k];
+        fx += a.x;
+        fy += a.y;
+        if (q == 1) {
+          const double2 b = g[k];
+          qx += b.x;
+          qy += b.y;
+        }
+        if constexpr (ENERGY) e += en[k];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
   }
 }

@@ -12,9 +12,10 @@ namespace dpm {
 #define ROWS_WAVES 8
 // waves per tile of the loops' start kernel when it builds near lists
 #define START_WAVES 4
-// waves per workgroup of the two persistent FIRE builds
-#define FS_WAVES 8
-#define FS_WAVES_WIDE 16
+// most waves per workgroup of the persistent FIRE kernel, and the LDS its near lists and positions may
+// take (of 160 KB, beside its static arrays)
+#define FS_WAVES 16
+constexpr unsigned kFireLds = 156 * 1024;
 
 __device__ __forceinline__ double shfl_d(double v, int src) { return __shfl(v, src, WAVE); }
 __device__ __forceinline__ int shfl_i(int v, int src) { return __shfl(v, src, WAVE); }
