@@ -12,6 +12,7 @@
 
 #include "../../include/dpmring.h"
 #include "dpm_internal.h"
+#include "dpm_tile.h"
 
 using namespace dpm;
 
@@ -358,9 +359,6 @@ double box_area(const dpm_set_s* S, long s) {
 
 int reduce_host(dpm_set_s* S) {
   HIPCHK(launch_reduce(S));
-  S->h_red.resize(S->nsys * 8);
-  HIPCHK(hipMemcpyAsync(S->h_red.data(), S->d_red, sizeof(double) * S->nsys * 8, hipMemcpyDeviceToHost,
-                        S->stream));
   HIPCHK(hipStreamSynchronize(S->stream));
   return DPM_OK;
 }
@@ -1143,7 +1141,19 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   A(S->d_part, (long)V.ntiles * 4);
   S->nwide = (long)S->h_wide.size();
   if (S->nwide > 0) A(S->d_wide, S->nwide);
-  A(S->d_red, numSystems * 8); A(S->d_scale, numSystems);
+  std::vector<int> chunkSys, chunkOff(1, 0);
+  for (long s = 0; s < numSystems; s++) {
+    const int n = (S->h_svoff[s + 1] - S->h_svoff[s] + REDUCE_CHUNK - 1) / REDUCE_CHUNK;
+    chunkSys.insert(chunkSys.end(), n, (int)s);
+    chunkOff.push_back((int)chunkSys.size());
+  }
+  S->redBlocks = (int)chunkSys.size();
+  A(S->d_red, (long)S->redBlocks * 8); A(S->d_scale, numSystems);
+  A(S->d_chunkSys, S->redBlocks); A(S->d_chunkOff, numSystems + 1);
+  if (hipHostMalloc((void**)&S->h_red, sizeof(double) * numSystems * 8) != hipSuccess) {
+    dpm_destroy(S);
+    return DPM_ERR_OOM;
+  }
 #undef A
   set_pos_view(S);
   hipStream_t st = S->stream;
@@ -1158,7 +1168,8 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
             up(V.rsys, S->h_rsys, st) == hipSuccess && up(V.svoff, S->h_svoff, st) == hipSuccess &&
             up(V.sroff, S->h_sroff, st) == hipSuccess && up(V.tile_v0, S->h_tile_v0, st) == hipSuccess &&
             up(V.tile_v1, S->h_tile_v1, st) == hipSuccess && up(V.tile_sys, S->h_tile_sys, st) == hipSuccess &&
-            up(V.stile, S->h_stile, st) == hipSuccess &&
+            up(V.stile, S->h_stile, st) == hipSuccess && up(S->d_chunkSys, chunkSys, st) == hipSuccess &&
+            up(S->d_chunkOff, chunkOff, st) == hipSuccess &&
             (S->nwide == 0 || up(S->d_wide, S->h_wide, st) == hipSuccess);
   // the persistent FIRE kernel's workgroup b runs system order[b]: the systems with the most tiles
   // first, so that the longest iterations start in the first wave of workgroups
@@ -1230,9 +1241,11 @@ int dpm_destroy(dpm_set_t h) {
                   S->d_contacts, S->d_ccount, S->d_x0, S->d_obs, S->mdCount[0], S->mdSlots[0], S->mdFlag[0],
                   S->mdFlag[1], S->mdFlag[2], S->mdFlag[3], S->mdGen[0], S->mdGen[1], S->mdGen[2], S->R.pvx, S->R.pvy, S->R.pw, S->R.pfx, S->R.pfy, S->R.ptq, S->R.moi,
                   S->R.prad, S->R.plx, S->R.ply, S->R.pla, S->R.vtq, S->d_rfire[0], S->d_rfire[1], S->d_rg,
-                  S->d_snap, S->d_ftape, S->d_ftapeState, S->d_fadj, S->d_wide, S->N.task, S->N.tcnt, S->N.span};
+                  S->d_snap, S->d_ftape, S->d_ftapeState, S->d_fadj, S->d_wide, S->N.task, S->N.tcnt, S->N.span,
+                  S->d_chunkSys, S->d_chunkOff};
   for (void* p : ptrs)
     if (p) hipFree(p);
+  if (S->h_red) hipHostFree(S->h_red);
   if (S->ownStream) hipStreamDestroy(S->ownStream);
   delete S;
   return DPM_OK;

@@ -218,9 +218,11 @@ struct dpm_set_s {
   int* d_sysOrder = nullptr;  // persistent FIRE: workgroup b runs system d_sysOrder[b] (most tiles first)
 
   // reductions
-  double* d_red = nullptr;   // per-system outputs [nsys * 8]
+  double* d_red = nullptr;   // partials of systems of several blocks [redBlocks * 8]
+  double* h_red = nullptr;   // per-system outputs [nsys * 8], pinned host memory the kernels write
+  int *d_chunkSys = nullptr, *d_chunkOff = nullptr;  // block -> system, system -> first block
+  int redBlocks = 0;
   double* d_scale = nullptr; // per-system scalars
-  std::vector<double> h_red;
 
   // adjoint tape (dpm_nve_forward / dpm_nve_backward)
   long tapeSteps = 0, tapeEvery = 0, tapeNck = 0;

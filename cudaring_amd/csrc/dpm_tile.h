@@ -8,6 +8,8 @@ namespace dpm {
 
 #define WAVE 64
 #define MAXSPLIT 8
+// vertices of a system per block of the reductions
+#define REDUCE_CHUNK 2048
 // waves per tile of the host-driven row build
 #define ROWS_WAVES 8
 // waves per tile of the loops' start kernel when it builds near lists
