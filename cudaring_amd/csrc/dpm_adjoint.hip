@@ -516,13 +516,48 @@ __global__ void k_copy_d(double* dst, const double* src, long n) {
   if (i < n) dst[i] = src[i];
 }
 
-// several copies in one launch: thread t copies word t of every segment, grid-stride
-__global__ void k_copy_segs(CopySegs c) {
+// several copies and fills in one launch: thread t takes word t of every segment, grid-stride
+__device__ __forceinline__ void fill_segs(const FillSegs& f) {
+  const long stride = (long)gridDim.x * blockDim.x;
+  for (int q = 0; q < f.n; q++) {
+    int* p = f.p[q];
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < f.words[q]; i += stride) p[i] = f.value[q];
+  }
+}
+__global__ void k_prologue(CopySegs c, FillSegs f) {
   const long stride = (long)gridDim.x * blockDim.x;
   for (int q = 0; q < c.n; q++) {
     const unsigned* src = c.src[q];
     unsigned* dst = c.dst[q];
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < c.words[q]; i += stride) dst[i] = src[i];
+  }
+  fill_segs(f);
+}
+
+// the end of a row build: its error bits and longest row for the host, its flags and cells clean
+__global__ void k_rebuild_end(FillSegs f, const int* err, const int* maxcnt, HostStat* stat) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    stat->err = *err;
+    stat->maxcnt = *maxcnt;
+  }
+  fill_segs(f);
+}
+
+// the end of a loop, one block: RNG call counters advanced by its draws, its error bits and
+// (with FIRE states) whether a system has not converged for the host
+__global__ __launch_bounds__(256) void k_loop_end(unsigned long long* ctr, long long addT, long long addA,
+                                                  const int* err, const FireState* fs, int nsys, HostStat* stat) {
+  int open = 0;
+  if (fs)
+    for (int s = threadIdx.x; s < nsys; s += 256) open |= !fs[s].converged;
+  open = __syncthreads_or(open);
+  if (threadIdx.x == 0) {
+    if (addT | addA) {
+      ctr[0] += (unsigned long long)addT;
+      ctr[1] += (unsigned long long)addA;
+    }
+    stat->err = *err;
+    stat->notDone = open;
   }
 }
 
@@ -606,12 +641,29 @@ hipError_t launch_fill_d(double* p, double value, long n, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_copy_segs(const CopySegs& segs, hipStream_t st) {
-  long most = 0;
-  for (int q = 0; q < segs.n; q++) most = segs.words[q] > most ? segs.words[q] : most;
-  if (most <= 0) return hipSuccess;
+static unsigned seg_blocks(long most) {
   const long blocks = (most + 255) / 256;
-  k_copy_segs<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, 0, st>>>(segs);
+  return (unsigned)std::max(1L, std::min(2048L, blocks));
+}
+
+hipError_t launch_prologue(const CopySegs& segs, const FillSegs& fills, hipStream_t st) {
+  long most = 0;
+  for (int q = 0; q < segs.n; q++) most = std::max(most, segs.words[q]);
+  for (int q = 0; q < fills.n; q++) most = std::max(most, fills.words[q]);
+  if (most <= 0) return hipSuccess;
+  k_prologue<<<seg_blocks(most), 256, 0, st>>>(segs, fills);
+  return hipGetLastError();
+}
+
+hipError_t launch_rebuild_end(dpm_set_s* S, const FillSegs& fills) {
+  long most = 0;
+  for (int q = 0; q < fills.n; q++) most = std::max(most, fills.words[q]);
+  k_rebuild_end<<<seg_blocks(most), 256, 0, S->stream>>>(fills, S->d_err, S->d_maxcnt, S->h_stat);
+  return hipGetLastError();
+}
+
+hipError_t launch_loop_end(dpm_set_s* S, long long addT, long long addA, const FireState* fs) {
+  k_loop_end<<<1, 256, 0, S->stream>>>(S->d_ctr, addT, addA, S->d_err, fs, (int)S->nsys, S->h_stat);
   return hipGetLastError();
 }
 

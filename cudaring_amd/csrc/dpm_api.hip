@@ -285,14 +285,21 @@ int rebuild(dpm_set_s* S, const std::vector<int>& flags, int countUpdates, bool 
     Vl.x = S->V.lx;
     Vl.y = S->V.ly;
   }
+  int any = 0;
+  bool every = true;
+  for (int f : flags) {
+    any |= f;
+    every = every && f == 1;
+  }
   for (int attempt = 0; attempt < 8; attempt++) {
-    int any = 0;
-    for (int f : flags) any |= f;
-    HIPCHK(hipMemcpyAsync(S->d_flag[b], flags.data(), sizeof(int) * S->nsys, hipMemcpyHostToDevice, S->stream));
-    HIPCHK(hipMemcpyAsync(S->d_any + b, &any, sizeof(int), hipMemcpyHostToDevice, S->stream));
-    HIPCHK(launch_fill_int(S->d_err, 0, 1, S->stream));
-    HIPCHK(launch_fill_int(S->d_maxcnt, 0, 1, S->stream));
-    HIPCHK(launch_fill_int(S->G.count[b], 0, S->G.ncells, S->stream));
+    FillSegs f{};
+    f.add(S->d_err, 0, 1);
+    f.add(S->d_maxcnt, 0, 1);
+    f.add(S->G.count[b], 0, S->G.ncells);
+    f.add(S->d_any + b, any, 1);
+    if (every) f.add(S->d_flag[b], 1, S->nsys);
+    else HIPCHK(hipMemcpyAsync(S->d_flag[b], flags.data(), sizeof(int) * S->nsys, hipMemcpyHostToDevice, S->stream));
+    HIPCHK(launch_prologue(CopySegs{}, f, S->stream));
     if (atListPositions) {
       HIPCHK(launch_bin_view(S, Vl, b));
       HIPCHK(launch_build_rows_view(S, Vl, b, countUpdates));
@@ -300,16 +307,14 @@ int rebuild(dpm_set_s* S, const std::vector<int>& flags, int countUpdates, bool 
       HIPCHK(launch_bin(S, 0, 0));
       HIPCHK(launch_build_rows(S, countUpdates));
     }
-    int err = 0, maxcnt = 0;
-    HIPCHK(hipMemcpyAsync(&err, S->d_err, sizeof(int), hipMemcpyDeviceToHost, S->stream));
-    HIPCHK(hipMemcpyAsync(&maxcnt, S->d_maxcnt, sizeof(int), hipMemcpyDeviceToHost, S->stream));
+    FillSegs c{};  // leave both parities' flags and the cells clean
+    c.add(S->d_flag[0], 0, S->nsys);
+    c.add(S->d_flag[1], 0, S->nsys);
+    c.add(S->d_any, 0, 2);
+    c.add(S->G.count[b], 0, S->G.ncells);
+    HIPCHK(launch_rebuild_end(S, c));
     HIPCHK(hipStreamSynchronize(S->stream));
-    // leave both parities' flags and the cells clean
-    HIPCHK(launch_fill_int(S->d_flag[0], 0, S->nsys, S->stream));
-    HIPCHK(launch_fill_int(S->d_flag[1], 0, S->nsys, S->stream));
-    HIPCHK(launch_fill_int(S->d_any, 0, 2, S->stream));
-    HIPCHK(launch_fill_int(S->G.count[b], 0, S->G.ncells, S->stream));
-    HIPCHK(hipStreamSynchronize(S->stream));
+    const int err = S->h_stat->err, maxcnt = S->h_stat->maxcnt;
     if (err & ERR_CELL_OVERFLOW) {
       S->G.cap *= 2;
       hipFree(S->G.slots);
@@ -342,13 +347,6 @@ int loop_status(dpm_set_s* S, int err) {
   if (err) return fail(S, DPM_ERR_OVERFLOW, err & ERR_LIST_OVERFLOW ? "neighbour list overflow during loop"
                                                                     : "cell overflow during loop");
   return DPM_OK;
-}
-
-int check_err_after_loop(dpm_set_s* S) {
-  int err = 0;
-  HIPCHK(hipMemcpyAsync(&err, S->d_err, sizeof(int), hipMemcpyDeviceToHost, S->stream));
-  HIPCHK(hipStreamSynchronize(S->stream));
-  return loop_status(S, err);
 }
 
 // area of system s's domain: the box, or pi R^2 for the round box (getPhi, DPM2D.cu:1208-1246)
@@ -400,7 +398,7 @@ std::vector<std::pair<unsigned*, long>> snap_fields(dpm_set_s* S, int what) {
   return f;
 }
 
-int snap_copy(dpm_set_s* S, int what, bool save) {
+int snap_copy(dpm_set_s* S, int what, bool save, const FillSegs& fills = FillSegs{}) {
   const auto f = snap_fields(S, what);
   long words = 0;
   for (auto& q : f) words += q.second;
@@ -421,15 +419,15 @@ int snap_copy(dpm_set_s* S, int what, bool save) {
     c.n++;
     off += q.second;
   }
-  HIPCHK(launch_copy_segs(c, S->stream));
+  HIPCHK(launch_prologue(c, fills, S->stream));
   return DPM_OK;
 }
 
-int snap_save(dpm_set_s* S, int what) {
+int snap_save(dpm_set_s* S, int what, const FillSegs& fills) {
   S->snapCur = S->cur;
   S->snapFireCur = S->fireCur;
   S->snapRfireCur = S->rfireCur;
-  return snap_copy(S, what, true);
+  return snap_copy(S, what, true, fills);
 }
 
 int snap_restore(dpm_set_s* S, int what) {
@@ -440,20 +438,44 @@ int snap_restore(dpm_set_s* S, int what) {
   return snap_copy(S, what, false);
 }
 
-// Run `loop` (which leaves its errors in d_err) from a copy of the state it changes, and again on
-// a wider list for as long as it reports ERR_LIST_OVERFLOW; returns the loop's status (one host
-// synchronisation per run).
+// What is cleared before a loop: the error word; for the step loops (LOOP_MD) cell lists 0 and 1 (the
+// start kernel bins the list positions into list 0, the first rebuild bins into list 1) and the flags
+// F[0] and F[1]; for the split FIRE step (LOOP_FIRE) the flags of its first drift's destination.
+enum : int { LOOP_MD = 1, LOOP_FIRE = 2 };
+FillSegs loop_fills(dpm_set_s* S, int kind) {
+  FillSegs f{};
+  f.add(S->d_err, 0, 1);
+  if (kind & LOOP_MD) {
+    f.add(S->mdCount[0], 0, 2L * (S->G.ncells > 0 ? S->G.ncells : 1));
+    f.add(S->mdFlag[0], 0, S->nsys);
+    f.add(S->mdFlag[1], 0, S->nsys);
+  }
+  if (kind & LOOP_FIRE) {
+    f.add(S->d_flag[1 - S->cur], 0, S->nsys);
+    f.add(S->d_any + 1 - S->cur, 0, 1);
+  }
+  return f;
+}
+
+// RNG calls of a loop, by which its end advances the counters
+struct Draws {
+  long long thermal = 0, active = 0;
+};
+
+// Run `loop` (which leaves its errors in d_err) from a copy of the state it changes (SNAP_* bits
+// `what`), and again on a wider list for as long as it reports ERR_LIST_OVERFLOW; returns the loop's
+// status.  Copy and clears are one launch, counters and status another, and the host waits once per run.
 template <class F>
-int with_replay(dpm_set_s* S, int what, F loop) {
-  int rc = snap_save(S, what);
+int with_replay(dpm_set_s* S, int what, int kind, Draws draws, F loop) {
+  int rc = snap_save(S, what, loop_fills(S, kind));
   if (rc) return rc;
   for (int attempt = 0; attempt < 6; attempt++) {
-    HIPCHK(launch_fill_int(S->d_err, 0, 1, S->stream));
+    if (attempt > 0) HIPCHK(launch_prologue(CopySegs{}, loop_fills(S, kind), S->stream));
     rc = loop();
     if (rc) return rc;
-    int err = 0;
-    HIPCHK(hipMemcpyAsync(&err, S->d_err, sizeof(int), hipMemcpyDeviceToHost, S->stream));
+    HIPCHK(launch_loop_end(S, draws.thermal, draws.active, what & SNAP_FIRE ? S->d_fire[S->fireCur] : nullptr));
     HIPCHK(hipStreamSynchronize(S->stream));
+    const int err = S->h_stat->err;
     if (!(err & ERR_LIST_OVERFLOW)) return loop_status(S, err);
     rc = snap_restore(S, what);
     if (rc) return rc;
@@ -517,15 +539,6 @@ bool near_loop(const dpm_set_s* S, long steps) {
   return S->N.task && steps >= NEAR_STEPS && (S->P.interaction == INT_VV || S->P.interaction == INT_SMOOTH);
 }
 
-// A step loop's cell protocol at its start: cell lists 0 and 1 cleared (the start kernel bins
-// the list positions into list 0, the first rebuild bins into list 1) and the flags of the first
-// step's drift destination F[1] cleared.
-int md_start(dpm_set_s* S) {
-  HIPCHK(launch_fill_int(S->mdCount[0], 0, 2L * (S->G.ncells > 0 ? S->G.ncells : 1), S->stream));
-  HIPCHK(launch_fill_int(S->mdFlag[1], 0, S->nsys, S->stream));
-  return DPM_OK;
-}
-
 long long active_draws(const dpm_set_s* S, long steps) { return S->P.particle != PART_PASSIVE ? steps : 0; }
 
 // Launch sequence of a velocity-Verlet loop (NVE / Langevin):
@@ -533,15 +546,12 @@ long long active_draws(const dpm_set_s* S, long steps) { return S->P.particle !=
 //          (buffer b -> 1-b)
 //   per step: step [rebuild rows if flagged; F(x'); thermostat; v += dt/2 F;
 //             unless last: v += dt/2 F, x'' = x' + dt v, displacement test of x'']
-//   end: RNG call counters advanced by the loop's draws.
 // The fused form performs the reference's operations in the reference's order.
 // With `rec` (slots of 2 nv doubles, x then y), the position after step i is also written to
 // slot i + 1 (the adjoint's recomputed segment).
 int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullptr) {
   const bool near = near_loop(S, steps);
   const long nv = S->nv;
-  int rc = md_start(S);
-  if (rc) return rc;
   if (rec) {
     // a recomputed segment starts from a restored checkpoint without a valid list: its list
     // positions become the start positions (whose cells the start kernel bins), and every
@@ -566,7 +576,6 @@ int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullp
     HIPCHK(launch_step(S, mode, A));
     if (more) swap_pos(S);
   }
-  HIPCHK(launch_ctr_add(S, langevin ? steps : 0, active_draws(S, steps)));
   return DPM_OK;
 }
 
@@ -575,8 +584,6 @@ int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullp
 // loop draws at counter ctr[0] + k.
 int baoab_sequence(dpm_set_s* S, long steps) {
   const bool near = near_loop(S, steps);
-  int rc = md_start(S);
-  if (rc) return rc;
   HIPCHK(launch_start_baoab(S, md_args(S, 0, 0, 0, near)));
   swap_pos(S);
   for (long i = 1; i <= steps; i++) {
@@ -585,7 +592,6 @@ int baoab_sequence(dpm_set_s* S, long steps) {
                        md_args(S, i, i, i - 1, near)));
     if (more) swap_pos(S);
   }
-  HIPCHK(launch_ctr_add(S, steps, active_draws(S, steps)));
   return DPM_OK;
 }
 
@@ -595,9 +601,6 @@ int baoab_sequence(dpm_set_s* S, long steps) {
 // test of x'].
 int brown_sequence(dpm_set_s* S, long steps, bool noisy) {
   // step i has rotation index i - 1: the prologue writes the flags F[0] and generations G[0]
-  int rc = md_start(S);
-  if (rc) return rc;
-  HIPCHK(launch_fill_int(S->mdFlag[0], 0, S->nsys, S->stream));
   const bool near = near_loop(S, steps);
   HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   for (long i = 1; i <= steps; i++) {
@@ -606,7 +609,6 @@ int brown_sequence(dpm_set_s* S, long steps, bool noisy) {
     HIPCHK(launch_step(S, mode, A));
     swap_pos(S);
   }
-  HIPCHK(launch_ctr_add(S, noisy ? steps : 0, active_draws(S, steps)));
   return DPM_OK;
 }
 
@@ -671,7 +673,9 @@ int run_verlet(dpm_set_s* S, long steps, bool langevin) {
   if (steps <= 0) return DPM_OK;
   int rc = require_list(S);
   if (rc) return rc;
-  return with_replay(S, 0, [&]() { return run_verlet_once(S, steps, langevin); });
+  const bool noisy = langevin && S->noiseType != NOISE_DRIVEN_BROWNIAN;
+  return with_replay(S, 0, LOOP_MD, Draws{noisy ? steps : 0, active_draws(S, steps)},
+                     [&]() { return run_verlet_once(S, steps, langevin); });
 }
 
 int fire_iteration(dpm_set_s* S) {
@@ -683,8 +687,6 @@ int fire_iteration(dpm_set_s* S) {
 }
 
 int fire_sequence(dpm_set_s* S, long iterations) {
-  HIPCHK(launch_fill_int(S->d_flag[1 - S->cur], 0, S->nsys, S->stream));
-  HIPCHK(launch_fill_int(S->d_any + 1 - S->cur, 0, 1, S->stream));
   HIPCHK(launch_fire_partials(S));
   for (long i = 0; i < iterations; i++) {
     int rc = fire_iteration(S);
@@ -726,11 +728,13 @@ int temperature_scale(dpm_set_s* S, double T) {
 // Flags, any-flags and both parities' cell counts cleared: the state the forward loops and the
 // adjoint's own rebuild protocol both start from.
 int clean_protocol(dpm_set_s* S) {
-  HIPCHK(launch_fill_int(S->d_flag[0], 0, S->nsys, S->stream));
-  HIPCHK(launch_fill_int(S->d_flag[1], 0, S->nsys, S->stream));
-  HIPCHK(launch_fill_int(S->d_any, 0, 2, S->stream));
-  HIPCHK(launch_fill_int(S->G.count[0], 0, S->G.ncells, S->stream));
-  HIPCHK(launch_fill_int(S->G.count[1], 0, S->G.ncells, S->stream));
+  FillSegs f{};
+  f.add(S->d_flag[0], 0, S->nsys);
+  f.add(S->d_flag[1], 0, S->nsys);
+  f.add(S->d_any, 0, 2);
+  f.add(S->G.count[0], 0, S->G.ncells);
+  f.add(S->G.count[1], 0, S->G.ncells);
+  HIPCHK(launch_prologue(CopySegs{}, f, S->stream));
   return DPM_OK;
 }
 
@@ -813,14 +817,19 @@ int record_segment(dpm_set_s* S, long len) {
   const long nv = S->nv;
   HIPCHK(launch_copy_d(S->d_seg, S->V.x, nv, S->stream));
   HIPCHK(launch_copy_d(S->d_seg + nv, S->V.y, nv, S->stream));
+  FillSegs fills = loop_fills(S, LOOP_MD);
+  fills.words[0] = 0;  // the error word gathers over the whole reverse pass
+  HIPCHK(launch_prologue(CopySegs{}, fills, S->stream));
   int rc;
   if (len < 4 || !graphs_enabled()) {
     rc = verlet_sequence(S, len, false, S->d_seg);
-    return rc;
+    if (rc) return rc;
+  } else {
+    rc = run_graph(S, std::make_tuple(4, len, S->cur), [&]() { return verlet_sequence(S, len, false, S->d_seg); });
+    if (rc) return rc;
+    if ((len % 2) == 1) swap_pos(S);
   }
-  rc = run_graph(S, std::make_tuple(4, len, S->cur), [&]() { return verlet_sequence(S, len, false, S->d_seg); });
-  if (rc) return rc;
-  if ((len % 2) == 1) swap_pos(S);
+  if (S->P.particle != PART_PASSIVE) HIPCHK(launch_ctr_add(S, 0, active_draws(S, len)));
   return DPM_OK;
 }
 
@@ -971,14 +980,11 @@ int rigid_clear(dpm_set_s* S) {
 //   start: half kick of the rings, centres and angles advanced, vertices moved (buffer b -> 1-b)
 //   per step: step [rebuild flagged rows; interaction F(x'); ring force, torque, moment of
 //             inertia; half kick; unless last: the next step's half kick and move]
-//   end: thermal call counter advanced by the loop's draws.
 // Both run the velocity-Verlet loop's protocol (a rebuilding step builds its rows from the cells
 // of the list positions and bins the new ones).  Langevin's kick adds unit Gaussian draws to the
 // ring velocities whatever the time step, so a ring can move far in one step: a drift longer than
 // cutoff / 3 flags its system FLAG_FAR, whose next rebuild searches all the system's vertices.
 int rigid_sequence(dpm_set_s* S, long steps, bool langevin) {
-  int rc = md_start(S);
-  if (rc) return rc;
   const bool near = near_loop(S, steps);
   HIPCHK(launch_rigid_start(S, langevin, md_args(S, 0, 0, 0, near)));
   swap_pos(S);
@@ -989,7 +995,6 @@ int rigid_sequence(dpm_set_s* S, long steps, bool langevin) {
     HIPCHK(launch_step(S, MODE_RIGID | MODE_KICK | (more ? MODE_START : 0) | (near ? MODE_NEAR : 0), A));
     if (more) swap_pos(S);
   }
-  if (langevin) HIPCHK(launch_ctr_add(S, steps, 0));
   return DPM_OK;
 }
 
@@ -998,7 +1003,7 @@ int run_rigid(dpm_set_s* S, long steps, bool langevin) {
   int rc = rigid_supported(S);
   if (rc) return rc;
   auto seq = [&]() -> int { return rigid_sequence(S, steps, langevin); };
-  return with_replay(S, SNAP_RIGID, [&]() -> int {
+  return with_replay(S, SNAP_RIGID, LOOP_MD, Draws{langevin ? steps : 0, 0}, [&]() -> int {
     if (steps < 4 || !graphs_enabled()) return seq();
     int r = run_graph(S, std::make_tuple(langevin ? 20 : 21, steps, S->cur), seq);
     if (!r && (steps % 2) == 1) swap_pos(S);
@@ -1016,9 +1021,6 @@ int rigid_fire_sequence(dpm_set_s* S, long iterations) {
   // F[i] (a drift longer than cutoff / 3 flags FLAG_FAR), and its step (rotation index i) reads
   // F[i], rebuilds flagged systems from the list-position cells (all pairs on FLAG_FAR) and clears
   // F[i + 2] for the move after next
-  int rc = md_start(S);
-  if (rc) return rc;
-  HIPCHK(launch_fill_int(S->mdFlag[0], 0, S->nsys, S->stream));
   const bool near = near_loop(S, iterations);
   HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   HIPCHK(launch_rigid_fire_partials(S));
@@ -1150,7 +1152,8 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   S->redBlocks = (int)chunkSys.size();
   A(S->d_red, (long)S->redBlocks * 8); A(S->d_scale, numSystems);
   A(S->d_chunkSys, S->redBlocks); A(S->d_chunkOff, numSystems + 1);
-  if (hipHostMalloc((void**)&S->h_red, sizeof(double) * numSystems * 8) != hipSuccess) {
+  if (hipHostMalloc((void**)&S->h_red, sizeof(double) * numSystems * 8) != hipSuccess ||
+      hipHostMalloc((void**)&S->h_stat, sizeof(HostStat)) != hipSuccess) {
     dpm_destroy(S);
     return DPM_ERR_OOM;
   }
@@ -1246,6 +1249,7 @@ int dpm_destroy(dpm_set_t h) {
   for (void* p : ptrs)
     if (p) hipFree(p);
   if (S->h_red) hipHostFree(S->h_red);
+  if (S->h_stat) hipHostFree(S->h_stat);
   if (S->ownStream) hipStreamDestroy(S->ownStream);
   delete S;
   return DPM_OK;
@@ -1789,14 +1793,13 @@ int dpm_nve_rescale_loop(dpm_set_t h, long steps) {
   if (S->simKind != 3) return fail(S, DPM_ERR_STATE, "dpm_init_nve_rescale not called");
   int rc = require_list(S);
   if (rc) return rc;
-  HIPCHK(launch_fill_int(S->d_err, 0, 1, S->stream));
   for (long i = 0; i < steps; i++) {
     rc = temperature_scale(S, S->Tinject);  // NVERescale::injectKineticEnergy, Simulator.cu:222-238
     if (rc) return rc;
-    rc = with_replay(S, 0, [&]() { return verlet_sequence(S, 1, false); });
+    rc = with_replay(S, 0, LOOP_MD, Draws{0, active_draws(S, 1)}, [&]() { return verlet_sequence(S, 1, false); });
     if (rc) return rc;
   }
-  return check_err_after_loop(S);
+  return DPM_OK;
 }
 
 int dpm_adjust_temperature(dpm_set_t h, double T) {
@@ -1854,7 +1857,7 @@ int dpm_fire_loop(dpm_set_t h, long iterations) {
     S->fp.tol = -1;
     bump(S);
   }
-  return with_replay(S, SNAP_FIRE, [&]() { return run_fire(S, iterations); });
+  return with_replay(S, SNAP_FIRE, LOOP_FIRE, Draws{}, [&]() { return run_fire(S, iterations); });
 }
 
 // The compressFIRE.cpp:121-131 loop for every system at once.  A system whose max |F_c| has
@@ -1871,7 +1874,6 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
     S->fp.maxIter = maxIter;
     bump(S);
   }
-  HIPCHK(launch_fill_int(S->d_err, 0, 1, S->stream));
   HIPCHK(launch_fire_resume(S));
   long done = 0;
   if (S->fireKernel == 1 && S->P.particle == PART_PASSIVE && S->P.geometry == GEOM_NORMAL && S->nwide == 0) {
@@ -1886,32 +1888,22 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
     }
     const long pchunk = 2048;
     while (done <= maxIter) {
-      rc = with_replay(S, SNAP_FIRE, [&]() -> int {
+      rc = with_replay(S, SNAP_FIRE, 0, Draws{}, [&]() -> int {
         HIPCHK(launch_fire_sys(S, (int)pchunk, waves));
         return DPM_OK;
       });
       if (rc) return rc;
       done += pchunk;
-      int notDone = 0;
-      HIPCHK(launch_fill_int(S->d_notDone, 0, 1, S->stream));
-      HIPCHK(launch_fire_done(S, S->d_notDone));
-      HIPCHK(hipMemcpyAsync(&notDone, S->d_notDone, sizeof(int), hipMemcpyDeviceToHost, S->stream));
-      HIPCHK(hipStreamSynchronize(S->stream));
-      if (!notDone) break;
+      if (!S->h_stat->notDone) break;
     }
     done = maxIter + 1;  // the graph path below is skipped
   }
   const long chunk = 256;
   while (done <= maxIter) {
-    rc = with_replay(S, SNAP_FIRE, [&]() { return run_fire(S, chunk); });
+    rc = with_replay(S, SNAP_FIRE, LOOP_FIRE, Draws{}, [&]() { return run_fire(S, chunk); });
     if (rc) return rc;
     done += chunk;
-    int notDone = 0;
-    HIPCHK(launch_fill_int(S->d_notDone, 0, 1, S->stream));
-    HIPCHK(launch_fire_done(S, S->d_notDone));
-    HIPCHK(hipMemcpyAsync(&notDone, S->d_notDone, sizeof(int), hipMemcpyDeviceToHost, S->stream));
-    HIPCHK(hipStreamSynchronize(S->stream));
-    if (!notDone) break;
+    if (!S->h_stat->notDone) break;
   }
   if (iterations) {
     std::vector<FireState> fs(S->nsys);
@@ -1920,7 +1912,7 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
     HIPCHK(hipStreamSynchronize(S->stream));
     for (long s = 0; s < S->nsys; s++) iterations[s] = fs[s].iters;
   }
-  return check_err_after_loop(S);
+  return DPM_OK;
 }
 
 int dpm_set_fire_kernel(dpm_set_t h, int persistent, int wavesPerSystem) {
@@ -2402,8 +2394,7 @@ int dpm_nve_forward(dpm_set_t h, long steps, long every) {
   }
   rc = save_state(S, S->d_fin, rings);
   if (rc) return rc;
-  rc = check_err_after_loop(S);
-  if (rc) return rc;
+  HIPCHK(hipStreamSynchronize(S->stream));
   S->tapeSteps = steps;
   S->tapeEvery = every;
   S->tapeNck = nck;
@@ -2439,7 +2430,7 @@ int dpm_fire_forward(dpm_set_t h, long iterations) {
   }
   // every iteration one at a time, its starting state recorded before it and its FIRE scalars
   // after its parameter update; replayed on a wider list as the loops are
-  rc = with_replay(S, SNAP_FIRE, [&]() -> int {
+  rc = with_replay(S, SNAP_FIRE, LOOP_FIRE, Draws{}, [&]() -> int {
     for (long k = 0; k < iterations; k++) {
       int r = save_state(S, S->d_ftape + k * 6 * nv);
       if (r) return r;
@@ -2679,7 +2670,7 @@ int dpm_rigid_fire_loop(dpm_set_t h, long iterations) {
   int rc = rigid_supported(S);
   if (rc) return rc;
   if (iterations <= 0) return DPM_OK;
-  return with_replay(S, SNAP_RIGID_FIRE, [&]() -> int {
+  return with_replay(S, SNAP_RIGID_FIRE, LOOP_MD, Draws{}, [&]() -> int {
     if (iterations < 4 || !graphs_enabled()) return rigid_fire_sequence(S, iterations);
     // the sequence flips the position and FIRE-state buffers once per iteration
     int r = run_graph(S, std::make_tuple(22 + S->rfireCur, iterations, S->cur),

@@ -111,6 +111,25 @@ struct CopySegs {
   int n;
 };
 
+// Up to kMaxFills int arrays set to a value in the same launch.
+constexpr int kMaxFills = 8;
+struct FillSegs {
+  int* p[kMaxFills];
+  long words[kMaxFills];
+  int value[kMaxFills];
+  int n;
+  void add(int* ptr, int v, long w) {
+    p[n] = ptr;
+    value[n] = v;
+    words[n++] = w;
+  }
+};
+
+// What the loops and list builds leave for the host, in pinned memory their last kernel writes.
+struct HostStat {
+  int err, maxcnt, notDone;
+};
+
 // Arguments of the H w kernel (dpm_adjoint.hip).
 struct AdjArgs {
   const int* flag;      // rebuild flags of this parity (rows rebuilt first when set), or null
@@ -222,6 +241,7 @@ struct dpm_set_s {
   double* h_red = nullptr;   // per-system outputs [nsys * 8], pinned host memory the kernels write
   int *d_chunkSys = nullptr, *d_chunkOff = nullptr;  // block -> system, system -> first block
   int redBlocks = 0;
+  dpm::HostStat* h_stat = nullptr;  // pinned host memory
   double* d_scale = nullptr; // per-system scalars
 
   // adjoint tape (dpm_nve_forward / dpm_nve_backward)
@@ -285,7 +305,6 @@ hipError_t launch_fire_begin(dpm_set_s* S);
 hipError_t launch_fire_mid(dpm_set_s* S);
 hipError_t launch_fire_partials(dpm_set_s* S);
 hipError_t launch_fire_step(dpm_set_s* S);
-hipError_t launch_fire_done(dpm_set_s* S, int* notDone);
 hipError_t launch_fire_resume(dpm_set_s* S);
 StepArgs loop_args(dpm_set_s* S);
 hipError_t launch_bin_view(dpm_set_s* S, const View& Vn, int parity);
@@ -307,7 +326,9 @@ hipError_t launch_displacement(dpm_set_s* S, const double* x, const double* y, c
                                long n, int rings, double waveNum, double* d2, double* sf);
 hipError_t launch_particle_stress(dpm_set_s* S, double* out);
 hipError_t launch_copy_d(double* dst, const double* src, long n, hipStream_t st);
-hipError_t launch_copy_segs(const CopySegs& segs, hipStream_t st);
+hipError_t launch_prologue(const CopySegs& segs, const FillSegs& fills, hipStream_t st);
+hipError_t launch_loop_end(dpm_set_s* S, long long addT, long long addA, const FireState* fs);
+hipError_t launch_rebuild_end(dpm_set_s* S, const FillSegs& fills);
 hipError_t launch_axpy(double* y, const double* x, double alpha, long n, hipStream_t st);
 hipError_t launch_build_rows_view(dpm_set_s* S, const View& Vn, int parity, int countUpdates);
 hipError_t launch_rigid_start(dpm_set_s* S, bool langevin, const StepArgs& A);

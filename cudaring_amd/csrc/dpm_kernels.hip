@@ -764,12 +764,6 @@ __global__ void k_fire_partials(View V, double* part) {
   }
 }
 
-// per-system FIRE summary after a minimisation: all-converged flag
-__global__ void k_fire_done(const FireState* fs, int nsys, int* notDone) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < nsys && !fs[s].converged) atomicOr(notDone, 1);
-}
-
 // a new minimisation call tests every system's stopping rule again (the driver's loop condition
 // is evaluated per call, compressFIRE.cpp:121-131)
 __global__ void k_fire_resume(FireState* fs, int nsys) {
@@ -1046,11 +1040,6 @@ hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves) {
 
 hipError_t launch_fire_resume(dpm_set_s* S) {
   k_fire_resume<<<grid_v(S->nsys), 256, 0, S->stream>>>(S->d_fire[S->fireCur], (int)S->nsys);
-  return hipGetLastError();
-}
-
-hipError_t launch_fire_done(dpm_set_s* S, int* notDone) {
-  k_fire_done<<<grid_v(S->nsys), 256, 0, S->stream>>>(S->d_fire[S->fireCur], (int)S->nsys, notDone);
   return hipGetLastError();
 }
 
