@@ -182,9 +182,10 @@ __device__ __forceinline__ void build_near_wave(const View& V, const Params& P, 
 // workgroup calls it (it holds barriers); lds holds rows_lds_ints(W, NEAR >= 0) ints; the caller
 // synchronises before reading the rows or reusing lds.
 //
-// Bound by latency: a chain of dependent loads (cell count, slot, position), shortened by fetching
-// ahead, and the fetch of its own instructions, which a rebuild runs cold (eight candidates unrolled
-// took longer than one after another); a vertex of the own ring is told by its index.
+// Bound by latency: a chain of dependent loads (cell count, slots, positions), shortened by fetching
+// ahead and four candidates at a time, and the fetch of its own instructions, which a rebuild runs cold
+// (eight candidates unrolled took longer than one after another).  A vertex of the own ring is told by
+// its index.  maxcnt: longest row for the host, or null (inside loops: one word for every tile).
 template <int NEAR>
 __device__ __forceinline__ void build_rows_tile(const View& V, const Params& P, const CellGrid& G, const int* count,
                                                 const int* slots, const Lane& L, int w, int nw, const Box& B, double x,
@@ -210,33 +211,42 @@ __device__ __forceinline__ void build_rows_tile(const View& V, const Params& P, 
       xx += xx < 0 ? ncx : (xx >= ncx ? -ncx : 0);
       return c0 + yy * ncx + xx;
     };
-    for (int k = w; k < 9; k += nw) {
-      const int cl = cell(k), m = min(count[cl], G.cap);
-      const int* sl = slots + (long)cl * G.cap;
-      // two candidates ahead: the slot of one, the position of the next
-      int j = 0, jn = 0;
-      double xj = 0, yj = 0, rj = 0;
-      if (m > 0) {
-        j = sl[0];
-        jn = sl[m > 1 ? 1 : 0];
-        xj = V.x[j];
-        yj = V.y[j];
-        rj = V.rad[j];
-      }
+    // a cell's count and first four slots are fetched while the cell before it is searched (slots past
+    // the count hold older vertices: in bounds, and not tested)
+    int cl = cell(w);
+    int m = count[cl];
+    int4 sj = *(const int4*)(slots + (long)cl * G.cap);
 #pragma unroll 1
-      for (int q = 0; q < m; q++) {
-        const int jc = j;
-        const double dx = pbx(x - xj, B), dy = pby(y - yj, B), sum = rv + rj;
-        j = jn;
-        jn = sl[q + 2 < m ? q + 2 : m - 1];
-        xj = V.x[j];
-        yj = V.y[j];
-        rj = V.rad[j];
-        if ((unsigned)(jc - L.f) >= (unsigned)L.n && in_list(P, dx * dx + dy * dy, sum)) {
-          const int idx = atomicAdd(&lcnt[lane], 1);
-          if (idx < W) lrow[idx * WAVE + lane] = jc;
+    for (int k = w; k < 9; k += nw) {
+      const int cn = cell(k + nw < 9 ? k + nw : k);
+      const int mn = count[cn];
+      const int4 sn = *(const int4*)(slots + (long)cn * G.cap);
+      const int* sl = slots + (long)cl * G.cap;
+      m = min(m, G.cap);
+#pragma unroll 1
+      for (int q = 0; q < m; q += 4) {
+        const int j[4] = {sj.x, sj.y, sj.z, sj.w};
+        double xj[4], yj[4], rj[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int u = q + i < m ? j[i] : v;
+          xj[i] = V.x[u];
+          yj[i] = V.y[u];
+          rj[i] = V.rad[u];
+        }
+        if (q + 4 < m) sj = *(const int4*)(sl + q + 4);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const double dx = pbx(x - xj[i], B), dy = pby(y - yj[i], B);
+          if (q + i < m && (unsigned)(j[i] - L.f) >= (unsigned)L.n && in_list(P, dx * dx + dy * dy, rv + rj[i])) {
+            const int idx = atomicAdd(&lcnt[lane], 1);
+            if (idx < W) lrow[idx * WAVE + lane] = j[i];
+          }
         }
       }
+      cl = cn;
+      m = mn;
+      sj = sn;
     }
   }
   double xp = 0, yp = 0;
@@ -250,7 +260,7 @@ __device__ __forceinline__ void build_rows_tile(const View& V, const Params& P, 
   const int n = c < W ? c : W;
   if (w == 0 && L.act) {
     if (c > W) atomicOr(err, ERR_LIST_OVERFLOW);
-    atomicMax(maxcnt, c);
+    if (maxcnt) atomicMax(maxcnt, c);
     V.ncnt[v] = n;
     V.lx[v] = x;
     V.ly[v] = y;

@@ -91,7 +91,7 @@ __device__ void build_row(const View& V, const Params& P, const CellGrid& G, con
     }
   }
   if (c > W) atomicOr(err, ERR_LIST_OVERFLOW);
-  atomicMax(maxcnt, c);
+  if (maxcnt) atomicMax(maxcnt, c);
   V.ncnt[v] = c < W ? c : W;
   V.lx[v] = x;
   V.ly[v] = y;

@@ -52,15 +52,6 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
         slots = M.slots;
         if (!A.rowsBuilt) {
           if (w == 0 && L.act && !allPairs) md_stale_test(V, P, B, L.v, x, y, A.err);
-          // these positions are the system's next list positions (its rows are built from them)
-          if (w == nw - 1 && L.act) bin_vertex(G, B, M.binCnt, M.binSlots, L.v, L.s, x, y, A.err);
-          if (!G.brute[L.s]) {
-            const int t0 = V.stile[L.s], nt = V.stile[L.s + 1] - t0;
-            const int n = G.ncx[L.s] * G.ncy[L.s];
-            int* clr = M.clear + G.coff[L.s];
-            for (int c = (L.tile - t0) * (int)blockDim.x + (int)threadIdx.x; c < n; c += nt * (int)blockDim.x)
-              clr[c] = 0;
-          }
         }
       }
     }
@@ -68,15 +59,28 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
     // the cell search shared by the tile's waves (rows in LDS) where the launch sized LDS for it
     const bool tileBuild = rebuild && !A.rowsBuilt && !allPairs && A.rowsLdsW == V.W && !G.brute[L.s];
     if (tileBuild) {
-      build_rows_tile<NEAR ? INTER : -1>(V, P, G, cells, slots, L, w, nw, B, x, y, (int*)red, A.err, A.maxcnt, A.near);
+      build_rows_tile<NEAR ? INTER : -1>(V, P, G, cells, slots, L, w, nw, B, x, y, (int*)red, A.err, nullptr, A.near);
     } else if (rebuild && w == 0 && L.act && !A.rowsBuilt) {
-      build_row(V, P, G, cells, slots, L.v, L.s, B, A.err, A.maxcnt, allPairs);
+      build_row(V, P, G, cells, slots, L.v, L.s, B, A.err, nullptr, allPairs);
     }
     if (rebuild) __syncthreads();
     if constexpr (NEAR) {
       if (rebuild && !tileBuild) {
         build_near_tile<INTER>(V, P, A.near, L, w, nw, B, V.x, V.y, G.brute[L.s] != 0, red);
         __syncthreads();
+      }
+    }
+    if (rebuild && A.genCur && !A.rowsBuilt && w == nw - 1) {
+      // these positions are the system's next list positions (its rows are built from them): binned into
+      // the next cell list, the one after cleared.  Nothing in this launch reads either, so one wave does
+      // it behind the rebuild's barriers, which would wait for the bins' atomics.
+      const MdCells M = md_cells(A, G, A.genCur[L.s]);
+      if (L.act) bin_vertex(G, B, M.binCnt, M.binSlots, L.v, L.s, x, y, A.err);
+      if (!G.brute[L.s]) {
+        const int t0 = V.stile[L.s], nt = V.stile[L.s + 1] - t0;
+        const int n = G.ncx[L.s] * G.ncy[L.s];
+        int* clr = M.clear + G.coff[L.s];
+        for (int c = (L.tile - t0) * WAVE + L.lane; c < n; c += nt * WAVE) clr[c] = 0;
       }
     }
   }
