@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "dpm_internal.h"
+#include "dpm_launch.h"
 #include "dpm_near.h"
 #include "dpm_rows.h"
 #include "dpm_tile.h"
@@ -575,7 +576,7 @@ hipError_t launch_adj_hvp(dpm_set_s* S, const View& Vn, AdjArgs A) {
   A.err = S->d_err;
   A.maxcnt = S->d_maxcnt;
   A.xcd = S->xcdMap;
-  const unsigned g = (unsigned)S->V.ntiles, b = WAVE * S->split;
+  const unsigned g = (unsigned)S->V.ntiles, b = WAVE * loop_waves(S);
   hipStream_t st = S->stream;
   // rows rebuilt by the whole workgroup need rows_lds_ints of LDS (W <= 64), in the region the gather
   // wave, W <= 64), in the region the gather partials use afterwards
@@ -583,7 +584,7 @@ hipError_t launch_adj_hvp(dpm_set_s* S, const View& Vn, AdjArgs A) {
   A.rowsLdsW = tileRows ? S->V.W : 0;
   const size_t rows = tileRows ? (size_t)rows_lds_ints(S->V.W, false) * sizeof(int) : 0;
   if (S->P.interaction == INT_SMOOTH) {
-    const size_t sh = std::max((size_t)(S->split - 1) * 4 * WAVE * sizeof(double), rows);
+    const size_t sh = std::max((size_t)(loop_waves(S) - 1) * 4 * WAVE * sizeof(double), rows);
     switch (S->P.potential) {
       case POT_HARMONIC: k_adj_hvp<INT_SMOOTH, POT_HARMONIC><<<g, b, sh, st>>>(Vn, S->P, S->G, A); break;
       case POT_LJ: k_adj_hvp<INT_SMOOTH, POT_LJ><<<g, b, sh, st>>>(Vn, S->P, S->G, A); break;
@@ -592,7 +593,7 @@ hipError_t launch_adj_hvp(dpm_set_s* S, const View& Vn, AdjArgs A) {
     }
     return hipGetLastError();
   }
-  const size_t sh = std::max((size_t)(S->split - 1) * 2 * WAVE * sizeof(double), rows);
+  const size_t sh = std::max((size_t)(loop_waves(S) - 1) * 2 * WAVE * sizeof(double), rows);
   switch (S->P.potential) {
     case POT_HARMONIC: k_adj_hvp<INT_VV, POT_HARMONIC><<<g, b, sh, st>>>(Vn, S->P, S->G, A); break;
     case POT_LJ: k_adj_hvp<INT_VV, POT_LJ><<<g, b, sh, st>>>(Vn, S->P, S->G, A); break;

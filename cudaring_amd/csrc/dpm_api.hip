@@ -709,6 +709,38 @@ int run_fire(dpm_set_s* S, long iterations) {
   return DPM_OK;
 }
 
+// FIRE iterations on every tile of the set, two launches each: the move (parameter update, drift and
+// displacement flags of every system, from tile partials) and the step kernel on near lists, with the
+// step loop's cell protocol as rigid FIRE runs it.  Stream launches: the host stays ahead of kernels of
+// five microseconds, and every dpm_init_fire would capture a graph anew.
+int fire_tile_sequence(dpm_set_s* S, long iterations) {
+  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], S->N));
+  HIPCHK(launch_fire_partials(S));
+  for (long it = 0; it < iterations; it++) {
+    HIPCHK(launch_fire_move(S, S->mdFlag[it % 3], S->d_any + 2));
+    S->fireCur = 1 - S->fireCur;
+    swap_pos(S);
+    StepArgs A = md_args(S, it, 0, 0, true);
+    A.fire = S->d_fire[S->fireCur];
+    A.part = S->d_part;
+    HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR, A));
+  }
+  return DPM_OK;
+}
+
+// Whether a minimisation of the set's systems runs on every tile rather than on one workgroup per
+// system, from what an iteration takes either way (us, harmonic vertex-vertex): 12 for the two launches
+// and 0.008 a tile of the set (measured 13.0 at 33 tiles, 13.4 at 85, 16.3 at 266, 59 at 5,333); or 3 and
+// 0.65 a tile of the largest system on its one CU, as often as the systems fill the chip (10.0 at 5
+// tiles, 13.5 at 10, 24.5 at 21, 32.6 at 33, 80 at 85 with frequent rebuilds, 31 at 60 without).
+bool fire_on_tiles(const dpm_set_s* S) {
+  if (!near_loop(S, NEAR_STEPS)) return false;
+  int most = 1;
+  for (long s = 0; s < S->nsys; s++) most = std::max(most, S->h_stile[s + 1] - S->h_stile[s]);
+  const double rounds = (double)((S->nsys + 255) / 256);
+  return 12 + 0.008 * S->V.ntiles < rounds * (3 + 0.65 * most);
+}
+
 int temperature_scale(dpm_set_s* S, double T) {
   int rc = reduce_host(S);
   if (rc) return rc;
@@ -1219,7 +1251,10 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   S->P.cutoff = 0;
   S->P.seed = 0;
   S->fp.tol = -1;
-  if (const char* e = getenv("DPM_SPLIT")) S->split = std::max(1, std::min(8, atoi(e)));
+  if (const char* e = getenv("DPM_SPLIT")) {
+    S->split = std::max(1, std::min(8, atoi(e)));
+    S->splitSet = true;
+  }
   if (const char* e = getenv("DPM_XCD_MAP")) S->xcdMap = atoi(e) != 0;
   if (alloc_list(S, 8) != DPM_OK) { dpm_destroy(S); return DPM_ERR_OOM; }
   *out = S;
@@ -1283,6 +1318,7 @@ int dpm_set_launch_config(dpm_set_t h, int wavesPerTile) {
   CHECK_HANDLE(h);
   if (wavesPerTile < 1 || wavesPerTile > 8) return fail(S, DPM_ERR_ARG, "wavesPerTile must be in 1..8");
   S->split = wavesPerTile;
+  S->splitSet = true;
   bump(S);
   return DPM_OK;
 }
@@ -1876,7 +1912,18 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
   }
   HIPCHK(launch_fire_resume(S));
   long done = 0;
-  if (S->fireKernel == 1 && S->P.particle == PART_PASSIVE && S->P.geometry == GEOM_NORMAL && S->nwide == 0) {
+  const bool plain = S->P.particle == PART_PASSIVE && S->P.geometry == GEOM_NORMAL && S->nwide == 0;
+  if (S->fireKernel < 0 && plain && fire_on_tiles(S)) {
+    const long tchunk = 256;
+    while (done < maxIter) {
+      const long n = std::min(tchunk, maxIter - done);
+      rc = with_replay(S, SNAP_FIRE, LOOP_MD, Draws{}, [&]() { return fire_tile_sequence(S, n); });
+      if (rc) return rc;
+      done += n;
+      if (!S->h_stat->notDone) break;
+    }
+    done = maxIter + 1;  // the other paths are skipped
+  } else if (S->fireKernel != 0 && plain) {
     // one workgroup per system, at most `pchunk` iterations per launch
     rc = clean_protocol(S);
     if (rc) return rc;

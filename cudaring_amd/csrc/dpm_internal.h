@@ -168,6 +168,7 @@ struct dpm_set_s {
   long nsys = 0, np = 0, nv = 0;
   std::string err;
   int split = 4;  // wavefronts per tile in the step kernel (1..8)
+  bool splitSet = false;  // by the caller, for every mode (else loop_waves in the loops)
   int xcdMap = 1; // XCD-aware workgroup -> tile mapping in the step kernel
   double cellScale = 1.0;  // cell side / (list radius + 2 cutoff / 3), >= 1 (dpm_set_cell_scale)
 
@@ -231,7 +232,8 @@ struct dpm_set_s {
   dpm::FireParams fp{};
   double* d_part = nullptr;  // per-tile partials [ntiles * 4]
   bool fireInit = false;
-  int fireKernel = 1;   // dpm_fire_minimize: 1 = one persistent workgroup per system, 0 = graph of step kernels
+  int fireKernel = -1;  // dpm_fire_minimize: 1 = one persistent workgroup per system, 0 = graph of step
+                        //   kernels, -1 = persistent or on every tile (fire_on_tiles)
   int fireWaves = 0;    // waves per system workgroup (0 = from the largest system's tile count)
   int* d_notDone = nullptr;
   int* d_sysOrder = nullptr;  // persistent FIRE: workgroup b runs system d_sysOrder[b] (most tiles first)
@@ -306,6 +308,7 @@ hipError_t launch_fire_mid(dpm_set_s* S);
 hipError_t launch_fire_partials(dpm_set_s* S);
 hipError_t launch_fire_step(dpm_set_s* S);
 hipError_t launch_fire_resume(dpm_set_s* S);
+hipError_t launch_fire_move(dpm_set_s* S, int* flagOut, int* anyOut);
 StepArgs loop_args(dpm_set_s* S);
 hipError_t launch_bin_view(dpm_set_s* S, const View& Vn, int parity);
 hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves);

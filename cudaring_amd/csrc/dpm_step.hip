@@ -6,6 +6,13 @@
 
 namespace dpm {
 
+// Single force calls and the split vertex FIRE step keep the reference's order of operations and a fixed
+// number of waves.
+template <int MODE>
+constexpr bool step_ref() {
+  return (MODE & (MODE_KICK | MODE_BROWN | MODE_NEAR)) == 0;
+}
+
 template <int INTER, int POT, int MODE>
 __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepArgs A, CellGrid G) {
   // partials of gather waves 1..nw-1: red[((w - 1) * 6 + q) * WAVE + lane], sized by the launch
@@ -15,8 +22,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   Lane L;
   constexpr bool WIDE = (MODE & MODE_WIDE) != 0;
   constexpr bool NEAR = (MODE & MODE_NEAR) != 0;
-  // single force calls and the vertex FIRE step keep the reference's order of operations
-  constexpr bool REF = (MODE & (MODE_KICK | MODE_BROWN)) == 0;
+  constexpr bool REF = step_ref<MODE>();
   constexpr int MB = MODE & ~(MODE_WIDE | MODE_NEAR);  // the integrator mode
   // A step of a velocity-Verlet, Langevin or BAOAB loop other than its last consumes the force it
   // computes in this launch (the closing and next opening half kicks); its force, energies, ring
@@ -84,6 +90,9 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       }
     }
   }
+  // FIRE on every tile: a converged system's positions, forces and partials stay as they are
+  if constexpr (NEAR && (MODE & MODE_FIRE) != 0 && (MODE & MODE_RIGID) == 0)
+    if (A.fire[L.s].converged) return;
   // wave 0's epilogue operands, fetched before the force work (lastPos after the rebuild above)
   double vx = 0, vy = 0, lx = 0, ly = 0;
   if (w == 0) {
@@ -251,9 +260,18 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
     const double f2 = L.act ? fmax(fx * fx, fy * fy) : -1.0;
     const double tP = wave_sum(pvf);
     const double tM = wave_max(f2);
+    double tV = 0, tF = 0;
+    if constexpr (NEAR) {  // the next move's sums (the split step sums them after its half kick)
+      tV = wave_sum(L.act ? vx * vx + vy * vy : 0.0);
+      tF = wave_sum(L.act ? fx * fx + fy * fy : 0.0);
+    }
     if (L.lane == 0) {
       A.part[L.tile * 4 + 0] = tP;
       A.part[L.tile * 4 + 3] = tM;
+      if constexpr (NEAR) {
+        A.part[L.tile * 4 + 1] = tV;
+        A.part[L.tile * 4 + 2] = tF;
+      }
     }
     if (!L.act) return;
     V.fx[L.v] = fx; V.fy[L.v] = fy; V.ev[L.v] = e;
@@ -320,18 +338,19 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
 // LDS of the step kernel: six partials per lane of each gather wave (eight with wide rings)
 // (or the results of the near list's evaluations), and in the same region the rows under construction
 template <int INTER, int MODE>
-static inline size_t step_lds(const dpm_set_s* S) {
+static inline size_t step_lds(const dpm_set_s* S, int nw) {
   constexpr bool STORE = (MODE & MODE_START) == 0 || (MODE & (MODE_BROWN | MODE_RIGID)) != 0;
   const size_t red = (MODE & MODE_NEAR) ? (size_t)near_slots_bytes<INTER, STORE>()
-                                        : (size_t)(S->split - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
+                                        : (size_t)(nw - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
   const size_t rows = S->V.W <= 64 ? (size_t)rows_lds_ints(S->V.W, (MODE & MODE_NEAR) != 0) * sizeof(int) : 0;
   return red > rows ? red : rows;
 }
 
 template <int INTER, int POT, int MODE>
 static hipError_t step_one(dpm_set_s* S, const StepArgs& A) {
+  const int nw = step_ref<MODE>() ? S->split : loop_waves(S);
   k_step<INTER, POT, MODE>
-      <<<S->V.ntiles, WAVE * S->split, step_lds<INTER, MODE>(S), S->stream>>>(S->V, S->P, A, S->G);
+      <<<S->V.ntiles, WAVE * nw, step_lds<INTER, MODE>(S, nw), S->stream>>>(S->V, S->P, A, S->G);
   return hipGetLastError();
 }
 
@@ -381,6 +400,7 @@ static hipError_t step_mode(dpm_set_s* S, int mode, const StepArgs& A) {
     return step_loop_mode<INTER, POT, MODE_WIDE>(S, mode, A);
   }
   if (mode & MODE_RIGID) return step_rigid<INTER, POT>(S, mode, A);
+  if (mode == (MODE_FIRE | MODE_NEAR)) return step_one<INTER, POT, MODE_FIRE | MODE_NEAR>(S, A);
   if (mode & MODE_NEAR) return step_loop_mode<INTER, POT, MODE_NEAR>(S, mode & ~MODE_NEAR, A);
   switch (mode) {
     case MODE_FORCE: return step_one<INTER, POT, MODE_FORCE>(S, A);

@@ -1,0 +1,44 @@
+"""fire_minimize on every tile of the set (the default choice for few systems) against one persistent
+workgroup per system: the same iterations, a system that stops early staying as it stopped.  The two
+add in different orders: an ulp of the forces, amplified a thousandfold per ten iterations where the
+contacts are stiff (WCA), so 20 iterations are compared there and 30 of the harmonic packing, to 1e-11."""
+import numpy as np
+import pytest
+
+from cudaring_amd import packing
+from tests.conftest import rel_err
+from tests.helpers import gpu_from_state, relaxed_state
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("pot,inter,iters", [("harmonic", "vertexVertex", 30), ("wca", "vertexSmooth", 20)])
+@pytest.mark.parametrize("sizes", [(60,), (64, 9), (70, 16, 40)])
+def test_tiles_match_persistent(pot, inter, iters, sizes):
+    systems = [relaxed_state(n, 0.8, 700 + n, final=(pot, inter)) for n in sizes]
+    cat = packing.concat_systems(systems)
+    sets = []
+    for persistent in (None, True):
+        g = gpu_from_state(cat, potential=pot, interaction=inter, costs=(1, 1, 0.1, 1),
+                           rings_per_system=cat["rings_per_system"])
+        g.calc_neighbor_list(g.set_displacement_cutoff(0.1, 2 * np.mean(cat["rad"])))
+        g.calc_force_energy()
+        dt = 0.01 * 2 * np.sqrt(np.mean(cat["a0"]) / np.pi)
+        g.init_fire([0.2, 0.5, 1.1, 0.99, dt, 10 * dt, 0.2], 20, 0)
+        if persistent:
+            g.set_fire_kernel(True, 0)
+        first = g.fire_minimize(0.0, iters)
+        # a second call whose tolerance the last system meets at once
+        tol = g.max_unbalanced_force()[-1] * 1.5 if len(sizes) > 1 else 0.0
+        second = g.fire_minimize(tol, iters + 3)
+        sets.append((g, first, second))
+    (a, fa, sa), (b, fb, sb) = sets
+    assert list(fa) == list(fb) == [iters] * len(sizes)
+    assert list(sa) == list(sb) and (len(sizes) == 1 or sa[-1] == iters)
+    for name in ("pos", "l0"):
+        assert rel_err(a.get(name), b.get(name), scale=1.0) < 1e-11
+    assert rel_err(a.get("force"), b.get("force")) < 1e-8
+    assert rel_err(a.get("energy"), b.get("energy")) < 1e-8
+    assert list(a.update_count()) == list(b.update_count())
+    for x in (a, b):
+        x.close()
