@@ -604,7 +604,8 @@ int brown_sequence(dpm_set_s* S, long steps, bool noisy) {
   const bool near = near_loop(S, steps);
   HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   for (long i = 1; i <= steps; i++) {
-    const int mode = MODE_BROWN | MODE_START | (noisy ? MODE_LANGEVIN : 0) | (near ? MODE_NEAR : 0);
+    const int mode = MODE_BROWN | MODE_START | (noisy ? MODE_LANGEVIN : 0) |
+                     (near ? MODE_NEAR | (i == steps ? MODE_OUT : 0) : 0);
     StepArgs A = md_args(S, i - 1, i - 1, i - 1, near);
     HIPCHK(launch_step(S, mode, A));
     swap_pos(S);
@@ -725,6 +726,11 @@ int fire_tile_sequence(dpm_set_s* S, long iterations) {
     A.part = S->d_part;
     HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR, A));
   }
+  StepArgs A = md_args(S, iterations, 0, 0, true);  // energies and ring geometry of the positions reached
+  A.fire = S->d_fire[S->fireCur];
+  A.part = S->d_part;
+  A.manage = 0;
+  HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR | MODE_OUT, A));
   return DPM_OK;
 }
 

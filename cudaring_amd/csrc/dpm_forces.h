@@ -266,7 +266,7 @@ __device__ __forceinline__ ShapeOut ring_shape_n(const View& V, const Params& P,
 
 // The ring centre alone (calcParticlePos, cudaKernel.cuh:365-388), as ring_shape computes it,
 // stored by the ring's first lane: the rigid rings' shape pass
-__device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, const Box& B, double x, double y) {
+__device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, const Box& B, double x, double y, bool write) {
   ShapeOut o{0, 0, 0, 0, 0};
   const double xn = shfl_d(x, L.nl), yn = shfl_d(y, L.nl);
   const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
@@ -278,7 +278,7 @@ __device__ __forceinline__ ShapeOut ring_centre(const View& V, const Lane& L, co
   const double ind = 1.0 / (double)L.n;
   o.cx = xf + sux * ind;
   o.cy = yf + suy * ind;
-  if (L.act && L.lane == L.segS) {
+  if (write && L.act && L.lane == L.segS) {
     V.cx[L.r] = o.cx;
     V.cy[L.r] = o.cy;
   }
@@ -484,7 +484,7 @@ __device__ __forceinline__ void rigid_fire_partials(const Lane& L, bool head, do
 // the next step's first half: last centre and angle stored, half kick with the next step's
 // draw, centre and angle advanced, vertices moved (RigidNVE / RigidLangevin::integrate,
 // Simulator.cu:241-252, 316-326).  With MODE_FIRE the half kick takes the system's FIRE step.
-template <int MODE, bool VV>
+template <int MODE, bool VV, bool STORE>
 __device__ __forceinline__ void rigid_epilogue(const View& V, const Params& P, const StepArgs& A, const Lane& L,
                                                const Box& B, double x, double y, double fx, double fy, double e,
                                                double cx, double cy, double lx, double ly, double z0, double z1) {
@@ -496,7 +496,7 @@ __device__ __forceinline__ void rigid_epilogue(const View& V, const Params& P, c
   const double Fy = seg_sum(L.act ? fy : 0.0, L.lane, L.segS, L.segE);
   const double T = seg_sum(L.act ? tq : 0.0, L.lane, L.segS, L.segE) / I;
   double E = 0;
-  if constexpr (VV) E = seg_sum(L.act ? e : 0.0, L.lane, L.segS, L.segE);
+  if constexpr (VV && STORE) E = seg_sum(L.act ? e : 0.0, L.lane, L.segS, L.segE);
   const bool head = L.act && L.lane == L.segS;
   double vx = 0, vy = 0, w = 0;
   if constexpr (MODE != MODE_RIGID) {
@@ -513,16 +513,18 @@ __device__ __forceinline__ void rigid_epilogue(const View& V, const Params& P, c
     rigid_fire_partials(L, head, vx, vy, Fx, Fy, A.part);
   }
   if (!L.act) return;
-  V.fx[L.v] = fx;
-  V.fy[L.v] = fy;
-  V.ev[L.v] = e;
-  R.vtq[L.v] = tq;
-  if (head) {
-    R.pfx[L.r] = Fx;
-    R.pfy[L.r] = Fy;
-    R.ptq[L.r] = T;
-    R.moi[L.r] = I;
-    if constexpr (VV) V.pe[L.r] = E;
+  if constexpr (STORE) {
+    V.fx[L.v] = fx;
+    V.fy[L.v] = fy;
+    V.ev[L.v] = e;
+    R.vtq[L.v] = tq;
+    if (head) {
+      R.pfx[L.r] = Fx;
+      R.pfy[L.r] = Fy;
+      R.ptq[L.r] = T;
+      R.moi[L.r] = I;
+      if constexpr (VV) V.pe[L.r] = E;
+    }
   }
   if constexpr (MODE == MODE_RIGID) return;
   if constexpr ((MODE & MODE_FIRE) == 0) {

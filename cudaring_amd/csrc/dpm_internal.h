@@ -21,7 +21,9 @@ namespace dpm {
 enum : int { MODE_FORCE = 0, MODE_KICK = 1, MODE_LANGEVIN = 2, MODE_START = 4, MODE_FIRE = 8, MODE_BAOAB = 16,
              MODE_BROWN = 32, MODE_RIGID = 64,
              MODE_WIDE = 128,   // the launch serves a set holding rings of more than 64 vertices
-     MODE_NEAR = 256 };  // the gather evaluates the tiles' near lists (dpm_near.h) instead of whole rows
+     MODE_NEAR = 256,   // the gather evaluates the tiles' near lists (dpm_near.h) instead of whole rows
+     MODE_OUT = 512 };  // near-list loops: a launch that stores the outputs (step_store): an overdamped
+                        // loop's last step, or (FIRE) outputs alone, after the iterations
 
 // noise types, simControlStruct::noiseEnum order (include/DPM2D.h:27)
 enum : int { NOISE_LANGEVIN = 0, NOISE_BAOAB = 1, NOISE_BROWNIAN = 2, NOISE_DRIVEN_BROWNIAN = 3 };

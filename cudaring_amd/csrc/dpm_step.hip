@@ -13,6 +13,17 @@ constexpr bool step_ref() {
   return (MODE & (MODE_KICK | MODE_BROWN | MODE_NEAR)) == 0;
 }
 
+// Whether the launch stores the force, energies, ring geometry and wall forces: what is read after a
+// loop.  A step of a velocity-Verlet, Langevin, BAOAB or rigid loop other than its last consumes the
+// force it computes (the closing and next opening half kicks); on near lists the overdamped loops and
+// FIRE store in a launch of MODE_OUT only.
+template <int MODE>
+constexpr bool step_store() {
+  if ((MODE & MODE_NEAR) != 0 && (MODE & MODE_RIGID) == 0 && (MODE & (MODE_BROWN | MODE_FIRE)) != 0)
+    return (MODE & MODE_OUT) != 0;
+  return (MODE & MODE_START) == 0 || (MODE & MODE_BROWN) != 0;
+}
+
 template <int INTER, int POT, int MODE>
 __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepArgs A, CellGrid G) {
   // partials of gather waves 1..nw-1: red[((w - 1) * 6 + q) * WAVE + lane], sized by the launch
@@ -23,11 +34,8 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   constexpr bool WIDE = (MODE & MODE_WIDE) != 0;
   constexpr bool NEAR = (MODE & MODE_NEAR) != 0;
   constexpr bool REF = step_ref<MODE>();
-  constexpr int MB = MODE & ~(MODE_WIDE | MODE_NEAR);  // the integrator mode
-  // A step of a velocity-Verlet, Langevin or BAOAB loop other than its last consumes the force it
-  // computes in this launch (the closing and next opening half kicks); its force, energies, ring
-  // geometry and wall forces are stored by the loop's last step only.
-  constexpr bool STORE = (MODE & MODE_START) == 0 || (MODE & (MODE_BROWN | MODE_RIGID)) != 0;
+  constexpr int MB = MODE & ~(MODE_WIDE | MODE_NEAR | MODE_OUT);  // the integrator mode
+  constexpr bool STORE = step_store<MODE>();
   lane_ctx<WIDE>(V, A.xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x, threadIdx.x & (WAVE - 1), L);
   const Box B = box_of(V, L.s);
   // own position first: the row rebuild below does not change it, so its load overlaps the
@@ -91,7 +99,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
     }
   }
   // FIRE on every tile: a converged system's positions, forces and partials stay as they are
-  if constexpr (NEAR && (MODE & MODE_FIRE) != 0 && (MODE & MODE_RIGID) == 0)
+  if constexpr (NEAR && (MODE & MODE_FIRE) != 0 && (MODE & (MODE_RIGID | MODE_OUT)) == 0)
     if (A.fire[L.s].converged) return;
   // wave 0's epilogue operands, fetched before the force work (lastPos after the rebuild above)
   double vx = 0, vy = 0, lx = 0, ly = 0;
@@ -144,7 +152,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   ShapeOut so{0, 0, 0};
   double zt0 = 0, zt1 = 0, ang = 0;
   if (w == 0) {
-    if constexpr ((MODE & MODE_RIGID) != 0) so = ring_centre(V, L, B, x, y);
+    if constexpr ((MODE & MODE_RIGID) != 0) so = ring_centre(V, L, B, x, y, STORE);
     else if constexpr (REF) so = ring_shape(V, P, L, B, x, y, STORE);
     else so = ring_shape_n(V, P, L, B, x, y, STORE);
     // one thermal draw per integrate call and ring: Langevin::updateThermalVel (Simulator.cu:54-77)
@@ -232,7 +240,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
     }
   }
   if constexpr ((MODE & MODE_RIGID) != 0) {
-    rigid_epilogue<MB, INTER == INT_VV>(V, P, A, L, B, x, y, fx, fy, e, so.cx, so.cy, lx, ly, zt0, zt1);
+    rigid_epilogue<MB, INTER == INT_VV, STORE>(V, P, A, L, B, x, y, fx, fy, e, so.cx, so.cy, lx, ly, zt0, zt1);
     return;
   }
   fx = so.fx + fx;
@@ -248,6 +256,10 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   if constexpr ((MODE & MODE_LANGEVIN) != 0 && (MODE & MODE_BROWN) == 0) {
     fx += P.noise * zt0 - P.gamma * vx;
     fy += P.noise * zt1 - P.gamma * vy;
+  }
+  if constexpr ((MODE & MODE_FIRE) != 0 && (MODE & MODE_OUT) != 0) {
+    if (L.act) V.ev[L.v] = e;
+    return;
   }
   if constexpr ((MODE & MODE_FIRE) != 0) {
     const FireState fs = A.fire[L.s];
@@ -274,7 +286,8 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       }
     }
     if (!L.act) return;
-    V.fx[L.v] = fx; V.fy[L.v] = fy; V.ev[L.v] = e;
+    V.fx[L.v] = fx; V.fy[L.v] = fy;
+    if constexpr (STORE) V.ev[L.v] = e;
     V.vx[L.v] = vx; V.vy[L.v] = vy;
     return;
   }
@@ -339,7 +352,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
 // (or the results of the near list's evaluations), and in the same region the rows under construction
 template <int INTER, int MODE>
 static inline size_t step_lds(const dpm_set_s* S, int nw) {
-  constexpr bool STORE = (MODE & MODE_START) == 0 || (MODE & (MODE_BROWN | MODE_RIGID)) != 0;
+  constexpr bool STORE = step_store<MODE>();
   const size_t red = (MODE & MODE_NEAR) ? (size_t)near_slots_bytes<INTER, STORE>()
                                         : (size_t)(nw - 1) * (S->nwide > 0 ? 8 : 6) * WAVE * sizeof(double);
   const size_t rows = S->V.W <= 64 ? (size_t)rows_lds_ints(S->V.W, (MODE & MODE_NEAR) != 0) * sizeof(int) : 0;
@@ -386,6 +399,13 @@ static hipError_t step_loop_mode(dpm_set_s* S, int mode, const StepArgs& A) {
     case MODE_BROWN | MODE_LANGEVIN | MODE_START:
       return step_one<INTER, POT, MODE_BROWN | MODE_LANGEVIN | MODE_START | XB>(S, A);
   }
+  if constexpr (XB == MODE_NEAR) {
+    switch (mode) {
+      case MODE_BROWN | MODE_START | MODE_OUT: return step_one<INTER, POT, MODE_BROWN | MODE_START | MODE_OUT | XB>(S, A);
+      case MODE_BROWN | MODE_LANGEVIN | MODE_START | MODE_OUT:
+        return step_one<INTER, POT, MODE_BROWN | MODE_LANGEVIN | MODE_START | MODE_OUT | XB>(S, A);
+    }
+  }
   return hipErrorInvalidValue;
 }
 
@@ -401,6 +421,7 @@ static hipError_t step_mode(dpm_set_s* S, int mode, const StepArgs& A) {
   }
   if (mode & MODE_RIGID) return step_rigid<INTER, POT>(S, mode, A);
   if (mode == (MODE_FIRE | MODE_NEAR)) return step_one<INTER, POT, MODE_FIRE | MODE_NEAR>(S, A);
+  if (mode == (MODE_FIRE | MODE_NEAR | MODE_OUT)) return step_one<INTER, POT, MODE_FIRE | MODE_NEAR | MODE_OUT>(S, A);
   if (mode & MODE_NEAR) return step_loop_mode<INTER, POT, MODE_NEAR>(S, mode & ~MODE_NEAR, A);
   switch (mode) {
     case MODE_FORCE: return step_one<INTER, POT, MODE_FORCE>(S, A);
