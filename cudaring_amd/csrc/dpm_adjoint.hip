@@ -211,13 +211,27 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_adj_hvp(View V, Params P, Ce
   if (A.cellOther)
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < A.ncells; c += gridDim.x * blockDim.x)
       A.cellOther[c] = 0;
+  if (A.flagClear)
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < V.nsys; t += gridDim.x * blockDim.x) A.flagClear[t] = 0;
   if (A.flag) {
-    const bool rebuild = A.flag[L.s] != 0;
-    if (rebuild && A.rowsLdsW == V.W && !G.brute[L.s])  // the tile's waves share the cell search
-      build_rows_tile<-1>(V, P, G, A.count, G.slots, L, w, nw, B, x, y, (int*)red, A.err, A.maxcnt, NearRows{});
+    const int flag = A.flag[L.s];
+    const bool rebuild = (flag & 1) != 0, allPairs = (flag & FLAG_FAR) != 0;
+    const int* cells = A.count;
+    const int* slots = G.slots;
+    MdCells M{};
+    if (A.genCur) {
+      const int g = A.genCur[L.s];
+      if (L.tile == V.stile[L.s] && threadIdx.x == 0) A.genOut[L.s] = rebuild ? g + 1 : g;
+      M = md_cells(A.cells, A.slots, G, g);
+      cells = M.cnt;
+      slots = M.slots;
+    }
+    if (rebuild && !allPairs && A.rowsLdsW == V.W && !G.brute[L.s])  // the tile's waves share the cell search
+      build_rows_tile<-1>(V, P, G, cells, slots, L, w, nw, B, x, y, (int*)red, A.err, A.maxcnt, NearRows{});
     else if (rebuild && w == 0 && L.act)
-      build_row(V, P, G, A.count, G.slots, L.v, L.s, B, A.err, A.maxcnt);
+      build_row(V, P, G, cells, slots, L.v, L.s, B, A.err, A.maxcnt, allPairs);
     if (rebuild) __syncthreads();
+    if (rebuild && A.genCur && w == nw - 1) md_bin_rebuilt(V, G, M, L, B, x, y, A.err);
   }
 
   // pair tangent along w: of sum_j g(d) (r_v - r_j) / d (kernelCalcVertexInteraction,
@@ -340,9 +354,10 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_adj_hvp(View V, Params P, Ce
   // Verlet-list validity at the positions processed next (checkDisplacement, DPM2D.cu:1390-1406);
   // a row rebuilt above was rebuilt by this lane, so lastPos is this lane's own write
   if (A.px) {
-    const double ddx = pbx(A.px[L.v] - V.lx[L.v], B), ddy = pby(A.py[L.v] - V.ly[L.v], B);
-    if (3 * sqrt(ddx * ddx + ddy * ddy) > P.cutoff) {
-      atomicOr(&A.flagOut[L.s], 1);
+    const double dx = A.px[L.v] - V.lx[L.v], dy = A.py[L.v] - V.ly[L.v];
+    if (moved_past(P, B, dx, dy)) {
+      // too far from its list position for the cells of those: all pairs (the step loop's protocol)
+      atomicOr(&A.flagOut[L.s], A.genCur && moved_past(P, B, dx, dy, 2.0) ? 1 | FLAG_FAR : 1);
       atomicOr(A.anyOut, 1);
     }
   }

@@ -602,7 +602,7 @@ int baoab_sequence(dpm_set_s* S, long steps) {
 int brown_sequence(dpm_set_s* S, long steps, bool noisy) {
   // step i has rotation index i - 1: the prologue writes the flags F[0] and generations G[0]
   const bool near = near_loop(S, steps);
-  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
+  HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   for (long i = 1; i <= steps; i++) {
     const int mode = MODE_BROWN | MODE_START | (noisy ? MODE_LANGEVIN : 0) |
                      (near ? MODE_NEAR | (i == steps ? MODE_OUT : 0) : 0);
@@ -715,7 +715,7 @@ int run_fire(dpm_set_s* S, long iterations) {
 // step loop's cell protocol as rigid FIRE runs it.  Stream launches: the host stays ahead of kernels of
 // five microseconds, and every dpm_init_fire would capture a graph anew.
 int fire_tile_sequence(dpm_set_s* S, long iterations) {
-  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], S->N));
+  HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], S->N));
   HIPCHK(launch_fire_partials(S));
   for (long it = 0; it < iterations; it++) {
     HIPCHK(launch_fire_move(S, S->mdFlag[it % 3], S->d_any + 2));
@@ -892,10 +892,20 @@ int backward_segment(dpm_set_s* S, long a, long top, long N) {
   HIPCHK(hipStreamSynchronize(S->stream));
   const bool single = !bad;
   auto seq = [&]() -> int {
-    int p = 0;
-    if (!single) {  // list validity at the first position processed, x_top
+    long i = 0;  // rotation index of the position's flags and generations
+    if (!single) {
+      // the step loop's cell protocol on the recorded positions, from x_top down: x_top the list
+      // positions (those of the rows just built lie half a segment away, and a system too far from its
+      // cells searches all its vertices), every system rebuilding its rows there
+      FillSegs fills = loop_fills(S, LOOP_MD);
+      fills.words[0] = 0;  // the error word gathers over the whole reverse pass
+      HIPCHK(launch_prologue(CopySegs{}, fills, S->stream));
       double* st = S->d_seg + (top - a) * 2 * nv;
-      HIPCHK(launch_adj_flag(S, view_at(S, st, st + nv), 0));
+      HIPCHK(launch_copy_d(S->V.lx, st, nv, S->stream));
+      HIPCHK(launch_copy_d(S->V.ly, st + nv, nv, S->stream));
+      HIPCHK(launch_bin_flag(S, view_at(S, st, st + nv), S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0],
+                             NearRows{}));
+      HIPCHK(launch_fill_int(S->mdFlag[0], 1, S->nsys, S->stream));
     }
     for (long n = top; n >= a; n--) {
       double* sx = S->d_seg + (n - a) * 2 * nv;
@@ -913,25 +923,25 @@ int backward_segment(dpm_set_s* S, long a, long top, long N) {
       A.mode = 1;
       A.update = n != 0;
       if (!single) {
-        // rebuild protocol of the step loop: bin the flagged systems, rebuild their rows in the
-        // kernel, which also tests the next position and clears the other parity's cells
-        HIPCHK(launch_bin_view(S, Vn, p));
-        A.flag = S->d_flag[p];
-        A.count = S->G.count[p];
-        A.cellOther = S->G.count[1 - p];
-        A.ncells = S->G.ncells;
+        // flagged systems rebuild their rows in the kernel, which also tests the next position
+        A.flag = S->mdFlag[i % 3];
+        A.cells = S->mdCount[0];
+        A.slots = S->mdSlots[0];
+        A.genCur = S->mdGen[i % 3];
+        A.genOut = S->mdGen[(i + 1) % 3];
+        A.flagOut = S->mdFlag[(i + 1) % 3];
+        A.flagClear = S->mdFlag[(i + 2) % 3];
+        A.anyOut = S->d_any + 2;  // not read
         if (n > a) {
           A.px = sx - 2 * nv;
           A.py = sx - nv;
-          A.flagOut = S->d_flag[1 - p];
-          A.anyOut = S->d_any + 1 - p;
         }
       }
       HIPCHK(launch_adj_hvp(S, Vn, A));
-      p ^= 1;
+      i++;
       S->wCur ^= 1;
     }
-    return single ? DPM_OK : clean_protocol(S);
+    return DPM_OK;
   };
   const int w0 = S->wCur;
   if (!graphs_enabled()) return seq();
@@ -1060,7 +1070,7 @@ int rigid_fire_sequence(dpm_set_s* S, long iterations) {
   // F[i], rebuilds flagged systems from the list-position cells (all pairs on FLAG_FAR) and clears
   // F[i + 2] for the move after next
   const bool near = near_loop(S, iterations);
-  HIPCHK(launch_bin_flag(S, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
+  HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], near ? S->N : NearRows{}));
   HIPCHK(launch_rigid_fire_partials(S));
   for (long it = 0; it < iterations; it++) {
     HIPCHK(launch_rigid_fire_move(S, S->mdFlag[it % 3], S->d_any + 2));

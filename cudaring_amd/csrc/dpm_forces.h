@@ -418,11 +418,25 @@ struct MdCells {
   int *binCnt, *binSlots;  // binned into
   int* clear;              // cleared
 };
-__device__ __forceinline__ MdCells md_cells(const StepArgs& A, const CellGrid& G, int g) {
+__device__ __forceinline__ MdCells md_cells(int* cells, int* slots, const CellGrid& G, int g) {
   const long C = G.ncells, CS = (long)G.ncells * G.cap;
   const int k0 = g % 3, k1 = (g + 1) % 3, k2 = (g + 2) % 3;
-  return MdCells{A.cellCur + k0 * C, A.slotsCur + k0 * CS, A.cellCur + k1 * C, A.slotsCur + k1 * CS,
-                 A.cellCur + k2 * C};
+  return MdCells{cells + k0 * C, slots + k0 * CS, cells + k1 * C, slots + k1 * CS, cells + k2 * C};
+}
+
+// A rebuild's own cells, by one wave of its tile: its positions are the system's next list positions (its
+// rows are built from them), binned into the next cell list, and the list after that cleared.  Nothing
+// in the launch reads either: the wave calls it behind the rebuild's barriers, which would wait for the
+// bins' atomics.
+__device__ __forceinline__ void md_bin_rebuilt(const View& V, const CellGrid& G, const MdCells& M, const Lane& L,
+                                               const Box& B, double x, double y, int* err) {
+  if (L.act) bin_vertex(G, B, M.binCnt, M.binSlots, L.v, L.s, x, y, err);
+  if (!G.brute[L.s]) {
+    const int t0 = V.stile[L.s], nt = V.stile[L.s + 1] - t0;
+    const int n = G.ncx[L.s] * G.ncy[L.s];
+    int* clr = M.clear + G.coff[L.s];
+    for (int c = (L.tile - t0) * WAVE + L.lane; c < n; c += nt * WAVE) clr[c] = 0;
+  }
 }
 
 // a rebuilding vertex at (x, y) farther than 2 cutoff / 3 from its list position: its cells may

@@ -159,6 +159,13 @@ struct AdjArgs {
   int update;
   int xcd;              // XCD-aware workgroup -> tile mapping
   int rowsLdsW;         // set by the launcher: list width the launch's LDS holds rows of
+  // with genCur, the step loop's cell protocol instead of `count` (md_cells): base of the three cell
+  // lists, generations, flags to clear
+  int* cells;
+  int* slots;
+  int* genCur;
+  int* genOut;
+  int* flagClear;
 };
 
 }  // namespace dpm
@@ -289,7 +296,8 @@ hipError_t launch_shape_only(dpm_set_s* S);
 hipError_t launch_step(dpm_set_s* S, int mode, const StepArgs& A);
 hipError_t launch_start_baoab(dpm_set_s* S, const StepArgs& A);
 hipError_t launch_start_md(dpm_set_s* S, const StepArgs& A);
-hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int* genOut, const NearRows& near);
+hipError_t launch_bin_flag(dpm_set_s* S, const View& Vn, int* count, int* slots, int* flag, int* genOut,
+                           const NearRows& near);
 hipError_t launch_near(dpm_set_s* S);
 hipError_t launch_ctr_add(dpm_set_s* S, long long addT, long long addA);
 hipError_t launch_bin(dpm_set_s* S, int bumpThermal, int bumpActive);

@@ -184,7 +184,7 @@ __global__ void k_rows_loop(View V, Params P, StepArgs A, CellGrid G) {
   if (A.genCur) {
     // step loop: the cells of the list positions (md_cells); the step kernel after this launch
     // advances the system's generation
-    const MdCells M = md_cells(A, G, A.genCur[s]);
+    const MdCells M = md_cells(A.cellCur, A.slotsCur, G, A.genCur[s]);
     const double x = V.x[v], y = V.y[v];
     if (!allPairs) md_stale_test(V, P, B, v, x, y, A.err);
     bin_vertex(G, B, M.binCnt, M.binSlots, v, s, x, y, A.err);
@@ -933,25 +933,26 @@ hipError_t launch_shape_only(dpm_set_s* S) {
 }
 
 template <int KIND>
-static hipError_t loop_start(dpm_set_s* S, const StepArgs& A) {
+static hipError_t loop_start(dpm_set_s* S, const View& Vn, const StepArgs& A) {
   if (KIND != START_NEAR && (!A.genOut || !A.flagOut || !A.anyOut || !A.cellCur || !A.slotsCur || !A.ctr))
     return hipErrorInvalidValue;
   if (KIND != START_NEAR && KIND != START_STAY && (!A.xout || !A.yout || !A.flagClear)) return hipErrorInvalidValue;
   const int threads = WAVE * (A.near.task ? START_WAVES : 1);
   if (S->P.interaction == INT_SMOOTH)
-    k_loop_start<KIND, INT_SMOOTH><<<S->V.ntiles, threads, 0, S->stream>>>(S->V, S->P, S->G, A);
+    k_loop_start<KIND, INT_SMOOTH><<<S->V.ntiles, threads, 0, S->stream>>>(Vn, S->P, S->G, A);
   else
-    k_loop_start<KIND, INT_VV><<<S->V.ntiles, threads, 0, S->stream>>>(S->V, S->P, S->G, A);
+    k_loop_start<KIND, INT_VV><<<S->V.ntiles, threads, 0, S->stream>>>(Vn, S->P, S->G, A);
   return hipGetLastError();
 }
 
-hipError_t launch_start_baoab(dpm_set_s* S, const StepArgs& A) { return loop_start<START_BAOAB>(S, A); }
+hipError_t launch_start_baoab(dpm_set_s* S, const StepArgs& A) { return loop_start<START_BAOAB>(S, S->V, A); }
 
-hipError_t launch_start_md(dpm_set_s* S, const StepArgs& A) { return loop_start<START_VERLET>(S, A); }
+hipError_t launch_start_md(dpm_set_s* S, const StepArgs& A) { return loop_start<START_VERLET>(S, S->V, A); }
 
-// the overdamped and rigid FIRE loops' start: flags of the current positions into `flag`, generation
-// 0 into `genOut`
-hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int* genOut, const NearRows& near) {
+// the start of the loops that begin at the positions of Vn as they are: their flags into `flag`,
+// generation 0 into `genOut`
+hipError_t launch_bin_flag(dpm_set_s* S, const View& Vn, int* count, int* slots, int* flag, int* genOut,
+                           const NearRows& near) {
   StepArgs A{};
   A.ctr = S->d_ctr;
   A.cellCur = count;
@@ -961,14 +962,14 @@ hipError_t launch_bin_flag(dpm_set_s* S, int* count, int* slots, int* flag, int*
   A.genOut = genOut;
   A.err = S->d_err;
   A.near = near;
-  return loop_start<START_STAY>(S, A);
+  return loop_start<START_STAY>(S, Vn, A);
 }
 
 // the near lists at the list positions
 hipError_t launch_near(dpm_set_s* S) {
   StepArgs A{};
   A.near = S->N;
-  return loop_start<START_NEAR>(S, A);
+  return loop_start<START_NEAR>(S, S->V, A);
 }
 
 hipError_t launch_ctr_add(dpm_set_s* S, long long addT, long long addA) {
@@ -1066,7 +1067,7 @@ hipError_t launch_scale_box(dpm_set_s* S) {
 hipError_t launch_rigid_start(dpm_set_s* S, bool langevin, const StepArgs& A) {
   StepArgs B = A;
   B.rigidLangevin = langevin ? 1 : 0;
-  return loop_start<START_RIGID>(S, B);
+  return loop_start<START_RIGID>(S, S->V, B);
 }
 
 hipError_t launch_rigid_inject(dpm_set_s* S, double amplitude, unsigned long long call) {

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       const int g = A.genCur[L.s];
       if (L.tile == V.stile[L.s] && threadIdx.x == 0) A.genOut[L.s] = rebuild ? g + 1 : g;
       if (rebuild) {
-        const MdCells M = md_cells(A, G, g);
+        const MdCells M = md_cells(A.cellCur, A.slotsCur, G, g);
         cells = M.cnt;
         slots = M.slots;
         if (!A.rowsBuilt) {
@@ -84,19 +84,8 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
         __syncthreads();
       }
     }
-    if (rebuild && A.genCur && !A.rowsBuilt && w == nw - 1) {
-      // these positions are the system's next list positions (its rows are built from them): binned into
-      // the next cell list, the one after cleared.  Nothing in this launch reads either, so one wave does
-      // it behind the rebuild's barriers, which would wait for the bins' atomics.
-      const MdCells M = md_cells(A, G, A.genCur[L.s]);
-      if (L.act) bin_vertex(G, B, M.binCnt, M.binSlots, L.v, L.s, x, y, A.err);
-      if (!G.brute[L.s]) {
-        const int t0 = V.stile[L.s], nt = V.stile[L.s + 1] - t0;
-        const int n = G.ncx[L.s] * G.ncy[L.s];
-        int* clr = M.clear + G.coff[L.s];
-        for (int c = (L.tile - t0) * WAVE + L.lane; c < n; c += nt * WAVE) clr[c] = 0;
-      }
-    }
+    if (rebuild && A.genCur && !A.rowsBuilt && w == nw - 1)
+      md_bin_rebuilt(V, G, md_cells(A.cellCur, A.slotsCur, G, A.genCur[L.s]), L, B, x, y, A.err);
   }
   // FIRE on every tile: a converged system's positions, forces and partials stay as they are
   if constexpr (NEAR && (MODE & MODE_FIRE) != 0 && (MODE & (MODE_RIGID | MODE_OUT)) == 0)
