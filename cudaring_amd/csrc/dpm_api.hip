@@ -532,8 +532,9 @@ StepArgs md_args(dpm_set_s* S, long r, long long offT, long long offA, bool near
   return A;
 }
 
-// Whether a loop of `steps` steps runs on near lists: building them costs its start kernel about what
-// they save in NEAR_STEPS steps.
+// Whether a loop of `steps` steps runs on near lists.  Building them takes its start kernel from 4.4 to
+// 10.0 us (1,024 rings, WCA vertex-segment) and each step from 10.8 to 7.2, so two steps pay for it; loops
+// shorter than the shortest captured as a graph stay on whole rows.
 constexpr long NEAR_STEPS = 4;
 bool near_loop(const dpm_set_s* S, long steps) {
   return S->N.task && steps >= NEAR_STEPS && (S->P.interaction == INT_VV || S->P.interaction == INT_SMOOTH);
@@ -546,7 +547,6 @@ long long active_draws(const dpm_set_s* S, long steps) { return S->P.particle !=
 //          (buffer b -> 1-b)
 //   per step: step [rebuild rows if flagged; F(x'); thermostat; v += dt/2 F;
 //             unless last: v += dt/2 F, x'' = x' + dt v, displacement test of x'']
-// The fused form performs the reference's operations in the reference's order.
 // With `rec` (slots of 2 nv doubles, x then y), the position after step i is also written to
 // slot i + 1 (the adjoint's recomputed segment).
 int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullptr) {
@@ -710,25 +710,37 @@ int run_fire(dpm_set_s* S, long iterations) {
   return DPM_OK;
 }
 
+// tiles of the set's largest system, and the waves of a system's sums (both one-system-one-block forms)
+int most_tiles(const dpm_set_s* S) {
+  int most = 1;
+  for (long s = 0; s < S->nsys; s++) most = std::max(most, S->h_stile[s + 1] - S->h_stile[s]);
+  return most;
+}
+int fire_waves(const dpm_set_s* S) {
+  return std::min(FS_WAVES, S->fireWaves > 0 ? S->fireWaves : most_tiles(S));
+}
+
 // FIRE iterations on every tile of the set, two launches each: the move (parameter update, drift and
-// displacement flags of every system, from tile partials) and the step kernel on near lists, with the
-// step loop's cell protocol as rigid FIRE runs it.  Stream launches: the host stays ahead of kernels of
-// five microseconds, and every dpm_init_fire would capture a graph anew.
+// displacement flags of every system) and the step kernel on near lists, with the step loop's cell
+// protocol as rigid FIRE runs it.  Stream launches: the host stays ahead of kernels of five
+// microseconds, and every dpm_init_fire would capture a graph anew.
 int fire_tile_sequence(dpm_set_s* S, long iterations) {
+  const int most = most_tiles(S), waves = fire_waves(S);
   HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], S->N));
-  HIPCHK(launch_fire_partials(S));
   for (long it = 0; it < iterations; it++) {
-    HIPCHK(launch_fire_move(S, S->mdFlag[it % 3], S->d_any + 2));
+    HIPCHK(launch_fire_move(S, most, waves, S->mdFlag[it % 3], S->d_any + 2));
     S->fireCur = 1 - S->fireCur;
     swap_pos(S);
     StepArgs A = md_args(S, it, 0, 0, true);
     A.fire = S->d_fire[S->fireCur];
     A.part = S->d_part;
+    A.vel = S->d_fireVel;
     HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR, A));
   }
   StepArgs A = md_args(S, iterations, 0, 0, true);  // energies and ring geometry of the positions reached
   A.fire = S->d_fire[S->fireCur];
   A.part = S->d_part;
+  A.vel = S->d_fireVel;
   A.manage = 0;
   HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR | MODE_OUT, A));
   return DPM_OK;
@@ -738,11 +750,12 @@ int fire_tile_sequence(dpm_set_s* S, long iterations) {
 // system, from what an iteration takes either way (us, harmonic vertex-vertex): 12 for the two launches
 // and 0.008 a tile of the set (measured 13.0 at 33 tiles, 13.4 at 85, 16.3 at 266, 59 at 5,333); or 3 and
 // 0.65 a tile of the largest system on its one CU, as often as the systems fill the chip (10.0 at 5
-// tiles, 13.5 at 10, 24.5 at 21, 32.6 at 33, 80 at 85 with frequent rebuilds, 31 at 60 without).
+// tiles, 13.5 at 10, 24.5 at 21, 32.6 at 33, 80 at 85 with frequent rebuilds, 31 at 60 without).  Those
+// are the times of the short forms; in the reference's order both sides take about 1.4 times as long (one
+// packing of 60 tiles on tiles 3.0 -> 4.3 ms, 512 packings on one workgroup each 10.0 -> 15.5).
 bool fire_on_tiles(const dpm_set_s* S) {
   if (!near_loop(S, NEAR_STEPS)) return false;
-  int most = 1;
-  for (long s = 0; s < S->nsys; s++) most = std::max(most, S->h_stile[s + 1] - S->h_stile[s]);
+  const int most = most_tiles(S);
   const double rounds = (double)((S->nsys + 255) / 256);
   return 12 + 0.008 * S->V.ntiles < rounds * (3 + 0.65 * most);
 }
@@ -1189,6 +1202,7 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   A(S->d_err, 1); A(S->d_maxcnt, 1); A(S->d_ctr, 4); A(S->d_notDone, 1); A(S->d_sysOrder, numSystems);
   A(S->d_fire[0], numSystems); A(S->d_fire[1], numSystems);
   A(S->d_part, (long)V.ntiles * 4);
+  A(S->d_fireVel, 2l * V.nv);
   S->nwide = (long)S->h_wide.size();
   if (S->nwide > 0) A(S->d_wide, S->nwide);
   std::vector<int> chunkSys, chunkOff(1, 0);
@@ -1290,7 +1304,7 @@ int dpm_destroy(dpm_set_t h) {
                   V.ncnt, V.nbr, V.nbrp, V.tile_v0, V.tile_v1, V.tile_sys, V.stile, S->G.ncx, S->G.ncy,
                   S->G.coff, S->G.brute, S->G.count[0], S->G.count[1], S->G.slots, S->G.cellSys, S->d_flag[0],
                   S->d_flag[1], S->d_any, S->d_updateCount, S->d_err, S->d_maxcnt, S->d_ctr, S->d_notDone,
-                  S->d_sysOrder, S->d_fire[0], S->d_fire[1], S->d_part, S->d_red, S->d_scale, V.kr,
+                  S->d_sysOrder, S->d_fire[0], S->d_fire[1], S->d_part, S->d_fireVel, S->d_red, S->d_scale, V.kr,
                   S->d_ck, S->d_fin, S->d_seg, S->d_adj, V.vinfo, V.l0r, V.mbx, V.mby, V.wfx, V.wfy,
                   S->d_contacts, S->d_ccount, S->d_x0, S->d_obs, S->mdCount[0], S->mdSlots[0], S->mdFlag[0],
                   S->mdFlag[1], S->mdFlag[2], S->mdFlag[3], S->mdGen[0], S->mdGen[1], S->mdGen[2], S->R.pvx, S->R.pvy, S->R.pw, S->R.pfx, S->R.pfy, S->R.ptq, S->R.moi,
@@ -1943,12 +1957,7 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
     // one workgroup per system, at most `pchunk` iterations per launch
     rc = clean_protocol(S);
     if (rc) return rc;
-    int waves = S->fireWaves;
-    if (waves <= 0) {
-      int maxTiles = 1;
-      for (long s = 0; s < S->nsys; s++) maxTiles = std::max(maxTiles, S->h_stile[s + 1] - S->h_stile[s]);
-      waves = std::min(16, maxTiles);
-    }
+    const int waves = fire_waves(S);
     const long pchunk = 2048;
     while (done <= maxIter) {
       rc = with_replay(S, SNAP_FIRE, 0, Draws{}, [&]() -> int {

@@ -17,75 +17,30 @@ namespace dpm {
 //
 // Bound by the vector instructions of one CU: a system of 200 rings is 60 tiles on 16 waves.  So an
 // iteration is one pass over the vertices up to the drift and one for the force, with two barriers:
-//   * the force phase evaluates the tile's near list (dpm_near.h), in the loops' short forms where the
-//     contacts are soft (a minimiser amplifies last bits a thousandfold per ten iterations of a stiff
-//     one, and the split FIRE step keeps the reference's order);
-//   * |v|^2 after the half kick is |v|^2 + 2 h P + h^2 |F|^2 (h^2 |F|^2 after a restart), from the sums
-//     made with P at the end of the iteration before: P > 0, so nothing cancels;
+//   * the force phase evaluates the tile's near list (dpm_near.h) instead of whole rows;
+//   * |v|^2 after the half kick is summed with v.F at the end of the iteration before (FireSums);
 //   * NEAR: the system's positions live in LDS (16 bytes a vertex), where the pair terms read them;
 //   * energies, ring geometry and the positions in memory are written once, when the launch ends.
+// Terms and sums keep the reference's order of operations and its rounding (quot, root): a minimiser
+// amplifies last bits, a thousandfold per ten iterations of a stiff contact.  The loops' short forms and
+// |v|^2 + 2 h P + h^2 |F|^2 took 512 packings of 16 to 256 rings through 2 x 60 iterations in 10.0 ms,
+// this takes 15.5 (whole rows from memory, four barriers: 19.1), but there single packings of a set left
+// the path: forces off by up to 9e-4 after a second compression.
 // Without near lists (rows of more than 64 entries, systems of more vertices than LDS holds, the
 // all-pairs interaction) it gathers over whole rows from memory.
-
-struct FireSums {
-  double P, vv, ff, m;  // v.F, |v|^2, |F|^2, max F_c^2
-};
-
-// workgroup sums of P, vv, ff and maximum of m (fixed order: lanes by butterfly, waves by index);
-// every thread passes another barrier between two calls
-__device__ __forceinline__ FireSums block_sums(FireSums a, double (*red)[4]) {
-  const int w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    a.P += __shfl_xor(a.P, d, WAVE);
-    a.vv += __shfl_xor(a.vv, d, WAVE);
-    a.ff += __shfl_xor(a.ff, d, WAVE);
-    a.m = fmax(a.m, __shfl_xor(a.m, d, WAVE));
-  }
-  if ((threadIdx.x & (WAVE - 1)) == 0) {
-    red[w][0] = a.P;
-    red[w][1] = a.vv;
-    red[w][2] = a.ff;
-    red[w][3] = a.m;
-  }
-  __syncthreads();
-  FireSums s{0, 0, 0, -1};
-  for (int q = 0; q < nw; q++) {
-    s.P += red[q][0];
-    s.vv += red[q][1];
-    s.ff += red[q][2];
-    s.m = fmax(s.m, red[q][3]);
-  }
-  return s;
-}
-
-__device__ __forceinline__ void add_vertex(FireSums& a, double vx, double vy, double fx, double fy) {
-  a.P += vx * fx + vy * fy;
-  a.vv += vx * vx + vy * vy;
-  a.ff += fx * fx + fy * fy;
-  a.m = fmax(a.m, fmax(fx * fx, fy * fy));
-}
-
-template <int INTER, int POT>
-constexpr bool fire_ref() {
-  return INTER == INT_SMOOTH || POT == POT_LJ || POT == POT_WCA;
-}
 
 // Force on the lane's vertex of tile t (and, STORE, its energy and the ring geometry into memory).
 template <int INTER, int POT, bool NEAR, bool STORE, class X>
 __device__ __forceinline__ void tile_force(const View& V, const Params& P, const NearRows& N, const Box& B,
                                            const Lane& L, X pos, double* res, double& fx, double& fy) {
-  constexpr bool REF = fire_ref<INTER, POT>();
   const double2 r = pos(L.v);
   double e = 0, es = 0, qx = 0, qy = 0, qnx = 0, qny = 0;  // sets with wide rings do not run this kernel
   fx = fy = 0;
   if constexpr (NEAR)
-    near_wave<INTER, POT, REF, STORE>(V, P, N, B, L, pos, res, fx, fy, INTER == INT_SMOOTH ? es : e, qx, qy);
+    near_wave<INTER, POT, true, STORE>(V, P, N, B, L, pos, res, fx, fy, INTER == INT_SMOOTH ? es : e, qx, qy);
   else
-    gather_pairs<INTER, POT, REF>(V, P, L, B, r.x, r.y, 0, 1, fx, fy, e, es, qx, qy, qnx, qny);
-  ShapeOut so;
-  if constexpr (REF) so = ring_shape(V, P, L, B, r.x, r.y, STORE);
-  else so = ring_shape_n(V, P, L, B, r.x, r.y, STORE);
+    gather_pairs<INTER, POT, true>(V, P, L, B, r.x, r.y, 0, 1, fx, fy, e, es, qx, qy, qnx, qny);
+  const ShapeOut so = ring_shape(V, P, L, B, r.x, r.y, STORE);
   if constexpr (INTER == INT_SMOOTH) {
     fx += shfl_d(qx, L.nl);
     fy += shfl_d(qy, L.nl);
@@ -107,7 +62,7 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, F
                                                              FireState* fst, int chunk, int* updateCount, int* err,
                                                              int* maxcnt, const int* order) {
   extern __shared__ double dyn[];  // NEAR: per wave near_wave_doubles, then the positions
-  __shared__ double red[FS_WAVES][4];
+  __shared__ double red[FS_WAVES][5];
   __shared__ int movedFlag[2];
   const int s = order[blockIdx.x];
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
@@ -120,43 +75,27 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, F
     else return make_double2(V.x[v], V.y[v]);
   };
   FireState fs = fst[s];
-  FireSums a{0, 0, 0, -1};
+  FireSums a{0, -1, 0, 0, 0};
+  const FireNext first(fp, fs);
   if (threadIdx.x < 2) movedFlag[threadIdx.x] = 0;
   for (int t = t0 + w; t < t1; t += nw) {
     Lane L;
     lane_ctx(V, t, lane, L);
     if (L.act) {
-      add_vertex(a, V.vx[L.v], V.vy[L.v], V.fx[L.v], V.fy[L.v]);
+      fire_add(a, first, V.vx[L.v], V.vy[L.v], V.fx[L.v], V.fy[L.v]);
       if constexpr (NEAR) lpos[L.v - b0] = make_double2(V.x[L.v], V.y[L.v]);
     }
     if constexpr (NEAR) build_near_wave<INTER>(V, P, N, L, B, V.lx, V.ly, G.brute[s] != 0);
   }
-  FireSums sum = block_sums(a, red);
+  FireSums sum = fire_block_sums(a, red, nw);
   bool ran = false;
   for (int it = 0; it < chunk; it++) {
     // ---- checkFIREParams (FIRE.cu:338-371) and the stopping rule
-    if (!fs.converged && (sqrt(sum.m) <= fp.tol || fs.iters >= fp.maxIter)) fs.converged = 1;
+    const bool reset = fire_update(fs, fp, sum);
     if (fs.converged) break;
     ran = true;
-    const bool reset = !(sum.P > 0);
-    fs.P = sum.P;
-    if (!reset) {
-      fs.numStep++;
-      if (fs.numStep > fp.minStep) {
-        fs.dt = fmin(fs.dt * fp.f_inc, fp.dt_max);
-        fs.a *= fp.f_a;
-      }
-    } else {
-      fs.numStep = 0;
-      fs.dt = fmax(fs.dt * fp.f_dec, fp.dt_max / 10);
-      fs.a = fp.a_start;
-    }
-    fs.iters++;
-    const double dt = fs.dt, h = 0.5 * dt, fa = fs.a;
-    // ---- back-step on reset (with the decreased dt), half kick, bendVertexVelocityTowardsForce
-    // (FIRE.cu:374-394), drift, displacement test
-    const double VV = reset ? h * h * sum.ff : sum.vv + 2 * h * sum.P + h * h * sum.ff;
-    const double bend = sum.ff > 0 ? fa * sqrt(VV / sum.ff) : 0.0, keep = sum.ff > 0 ? 1 - fa : 1.0;
+    const double h = 0.5 * fs.dt;
+    // ---- back-step on reset, half kick, mixing, drift, displacement test
     int moved = 0;
     for (int t = t0 + w; t < t1; t += nw) {
       const int v = V.tile_v0[t] + lane;
@@ -164,16 +103,7 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, F
         double vx = V.vx[v], vy = V.vy[v];
         const double fx = V.fx[v], fy = V.fy[v], lx = V.lx[v], ly = V.ly[v];
         double2 r = pos(v);
-        if (reset) {
-          r.x -= h * vx;
-          r.y -= h * vy;
-          vx = 0;
-          vy = 0;
-        }
-        vx = keep * (vx + h * fx) + bend * fx;
-        vy = keep * (vy + h * fy) + bend * fy;
-        r.x += dt * vx;
-        r.y += dt * vy;
+        fire_move(fs, sum, reset, fx, fy, r.x, r.y, vx, vy);
         V.vx[v] = vx;
         V.vy[v] = vy;
         if constexpr (NEAR) {
@@ -217,7 +147,8 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, F
       if (threadIdx.x == 0) updateCount[s] += 1;
     }
     // ---- calcForceEnergy (shape + interaction) and the second half kick
-    a = FireSums{0, 0, 0, -1};
+    a = FireSums{0, -1, 0, 0, 0};
+    const FireNext next(fp, fs);
     for (int t = t0 + w; t < t1; t += nw) {
       Lane L;
       lane_ctx(V, t, lane, L);
@@ -229,10 +160,10 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, F
         V.fy[L.v] = fy;
         V.vx[L.v] = vx;
         V.vy[L.v] = vy;
-        add_vertex(a, vx, vy, fx, fy);
+        fire_add(a, next, vx, vy, fx, fy);
       }
     }
-    sum = block_sums(a, red);
+    sum = fire_block_sums(a, red, nw);
   }
   if (ran) {  // what the last force phase left out
     for (int t = t0 + w; t < t1; t += nw) {

@@ -46,7 +46,7 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
     const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
     const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
     theta = atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);  // calcAngle 423-427
-    seglen = sqrt(dnx * dnx + dny * dny);
+    seglen = root(dnx * dnx + dny * dny);
     // Unwrapped position relative to the first vertex: the reference walks the ring one
     // minimum-image segment at a time; here that walk is an exclusive segmented scan of the
     // segment vectors, valid for rings wider than half the box.
@@ -59,7 +59,7 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
     const double shoeSum = seg_sum(shoe, L.lane, L.segS, L.segE);
     const double sux = seg_sum(ux, L.lane, L.segS, L.segE);
     const double suy = seg_sum(uy, L.lane, L.segS, L.segE);
-    const double ind = 1.0 / (double)L.n;
+    const double ind = quot(1.0, (double)L.n);
     area = fabs(shoeSum) * 0.5;
     comx = xf + sux * ind;
     comy = yf + suy * ind;
@@ -72,7 +72,7 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
     xp = V.x[vp]; yp = V.y[vp];
     theta = vertex_theta(B, x, y, xn, yn, xp, yp);
     const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-    seglen = sqrt(dnx * dnx + dny * dny);
+    seglen = root(dnx * dnx + dny * dny);
     area = V.area[L.r];
     perim = V.perim[L.r];
     comx = V.cx[L.r];
@@ -90,7 +90,7 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
       V.cy[L.r] = comy;
     }
   }
-  const double ind = 1.0 / (double)L.n;
+  const double ind = quot(1.0, (double)L.n);
   // positions relative to the ring centre (getRelativeVertexPos 273-279)
   const double rvx = pbx(x - comx, B), rvy = pby(y - comy, B);
   const double rnx = pbx(xn - comx, B), rny = pby(yn - comy, B);
@@ -101,23 +101,23 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
   const double el = V.kr ? V.kr[V.np + L.r] : P.el;
   const double eb = V.kr ? V.kr[2 * V.np + L.r] : P.eb;
   // area term (calcAreaForceEnergy 429-435)
-  const double deltaA = (area / a0) - 1.;
-  const double gmA = ea * deltaA / a0;
+  const double deltaA = quot(area, a0) - 1.;
+  const double gmA = quot(ea * deltaA, a0);
   double fx = 0.5 * gmA * (rpy - rny);
   double fy = 0.5 * gmA * (rnx - rpx);
   double e = (0.5 * ea * deltaA * deltaA) * ind;
   // perimeter term (calcPerimeterForceEnergy 437-447 / FENE 449-455)
   const double nsx = rnx - rvx, nsy = rny - rvy;
   const double qsx = rvx - rpx, qsy = rvy - rpy;
-  const double pLen = sqrt(qsx * qsx + qsy * qsy);
-  const double nLen = sqrt(nsx * nsx + nsy * nsy);
+  const double pLen = root(qsx * qsx + qsy * qsy);
+  const double nLen = root(nsx * nsx + nsy * nsy);
   const double l0v = V.l0[L.v];
   const double l0s = shfl_d(l0v, L.pl);
   const double l0p = L.wide ? V.l0[vp] : l0s;
   if (P.monomer == MONO_HARMONIC) {
-    const double pDelta = (pLen / l0p) - 1.;
-    const double nDelta = (nLen / l0v) - 1.;
-    const double cn = nDelta / (l0v * nLen), cp = pDelta / (l0p * pLen);
+    const double pDelta = quot(pLen, l0p) - 1.;
+    const double nDelta = quot(nLen, l0v) - 1.;
+    const double cn = quot(nDelta, l0v * nLen), cp = quot(pDelta, l0p * pLen);
     fx += el * ((cn * (rnx - rvx)) - (cp * (rvx - rpx)));
     fy += el * ((cn * (rny - rvy)) - (cp * (rvy - rpy)));
     e += (0.5 * el * pDelta * pDelta);
@@ -137,8 +137,8 @@ __device__ __forceinline__ ShapeOut ring_shape(const View& V, const Params& P, c
     Dp = vertex_theta(B, xp, yp, x, y, V.x[vpp], V.y[vpp]) - V.th0[vp];
     Dn = vertex_theta(B, xn, yn, V.x[vnn], V.y[vnn], x, y) - V.th0[vn];
   }
-  const double preVar = (D - Dp) / (qsx * qsx + qsy * qsy);
-  const double nextVar = (D - Dn) / (nsx * nsx + nsy * nsy);
+  const double preVar = quot(D - Dp, qsx * qsx + qsy * qsy);
+  const double nextVar = quot(D - Dn, nsx * nsx + nsy * nsy);
   fx += eb * (preVar * qsy + nextVar * nsy);
   fy += eb * (preVar * (-qsx) + nextVar * (-nsx));
   e += (0.5 * eb * D * D);
@@ -444,6 +444,99 @@ __device__ __forceinline__ void md_bin_rebuilt(const View& V, const CellGrid& G,
 __device__ __forceinline__ void md_stale_test(const View& V, const Params& P, const Box& B, int v, double x, double y,
                                               int* err) {
   if (moved_past(P, B, x - V.lx[v], y - V.ly[v], 2.0)) atomicOr(err, ERR_STALE_BINS);
+}
+
+// ------------------------------------------------------------------ FIRE ---
+// Sums an iteration starts from: v.F, max F_c^2, |F|^2, and |v|^2 after the half kick.  The step of that
+// kick is known before v.F but for its sign: h1 when it is positive, h2 of a restart (which clears v first),
+// so one exchange carries both outcomes, each vertex's half-kicked velocity rounded as the kick rounds it.
+struct FireSums {
+  double P, m, ff, v1, v2;
+};
+struct FireNext {
+  double h1, h2;
+  __device__ __forceinline__ FireNext(const FireParams& fp, const FireState& fs)
+      : h1(0.5 * (fs.numStep + 1 > fp.minStep ? fmin(fs.dt * fp.f_inc, fp.dt_max) : fs.dt)),
+        h2(0.5 * fmax(fs.dt * fp.f_dec, fp.dt_max / 10)) {}
+};
+__device__ __forceinline__ void fire_add(FireSums& a, const FireNext& n, double vx, double vy, double fx, double fy) {
+  const double ux = vx + n.h1 * fx, uy = vy + n.h1 * fy, wx = n.h2 * fx, wy = n.h2 * fy;
+  a.P += vx * fx + vy * fy;
+  a.m = fmax(a.m, fmax(fx * fx, fy * fy));
+  a.ff += fx * fx + fy * fy;
+  a.v1 += ux * ux + uy * uy;
+  a.v2 += wx * wx + wy * wy;
+}
+// workgroup sums (fixed order: lanes by butterfly, the first nw waves by index); every thread passes
+// another barrier between two calls
+__device__ __forceinline__ FireSums fire_block_sums(FireSums a, double (*red)[5], int nw) {
+  const int w = threadIdx.x / WAVE;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    a.P += __shfl_xor(a.P, d, WAVE);
+    a.m = fmax(a.m, __shfl_xor(a.m, d, WAVE));
+    a.ff += __shfl_xor(a.ff, d, WAVE);
+    a.v1 += __shfl_xor(a.v1, d, WAVE);
+    a.v2 += __shfl_xor(a.v2, d, WAVE);
+  }
+  if ((threadIdx.x & (WAVE - 1)) == 0) {
+    red[w][0] = a.P;
+    red[w][1] = a.m;
+    red[w][2] = a.ff;
+    red[w][3] = a.v1;
+    red[w][4] = a.v2;
+  }
+  __syncthreads();
+  FireSums s{0, -1, 0, 0, 0};
+  for (int q = 0; q < nw; q++) {
+    s.P += red[q][0];
+    s.m = fmax(s.m, red[q][1]);
+    s.ff += red[q][2];
+    s.v1 += red[q][3];
+    s.v2 += red[q][4];
+  }
+  return s;
+}
+// checkFIREParams (FIRE.cu:338-371) with the stopping rule; true when the iteration restarts
+__device__ __forceinline__ bool fire_update(FireState& fs, const FireParams& fp, const FireSums& s) {
+  if (!fs.converged && (sqrt(s.m) <= fp.tol || fs.iters >= fp.maxIter)) fs.converged = 1;
+  if (fs.converged) return false;
+  const bool reset = !(s.P > 0);
+  fs.P = s.P;
+  if (!reset) {
+    fs.numStep++;
+    if (fs.numStep > fp.minStep) {
+      fs.dt = fmin(fs.dt * fp.f_inc, fp.dt_max);
+      fs.a *= fp.f_a;
+    }
+  } else {
+    fs.numStep = 0;
+    fs.dt = fmax(fs.dt * fp.f_dec, fp.dt_max / 10);
+    fs.a = fp.a_start;
+  }
+  fs.iters++;
+  return reset;
+}
+// back-step on reset (with the decreased dt), half kick, bendVertexVelocityTowardsForce
+// (FIRE.cu:374-394) and drift of one vertex
+__device__ __forceinline__ void fire_move(const FireState& fs, const FireSums& s, bool reset, double fx, double fy,
+                                          double& x, double& y, double& vx, double& vy) {
+  const double h = 0.5 * fs.dt, fa = fs.a;
+  if (reset) {
+    x -= h * vx;
+    y -= h * vy;
+    vx = 0;
+    vy = 0;
+  }
+  vx += h * fx;
+  vy += h * fy;
+  if (s.ff > 0) {
+    const double ratio = sqrt((reset ? s.v2 : s.v1) / s.ff);
+    vx = (1 - fa) * vx + fa * fx * ratio;
+    vy = (1 - fa) * vy + fa * fy * ratio;
+  }
+  x += fs.dt * vx;
+  y += fs.dt * vy;
 }
 
 // ---------------------------------------------------------- rigid rings ---

@@ -1,5 +1,6 @@
 // dpm_internal.h -- host-side handle of a system set and the launcher interface
-// between the C ABI (dpm_api.hip) and the kernels (dpm_kernels.hip).
+// between the C ABI (dpm_api.hip) and the kernels (dpm_kernels.hip, dpm_step.hip, dpm_fire.hip,
+// dpm_adjoint.hip, dpm_observe.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -93,6 +94,7 @@ struct StepArgs {
   long long ctrOffT, ctrOffA;     // call index of this step's draws = ctr[k] + offset
   FireState* fire;                // MODE_FIRE: per-system state of this iteration
   double* part;                   // MODE_FIRE: per-tile partial sums [ntiles * 4]
+  const double* vel;              // MODE_FIRE | MODE_NEAR: velocities after the drift [2 * nv]
   int* err;
   int* maxcnt;
   int* updateCount;
@@ -104,7 +106,7 @@ struct StepArgs {
   NearRows near;                  // step loops with near lists (MODE_NEAR); start kernels build them when task is set
 };
 
-// Up to kMaxCopySegs device-to-device copies in one launch (k_copy_segs): 4-byte words.
+// Up to kMaxCopySegs device-to-device copies in one launch (k_prologue): 4-byte words.
 constexpr int kMaxCopySegs = 32;
 struct CopySegs {
   const unsigned* src[kMaxCopySegs];
@@ -240,6 +242,7 @@ struct dpm_set_s {
   int fireCur = 0;
   dpm::FireParams fp{};
   double* d_part = nullptr;  // per-tile partials [ntiles * 4]
+  double* d_fireVel = nullptr;  // FIRE on tiles: velocities between the move and the step [2 * nv]
   bool fireInit = false;
   int fireKernel = -1;  // dpm_fire_minimize: 1 = one persistent workgroup per system, 0 = graph of step
                         //   kernels, -1 = persistent or on every tile (fire_on_tiles)
@@ -291,7 +294,7 @@ struct dpm_set_s {
 
 namespace dpm {
 
-// launchers (dpm_kernels.hip); all return hipError_t of the last launch
+// launchers (dpm_kernels.hip, dpm_adjoint.hip, dpm_observe.hip); all return hipError_t of the last launch
 hipError_t launch_shape_only(dpm_set_s* S);
 hipError_t launch_step(dpm_set_s* S, int mode, const StepArgs& A);
 hipError_t launch_start_baoab(dpm_set_s* S, const StepArgs& A);
@@ -318,7 +321,7 @@ hipError_t launch_fire_mid(dpm_set_s* S);
 hipError_t launch_fire_partials(dpm_set_s* S);
 hipError_t launch_fire_step(dpm_set_s* S);
 hipError_t launch_fire_resume(dpm_set_s* S);
-hipError_t launch_fire_move(dpm_set_s* S, int* flagOut, int* anyOut);
+hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut);
 StepArgs loop_args(dpm_set_s* S);
 hipError_t launch_bin_view(dpm_set_s* S, const View& Vn, int parity);
 hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves);

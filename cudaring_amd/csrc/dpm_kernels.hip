@@ -8,18 +8,22 @@
 //     neighbours (prev/next vertex, their angles and rest lengths) come from lane
 //     shuffles, so the reference's three shape kernels collapse into one pass;
 //     it also draws the ring's Philox numbers;
-//   * meanwhile waves 1..nw-1 share the interparticle gather over the ELL
-//     neighbour list and reduce their partial forces through LDS in a fixed
-//     order (with nw = 1 wave 0 does the gather itself);
+//   * meanwhile waves 1..nw-1 share the interparticle gather (with nw = 1 wave 0
+//     does it itself): in loops over the tile's near list, one evaluation per
+//     lane (dpm_near.h), in single force calls over the rows of the ELL neighbour
+//     list; the partial forces are added through LDS in a fixed order;
 //   * wave 0 applies the integrator epilogue (thermostat, kicks, drift,
 //     displacement test).
-// Neighbour rows are rebuilt inside the step kernel when the system's rebuild
-// flag is set, and a tile's rows are all built by its own workgroup before its
+// Neighbour rows and near lists are rebuilt inside the step kernel when the
+// system's rebuild flag is set, each tile's by its own workgroup before its
 // gather starts.  In the step loops the cells searched are those of the list
 // positions (the positions of the system's last rebuild, binned by that rebuild:
 // md_cells), so a step is one launch with no binning and no host
-// synchronisation; the FIRE graph path bins the current positions in a k_bin
+// synchronisation; the split FIRE step bins the current positions in a k_bin
 // launch before each step kernel.
+// This file: list builds, loop starts, reductions, stage kernels, the split FIRE
+// step and the moves of rigid and tile-parallel FIRE.  dpm_step.hip holds the step
+// kernel, dpm_fire.hip the persistent FIRE kernel, dpm_forces.h what they share.
 #include "dpm_forces.h"
 #include "dpm_launch.h"
 #include "dpm_near.h"
@@ -746,105 +750,66 @@ __global__ void k_fire_mid(View V, Params P, const FireState* fcur, const double
   }
 }
 
-// per-tile partials of P = v.F, |v|^2, |F|^2 and max F_c^2 for the current state (start of a FIRE call)
+// per-tile partials of P = v.F and max F_c^2 for the current state (start of a FIRE call)
 __global__ void k_fire_partials(View V, double* part) {
   Lane L;
   if (!wave_tile_ctx(V, L)) return;
-  double pvf = 0, v2 = 0, ff = 0, f2 = -1;
+  double pvf = 0, f2 = -1;
   if (L.act) {
     const double vx = V.vx[L.v], vy = V.vy[L.v], fx = V.fx[L.v], fy = V.fy[L.v];
     pvf = vx * fx + vy * fy;
-    v2 = vx * vx + vy * vy;
-    ff = fx * fx + fy * fy;
     f2 = fmax(fx * fx, fy * fy);
   }
   const double tP = wave_sum(pvf);
-  const double tV = wave_sum(v2);
-  const double tF = wave_sum(ff);
   const double tM = wave_max(f2);
   if (L.lane == 0) {
     part[L.tile * 4 + 0] = tP;
-    part[L.tile * 4 + 1] = tV;
-    part[L.tile * 4 + 2] = tF;
     part[L.tile * 4 + 3] = tM;
   }
 }
 
-// An iteration of FIRE on every tile up to the drift, one wave per tile (the step kernel of
-// MODE_FIRE | MODE_NEAR follows): every wave adds its system's tile partials, takes the stopping rule and
-// the parameter update (checkFIREParams 338-371), and moves its vertices as the persistent kernel does
-// (dpm_fire.hip), into the other position buffer, with the step loop's flags.
-__global__ void k_fire_move(View V, Params P, FireParams fp, const FireState* fin, FireState* fout, const double* part,
-                            double* xo, double* yo, int* flagOut, int* anyOut) {
-  Lane L;
-  if (!wave_tile_ctx(V, L)) return;
-  const int t0 = V.stile[L.s], t1 = V.stile[L.s + 1];
-  FireState fs = fin[L.s];
-  const double x = V.x[L.v], y = V.y[L.v];
-  double vx = V.vx[L.v], vy = V.vy[L.v];
-  const double fx = V.fx[L.v], fy = V.fy[L.v];
-  double p = 0, vv = 0, ff = 0, m = -1;
-  for (int t = t0 + L.lane; t < t1; t += WAVE) {
-    p += part[t * 4 + 0];
-    vv += part[t * 4 + 1];
-    ff += part[t * 4 + 2];
-    m = fmax(m, part[t * 4 + 3]);
+// An iteration of FIRE on every tile up to the drift (the step kernel of MODE_FIRE | MODE_NEAR follows):
+// `per` blocks a system, of one wave per tile.  Every block sums its whole system
+// first, over the vertices in the order of the persistent kernel with as many waves (so that both follow
+// the same path to the last bit), then takes the stopping rule and the parameter update and moves its
+// vertices into the other position buffer and vxn, vyn (other blocks still sum vx, vy), with the step
+// loop's flags.
+__global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_move(View V, Params P, FireParams fp, int per,
+                                                              const FireState* fin, FireState* fout, double* xo,
+                                                              double* yo, double* vxn, double* vyn, int* flagOut,
+                                                              int* anyOut) {
+  __shared__ double red[FS_WAVES][5];
+  const int s = blockIdx.x / per, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x & (WAVE - 1);
+  const int t0 = V.stile[s], t1 = V.stile[s + 1], tile = t0 + (blockIdx.x % per) * nw + w;
+  FireState fs = fin[s];
+  const FireNext next(fp, fs);
+  FireSums a{0, -1, 0, 0, 0};
+  for (int t = t0 + w; t < t1; t += nw) {
+    const int v = V.tile_v0[t] + lane;
+    if (v < V.tile_v1[t]) fire_add(a, next, V.vx[v], V.vy[v], V.fx[v], V.fy[v]);
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    p += __shfl_xor(p, d, WAVE);
-    vv += __shfl_xor(vv, d, WAVE);
-    ff += __shfl_xor(ff, d, WAVE);
-    m = fmax(m, __shfl_xor(m, d, WAVE));
-  }
-  if (!fs.converged && (sqrt(m) <= fp.tol || fs.iters >= fp.maxIter)) fs.converged = 1;
-  const bool reset = !(p > 0);
-  if (!fs.converged) {
-    fs.P = p;
-    if (!reset) {
-      fs.numStep++;
-      if (fs.numStep > fp.minStep) {
-        fs.dt = fmin(fs.dt * fp.f_inc, fp.dt_max);
-        fs.a *= fp.f_a;
-      }
-    } else {
-      fs.numStep = 0;
-      fs.dt = fmax(fs.dt * fp.f_dec, fp.dt_max / 10);
-      fs.a = fp.a_start;
-    }
-    fs.iters++;
-  }
-  if (L.tile == t0 && L.lane == 0) fout[L.s] = fs;
-  if (!L.act) return;
-  if (fs.converged) {
-    xo[L.v] = x;
-    yo[L.v] = y;
-    return;
-  }
-  const double h = 0.5 * fs.dt;
-  const double VV = reset ? h * h * ff : vv + 2 * h * p + h * h * ff;
-  const double bend = ff > 0 ? fs.a * sqrt(VV / ff) : 0.0, keep = ff > 0 ? 1 - fs.a : 1.0;
+  const FireSums sum = fire_block_sums(a, red, nw);
+  const bool reset = fire_update(fs, fp, sum);
+  if (tile == t0 && lane == 0) fout[s] = fs;
+  if (tile >= t1) return;
+  const int v = V.tile_v0[tile] + lane;
+  if (v >= V.tile_v1[tile]) return;
+  const double x = V.x[v], y = V.y[v];
   double xn = x, yn = y;
-  if (reset) {
-    xn -= h * vx;
-    yn -= h * vy;
-    vx = 0;
-    vy = 0;
+  if (!fs.converged) {
+    double vx = V.vx[v], vy = V.vy[v];
+    fire_move(fs, sum, reset, V.fx[v], V.fy[v], xn, yn, vx, vy);
+    vxn[v] = vx;
+    vyn[v] = vy;
+    const Box B = box_of(V, s);
+    if (moved_past(P, B, xn - V.lx[v], yn - V.ly[v])) {
+      atomicOr(&flagOut[s], 1);
+      atomicOr(anyOut, 1);
+    }
+    far_test(P, B, xn - x, yn - y, flagOut + s);
   }
-  vx = keep * (vx + h * fx) + bend * fx;
-  vy = keep * (vy + h * fy) + bend * fy;
-  xn += fs.dt * vx;
-  yn += fs.dt * vy;
-  V.vx[L.v] = vx;
-  V.vy[L.v] = vy;
-  xo[L.v] = xn;
-  yo[L.v] = yn;
-  const Box B = box_of(V, L.s);
-  if (moved_past(P, B, xn - V.lx[L.v], yn - V.ly[L.v])) {
-    atomicOr(&flagOut[L.s], 1);
-    atomicOr(anyOut, 1);
-  }
-  far_test(P, B, xn - x, yn - y, flagOut + L.s);
+  xo[v] = xn;
+  yo[v] = yn;
 }
 
 // a new minimisation call tests every system's stopping rule again (the driver's loop condition
@@ -1108,12 +1073,13 @@ hipError_t launch_fire_mid(dpm_set_s* S) {
   return hipGetLastError();
 }
 
-hipError_t launch_fire_move(dpm_set_s* S, int* flagOut, int* anyOut) {
-  if (!flagOut || !anyOut) return hipErrorInvalidValue;
+hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut) {
+  if (!flagOut || !anyOut || waves < 1 || waves > FS_WAVES) return hipErrorInvalidValue;
   const int nb = 1 - S->cur;
-  k_fire_move<<<grid_w(S->V.ntiles), 256, 0, S->stream>>>(
-      S->V, S->P, S->fp, S->d_fire[S->fireCur], S->d_fire[1 - S->fireCur], S->d_part, S->pos[nb][0], S->pos[nb][1],
-      flagOut, anyOut);
+  const int per = (most + waves - 1) / waves;
+  k_fire_move<<<(unsigned)(S->nsys * per), WAVE * waves, 0, S->stream>>>(
+      S->V, S->P, S->fp, per, S->d_fire[S->fireCur], S->d_fire[1 - S->fireCur], S->pos[nb][0], S->pos[nb][1], S->d_fireVel,
+      S->d_fireVel + S->V.nv, flagOut, anyOut);
   return hipGetLastError();
 }
 

@@ -295,7 +295,7 @@ constexpr int near_slots_bytes() {
 
 // Evaluations [base, base + NEAR_WIN) of both roles of a tile, dealt in chunks of 64 to the gather
 // waves w of nw (roles alternate, so that the first chunks of both start at once).
-template <int INTER, int POT, bool ENERGY>
+template <int INTER, int POT, bool REF, bool ENERGY>
 __device__ __forceinline__ void eval_near(const View& V, const Params& P, const NearRows& N, const Box& B, int tile,
                                           int v0, int2 cnt, int base, int lane, int w, int nw, void* lds) {
   constexpr int NR = INTER == INT_SMOOTH ? 2 : 1;
@@ -317,10 +317,10 @@ __device__ __forceinline__ void eval_near(const View& V, const Params& P, const 
         const double sum = V.rad[v] + V.rad[u];
         double fx = 0, fy = 0, e;
         if constexpr (NR == 1) {
-          e = pair_force_n<POT>(P, pbx(x - xu, B), pby(y - yu, B), sum, fx, fy);
+          e = pair_of<POT, REF>(P, pbx(x - xu, B), pby(y - yu, B), sum, fx, fy);
         } else {
           const int p1 = u - (((t.y >> 8) & 255) - 64), p2 = u - (((t.y >> 16) & 255) - 64);
-          e = smooth_this_n<POT>(P, B, x, y, xu, yu, V.x[p1], V.y[p1], V.x[p2], V.y[p2], sum, fx, fy);
+          e = smooth_this_of<POT, REF>(P, B, x, y, xu, yu, V.x[p1], V.y[p1], V.x[p2], V.y[p2], sum, fx, fy);
         }
         fT[i] = make_double2(fx, fy);
         if constexpr (ENERGY) eT[i] = e;
@@ -331,7 +331,7 @@ __device__ __forceinline__ void eval_near(const View& V, const Params& P, const 
         const int v = v0 + (t.y & 63), u = t.x;
         const int p1 = v - (((t.y >> 8) & 255) - 64), p2 = v - (((t.y >> 16) & 255) - 64);
         double fx = 0, fy = 0, qx = 0, qy = 0;
-        const double e = smooth_op_n<POT>(P, B, V.x[u], V.y[u], V.x[v], V.y[v], V.x[p1], V.y[p1], V.x[p2], V.y[p2],
+        const double e = smooth_op_of<POT, REF>(P, B, V.x[u], V.y[u], V.x[v], V.y[v], V.x[p1], V.y[p1], V.x[p2], V.y[p2],
                                              V.rad[v] + V.rad[u], fx, fy, qx, qy);
         fO[i] = make_double2(fx, fy);
         qO[i] = make_double2(qx, qy);

@@ -6,11 +6,11 @@
 
 namespace dpm {
 
-// Single force calls and the split vertex FIRE step keep the reference's order of operations and a fixed
-// number of waves.
+// Single force calls and the vertex FIRE steps keep the reference's order of operations, over whole rows
+// with a fixed number of waves too (whose sums they set).
 template <int MODE>
 constexpr bool step_ref() {
-  return (MODE & (MODE_KICK | MODE_BROWN | MODE_NEAR)) == 0;
+  return (MODE & (MODE_KICK | MODE_BROWN)) == 0 && (MODE & (MODE_RIGID | MODE_NEAR)) != (MODE_RIGID | MODE_NEAR);
 }
 
 // Whether the launch stores the force, energies, ring geometry and wall forces: what is read after a
@@ -94,8 +94,9 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
   double vx = 0, vy = 0, lx = 0, ly = 0;
   if (w == 0) {
     if constexpr (MB != MODE_FORCE && (MODE & MODE_RIGID) == 0) {
-      vx = V.vx[L.v];
-      vy = V.vy[L.v];
+      constexpr bool MOVED = NEAR && MB == MODE_FIRE;  // the velocities k_fire_move wrote
+      vx = MOVED ? A.vel[L.v] : V.vx[L.v];
+      vy = MOVED ? A.vel[V.nv + L.v] : V.vy[L.v];
     }
     if constexpr ((MODE & MODE_START) != 0) {
       lx = V.lx[L.v];
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       spanT = A.near.span[L.v];
       if constexpr (INTER == INT_SMOOTH) spanO = A.near.span[V.nv + L.v];
     }
-    if (w >= g0) eval_near<INTER, POT, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, 0, L.lane, w - g0, ng, red);
+    if (w >= g0) eval_near<INTER, POT, REF, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, 0, L.lane, w - g0, ng, red);
   } else {
     if (w >= g0) gather_pairs<INTER, POT, REF>(V, P, L, B, x, y, w - g0, ng, fx, fy, e, es, qx, qy, qnx, qny);
     if (nw > 1 && w > 0) {
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       base += NEAR_WIN;
       if (base >= most) break;
       __syncthreads();
-      if (w >= g0) eval_near<INTER, POT, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, base, L.lane, w - g0, ng, red);
+      if (w >= g0) eval_near<INTER, POT, REF, STORE>(V, P, A.near, B, L.tile, L.v0, cnt, base, L.lane, w - g0, ng, red);
     }
     if (w > 0) return;
   } else if (nw > 1) {
@@ -257,21 +258,14 @@ __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepA
       vx += h * fx;
       vy += h * fy;
     }
-    const double pvf = L.act ? (vx * fx + vy * fy) : 0.0;
-    const double f2 = L.act ? fmax(fx * fx, fy * fy) : -1.0;
-    const double tP = wave_sum(pvf);
-    const double tM = wave_max(f2);
-    double tV = 0, tF = 0;
-    if constexpr (NEAR) {  // the next move's sums (the split step sums them after its half kick)
-      tV = wave_sum(L.act ? vx * vx + vy * vy : 0.0);
-      tF = wave_sum(L.act ? fx * fx + fy * fy : 0.0);
-    }
-    if (L.lane == 0) {
-      A.part[L.tile * 4 + 0] = tP;
-      A.part[L.tile * 4 + 3] = tM;
-      if constexpr (NEAR) {
-        A.part[L.tile * 4 + 1] = tV;
-        A.part[L.tile * 4 + 2] = tF;
+    if constexpr (!NEAR) {  // (the move on near lists sums over the vertices)
+      const double pvf = L.act ? (vx * fx + vy * fy) : 0.0;
+      const double f2 = L.act ? fmax(fx * fx, fy * fy) : -1.0;
+      const double tP = wave_sum(pvf);
+      const double tM = wave_max(f2);
+      if (L.lane == 0) {
+        A.part[L.tile * 4 + 0] = tP;
+        A.part[L.tile * 4 + 3] = tM;
       }
     }
     if (!L.act) return;
@@ -350,7 +344,7 @@ static inline size_t step_lds(const dpm_set_s* S, int nw) {
 
 template <int INTER, int POT, int MODE>
 static hipError_t step_one(dpm_set_s* S, const StepArgs& A) {
-  const int nw = step_ref<MODE>() ? S->split : loop_waves(S);
+  const int nw = step_ref<MODE>() && !(MODE & MODE_NEAR) ? S->split : loop_waves(S);
   k_step<INTER, POT, MODE>
       <<<S->V.ntiles, WAVE * nw, step_lds<INTER, MODE>(S, nw), S->stream>>>(S->V, S->P, A, S->G);
   return hipGetLastError();
