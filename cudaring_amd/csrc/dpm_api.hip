@@ -1943,29 +1943,26 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
   HIPCHK(launch_fire_resume(S));
   long done = 0;
   const bool plain = S->P.particle == PART_PASSIVE && S->P.geometry == GEOM_NORMAL && S->nwide == 0;
-  if (S->fireKernel < 0 && plain && fire_on_tiles(S)) {
-    const long tchunk = 256;
-    while (done < maxIter) {
-      const long n = std::min(tchunk, maxIter - done);
-      rc = with_replay(S, SNAP_FIRE, LOOP_MD, Draws{}, [&]() { return fire_tile_sequence(S, n); });
-      if (rc) return rc;
-      done += n;
-      if (!S->h_stat->notDone) break;
-    }
-    done = maxIter + 1;  // the other paths are skipped
-  } else if (S->fireKernel != 0 && plain) {
-    // one workgroup per system, at most `pchunk` iterations per launch
-    rc = clean_protocol(S);
-    if (rc) return rc;
+  if (S->fireKernel != 0 && plain) {
+    // on every tile, or one workgroup per system with at most `pchunk` iterations per launch
     const int waves = fire_waves(S);
-    const long pchunk = 2048;
-    while (done <= maxIter) {
-      rc = with_replay(S, SNAP_FIRE, 0, Draws{}, [&]() -> int {
-        HIPCHK(launch_fire_sys(S, (int)pchunk, waves));
+    const long tchunk = 256, pchunk = 2048;
+    bool tiles = S->fireKernel < 0 && fire_on_tiles(S);
+    while (tiles ? done < maxIter : done <= maxIter) {
+      long n = 0;
+      rc = with_replay(S, SNAP_FIRE, tiles ? LOOP_MD : 0, Draws{}, [&]() -> int {
+        // a replay's wider list may have no near lists, without which the tiles cannot run: one workgroup
+        // per system goes on from the restored state
+        tiles = tiles && near_loop(S, NEAR_STEPS);
+        n = tiles ? std::min(tchunk, maxIter - done) : pchunk;
+        if (tiles) return fire_tile_sequence(S, n);
+        const int r = clean_protocol(S);
+        if (r) return r;
+        HIPCHK(launch_fire_sys(S, (int)n, waves));
         return DPM_OK;
       });
       if (rc) return rc;
-      done += pchunk;
+      done += n;
       if (!S->h_stat->notDone) break;
     }
     done = maxIter + 1;  // the graph path below is skipped

@@ -875,6 +875,7 @@ static hipError_t launch_step_kernel(dpm_set_s* S, int mode, const StepArgs& A0)
   if (S->P.particle == PART_ACTIVE_SHAPE && !S->V.l0r) return hipErrorInvalidValue;
   if ((mode & MODE_FIRE) && (!A.fire || !A.part)) return hipErrorInvalidValue;
   if ((mode & MODE_RIGID) && S->P.interaction == INT_ALL) return hipErrorInvalidValue;
+  if ((mode & MODE_NEAR) && (!A.near.task || S->V.W > 64)) return hipErrorInvalidValue;  // masks of 64 entries
   if ((mode & MODE_START) && (!A.xout || !A.yout || !A.flagOut || !A.anyOut)) return hipErrorInvalidValue;
   if (A.manage && (!A.flagCur || !A.cellCur || !A.slotsCur || (A.genCur && !A.genOut) || !A.err || !A.maxcnt ||
                    !A.updateCount))

@@ -91,3 +91,30 @@ def test_fire_minimize_widens_list_and_matches_oracle(oracle_mod):
     o.fire(300)
     for pos in runs:
         assert rel_err(pos, o.get("pos"), 1.0) < 1e-10
+
+
+def test_fire_minimize_outgrows_near_lists(oracle_mod):
+    """The library's own choice of kernel for one packing of 100 rings (every tile, on near lists, which
+    hold rows of at most 64 entries) from rows 64 wide to positions, pulled together without a rebuild,
+    whose rows are longer: the replay has no near lists and goes on in the persistent kernel."""
+    from cudaring_amd import packing
+    st = packing.lattice_system(100, 0.3, 11, n_small=16, n_large=22, perturb=0.1)
+    size, L = 2 * float(np.mean(st["rad"])), st["box"][0]
+    pos = st["pos"].reshape(-1, 2).copy()
+    first = np.concatenate([[0], np.cumsum(st["nvp"])])
+    for a, b in zip(first[:-1], first[1:]):
+        pos[a:b] += 0.3 * (L / 2 - pos[a:b].mean(0))
+    g, o = gpu_from_state(st), oracle_from_state(oracle_mod, st)
+    for s in (g, o):
+        s.calc_neighbor_list(s.set_displacement_cutoff(7.0, size))
+        s.set("pos", pos.ravel())
+        s.calc_force_energy()
+        s.init_fire((0.2, 0.5, 1.1, 0.99, 1e-3, 1e-2, 0.2), 20, 0)
+    assert g.neighbors()[1] == 64
+    print("case fire default choice, rows 64 -> 128", flush=True)
+    g.fire_minimize(0.0, 40)
+    o.fire(40)
+    assert g.neighbors()[1] == 128
+    assert rel_err(g.get("pos"), o.get("pos"), 1.0) < 1e-10
+    assert rel_err(g.get("force"), o.get("force")) < 1e-9
+    g.close()
