@@ -1079,7 +1079,7 @@ int run_rigid(dpm_set_s* S, long steps, bool langevin) {
 int rigid_fire_sequence(dpm_set_s* S, long iterations) {
   // the step loop's cell protocol: the list positions binned into cell list 0 and the current
   // positions' list validity in F[0]; iteration i's move ORs its moved positions' validity into
-  // F[i] (a drift longer than cutoff / 3 flags FLAG_FAR), and its step (rotation index i) reads
+  // F[i] (FLAG_FAR beyond 2 cutoff / 3 from a list position), and its step (rotation index i) reads
   // F[i], rebuilds flagged systems from the list-position cells (all pairs on FLAG_FAR) and clears
   // F[i + 2] for the move after next
   const bool near = near_loop(S, iterations);

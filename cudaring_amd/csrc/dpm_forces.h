@@ -407,6 +407,15 @@ __device__ __forceinline__ void far_test(const Params& P, const Box& B, double d
   if (moved_past(P, B, dx, dy)) atomicOr(flag, FLAG_FAR);
 }
 
+// Rebuild flag of a vertex (dx, dy) from its list position: the displacement test, with FLAG_FAR beyond the
+// 2 cutoff / 3 that the cells of the list positions allow for, however the vertex came there
+__device__ __forceinline__ void moved_test(const Params& P, const Box& B, double dx, double dy, int* flag, int* any) {
+  if (moved_past(P, B, dx, dy)) {
+    atomicOr(flag, moved_past(P, B, dx, dy, 2.0) ? 1 | FLAG_FAR : 1);
+    if (any) atomicOr(any, 1);
+  }
+}
+
 // The step loop's cell lists of a system whose list positions (the positions of its last
 // rebuild) have generation g: its rows are rebuilt from list g % 3, the rebuild bins its own
 // positions (the next list positions) into list (g + 1) % 3, cleared by the rebuild before, and

@@ -33,8 +33,8 @@ enum : int { NOISE_LANGEVIN = 0, NOISE_BAOAB = 1, NOISE_BROWNIAN = 2, NOISE_DRIV
 enum : int { ERR_LIST_OVERFLOW = 1, ERR_CELL_OVERFLOW = 2, ERR_STALE_BINS = 4 };
 
 // rebuild-flag bits (per system): 1 = rebuild, FLAG_FAR = a vertex moved more than cutoff / 3 in
-// the drift that produced these positions, or (first positions of a step loop) lies more than
-// 2 cutoff / 3 from its list position: the cells of the list positions may miss its neighbours
+// the drift that produced these positions, or (first positions of a step loop, FIRE's moves) lies more
+// than 2 cutoff / 3 from its list position: the cells of the list positions may miss its neighbours
 enum : int { FLAG_FAR = 2 };
 
 // per-system FIRE scalars (double buffered by iteration parity)

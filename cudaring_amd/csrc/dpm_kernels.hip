@@ -220,10 +220,7 @@ __device__ __forceinline__ void md_prologue(const View& V, const Params& P, cons
                                             const Box& B, int v, int s, double x, double y, int* flag, int* any) {
   const double lx = V.lx[v], ly = V.ly[v];
   bin_vertex(G, B, A.cellCur, A.slotsCur, v, s, lx, ly, A.err);
-  if (moved_past(P, B, x - lx, y - ly)) {
-    atomicOr(flag, moved_past(P, B, x - lx, y - ly, 2.0) ? 1 | FLAG_FAR : 1);
-    if (any) atomicOr(any, 1);
-  }
+  moved_test(P, B, x - lx, y - ly, flag, any);
 }
 
 // Start of a step loop, one workgroup per tile: wave 0 takes the loop's opening move, all waves
@@ -641,11 +638,7 @@ __global__ void k_rigid_fire_move(View V, Params P, FireParams fp, const FireSta
   rigid_move(B, V.x[L.v], V.y[L.v], lcx, lcy, cx, cy, cos(dth), sin(dth), xn, yn);
   xo[L.v] = xn;
   yo[L.v] = yn;
-  if (moved_past(P, B, xn - V.lx[L.v], yn - V.ly[L.v])) {
-    atomicOr(&flagOut[L.s], 1);
-    atomicOr(anyOut, 1);
-  }
-  far_test(P, B, xn - V.x[L.v], yn - V.y[L.v], flagOut + L.s);
+  moved_test(P, B, xn - V.lx[L.v], yn - V.ly[L.v], flagOut + L.s, anyOut);
   if (L.lane == L.segS) {
     R.plx[L.r] = lcx;
     R.ply[L.r] = lcy;
@@ -801,12 +794,7 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_move(View V, Params P, 
     fire_move(fs, sum, reset, V.fx[v], V.fy[v], xn, yn, vx, vy);
     vxn[v] = vx;
     vyn[v] = vy;
-    const Box B = box_of(V, s);
-    if (moved_past(P, B, xn - V.lx[v], yn - V.ly[v])) {
-      atomicOr(&flagOut[s], 1);
-      atomicOr(anyOut, 1);
-    }
-    far_test(P, B, xn - x, yn - y, flagOut + s);
+    moved_test(P, box_of(V, s), xn - V.lx[v], yn - V.ly[v], flagOut + s, anyOut);
   }
   xo[v] = xn;
   yo[v] = yn;

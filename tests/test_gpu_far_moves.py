@@ -110,3 +110,65 @@ def test_fast_rigid_rings_langevin(oracle_mod):
         assert rel_err(g.get("pvel"), o.get("pvel")) < 1e-10, chunk
     assert g.update_count()[0] >= 2  # the list was rebuilt (all pairs) in these steps
     g.close()
+
+
+def drifting(g, st, force, size, cutoff, dt):
+    """`g` moved by 0.6 cutoff from its list positions without a list build (a translation of the whole
+    packing, which keeps every pair distance), drifting on at 0.25 cutoff per `dt`; a little of the force
+    in the velocities keeps FIRE's power positive.  Returns the velocities."""
+    u = np.array([np.cos(0.7), np.sin(0.7)]) * cutoff * size
+    g.set("pos", st["pos"] + np.tile(0.6 * u, len(st["rad"])))
+    return np.tile(0.25 * u / dt, len(force) // 2) + 1e-3 * force
+
+
+@pytest.mark.parametrize("inter", ["vertexVertex", "vertexSmooth"])
+def test_fire_minimize_starts_beyond_displacement_test(inter):
+    """A start farther than cutoff / 3 from the list positions and a first drift (below cutoff / 3 itself)
+    past 2 cutoff / 3, which the cells of the list positions do not cover: FIRE on every tile (the
+    library's choice for one packing of 60 rings) rebuilds as the persistent kernel does."""
+    from cudaring_amd import packing
+    print(f"case far_moves fire tiles {inter}", flush=True)
+    st = packing.lattice_system(60, 0.8, 21, n_small=16, n_large=22, perturb=0.05)
+    size = 2 * float(st["rad"].mean())
+    dt = 1e-2
+    out = []
+    for persistent in (False, True):
+        g = gpu_from_state(st, interaction=inter, costs=(1, 1, 0.1, 1))
+        g.calc_neighbor_list(g.set_displacement_cutoff(0.5, size))
+        g.calc_force_energy()
+        g.set("vel", drifting(g, st, g.get("force"), size, 0.5, dt))
+        g.calc_force_energy()
+        g.init_fire((0.2, 0.5, 1.1, 0.99, dt, dt, 0.02), 20, 0)
+        if persistent:
+            g.set_fire_kernel(True, 0)
+        g.fire_minimize(0.0, 5)
+        out.append((g.get("pos"), g.get("force"), list(g.update_count())))
+        g.close()
+    assert out[0][2] == out[1][2] and out[0][2][0] >= 1
+    assert rel_err(out[0][0], out[1][0], scale=1.0) < 1e-11
+    assert rel_err(out[0][1], out[1][1]) < 1e-10
+
+
+def test_rigid_fire_starts_beyond_displacement_test():
+    """The same start for rigid FIRE, against a set whose list is built at the start positions."""
+    print("case far_moves rigid fire", flush=True)
+    st = ring_block(gap=1.5, seed=9)
+    size = 2 * st["rad"].mean()
+    dt = 1e-2
+    out = []
+    for fresh in (False, True):
+        g = gpu_from_state(st, costs=(0, 0, 0, 1))
+        cut = g.set_displacement_cutoff(0.5, size)
+        g.calc_neighbor_list(cut)
+        g.calc_rigid_force_energy()
+        v = drifting(g, st, g.get("pforce"), size, 0.5, dt)
+        if fresh:
+            g.calc_neighbor_list(cut)
+        g.calc_rigid_force_energy()
+        g.init_rigid_fire([0.2, 0.5, 1.1, 0.99, dt, dt, 0.2], 20, 0)
+        g.set("pvel", v)
+        g.rigid_fire(5)
+        out.append((g.get("pos"), g.get("pforce")))
+        g.close()
+    assert rel_err(out[0][0], out[1][0], scale=1.0) < 1e-11
+    assert rel_err(out[0][1], out[1][1]) < 1e-10
