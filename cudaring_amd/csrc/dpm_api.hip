@@ -726,7 +726,9 @@ int fire_waves(const dpm_set_s* S) {
 // microseconds, and every dpm_init_fire would capture a graph anew.
 int fire_tile_sequence(dpm_set_s* S, long iterations) {
   const int most = most_tiles(S), waves = fire_waves(S);
-  HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[0], S->mdGen[0], S->N));
+  // the start positions' flags go to the sink: the rows serve the positions after the first move, which
+  // flags those (a system that stops before it moves keeps its rows)
+  HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[3], S->mdGen[0], S->N));
   for (long it = 0; it < iterations; it++) {
     HIPCHK(launch_fire_move(S, most, waves, S->mdFlag[it % 3], S->d_any + 2));
     S->fireCur = 1 - S->fireCur;

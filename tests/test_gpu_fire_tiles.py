@@ -42,3 +42,24 @@ def test_tiles_match_persistent(pot, inter, iters, sizes):
     assert list(a.update_count()) == list(b.update_count())
     for x in (a, b):
         x.close()
+
+
+def test_stopped_system_keeps_its_rows():
+    """A system that meets its tolerance before it moves, displaced past the displacement test: neither
+    path rebuilds its rows."""
+    st = packing.lattice_system(60, 0.8, 21, n_small=16, n_large=22, perturb=0.05)
+    size = 2 * float(st["rad"].mean())
+    for persistent in (False, True):
+        g = gpu_from_state(st)
+        g.calc_neighbor_list(g.set_displacement_cutoff(0.5, size))
+        last = g.get("lastpos")
+        g.set("pos", st["pos"] + 0.25 * size)
+        g.calc_force_energy()
+        g.init_fire([0.2, 0.5, 1.1, 0.99, 1e-2, 1e-1, 0.2], 20, 0)
+        if persistent:
+            g.set_fire_kernel(True, 0)
+        before = list(g.update_count())
+        assert list(g.fire_minimize(1e9, 10)) == [0]
+        assert list(g.update_count()) == before
+        assert np.array_equal(g.get("lastpos"), last)
+        g.close()
