@@ -199,7 +199,7 @@ __global__ void k_adj_seg_check(View V, Params P, const double* seg, int slots, 
 template <int INTER, int POT>
 __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_adj_hvp(View V, Params P, CellGrid G, AdjArgs A) {
   // partials of gather waves 1..nw-1: red[((w - 1) * NR + q) * WAVE + lane], sized by the launch
-  extern __shared__ double red[];
+  extern __shared__ __align__(16) double red[];
   constexpr int NR = INTER == INT_SMOOTH ? 4 : 2;
   const int w = threadIdx.x / WAVE;
   const int nw = blockDim.x / WAVE;

@@ -61,7 +61,9 @@ template <int INTER, int POT, bool NEAR>
 __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, FireParams fp, CellGrid G, NearRows N,
                                                              FireState* fst, int chunk, int* updateCount, int* err,
                                                              int* maxcnt, const int* order) {
-  extern __shared__ double dyn[];  // NEAR: per wave near_wave_doubles, then the positions
+  // NEAR: per wave near_wave_doubles, then the positions, both read and written as double2
+  extern __shared__ __align__(16) double dyn[];
+  static_assert(__alignof__(dyn) % alignof(double2) == 0, "128-bit LDS accesses");
   __shared__ double red[FS_WAVES][5];
   __shared__ int movedFlag[2];
   const int s = order[blockIdx.x];

@@ -26,8 +26,10 @@ constexpr bool step_store() {
 
 template <int INTER, int POT, int MODE>
 __global__ __launch_bounds__(WAVE* MAXSPLIT) void k_step(View V, Params P, StepArgs A, CellGrid G) {
-  // partials of gather waves 1..nw-1: red[((w - 1) * 6 + q) * WAVE + lane], sized by the launch
-  extern __shared__ double red[];
+  // partials of gather waves 1..nw-1: red[((w - 1) * 6 + q) * WAVE + lane], sized by the launch; near
+  // lists' results as double2
+  extern __shared__ __align__(16) double red[];
+  static_assert(__alignof__(red) % alignof(double2) == 0, "128-bit LDS accesses");
   const int w = threadIdx.x / WAVE;
   const int nw = blockDim.x / WAVE;
   Lane L;
