@@ -723,14 +723,26 @@ int fire_waves(const dpm_set_s* S) {
 // FIRE iterations on every tile of the set, two launches each: the move (parameter update, drift and
 // displacement flags of every system) and the step kernel on near lists, with the step loop's cell
 // protocol as rigid FIRE runs it.  Stream launches: the host stays ahead of kernels of five
-// microseconds, and every dpm_init_fire would capture a graph anew.
+// microseconds, and every dpm_init_fire would capture a graph anew.  It ends with the last system: the
+// moves of iterations 2, 6, 14, 30 and of every 32nd from there tell the host whether a system goes on,
+// which looks with the next iterations already enqueued: the kernels never wait for the host, and at
+// most 64 iterations of two short launches follow the last system's.
 int fire_tile_sequence(dpm_set_s* S, long iterations) {
   const int most = most_tiles(S), waves = fire_waves(S);
+  for (hipEvent_t& e : S->fireEvent)
+    if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  long part = 2, look = part;  // iterations up to the next look
+  int looks = 0;
   // the start positions' flags go to the sink: the rows serve the positions after the first move, which
   // flags those (a system that stops before it moves keeps its rows)
   HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[3], S->mdGen[0], S->N));
   for (long it = 0; it < iterations; it++) {
-    HIPCHK(launch_fire_move(S, most, waves, S->mdFlag[it % 3], S->d_any + 2));
+    volatile int* open = nullptr;
+    if (it + 1 == look) {
+      open = S->h_stat->open + looks % 4;
+      *open = 0;
+    }
+    HIPCHK(launch_fire_move(S, most, waves, S->mdFlag[it % 3], S->d_any + 2, (int*)open));
     S->fireCur = 1 - S->fireCur;
     swap_pos(S);
     StepArgs A = md_args(S, it, 0, 0, true);
@@ -738,8 +750,18 @@ int fire_tile_sequence(dpm_set_s* S, long iterations) {
     A.part = S->d_part;
     A.vel = S->d_fireVel;
     HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR, A));
+    if (open) {
+      HIPCHK(hipEventRecord(S->fireEvent[looks % 2], S->stream));
+      if (looks > 0) {
+        HIPCHK(hipEventSynchronize(S->fireEvent[1 - looks % 2]));
+        if (!*(volatile int*)(S->h_stat->open + (looks - 1) % 4)) break;
+      }
+      looks++;
+      part = std::min(2 * part, 32L);
+      look += part;
+    }
   }
-  StepArgs A = md_args(S, iterations, 0, 0, true);  // energies and ring geometry of the positions reached
+  StepArgs A = md_args(S, 0, 0, 0, true);  // energies and ring geometry of the positions reached
   A.fire = S->d_fire[S->fireCur];
   A.part = S->d_part;
   A.vel = S->d_fireVel;
@@ -1317,6 +1339,8 @@ int dpm_destroy(dpm_set_t h) {
     if (p) hipFree(p);
   if (S->h_red) hipHostFree(S->h_red);
   if (S->h_stat) hipHostFree(S->h_stat);
+  for (hipEvent_t e : S->fireEvent)
+    if (e) hipEventDestroy(e);
   if (S->ownStream) hipStreamDestroy(S->ownStream);
   delete S;
   return DPM_OK;

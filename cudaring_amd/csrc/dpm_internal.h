@@ -132,6 +132,7 @@ struct FillSegs {
 // What the loops and list builds leave for the host, in pinned memory their last kernel writes.
 struct HostStat {
   int err, maxcnt, notDone;
+  int open[4];  // FIRE on tiles: set by a move that leaves a system to go on, one word per look
 };
 
 // Arguments of the H w kernel (dpm_adjoint.hip).
@@ -243,6 +244,7 @@ struct dpm_set_s {
   dpm::FireParams fp{};
   double* d_part = nullptr;  // per-tile partials [ntiles * 4]
   double* d_fireVel = nullptr;  // FIRE on tiles: velocities between the move and the step [2 * nv]
+  hipEvent_t fireEvent[2] = {nullptr, nullptr};  // FIRE on tiles: behind the moves of the last two looks
   bool fireInit = false;
   int fireKernel = -1;  // dpm_fire_minimize: 1 = one persistent workgroup per system, 0 = graph of step
                         //   kernels, -1 = persistent or on every tile (fire_on_tiles)
@@ -321,7 +323,7 @@ hipError_t launch_fire_mid(dpm_set_s* S);
 hipError_t launch_fire_partials(dpm_set_s* S);
 hipError_t launch_fire_step(dpm_set_s* S);
 hipError_t launch_fire_resume(dpm_set_s* S);
-hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut);
+hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut, int* open);
 StepArgs loop_args(dpm_set_s* S);
 hipError_t launch_bin_view(dpm_set_s* S, const View& Vn, int parity);
 hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves);

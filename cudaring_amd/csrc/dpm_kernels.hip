@@ -766,24 +766,31 @@ __global__ void k_fire_partials(View V, double* part) {
 // first, over the vertices in the order of the persistent kernel with as many waves (so that both follow
 // the same path to the last bit), then takes the stopping rule and the parameter update and moves its
 // vertices into the other position buffer and vxn, vyn (other blocks still sum vx, vy), with the step
-// loop's flags.
+// loop's flags.  A system that has stopped only keeps its positions in the buffer that is read next.
 __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_move(View V, Params P, FireParams fp, int per,
                                                               const FireState* fin, FireState* fout, double* xo,
                                                               double* yo, double* vxn, double* vyn, int* flagOut,
-                                                              int* anyOut) {
+                                                              int* anyOut, int* open) {
   __shared__ double red[FS_WAVES][5];
   const int s = blockIdx.x / per, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x & (WAVE - 1);
   const int t0 = V.stile[s], t1 = V.stile[s + 1], tile = t0 + (blockIdx.x % per) * nw + w;
   FireState fs = fin[s];
-  const FireNext next(fp, fs);
-  FireSums a{0, -1, 0, 0, 0};
-  for (int t = t0 + w; t < t1; t += nw) {
-    const int v = V.tile_v0[t] + lane;
-    if (v < V.tile_v1[t]) fire_add(a, next, V.vx[v], V.vy[v], V.fx[v], V.fy[v]);
+  FireSums sum{0, -1, 0, 0, 0};
+  bool reset = false;
+  if (!fs.converged) {
+    const FireNext next(fp, fs);
+    FireSums a{0, -1, 0, 0, 0};
+    for (int t = t0 + w; t < t1; t += nw) {
+      const int v = V.tile_v0[t] + lane;
+      if (v < V.tile_v1[t]) fire_add(a, next, V.vx[v], V.vy[v], V.fx[v], V.fy[v]);
+    }
+    sum = fire_block_sums(a, red, nw);
+    reset = fire_update(fs, fp, sum);
   }
-  const FireSums sum = fire_block_sums(a, red, nw);
-  const bool reset = fire_update(fs, fp, sum);
-  if (tile == t0 && lane == 0) fout[s] = fs;
+  if (tile == t0 && lane == 0) {
+    fout[s] = fs;
+    if (open && !fs.converged) *open = 1;  // for the host (pinned memory); every writer writes 1
+  }
   if (tile >= t1) return;
   const int v = V.tile_v0[tile] + lane;
   if (v >= V.tile_v1[tile]) return;
@@ -1062,13 +1069,13 @@ hipError_t launch_fire_mid(dpm_set_s* S) {
   return hipGetLastError();
 }
 
-hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut) {
+hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut, int* open) {
   if (!flagOut || !anyOut || waves < 1 || waves > FS_WAVES) return hipErrorInvalidValue;
   const int nb = 1 - S->cur;
   const int per = (most + waves - 1) / waves;
   k_fire_move<<<(unsigned)(S->nsys * per), WAVE * waves, 0, S->stream>>>(
       S->V, S->P, S->fp, per, S->d_fire[S->fireCur], S->d_fire[1 - S->fireCur], S->pos[nb][0], S->pos[nb][1], S->d_fireVel,
-      S->d_fireVel + S->V.nv, flagOut, anyOut);
+      S->d_fireVel + S->V.nv, flagOut, anyOut, open);
   return hipGetLastError();
 }
 

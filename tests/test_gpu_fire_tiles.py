@@ -2,6 +2,8 @@
 workgroup per system: the same iterations, a system that stops early staying as it stopped.  The two
 add in different orders: an ulp of the forces, amplified a thousandfold per ten iterations where the
 contacts are stiff (WCA), so 20 iterations are compared there and 30 of the harmonic packing, to 1e-11."""
+import time
+
 import numpy as np
 import pytest
 
@@ -63,3 +65,26 @@ def test_stopped_system_keeps_its_rows():
         assert list(g.update_count()) == before
         assert np.array_equal(g.get("lastpos"), last)
         g.close()
+
+
+def test_call_on_relaxed_packing_ends_at_once():
+    """A minimisation whose system has stopped does not run on to the end of its launches' chunk: on a
+    packing of 200 rings that meets its tolerance at once, the tiles take a few launches more than the
+    persistent kernel's one (512 launches took forty times as long; ten is allowed)."""
+    st = packing.lattice_system(200, 0.8, 22, n_small=16, n_large=22, perturb=0.05)
+    best = []
+    for persistent in (False, True):
+        g = gpu_from_state(st)
+        g.calc_neighbor_list(g.set_displacement_cutoff(0.5, 2 * float(st["rad"].mean())))
+        g.calc_force_energy()
+        g.init_fire([0.2, 0.5, 1.1, 0.99, 1e-2, 1e-1, 0.2], 20, 0)
+        if persistent:
+            g.set_fire_kernel(True, 0)
+        times = []
+        for _ in range(6):
+            t0 = time.perf_counter()
+            assert list(g.fire_minimize(1e9, 10000)) == [0]
+            times.append(time.perf_counter() - t0)
+        best.append(min(times))
+        g.close()
+    assert best[0] < 10 * best[1], best
