@@ -253,7 +253,7 @@ def fire_setup(s, size, skin=0.3, cell_scale=1.0):
 def fire_step(s, cut, mode):
     """One compression step of every system in `s` (compressFIRE.cpp:104-131, 153): grow by
     sqrt((phi + dphi) / phi), rebuild, FIRE to max|F_c| <= tol.  `mode` "engine": the set's own
-    fire_minimize (every system to its own convergence, persistent kernel); "host": the reference
+    fire_minimize (every system to its own convergence); "host": the reference
     driver's loop, one FIRE iteration and one host check of max|F_c| per call.  Returns
     iterations per system."""
     phi = s.phi()
@@ -274,7 +274,8 @@ def fire_step(s, cut, mode):
 
 def batched_fire(args):
     """cfg3: packings/s of the batched set against two one-system paths on a stratified sample of
-    the same packings: the engine's own fire_minimize on a set holding one system, and the
+    the same packings: the engine's own fire_minimize, on the library's own kernel, on a set holding one
+    system, and the
     reference driver's loop (one iteration, one host check per call)."""
     from cudaring_amd import DPMSet, autotune, packing
     systems = fire_systems()
@@ -322,7 +323,6 @@ def batched_fire(args):
             p.load_state(sub)
             p.set("vel", start["vel"][2 * voff[i]:2 * voff[i + 1]])
             pcut = fire_setup(p, size, skin, cell_scale)
-            p.set_fire_kernel(*fire_kernel)
             p.synchronize()
             t0 = time.perf_counter()
             for _ in range(args.fire_steps):
@@ -351,7 +351,7 @@ def batched_fire(args):
                       f"{t_path['engine']:.2f} s; the driver loop with a host check per iteration "
                       f"{it_path['host']} iterations in {t_path['host']:.2f} s",
             "start_relax_iterations_max": int(it0.max()), "start_relax_s": round(relax_s, 2),
-            "fire_kernel": {"persistent": bool(fire_kernel[0]), "waves": int(fire_kernel[1])},
+            "fire_kernel": {"persistent": int(fire_kernel[0]), "waves": int(fire_kernel[1])},
             "fire_tune_s": fire_tune, "skin": skin, "cell_scale": cell_scale, "neighbor_tune_s": nbr_tune,
             "cpu": cpu}
 

@@ -71,9 +71,9 @@ def tune_skin(s, size, candidates=(0.2, 0.3, 0.5, 0.8), steps=400, kind="langevi
     return best, times
 
 
-def tune_fire(s, params7, cut, candidates=((1, 2), (1, 4), (1, 8), (1, 16), (0, 0)), iters=200):
-    """Pick the fire_minimize kernel (persistent workgroup per system with 2/4/8/16 waves, or graphs
-    of the split step kernels) by timing `iters` iterations of each from the caller's state,
+def tune_fire(s, params7, cut, candidates=((-1, 0), (1, 2), (1, 4), (1, 8), (1, 16), (0, 0)), iters=200):
+    """Pick the fire_minimize kernel (the library's choice, the persistent workgroup per system with
+    2/4/8/16 waves, or graphs of the split step kernels) by timing `iters` iterations of each from the caller's state,
     which is restored after every trial and at the end."""
     keep = {k: s.get(k) for k in ("pos", "vel")}
     times = {}
@@ -95,7 +95,8 @@ def tune_fire(s, params7, cut, candidates=((1, 2), (1, 4), (1, 8), (1, 16), (0, 
     s.calc_neighbor_list(cut)
     s.calc_force_energy()
     s.set_fire_kernel(*best)
-    return best, {f"{'persistent' if p else 'graph'}{w or ''}": round(t, 4) for (p, w), t in times.items()}
+    name = {-1: "automatic", 0: "graph", 1: "persistent"}
+    return best, {f"{name[int(p)]}{w or ''}": round(t, 4) for (p, w), t in times.items()}
 
 
 def tune_fire_neighbors(s, params7, size, skins=(0.2, 0.3, 0.5, 0.8), scales=(1.0, 1.5, 2.0), iters=200):

@@ -2012,9 +2012,9 @@ int dpm_fire_minimize(dpm_set_t h, double tol, long maxIter, long* iterations) {
 
 int dpm_set_fire_kernel(dpm_set_t h, int persistent, int wavesPerSystem) {
   CHECK_HANDLE(h);
-  if (persistent < 0 || persistent > 1 || wavesPerSystem < 0 || wavesPerSystem > 16)
-    return fail(S, DPM_ERR_ARG, "dpm_set_fire_kernel: persistent in {0, 1}, waves in 0..16");
-  if (persistent && S->nwide > 0)
+  if (persistent < -1 || persistent > 1 || wavesPerSystem < 0 || wavesPerSystem > 16)
+    return fail(S, DPM_ERR_ARG, "dpm_set_fire_kernel: persistent in {-1, 0, 1}, waves in 0..16");
+  if (persistent == 1 && S->nwide > 0)
     return fail(S, DPM_ERR_UNSUPPORTED, "one-workgroup-per-system FIRE: rings of at most 64 vertices only");
   S->fireKernel = persistent;
   S->fireWaves = wavesPerSystem;

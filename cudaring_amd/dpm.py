@@ -423,8 +423,10 @@ class DPMSet:
 
     def set_fire_kernel(self, persistent=True, waves=0):
         """fire_minimize on one persistent workgroup per system (waves 1..16, 0 = one per tile of
-        the largest system up to 16), or on graphs of step kernels."""
-        self._chk(self.L.dpm_set_fire_kernel(self.h, int(bool(persistent)), int(waves)), "set_fire_kernel")
+        the largest system up to 16), or on graphs of step kernels; persistent = -1: the library's
+        choice, which a new set starts with (persistent, or every tile for few systems)."""
+        kind = -1 if persistent == -1 else int(bool(persistent))
+        self._chk(self.L.dpm_set_fire_kernel(self.h, kind, int(waves)), "set_fire_kernel")
 
     def fire_minimize(self, tol, max_iter):
         it = np.zeros(self.nsys, dtype=np.int64)

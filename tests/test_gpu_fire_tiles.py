@@ -67,6 +67,25 @@ def test_stopped_system_keeps_its_rows():
         g.close()
 
 
+def test_choice_can_be_given_back():
+    """set_fire_kernel(-1) gives the choice back to the library, and the tuner tries that choice too."""
+    from cudaring_amd import autotune
+    from cudaring_amd.dpm import DPMError
+    st = packing.lattice_system(60, 0.8, 21, n_small=16, n_large=22, perturb=0.05)
+    g = gpu_from_state(st)
+    cut = g.set_displacement_cutoff(0.5, 2 * float(st["rad"].mean()))
+    best, times = autotune.tune_fire(g, [0.2, 0.5, 1.1, 0.99, 1e-2, 1e-1, 0.2], cut, iters=20)
+    assert "automatic" in times and len(times) == 6
+    for kind in (1, -1, 0, -1):
+        g.set_fire_kernel(kind, 0)
+        g.init_fire([0.2, 0.5, 1.1, 0.99, 1e-2, 1e-1, 0.2], 20, 0)
+        assert list(g.fire_minimize(0.0, 5)) == [5]
+    for kind, waves in ((-2, 0), (2, 0), (-1, 17)):
+        with pytest.raises(DPMError, match="bad argument"):
+            g._chk(g.L.dpm_set_fire_kernel(g.h, kind, waves), "set_fire_kernel")
+    g.close()
+
+
 def test_call_on_relaxed_packing_ends_at_once():
     """A minimisation whose system has stopped does not run on to the end of its launches' chunk: on a
     packing of 200 rings that meets its tolerance at once, the tiles take a few launches more than the
