@@ -24,8 +24,11 @@ namespace dpm {
 // Terms and sums keep the reference's order of operations and its rounding (quot, root): a minimiser
 // amplifies last bits, a thousandfold per ten iterations of a stiff contact.  The loops' short forms and
 // |v|^2 + 2 h P + h^2 |F|^2 took 512 packings of 16 to 256 rings through 2 x 60 iterations in 10.0 ms,
-// this takes 15.5 (whole rows from memory, four barriers: 19.1), but there single packings of a set left
+// this takes 15.3 (whole rows from memory, four barriers: 19.1), but there single packings of a set left
 // the path: forces off by up to 9e-4 after a second compression.
+// MAXW 8: up to eight waves a lane may hold 256 registers, and nothing spills (200 to 214 in use); 16 waves
+// have 128, of which 63 to 114 spill.  512 packings of 16 to 256 rings, 200 iterations: 8 waves 63.4 -> 51.0 ms
+// and 4 waves 93.1 -> 79.3 against the 16-wave build (12 waves take 54.0, 16 take 48.0).
 // Without near lists (rows of more than 64 entries, systems of more vertices than LDS holds, the
 // all-pairs interaction) it gathers over whole rows from memory.
 
@@ -57,14 +60,14 @@ __device__ __forceinline__ void tile_force(const View& V, const Params& P, const
   if (STORE && L.act) V.ev[L.v] = so.e + e;
 }
 
-template <int INTER, int POT, bool NEAR>
-__global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, FireParams fp, CellGrid G, NearRows N,
+template <int INTER, int POT, bool NEAR, int MAXW>
+__global__ __launch_bounds__(WAVE* MAXW) void k_fire_sys(View V, Params P, FireParams fp, CellGrid G, NearRows N,
                                                              FireState* fst, int chunk, int* updateCount, int* err,
                                                              int* maxcnt, const int* order) {
   // NEAR: per wave near_wave_doubles, then the positions, both read and written as double2
   extern __shared__ __align__(16) double dyn[];
   static_assert(__alignof__(dyn) % alignof(double2) == 0, "128-bit LDS accesses");
-  __shared__ double red[FS_WAVES][5];
+  __shared__ double red[MAXW][5];
   __shared__ int movedFlag[2];
   const int s = order[blockIdx.x];
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
@@ -186,8 +189,8 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_sys(View V, Params P, F
 #if !defined(FIRE_INTER) || !defined(FIRE_POT)
 #error "compile with -DFIRE_INTER and -DFIRE_POT"
 #endif
-template <>
-hipError_t fire_launch<FIRE_INTER, FIRE_POT>(dpm_set_s* S, int chunk, int threads) {
+template <int MAXW>
+static hipError_t fire_waves_launch(dpm_set_s* S, int chunk, int threads) {
   const unsigned g = (unsigned)S->nsys;
 #if FIRE_INTER != 3
   int most = 0;
@@ -195,7 +198,7 @@ hipError_t fire_launch<FIRE_INTER, FIRE_POT>(dpm_set_s* S, int chunk, int thread
   const size_t lds = (size_t)(threads / WAVE) * near_wave_doubles<FIRE_INTER>() * sizeof(double) +
                      (size_t)most * sizeof(double2);
   if (S->N.task && lds <= kFireLds) {
-    auto k = k_fire_sys<FIRE_INTER, FIRE_POT, true>;
+    auto k = k_fire_sys<FIRE_INTER, FIRE_POT, true, MAXW>;
     hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFireLds);
     if (e != hipSuccess) return e;
     k<<<g, threads, lds, S->stream>>>(S->V, S->P, S->fp, S->G, S->N, S->d_fire[S->fireCur], chunk, S->d_updateCount,
@@ -203,10 +206,16 @@ hipError_t fire_launch<FIRE_INTER, FIRE_POT>(dpm_set_s* S, int chunk, int thread
     return hipGetLastError();
   }
 #endif
-  k_fire_sys<FIRE_INTER, FIRE_POT, false>
+  k_fire_sys<FIRE_INTER, FIRE_POT, false, MAXW>
       <<<g, threads, 0, S->stream>>>(S->V, S->P, S->fp, S->G, S->N, S->d_fire[S->fireCur], chunk, S->d_updateCount,
                                      S->d_err, S->d_maxcnt, S->d_sysOrder);
   return hipGetLastError();
+}
+
+template <>
+hipError_t fire_launch<FIRE_INTER, FIRE_POT>(dpm_set_s* S, int chunk, int threads) {
+  return threads <= WAVE * FS_WAVES_FEW ? fire_waves_launch<FS_WAVES_FEW>(S, chunk, threads)
+                                        : fire_waves_launch<FS_WAVES>(S, chunk, threads);
 }
 
 }  // namespace dpm
