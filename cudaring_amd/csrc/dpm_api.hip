@@ -771,17 +771,18 @@ int fire_tile_sequence(dpm_set_s* S, long iterations) {
 }
 
 // Whether a minimisation of the set's systems runs on every tile rather than on one workgroup per
-// system, from what an iteration takes either way (us, harmonic vertex-vertex): 12 for the two launches
-// and 0.008 a tile of the set (measured 13.0 at 33 tiles, 13.4 at 85, 16.3 at 266, 59 at 5,333); or 3 and
-// 0.65 a tile of the largest system on its one CU, as often as the systems fill the chip (10.0 at 5
-// tiles, 13.5 at 10, 24.5 at 21, 32.6 at 33, 80 at 85 with frequent rebuilds, 31 at 60 without).  Those
-// are the times of the short forms; in the reference's order both sides take about 1.4 times as long (one
-// packing of 60 tiles on tiles 3.0 -> 4.3 ms, 512 packings on one workgroup each 10.0 -> 15.5).
+// system, from what an iteration without rebuilds takes either way (us): 14.5 for the two launches and
+// 0.010 a tile of the set; or 5 and 0.85 a tile of the largest system on its one CU, or the same summed
+// over the systems and shared by 256 CUs where that is more.  Measured (tiles of the set, harmonic
+// vertex-vertex and WCA vertex-segment; persistent against tiles): one system of 8 tiles 8.5, 12.4 against
+// 13.4, 14.2; of 10 12.7, 18.2 against 14.7, 15.5; of 13 15.7, 19.5 against 15.8, 16.6; of 66 47, 65 against
+// 19, 20; 64 systems of up to 21 (827) 22, 28 against 20, 20; 128 of up to 42 (2,995) 43, 53 against 42, 42;
+// 300 of up to 21 (3,875) 36, 43 against 50, 51; 512 of up to 85 (22,714) 120, 141 against 229, 246.  Where
+// every few iterations rebuild, the tiles gain more (827 tiles: 47 against 29).  Both give the same bits.
 bool fire_on_tiles(const dpm_set_s* S) {
   if (!near_loop(S, NEAR_STEPS)) return false;
-  const int most = most_tiles(S);
-  const double rounds = (double)((S->nsys + 255) / 256);
-  return 12 + 0.008 * S->V.ntiles < rounds * (3 + 0.65 * most);
+  const double shared = (5.0 * S->nsys + 0.85 * S->V.ntiles) / 256;
+  return 14.5 + 0.010 * S->V.ntiles < std::max(5 + 0.85 * most_tiles(S), shared);
 }
 
 int temperature_scale(dpm_set_s* S, double T) {
