@@ -729,20 +729,16 @@ int fire_waves(const dpm_set_s* S) {
 // most 64 iterations of two short launches follow the last system's.
 int fire_tile_sequence(dpm_set_s* S, long iterations) {
   const int most = most_tiles(S), waves = fire_waves(S);
-  for (hipEvent_t& e : S->fireEvent)
-    if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  long part = 2, look = part;  // iterations up to the next look
-  int looks = 0;
+  if (S->fireLook > 1 << 29) S->fireLook = S->h_stat->look = 0;
+  long part = 2, next = part;  // iterations up to the next look
+  int last = 0, tell = 0;      // the look before; the look to tell of
   // the start positions' flags go to the sink: the rows serve the positions after the first move, which
   // flags those (a system that stops before it moves keeps its rows)
   HIPCHK(launch_bin_flag(S, S->V, S->mdCount[0], S->mdSlots[0], S->mdFlag[3], S->mdGen[0], S->N));
   for (long it = 0; it < iterations; it++) {
-    volatile int* open = nullptr;
-    if (it + 1 == look) {
-      open = S->h_stat->open + looks % 4;
-      *open = 0;
-    }
-    HIPCHK(launch_fire_move(S, most, waves, S->mdFlag[it % 3], S->d_any + 2, (int*)open));
+    const int look = it + 1 == next ? ++S->fireLook : 0;
+    HIPCHK(launch_fire_move(S, most, waves, S->mdFlag[it % 3], S->d_any + 2, look, tell));
+    tell = look;
     S->fireCur = 1 - S->fireCur;
     swap_pos(S);
     StepArgs A = md_args(S, it, 0, 0, true);
@@ -750,15 +746,22 @@ int fire_tile_sequence(dpm_set_s* S, long iterations) {
     A.part = S->d_part;
     A.vel = S->d_fireVel;
     HIPCHK(launch_step(S, MODE_FIRE | MODE_NEAR, A));
-    if (open) {
-      HIPCHK(hipEventRecord(S->fireEvent[looks % 2], S->stream));
-      if (looks > 0) {
-        HIPCHK(hipEventSynchronize(S->fireEvent[1 - looks % 2]));
-        if (!*(volatile int*)(S->h_stat->open + (looks - 1) % 4)) break;
+    if (look) {
+      if (last) {
+        // wait for the look before, of which the move after it tells (an event between the kernels costs
+        // more than the words it saves); an idle or failed stream ends the wait
+        volatile int& told = S->h_stat->look;
+        for (long spin = 1; (told >> 1) < last; spin++)
+          if (spin % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(S->stream);
+            if (e == hipSuccess) break;
+            if (e != hipErrorNotReady) HIPCHK(e);
+          }
+        if (told == 2 * last) break;
       }
-      looks++;
+      last = look;
       part = std::min(2 * part, 32L);
-      look += part;
+      next += part;
     }
   }
   StepArgs A = md_args(S, 0, 0, 0, true);  // energies and ring geometry of the positions reached
@@ -1227,7 +1230,7 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   A(S->d_err, 1); A(S->d_maxcnt, 1); A(S->d_ctr, 4); A(S->d_notDone, 1); A(S->d_sysOrder, numSystems);
   A(S->d_fire[0], numSystems); A(S->d_fire[1], numSystems);
   A(S->d_part, (long)V.ntiles * 4);
-  A(S->d_fireVel, 2l * V.nv);
+  A(S->d_fireVel, 2l * V.nv); A(S->d_look, 1);
   S->nwide = (long)S->h_wide.size();
   if (S->nwide > 0) A(S->d_wide, S->nwide);
   std::vector<int> chunkSys, chunkOff(1, 0);
@@ -1244,6 +1247,7 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
     dpm_destroy(S);
     return DPM_ERR_OOM;
   }
+  *S->h_stat = HostStat{};
 #undef A
   set_pos_view(S);
   hipStream_t st = S->stream;
@@ -1286,6 +1290,7 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   ok = ok && hipMemsetAsync(S->d_any, 0, sizeof(int) * 2, st) == hipSuccess;
   ok = ok && hipMemsetAsync(S->d_updateCount, 0, sizeof(int) * numSystems, st) == hipSuccess;
   ok = ok && hipMemsetAsync(S->d_err, 0, sizeof(int), st) == hipSuccess;
+  ok = ok && hipMemsetAsync(S->d_look, 0, sizeof(int), st) == hipSuccess;
   ok = ok && hipMemsetAsync(S->d_ctr, 0, sizeof(unsigned long long) * 4, st) == hipSuccess;
   ok = ok && hipMemsetAsync(S->d_part, 0, sizeof(double) * V.ntiles * 4, st) == hipSuccess;
   ok = ok && hipStreamSynchronize(st) == hipSuccess;
@@ -1329,7 +1334,7 @@ int dpm_destroy(dpm_set_t h) {
                   V.ncnt, V.nbr, V.nbrp, V.tile_v0, V.tile_v1, V.tile_sys, V.stile, S->G.ncx, S->G.ncy,
                   S->G.coff, S->G.brute, S->G.count[0], S->G.count[1], S->G.slots, S->G.cellSys, S->d_flag[0],
                   S->d_flag[1], S->d_any, S->d_updateCount, S->d_err, S->d_maxcnt, S->d_ctr, S->d_notDone,
-                  S->d_sysOrder, S->d_fire[0], S->d_fire[1], S->d_part, S->d_fireVel, S->d_red, S->d_scale, V.kr,
+                  S->d_sysOrder, S->d_fire[0], S->d_fire[1], S->d_part, S->d_fireVel, S->d_look, S->d_red, S->d_scale, V.kr,
                   S->d_ck, S->d_fin, S->d_seg, S->d_adj, V.vinfo, V.l0r, V.mbx, V.mby, V.wfx, V.wfy,
                   S->d_contacts, S->d_ccount, S->d_x0, S->d_obs, S->mdCount[0], S->mdSlots[0], S->mdFlag[0],
                   S->mdFlag[1], S->mdFlag[2], S->mdFlag[3], S->mdGen[0], S->mdGen[1], S->mdGen[2], S->R.pvx, S->R.pvy, S->R.pw, S->R.pfx, S->R.pfy, S->R.ptq, S->R.moi,
@@ -1340,8 +1345,6 @@ int dpm_destroy(dpm_set_t h) {
     if (p) hipFree(p);
   if (S->h_red) hipHostFree(S->h_red);
   if (S->h_stat) hipHostFree(S->h_stat);
-  for (hipEvent_t e : S->fireEvent)
-    if (e) hipEventDestroy(e);
   if (S->ownStream) hipStreamDestroy(S->ownStream);
   delete S;
   return DPM_OK;

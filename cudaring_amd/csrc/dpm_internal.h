@@ -132,7 +132,7 @@ struct FillSegs {
 // What the loops and list builds leave for the host, in pinned memory their last kernel writes.
 struct HostStat {
   int err, maxcnt, notDone;
-  int open[4];  // FIRE on tiles: set by a move that leaves a system to go on, one word per look
+  int look;  // FIRE on tiles: 2 x the last look's number, + 1 if it left a system to go on
 };
 
 // Arguments of the H w kernel (dpm_adjoint.hip).
@@ -244,7 +244,8 @@ struct dpm_set_s {
   dpm::FireParams fp{};
   double* d_part = nullptr;  // per-tile partials [ntiles * 4]
   double* d_fireVel = nullptr;  // FIRE on tiles: velocities between the move and the step [2 * nv]
-  hipEvent_t fireEvent[2] = {nullptr, nullptr};  // FIRE on tiles: behind the moves of the last two looks
+  int* d_look = nullptr;        //   the last look that left a system to go on
+  int fireLook = 0;             //   looks so far
   bool fireInit = false;
   int fireKernel = -1;  // dpm_fire_minimize: 1 = one persistent workgroup per system, 0 = graph of step
                         //   kernels, -1 = persistent or on every tile (fire_on_tiles)
@@ -323,7 +324,7 @@ hipError_t launch_fire_mid(dpm_set_s* S);
 hipError_t launch_fire_partials(dpm_set_s* S);
 hipError_t launch_fire_step(dpm_set_s* S);
 hipError_t launch_fire_resume(dpm_set_s* S);
-hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut, int* open);
+hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut, int look, int tell);
 StepArgs loop_args(dpm_set_s* S);
 hipError_t launch_bin_view(dpm_set_s* S, const View& Vn, int parity);
 hipError_t launch_fire_sys(dpm_set_s* S, int chunk, int waves);

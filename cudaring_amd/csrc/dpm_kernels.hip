@@ -766,14 +766,18 @@ __global__ void k_fire_partials(View V, double* part) {
 // first, over the vertices in the order of the persistent kernel with as many waves (so that both follow
 // the same path to the last bit), then takes the stopping rule and the parameter update and moves its
 // vertices into the other position buffer and vxn, vyn (other blocks still sum vx, vy), with the step
-// loop's flags.  A system that has stopped only keeps its positions in the buffer that is read next.
+// loop's flags.  A system that has stopped only keeps its positions in the buffer that is read next.  Look
+// `look` (not 0) notes whether a system goes on, and the launch after it tells the host.
 __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_move(View V, Params P, FireParams fp, int per,
                                                               const FireState* fin, FireState* fout, double* xo,
                                                               double* yo, double* vxn, double* vyn, int* flagOut,
-                                                              int* anyOut, int* open) {
+                                                              int* anyOut, int* open, int look, int* told,
+                                                              int tell) {
   __shared__ double red[FS_WAVES][5];
   const int s = blockIdx.x / per, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x & (WAVE - 1);
   const int t0 = V.stile[s], t1 = V.stile[s + 1], tile = t0 + (blockIdx.x % per) * nw + w;
+  // what the launch before, look `tell`, found, for the host (pinned memory)
+  if (tell && blockIdx.x == 0 && threadIdx.x == 0) *(volatile int*)told = 2 * tell + (*open == tell);
   FireState fs = fin[s];
   FireSums sum{0, -1, 0, 0, 0};
   bool reset = false;
@@ -789,7 +793,7 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_move(View V, Params P, 
   }
   if (tile == t0 && lane == 0) {
     fout[s] = fs;
-    if (open && !fs.converged) *open = 1;  // for the host (pinned memory); every writer writes 1
+    if (look && !fs.converged) *open = look;
   }
   if (tile >= t1) return;
   const int v = V.tile_v0[tile] + lane;
@@ -1069,13 +1073,13 @@ hipError_t launch_fire_mid(dpm_set_s* S) {
   return hipGetLastError();
 }
 
-hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut, int* open) {
+hipError_t launch_fire_move(dpm_set_s* S, int most, int waves, int* flagOut, int* anyOut, int look, int tell) {
   if (!flagOut || !anyOut || waves < 1 || waves > FS_WAVES) return hipErrorInvalidValue;
   const int nb = 1 - S->cur;
   const int per = (most + waves - 1) / waves;
   k_fire_move<<<(unsigned)(S->nsys * per), WAVE * waves, 0, S->stream>>>(
       S->V, S->P, S->fp, per, S->d_fire[S->fireCur], S->d_fire[1 - S->fireCur], S->pos[nb][0], S->pos[nb][1], S->d_fireVel,
-      S->d_fireVel + S->V.nv, flagOut, anyOut, open);
+      S->d_fireVel + S->V.nv, flagOut, anyOut, S->d_look, look, &S->h_stat->look, tell);
   return hipGetLastError();
 }
 
