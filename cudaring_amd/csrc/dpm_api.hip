@@ -387,7 +387,9 @@ std::vector<std::pair<unsigned*, long>> snap_fields(dpm_set_s* S, int what) {
       w(S->V.fx, 8 * nv), w(S->V.fy, 8 * nv), w(S->V.lx, 8 * nv), w(S->V.ly, 8 * nv),
       w(S->V.l0, 8 * nv), w(S->V.ang, 8 * np), w(S->V.cx, 8 * np), w(S->V.cy, 8 * np),
       w(S->d_ctr, 4 * sizeof(unsigned long long)), w(S->d_updateCount, 4 * ns),
-      w(S->d_flag[0], 4 * ns), w(S->d_flag[1], 4 * ns), w(S->d_any, 4 * 3)};
+      // the flags of the positions the loop starts from; the other parity's are clean, or cleared by the
+      // launch that takes the snapshot (loop_fills), which copies and clears in no order
+      w(S->d_flag[S->cur], 4 * ns), w(S->d_any + S->cur, 4)};
   if (what & SNAP_FIRE) f.push_back(w(S->d_fire[S->fireCur], sizeof(FireState) * ns));
   if (what & (SNAP_RIGID | SNAP_RIGID_FIRE)) {
     const Rigid& R = S->R;
