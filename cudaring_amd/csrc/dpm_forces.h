@@ -160,8 +160,27 @@ __device__ __forceinline__ void ring_walk(const Lane& L, const Box& B, double x,
   uy = L.act ? seg_scan(L.act ? dny : 0.0, L.lane, L.segS) - dny : 0.0;
 }
 
+// ring_walk for ring_shape_n.  True when a ring of the wave reaches past half the box from its centre
+// (cx, cy), set only then: there the reference's centre-relative positions, a minimum image each
+// (getRelativeVertexPos 273-279), differ by a box length more than the segments.  Rings within a quarter
+// of the box of their first vertex, the usual case, are told by that.
+__device__ __forceinline__ bool ring_walk_past_half(const Lane& L, const Box& B, double x, double y, double dnx,
+                                                    double dny, double& ux, double& uy, double& cx, double& cy) {
+  const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
+  ux = L.act ? pbx(x - xf, B) : 0.0;
+  uy = L.act ? pby(y - yf, B) : 0.0;
+  if (__all(fabs(ux * B.mx) < 0.25 && fabs(uy * B.my) < 0.25)) return false;
+  ring_walk(L, B, x, y, xf, yf, dnx, dny, ux, uy);
+  const double ind = quot(1.0, (double)L.n);
+  const double mx = seg_sum(ux, L.lane, L.segS, L.segE) * ind, my = seg_sum(uy, L.lane, L.segS, L.segE) * ind;
+  cx = xf + mx;
+  cy = yf + my;
+  return __any(L.act && !(fabs((ux - mx) * B.mx) < 0.4999 && fabs((uy - my) * B.my) < 0.4999));
+}
+
 // ring_shape for the step loops.  With dn = (v, next) and ps = (prev, v): the centre-relative differences of the reference's terms
-// (getRelativeVertexPos 273-279) are sums of the two, so the force needs no centre; the previous
+// (getRelativeVertexPos 273-279) are sums of the two, so the force needs no centre (rings reaching past
+// half the box from theirs excepted); the previous
 // segment's factors are the previous lane's own.  `write`: theta, length, energy, and the ring's area,
 // perimeter and centre, which nothing inside a step needs.
 __device__ __forceinline__ ShapeOut ring_shape_n(const View& V, const Params& P, const Lane& L, const Box& B,
@@ -181,17 +200,19 @@ __device__ __forceinline__ ShapeOut ring_shape_n(const View& V, const Params& P,
     xn = V.x[vn]; yn = V.y[vn];
     xp = V.x[vp]; yp = V.y[vp];
   }
-  const double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
-  const double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
+  double dnx = pbx(xn - x, B), dny = pby(yn - y, B);
+  double psx = -pbx(xp - x, B), psy = -pby(yp - y, B);
   const double theta = atan2(dnx * psy - dny * psx, dnx * psx + dny * psy);  // calcAngle 423-427
-  const double n2 = dnx * dnx + dny * dny, in = rsqrt_n(n2), seglen = n2 > 0 ? sqrt_from(n2, in) : n2;
+  double n2 = dnx * dnx + dny * dny, in = rsqrt_n(n2), seglen = n2 > 0 ? sqrt_from(n2, in) : n2;
+  bool past;  // a ring of the wave reaches past half the box from its centre (cx, cy)
+  double cx = 0, cy = 0;
   if (!L.wide) {
-    const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
     double ux, uy;
-    ring_walk(L, B, x, y, xf, yf, dnx, dny, ux, uy);
+    past = ring_walk_past_half(L, B, x, y, dnx, dny, ux, uy, cx, cy);
     const double shoe = L.act ? (ux * dny - dnx * uy) : 0.0;  // shoelace: cur x next = cur x delta
     area = fabs(seg_sum(shoe, L.lane, L.segS, L.segE)) * 0.5;
     if (write) {
+      const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
       perim = seg_sum(L.act ? seglen : 0.0, L.lane, L.segS, L.segE);
       const double ind = 1.0 / (double)L.n;
       o.cx = xf + seg_sum(ux, L.lane, L.segS, L.segE) * ind;
@@ -199,6 +220,11 @@ __device__ __forceinline__ ShapeOut ring_shape_n(const View& V, const Params& P,
     }
   } else {
     area = V.area[L.r];
+    cx = V.cx[L.r];
+    cy = V.cy[L.r];
+    const double rx = pbx(x - cx, B), ry = pby(y - cy, B);
+    past = __any(L.act && !(fabs((rx + dnx) * B.mx) < 0.4999 && fabs((ry + dny) * B.my) < 0.4999 &&
+                            fabs((rx - psx) * B.mx) < 0.4999 && fabs((ry - psy) * B.my) < 0.4999));
   }
   if (write && L.act) {
     V.th[L.v] = theta;
@@ -209,6 +235,16 @@ __device__ __forceinline__ ShapeOut ring_shape_n(const View& V, const Params& P,
       V.cx[L.r] = o.cx;
       V.cy[L.r] = o.cy;
     }
+  }
+  if (past) {  // the terms' differences of centre-relative positions, as ring_shape forms them
+    const double rvx = pbx(x - cx, B), rvy = pby(y - cy, B);
+    dnx = pbx(xn - cx, B) - rvx;
+    dny = pby(yn - cy, B) - rvy;
+    psx = rvx - pbx(xp - cx, B);
+    psy = rvy - pby(yp - cy, B);
+    n2 = dnx * dnx + dny * dny;
+    in = rsqrt_n(n2);
+    seglen = n2 > 0 ? sqrt_from(n2, in) : n2;
   }
   const double a0 = V.a0[L.r], ia0 = recip(a0);
   // shape costs: the global ea, el, eb, or per-ring values when the caller set them
