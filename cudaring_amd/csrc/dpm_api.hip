@@ -712,6 +712,15 @@ int run_fire(dpm_set_s* S, long iterations) {
   return DPM_OK;
 }
 
+// before a fixed number of iterations: no system stops, nor stays where a minimisation stopped it
+int fire_all_go_on(dpm_set_s* S) {
+  if (S->fp.tol < 0) return DPM_OK;
+  S->fp.tol = -1;
+  bump(S);
+  HIPCHK(launch_fire_resume(S));
+  return DPM_OK;
+}
+
 // tiles of the set's largest system, and the waves of a system's sums (both one-system-one-block forms)
 int most_tiles(const dpm_set_s* S) {
   int most = 1;
@@ -1951,10 +1960,8 @@ int dpm_fire_loop(dpm_set_t h, long iterations) {
   if (!S->fireInit) return fail(S, DPM_ERR_STATE, "dpm_init_fire not called");
   int rc = require_list(S);
   if (rc) return rc;
-  if (S->fp.tol >= 0) {
-    S->fp.tol = -1;
-    bump(S);
-  }
+  rc = fire_all_go_on(S);
+  if (rc) return rc;
   return with_replay(S, SNAP_FIRE, LOOP_FIRE, Draws{}, [&]() { return run_fire(S, iterations); });
 }
 
@@ -2525,10 +2532,8 @@ int dpm_fire_forward(dpm_set_t h, long iterations) {
     HIPCHK(dalloc(&S->d_fadj, 10 * nv));
     S->fireTapeCap = iterations;
   }
-  if (S->fp.tol >= 0) {  // a fixed number of iterations: no system stops
-    S->fp.tol = -1;
-    bump(S);
-  }
+  rc = fire_all_go_on(S);
+  if (rc) return rc;
   // every iteration one at a time, its starting state recorded before it and its FIRE scalars
   // after its parameter update; replayed on a wider list as the loops are
   rc = with_replay(S, SNAP_FIRE, LOOP_FIRE, Draws{}, [&]() -> int {

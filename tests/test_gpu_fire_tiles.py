@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from cudaring_amd import packing
-from tests.helpers import gpu_from_state, relaxed_state
+from tests.conftest import rel_err
+from tests.helpers import gpu_from_state, oracle_from_state, relaxed_state
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +62,26 @@ def test_stopped_system_keeps_its_rows():
         assert list(g.update_count()) == before
         assert np.array_equal(g.get("lastpos"), last)
         g.close()
+
+
+@pytest.mark.parametrize("persistent", [-1, 1, 0])
+@pytest.mark.parametrize("tol,max_iter", [(1e9, 20), (0.0, 20)])
+def test_fire_loop_goes_on_after_a_minimisation(oracle_mod, persistent, tol, max_iter):
+    """fire(n) advances every system (dpmring.h), also one that a minimisation before it stopped, by its
+    tolerance or by its number of iterations."""
+    st = packing.lattice_system(60, 0.8, 21, n_small=16, n_large=22, perturb=0.05)
+    g, o = gpu_from_state(st), oracle_from_state(oracle_mod, st)
+    for s in (g, o):
+        s.calc_neighbor_list(s.set_displacement_cutoff(0.5, 2 * float(st["rad"].mean())))
+        s.calc_force_energy()
+        s.init_fire([0.2, 0.5, 1.1, 0.99, 1e-2, 1e-1, 0.2], 20, 0)
+    g.set_fire_kernel(persistent, 0)
+    for s in (g, o):
+        s.fire_minimize(tol, max_iter)
+        s.fire(10)
+    assert list(g.fire_state()["iters"]) == [10 + (0 if tol else max_iter)]
+    assert rel_err(g.get("pos"), o.get("pos"), scale=1.0) < 1e-11
+    g.close()
 
 
 def test_choice_can_be_given_back():
