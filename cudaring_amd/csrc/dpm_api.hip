@@ -557,15 +557,16 @@ int verlet_sequence(dpm_set_s* S, long steps, bool langevin, double* rec = nullp
   if (rec) {
     // a recomputed segment starts from a restored checkpoint without a valid list: its list
     // positions become the start positions (whose cells the start kernel bins), and every
-    // system rebuilds its rows in the first step (below)
+    // system rebuilds its rows in the first step
     HIPCHK(launch_copy_d(S->V.lx, S->V.x, nv, S->stream));
     HIPCHK(launch_copy_d(S->V.ly, S->V.y, nv, S->stream));
+    // before the start kernel, which adds FLAG_FAR where the first drift is long
+    HIPCHK(launch_fill_int(S->mdFlag[1], 1, S->nsys, S->stream));
   }
   StepArgs A0 = md_args(S, 0, 0, 0, near);
   A0.recx = rec ? rec + 2 * nv : nullptr;
   A0.recy = rec ? rec + 3 * nv : nullptr;
   HIPCHK(launch_start_md(S, A0));
-  if (rec) HIPCHK(launch_fill_int(S->mdFlag[1], 1, S->nsys, S->stream));
   swap_pos(S);
   for (long i = 1; i <= steps; i++) {
     const bool more = i < steps;

@@ -4,6 +4,7 @@ cudaKernel.cuh:1735-1763) instead of the previous positions' cells, and the traj
 matches the oracle, which rebuilds from scratch."""
 import numpy as np
 import pytest
+import torch
 
 from tests.conftest import rel_err
 from tests.helpers import gpu_from_state, oracle_from_state
@@ -172,3 +173,41 @@ def test_rigid_fire_starts_beyond_displacement_test():
         g.close()
     assert rel_err(out[0][0], out[1][0], scale=1.0) < 1e-11
     assert rel_err(out[0][1], out[1][1]) < 1e-10
+
+
+def gradient(g, st, steps, every, seed):
+    """Gradients (x0, v0, ring costs, l0) of seed . (x_N, v_N) through `steps` NVE steps."""
+    nv = len(st["rad"])
+    c = torch.as_tensor(np.random.default_rng(seed).standard_normal(4 * nv), device="cuda")
+    ax, av = c[:2 * nv].clone(), c[2 * nv:].clone()
+    gx, gv = torch.empty_like(ax), torch.empty_like(ax)
+    gring = torch.empty(3 * len(st["nvp"]), dtype=torch.float64, device="cuda")
+    gl0 = torch.empty(nv, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    g.nve_forward(steps, every)
+    g.nve_backward(*(t.data_ptr() for t in (ax, av, gx, gv, gring, gl0)))
+    return [t.cpu().numpy() for t in (gx, gv, gring, gl0)]
+
+
+def test_recomputed_segment_of_fast_rings():
+    """The reverse pass recomputes its segments with every system flagged for a rebuild in the first step; a
+    first drift of 0.8 cutoff keeps its far-move mark, and the gradient is the one of a wide skin, whose
+    recomputation makes no far move."""
+    from cudaring_amd import packing
+    print("case far_moves reverse pass", flush=True)
+    st = packing.lattice_system(25, 0.8, 23, n_small=16, n_large=22, perturb=0.05)
+    size, dt = 2 * float(st["rad"].mean()), 1e-3
+    rng = np.random.default_rng(8)
+    nv = len(st["rad"])
+    vel = np.tile(0.8 * 0.3 * size / dt * np.array([np.cos(0.7), np.sin(0.7)]), nv) + 0.1 * rng.standard_normal(2 * nv)
+    out = []
+    for skin in (0.3, 2.0):
+        g = gpu_from_state(st, dt=dt)
+        g.calc_neighbor_list(g.set_displacement_cutoff(skin, size))
+        g.set("vel", vel)
+        g.calc_force_energy()
+        out.append(gradient(g, st, 6, 6, 8))
+        g.close()
+    for a, b in zip(*out):
+        assert rel_err(a, b) < 1e-11
+
