@@ -817,15 +817,21 @@ int temperature_scale(dpm_set_s* S, double T) {
 
 // ------------------------------------------------------------------ adjoint ---
 // Flags, any-flags and both parities' cell counts cleared: the state the forward loops and the
-// adjoint's own rebuild protocol both start from.
-int clean_protocol(dpm_set_s* S) {
+// adjoint's own rebuild protocol both start from.  `errTo`: where to keep a copy of the error word.
+int clean_protocol(dpm_set_s* S, int* errTo = nullptr) {
   FillSegs f{};
   f.add(S->d_flag[0], 0, S->nsys);
   f.add(S->d_flag[1], 0, S->nsys);
   f.add(S->d_any, 0, 2);
   f.add(S->G.count[0], 0, S->G.ncells);
   f.add(S->G.count[1], 0, S->G.ncells);
-  HIPCHK(launch_prologue(CopySegs{}, f, S->stream));
+  CopySegs c{};
+  if (errTo) {
+    c.src[0] = (const unsigned*)S->d_err;
+    c.dst[0] = (unsigned*)errTo;
+    c.words[0] = c.n = 1;
+  }
+  HIPCHK(launch_prologue(c, f, S->stream));
   return DPM_OK;
 }
 
@@ -908,9 +914,7 @@ int record_segment(dpm_set_s* S, long len) {
   const long nv = S->nv;
   HIPCHK(launch_copy_d(S->d_seg, S->V.x, nv, S->stream));
   HIPCHK(launch_copy_d(S->d_seg + nv, S->V.y, nv, S->stream));
-  FillSegs fills = loop_fills(S, LOOP_MD);
-  fills.words[0] = 0;  // the error word gathers over the whole reverse pass
-  HIPCHK(launch_prologue(CopySegs{}, fills, S->stream));
+  HIPCHK(launch_prologue(CopySegs{}, loop_fills(S, LOOP_MD), S->stream));
   int rc;
   if (len < 4 || !graphs_enabled()) {
     rc = verlet_sequence(S, len, false, S->d_seg);
@@ -924,35 +928,42 @@ int record_segment(dpm_set_s* S, long len) {
   return DPM_OK;
 }
 
-// reverse pass over positions n = top .. a of the recorded segment starting at step a
-int backward_segment(dpm_set_s* S, long a, long top, long N) {
+// One list for a whole recorded segment of `count` positions when it can serve every one (`single`): rows
+// built at the middle slot, checked against all slots.  Otherwise each position runs the rebuild
+// protocol (displacement flags, binning, in-kernel row rebuild).  The host's one wait per segment also
+// brings the error words of the reverse pass over the segment before (`before`) and of the recording
+// (`recorded`), which the row build here clears.
+int segment_list(dpm_set_s* S, long count, bool* single, int* before, int* recorded) {
   const long nv = S->nv;
-  const long count = top - a + 1;
-  const bool hasTop = (top == N), hasZero = (a == 0);
-  // One list for the whole segment when it can serve every recorded position: rows built at
-  // the middle slot, checked against all slots.  Otherwise each position runs the rebuild
-  // protocol (displacement flags, binning, in-kernel row rebuild).
   const long mid = (count - 1) / 2;
   HIPCHK(launch_copy_d(S->V.x, S->d_seg + mid * 2 * nv, nv, S->stream));
   HIPCHK(launch_copy_d(S->V.y, S->d_seg + mid * 2 * nv + nv, nv, S->stream));
   std::vector<int> all(S->nsys, 1);
   int rc = rebuild(S, all, 0);
   if (rc) return rc;
-  int bad = 0;
+  int got[3];
   HIPCHK(launch_fill_int(S->d_notDone, 0, 1, S->stream));
   HIPCHK(launch_adj_seg_check(S, S->d_seg, (int)count, S->d_notDone));
-  HIPCHK(hipMemcpyAsync(&bad, S->d_notDone, sizeof(int), hipMemcpyDeviceToHost, S->stream));
+  HIPCHK(hipMemcpyAsync(got, S->d_notDone, sizeof(got), hipMemcpyDeviceToHost, S->stream));
   HIPCHK(hipStreamSynchronize(S->stream));
-  const bool single = !bad;
+  *single = !got[0];
+  *before = got[1];
+  *recorded = got[2];
+  return DPM_OK;
+}
+
+// reverse pass over positions n = top .. a of the recorded segment starting at step a
+int backward_segment(dpm_set_s* S, long a, long top, long N, bool single) {
+  const long nv = S->nv;
+  const long count = top - a + 1;
+  const bool hasTop = (top == N), hasZero = (a == 0);
   auto seq = [&]() -> int {
     long i = 0;  // rotation index of the position's flags and generations
     if (!single) {
       // the step loop's cell protocol on the recorded positions, from x_top down: x_top the list
       // positions (those of the rows just built lie half a segment away, and a system too far from its
       // cells searches all its vertices), every system rebuilding its rows there
-      FillSegs fills = loop_fills(S, LOOP_MD);
-      fills.words[0] = 0;  // the error word gathers over the whole reverse pass
-      HIPCHK(launch_prologue(CopySegs{}, fills, S->stream));
+      HIPCHK(launch_prologue(CopySegs{}, loop_fills(S, LOOP_MD), S->stream));
       double* st = S->d_seg + (top - a) * 2 * nv;
       HIPCHK(launch_copy_d(S->V.lx, st, nv, S->stream));
       HIPCHK(launch_copy_d(S->V.ly, st + nv, nv, S->stream));
@@ -999,7 +1010,7 @@ int backward_segment(dpm_set_s* S, long a, long top, long N) {
   const int w0 = S->wCur;
   if (!graphs_enabled()) return seq();
   const int kind = 256 | (hasTop ? 1 : 0) | (hasZero ? 2 : 0) | (single ? 4 : 0);
-  rc = run_graph(S, std::make_tuple(kind, count, w0), [&]() {
+  const int rc = run_graph(S, std::make_tuple(kind, count, w0), [&]() {
     int r = seq();
     S->wCur = w0;
     return r;
@@ -1239,7 +1250,7 @@ int dpm_create(dpm_set_t* out, int device, long numSystems, const long* ringsPer
   A(V.stile, numSystems + 1);
   A(S->G.ncx, numSystems); A(S->G.ncy, numSystems); A(S->G.coff, numSystems); A(S->G.brute, numSystems);
   A(S->d_flag[0], numSystems); A(S->d_flag[1], numSystems); A(S->d_any, 3); A(S->d_updateCount, numSystems);
-  A(S->d_err, 1); A(S->d_maxcnt, 1); A(S->d_ctr, 4); A(S->d_notDone, 1); A(S->d_sysOrder, numSystems);
+  A(S->d_err, 1); A(S->d_maxcnt, 1); A(S->d_ctr, 4); A(S->d_notDone, 3); A(S->d_sysOrder, numSystems);
   A(S->d_fire[0], numSystems); A(S->d_fire[1], numSystems);
   A(S->d_part, (long)V.ntiles * 4);
   A(S->d_fireVel, 2l * V.nv); A(S->d_look, 1);
@@ -2658,17 +2669,34 @@ int dpm_nve_backward(dpm_set_t h, const double* ax, const double* av, double* gx
   std::vector<int> all(S->nsys, 1);
   for (long k = S->tapeNck - 1; k >= 0; k--) {
     const long a = k * every, b = std::min(a + every, N);
-    // restore the checkpoint, recompute the segment (its first step rebuilds every row), then
-    // the reverse pass over it; no host synchronisation until the end
-    rc = load_state(S, S->d_ck + k * words, rings);
-    if (rc) return rc;
-    rc = clean_protocol(S);
-    if (rc) return rc;
-    rc = record_segment(S, b - a);
-    if (rc) return rc;
-    rc = clean_protocol(S);
-    if (rc) return rc;
-    rc = backward_segment(S, a, (k == S->tapeNck - 1) ? b : b - 1, N);
+    const long top = (k == S->tapeNck - 1) ? b : b - 1;
+    // restore the checkpoint, recompute the segment (its first step rebuilds every row; again on a wider
+    // list when a row did not fit), then the reverse pass over it
+    bool single = false;
+    for (int attempt = 0;; attempt++) {
+      rc = load_state(S, S->d_ck + k * words, rings);
+      if (rc) return rc;
+      rc = clean_protocol(S, S->d_notDone + 1);
+      if (rc) return rc;
+      rc = record_segment(S, b - a);
+      if (rc) return rc;
+      rc = clean_protocol(S, S->d_notDone + 2);
+      if (rc) return rc;
+      const int W = S->V.W;
+      int before = 0, recorded = 0;
+      rc = segment_list(S, top - a + 1, &single, &before, &recorded);
+      if (rc) return rc;
+      if (before) return fail(S, DPM_ERR_OVERFLOW, "dpm_nve_backward: neighbour list overflow");
+      if (!(recorded & ERR_LIST_OVERFLOW)) {
+        rc = loop_status(S, recorded);
+        if (rc) return rc;
+        break;
+      }
+      if (attempt == 5) return fail(S, DPM_ERR_OVERFLOW, "dpm_nve_backward: neighbour list overflow");
+      if (S->V.W < 2 * W) rc = alloc_list(S, 2 * W);
+      if (rc) return rc;
+    }
+    rc = backward_segment(S, a, top, N, single);
     if (rc) return rc;
   }
   {

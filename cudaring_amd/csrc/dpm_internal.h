@@ -250,7 +250,7 @@ struct dpm_set_s {
   int fireKernel = -1;  // dpm_fire_minimize: 1 = one persistent workgroup per system, 0 = graph of step
                         //   kernels, -1 = persistent or on every tile (fire_on_tiles)
   int fireWaves = 0;    // waves per system workgroup (0 = from the largest system's tile count)
-  int* d_notDone = nullptr;
+  int* d_notDone = nullptr;   // scratch flag; [1], [2]: the reverse pass's error words (segment_list)
   int* d_sysOrder = nullptr;  // persistent FIRE: workgroup b runs system d_sysOrder[b] (most tiles first)
 
   // reductions

@@ -211,3 +211,27 @@ def test_recomputed_segment_of_fast_rings():
     for a, b in zip(*out):
         assert rel_err(a, b) < 1e-11
 
+
+@pytest.mark.parametrize("every", [12, 5])
+def test_recomputed_segment_widens_list(every):
+    """Rows built for a narrow skin serve a slow forward pass under a wide one (nothing moves past its
+    displacement test); the reverse pass rebuilds them, finds rows longer than the list is wide, and
+    recomputes on a wider list: the gradient is the one of rows built for the wide skin."""
+    from cudaring_amd import packing
+    print("case reverse pass widens list", flush=True)
+    st = packing.lattice_system(25, 0.8, 23, n_small=16, n_large=22, perturb=0.05)
+    size = 2 * float(st["rad"].mean())
+    vel = 0.1 * np.random.default_rng(8).standard_normal(2 * len(st["rad"]))
+    out = []
+    for first in (0.1, 3.0):
+        g = gpu_from_state(st, dt=1e-3)
+        g.calc_neighbor_list(g.set_displacement_cutoff(first, size))
+        w0 = g.neighbors()[1]
+        g.set_displacement_cutoff(3.0, size)
+        g.set("vel", vel)
+        g.calc_force_energy()
+        out.append(gradient(g, st, 12, every, 9))
+        assert first == 3.0 or g.neighbors()[1] > w0
+        g.close()
+    for a, b in zip(*out):
+        assert rel_err(a, b) < 1e-11
