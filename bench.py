@@ -34,11 +34,11 @@ DT_UNITS = 1e-3                # dt = 1e-3 * sigma / sqrt(ec), sigma = mean part
 CHUNK = 250                    # steps per graph replay
 # HBM bytes per launch of the step kernel on this workload, from the FETCH_SIZE and WRITE_SIZE
 # counter runs of `bench.py --traffic` (the line's own warm-up and timed steps, so the same state
-# and mean neighbour count 4.460; each counter scaled by its reading for a 1 GiB device copy:
-# 2.000 and 1.000): 2 x 1878.63 KiB + 608.66 KiB.  The summary with its commands is
+# and mean neighbour count 4.462; each counter scaled by its reading for a 1 GiB device copy:
+# 2.000 and 1.000): 2 x 1877.56 KiB + 608.66 KiB.  The summary with its commands is
 # profiles/k_step_traffic_nvt1024_wca_smooth.md; re-measure after changing the step kernel.
-TRAFFIC_BYTES_PER_LAUNCH = 4470688
-TRAFFIC_MEAN_NEIGHBORS = 4.460
+TRAFFIC_BYTES_PER_LAUNCH = 4468512
+TRAFFIC_MEAN_NEIGHBORS = 4.462
 
 
 def alg_bytes_per_step(nv, np_, kbar):

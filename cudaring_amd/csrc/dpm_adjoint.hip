@@ -595,7 +595,7 @@ hipError_t launch_adj_hvp(dpm_set_s* S, const View& Vn, AdjArgs A) {
   const unsigned g = (unsigned)S->V.ntiles, b = WAVE * loop_waves(S);
   hipStream_t st = S->stream;
   // rows rebuilt by the whole workgroup need rows_lds_ints of LDS (W <= 64), in the region the gather
-  // wave, W <= 64), in the region the gather partials use afterwards
+  // partials use afterwards
   const bool tileRows = A.flag && S->V.W <= 64;
   A.rowsLdsW = tileRows ? S->V.W : 0;
   const size_t rows = tileRows ? (size_t)rows_lds_ints(S->V.W, false) * sizeof(int) : 0;

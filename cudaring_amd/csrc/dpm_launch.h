@@ -10,9 +10,10 @@ namespace dpm {
 static inline int grid_v(long n) { return (int)((n + 255) / 256); }
 static inline int grid_w(int ntiles) { return (ntiles + 3) / 4; }
 
-// Waves per tile of the loops where the caller set none: 8 while two workgroups a CU hold the set (32 to
-// 1,024 rings: 2 to 5% faster than 4, a rebuild or the tile's longest wave being what a step waits for), 4
-// beyond (2,000 rings 679 us against 970 with 8 and 715 with 2).
+// Waves per tile of the loops where the caller set none: 8 while two workgroups a CU, all that registers
+// leave room for, hold the set (32 to 1,024 rings: 2 to 5% faster than 4 where a step waits for a rebuild or
+// the tile's longest wave; without rebuilds the same, 459 tiles 7.2 us a vertex-vertex step with either), 4
+// beyond (590 tiles 7.1 us against 11.1 with 8; vertex-segment 8.1 against 12.3).
 static inline int loop_waves(const dpm_set_s* S) { return S->splitSet ? S->split : (S->V.ntiles <= 512 ? 8 : 4); }
 
 // the step kernel of MODE bits `mode` on every tile of the set
