@@ -776,9 +776,9 @@ __global__ __launch_bounds__(WAVE* FS_WAVES) void k_fire_move(View V, Params P, 
   __shared__ double red[FS_WAVES][5];
   const int s = blockIdx.x / per, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE, lane = threadIdx.x & (WAVE - 1);
   const int t0 = V.stile[s], t1 = V.stile[s + 1], tile = t0 + (blockIdx.x % per) * nw + w;
+  FireState fs = fin[s];  // (before the store below, which would take it from the scalar cache)
   // what the launch before, look `tell`, found, for the host (pinned memory)
   if (tell && blockIdx.x == 0 && threadIdx.x == 0) *(volatile int*)told = 2 * tell + (*open == tell);
-  FireState fs = fin[s];
   FireSums sum{0, -1, 0, 0, 0};
   bool reset = false;
   if (!fs.converged) {
