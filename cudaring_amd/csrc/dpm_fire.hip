@@ -26,9 +26,10 @@ namespace dpm {
 // |v|^2 + 2 h P + h^2 |F|^2 took 512 packings of 16 to 256 rings through 2 x 60 iterations in 10.0 ms,
 // this takes 15.3 (whole rows from memory, four barriers: 19.1), but there single packings of a set left
 // the path: forces off by up to 9e-4 after a second compression.
-// MAXW 8: up to eight waves a lane may hold 256 registers, and nothing spills (200 to 214 in use); 16 waves
-// have 128, of which 63 to 114 spill.  512 packings of 16 to 256 rings, 200 iterations: 8 waves 63.4 -> 51.0 ms
-// and 4 waves 93.1 -> 79.3 against the 16-wave build (12 waves take 54.0, 16 take 48.0).
+// MAXW: a lane may hold 256 registers with up to 8 waves (200 to 214 in use, nothing spills), 168 with up to
+// 12 (23 to 49 spill), 128 with 16 (63 to 114).  Against the 16-wave build alone: 512 packings of 16 to 256
+// rings, 200 iterations, 4 waves 93.1 -> 79.2 ms, 8 waves 63.4 -> 51.0, 12 waves 54.1 -> 45.1 (16 waves take
+// 47.7); 512 packings of 16 to 24 rings (5 to 9 tiles), 8 waves 8.4 -> 7.5, 9 waves 10.2 -> 7.8.
 // Without near lists (rows of more than 64 entries, systems of more vertices than LDS holds, the
 // all-pairs interaction) it gathers over whole rows from memory.
 
@@ -214,8 +215,9 @@ static hipError_t fire_waves_launch(dpm_set_s* S, int chunk, int threads) {
 
 template <>
 hipError_t fire_launch<FIRE_INTER, FIRE_POT>(dpm_set_s* S, int chunk, int threads) {
-  return threads <= WAVE * FS_WAVES_FEW ? fire_waves_launch<FS_WAVES_FEW>(S, chunk, threads)
-                                        : fire_waves_launch<FS_WAVES>(S, chunk, threads);
+  if (threads <= WAVE * FS_WAVES_FEW) return fire_waves_launch<FS_WAVES_FEW>(S, chunk, threads);
+  if (threads <= WAVE * FS_WAVES_SOME) return fire_waves_launch<FS_WAVES_SOME>(S, chunk, threads);
+  return fire_waves_launch<FS_WAVES>(S, chunk, threads);
 }
 
 }  // namespace dpm

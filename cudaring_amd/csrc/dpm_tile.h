@@ -17,8 +17,9 @@ namespace dpm {
 // most waves per workgroup of the persistent FIRE kernel, and the LDS its near lists and positions may
 // take (of 160 KB, beside its static arrays)
 #define FS_WAVES 16
-// up to this many waves, the persistent FIRE kernel's build that holds 256 registers a lane
+// up to as many waves, the persistent FIRE kernel's builds that hold 256 and 168 registers a lane
 #define FS_WAVES_FEW 8
+#define FS_WAVES_SOME 12
 constexpr unsigned kFireLds = 156 * 1024;
 
 __device__ __forceinline__ double shfl_d(double v, int src) { return __shfl(v, src, WAVE); }

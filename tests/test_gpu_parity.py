@@ -265,7 +265,7 @@ def test_cfg1_nve_full_length(oracle_mod):
     assert np.all(np.isfinite(g.get("pos")))
 
 
-@pytest.mark.parametrize("waves", [0, 16])
+@pytest.mark.parametrize("waves", [0, 12, 16])
 @pytest.mark.parametrize("pot,inter", [("harmonic", "vertexVertex"), ("wca", "vertexSmooth")])
 def test_persistent_fire_matches_step_kernels(pot, inter, waves):
     """fire_minimize on one workgroup per system (tol 0, 30 iterations) against 30 iterations of
@@ -287,7 +287,7 @@ def test_persistent_fire_matches_step_kernels(pot, inter, waves):
         g.init_fire([0.2, 0.5, 1.1, 0.99, dt, 10 * dt, 0.2], 20, 0)
         sets.append(g)
     a, b = sets
-    a.set_fire_kernel(True, waves)  # 0: one wave per tile of the larger system (512-lane build); 16: the 1024-lane build
+    a.set_fire_kernel(True, waves)  # 0: one wave per tile of the larger system (512-lane build); 12, 16: the 768- and 1024-lane builds
     it = a.fire_minimize(0.0, 30)
     b.fire(30)
     assert list(it) == [30, 30]
