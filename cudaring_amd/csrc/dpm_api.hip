@@ -790,7 +790,7 @@ int fire_tile_sequence(dpm_set_s* S, long iterations) {
 // 0.010 a tile of the set; or 5 and 0.85 a tile of the largest system on its one CU, or the same summed
 // over the systems and shared by 256 CUs where that is more.  Measured (tiles of the set, harmonic
 // vertex-vertex and WCA vertex-segment; persistent against tiles): one system of 8 tiles 8.5, 12.4 against
-// 13.4, 14.2; of 10 12.7, 18.2 against 14.7, 15.5; of 13 15.7, 19.5 against 15.8, 16.6; of 66 47, 65 against
+// 13.4, 14.2; of 10 10.7, 16.8 against 14.7, 15.5; of 13 15.7, 19.4 against 15.8, 16.6; of 66 47, 65 against
 // 19, 20; 64 systems of up to 21 (827) 22, 28 against 20, 20; 128 of up to 42 (2,995) 43, 53 against 42, 42;
 // 300 of up to 21 (3,875) 36, 43 against 50, 51; 512 of up to 85 (22,714) 120, 141 against 229, 246.  Where
 // every few iterations rebuild, the tiles gain more (827 tiles: 47 against 29).  Both give the same bits.
