@@ -160,19 +160,40 @@ __device__ __forceinline__ void ring_walk(const Lane& L, const Box& B, double x,
   uy = L.act ? seg_scan(L.act ? dny : 0.0, L.lane, L.segS) - dny : 0.0;
 }
 
+// seg_scan of a pair as a loop: the walk's rare path, small rather than fast (a step's time is the
+// length of its instruction stream, also of what it jumps over)
+__device__ __forceinline__ void seg_scan_pair(double& a, double& b, int lane, int segS) {
+#pragma unroll 1
+  for (int d = 1; d < WAVE; d <<= 1) {
+    const double s = __shfl_up(a, d, WAVE), t = __shfl_up(b, d, WAVE);
+    if (lane - d >= segS) {
+      a += s;
+      b += t;
+    }
+  }
+}
+
 // ring_walk for ring_shape_n.  True when a ring of the wave reaches past half the box from its centre
 // (cx, cy), set only then: there the reference's centre-relative positions, a minimum image each
 // (getRelativeVertexPos 273-279), differ by a box length more than the segments.  Rings within a quarter
-// of the box of their first vertex, the usual case, are told by that.
+// of the box of the middle between their first vertex and the opposite one, the usual case down to packings
+// of ten rings, are told by that: their centre lies there too, and the walk is the minimum image itself.
 __device__ __forceinline__ bool ring_walk_past_half(const Lane& L, const Box& B, double x, double y, double dnx,
                                                     double dny, double& ux, double& uy, double& cx, double& cy) {
   const double xf = shfl_d(x, L.segS), yf = shfl_d(y, L.segS);
   ux = L.act ? pbx(x - xf, B) : 0.0;
   uy = L.act ? pby(y - yf, B) : 0.0;
-  if (__all(fabs(ux * B.mx) < 0.25 && fabs(uy * B.my) < 0.25)) return false;
-  ring_walk(L, B, x, y, xf, yf, dnx, dny, ux, uy);
-  const double ind = quot(1.0, (double)L.n);
-  const double mx = seg_sum(ux, L.lane, L.segS, L.segE) * ind, my = seg_sum(uy, L.lane, L.segS, L.segE) * ind;
+  const int opposite = (L.segS + (L.n >> 1)) & (WAVE - 1);
+  const double hx = 0.5 * shfl_d(ux, opposite), hy = 0.5 * shfl_d(uy, opposite);
+  if (__all(!L.act || (fabs((ux - hx) * B.mx) < 0.25 && fabs((uy - hy) * B.my) < 0.25))) return false;
+  double ax = L.act ? dnx : 0.0, ay = L.act ? dny : 0.0;  // the walk, one segment at a time
+  seg_scan_pair(ax, ay, L.lane, L.segS);
+  ux = L.act ? ax - dnx : 0.0;
+  uy = L.act ? ay - dny : 0.0;
+  ax = ux;
+  ay = uy;
+  seg_scan_pair(ax, ay, L.lane, L.segS);
+  const double ind = quot(1.0, (double)L.n), mx = shfl_d(ax, L.segE) * ind, my = shfl_d(ay, L.segE) * ind;
   cx = xf + mx;
   cy = yf + my;
   return __any(L.act && !(fabs((ux - mx) * B.mx) < 0.4999 && fabs((uy - my) * B.my) < 0.4999));

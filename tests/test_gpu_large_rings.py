@@ -23,9 +23,10 @@ def state(n, reach):
     return {"nvp": nvp, "box": np.array([L, 1.1 * L]), "pos": pos.ravel(), "rad": rad, "l0": l0, "theta0": th0, "a0": a0}
 
 
-# radius in box lengths: 0.2 (past a quarter of the box from the first vertex, within half from the
-# centre), 0.47 and 0.53 (about the line), 0.6; 40 vertices in one tile, 90 in two slices
-@pytest.mark.parametrize("reach", [0.2, 0.47, 0.53, 0.6])
+# radius in box lengths: 0.2 (past a quarter of the box from the first vertex, within one from the middle),
+# 0.3 (past that, within half from the centre), 0.47 and 0.53 (about the line), 0.6; 40 vertices in one
+# tile, 90 in two slices
+@pytest.mark.parametrize("reach", [0.2, 0.3, 0.47, 0.53, 0.6])
 @pytest.mark.parametrize("n", [40, 90])
 @pytest.mark.parametrize("inter", ["vertexVertex", "vertexSmooth"])
 def test_loops_give_the_force_call(oracle_mod, n, reach, inter):
