@@ -184,8 +184,8 @@ __device__ __forceinline__ bool ring_walk_past_half(const Lane& L, const Box& B,
   ux = L.act ? pbx(x - xf, B) : 0.0;
   uy = L.act ? pby(y - yf, B) : 0.0;
   const int opposite = (L.segS + (L.n >> 1)) & (WAVE - 1);
-  const double hx = 0.5 * shfl_d(ux, opposite), hy = 0.5 * shfl_d(uy, opposite);
-  if (__all(!L.act || (fabs((ux - hx) * B.mx) < 0.25 && fabs((uy - hy) * B.my) < 0.25))) return false;
+  const double hx = __builtin_fma(-0.5, shfl_d(ux, opposite), ux), hy = __builtin_fma(-0.5, shfl_d(uy, opposite), uy);
+  if (__all(!L.act || (fabs(hx) < 0.25 * B.Lx && fabs(hy) < 0.25 * B.Ly))) return false;
   double ax = L.act ? dnx : 0.0, ay = L.act ? dny : 0.0;  // the walk, one segment at a time
   seg_scan_pair(ax, ay, L.lane, L.segS);
   ux = L.act ? ax - dnx : 0.0;
